@@ -232,8 +232,12 @@ class ModelRunner:
             + [p.shape[0] for p in self.params.values() if p.dim() == 2 and p.shape[0] != self.spec.vocab_size]
         )
         parts = list(self.model.all_parts())
+        wide = [tuple(p.shape) for p in self.params.values() if p.dim() == 2 and p.dtype == torch.float32]
         total = 0
         for rows in sizes:
+            # a float32 product's partial results, given back behind it
+            scratch = max((ops.f32_scratch_bytes(rows, *shape) for shape in wide), default=0)
+            total += len(bounds) * scratch
             for bound in bounds:
                 kept = max((p.recorded_step_bytes(rows, bound, e.page_size) for p in parts), default=0)
                 total += rows * 4 * (self.spec.vocab_size + 8 * widest) + 2 * kept

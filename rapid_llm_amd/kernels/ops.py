@@ -8,6 +8,7 @@ GPU or without the compiled library these raise.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional
 
@@ -978,8 +979,54 @@ def head_product(
     )
 
 
+# The float32 product's tiles (rows of A a workgroup takes): rows of W, and microseconds a chunk of 32 k
+# takes with one, two, .. workgroups on every compute unit, as many as a unit holds (measured over the
+# family's matrices at 17 to 2,048 rows; the estimate built from them is within 10% of what was measured,
+# save below 20 us, where a launch's start counts as much).
+_F32_TILES = {32: (64, (0.57, 0.66, 0.77, 0.90)), 64: (64, (0.68, 0.95, 1.29)), 128: (128, (1.68, 2.45))}
+_F32_SHARED = 4.0  # microseconds of the kernel that adds the runs, beside the runs' bytes
+_F32_RUN_BYTES = 8e6  # bytes a microsecond at which the runs' results are written and read again
+_F32_READ_BYTES = 5.5e6  # and at which weights arrive
+_F32_MOST_SCRATCH = 1 << 27  # bytes of partial results a product may take
+
+
+@functools.lru_cache(maxsize=4096)
+def f32_plan(m: int, n: int, k: int, units: int) -> tuple[int, int]:
+    """(tile, workgroups that share a tile's runs of K) of the float32 product.  Up to 16 rows the kernel that
+    streams the weights: one tile of 16 weight rows a workgroup, or two (tile 1 or 2) where that makes one
+    round of what would be a round and a half (6,144 weight rows on 256 units, 8 rows: 25.2 against 26.3 us;
+    a single row, whose time is the first loads': 23.3 against 22.1), and, from 13 rows on, where the rows read
+    again by every workgroup weigh as much as its weights (24,576 x 4,096, 16 rows: 92 against 98 us; 8 rows:
+    87 against 76).  More rows: the tile and the sharing for which the estimate is lowest; sharing fills
+    the chip where the tiles do not, and writes and reads eight partial results for it."""
+    if m <= 16:
+        tiles = -(-n // 16)
+        return (2 if (units < tiles <= 2 * units and m > 4) or (tiles > 2 * units and m > 12) else 1), 1
+    best = None
+    for tile in (32,) if m <= 32 else (64,) if m <= 64 else (64, 128):
+        width, costs = _F32_TILES[tile]
+        count = -(-m // tile) * -(-n // width)
+        for groups in (1, 2, 4, 8):
+            rounds, rest = divmod(count * groups, len(costs) * units)
+            chunk = rounds * costs[-1] + (costs[-(-rest // units) - 1] if rest else 0.0)
+            # never below what the weights' bytes take
+            time = max(chunk * -(-k // (32 * groups)), 4.0 * n * k / _F32_READ_BYTES)
+            if groups > 1:
+                if 32 * m * n > _F32_MOST_SCRATCH or m > 65535:  # the adding kernel's grid has a row of blocks a row
+                    break
+                time += _F32_SHARED + 64.0 * m * n / _F32_RUN_BYTES
+            if best is None or time < best[0]:
+                best = (time, tile, groups)
+    return best[1], best[2]
+
+
+def f32_scratch_bytes(m: int, n: int, k: int) -> int:
+    """What a float32 product of ``m`` rows over ``[n, k]`` weights takes for its runs' results."""
+    return 32 * m * n if f32_plan(m, n, k, chip().units)[1] > 1 else 0
+
+
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
-    """``out[M,N] = a[M,K] @ w[N,K]^T`` in true float32.  Rows may be strided (views of wider
+    """``out[M,N] = a[M,K] @ w[N,K]^T`` in float32.  Rows may be strided (views of wider
     matrices); the inner dimension must be contiguous."""
     for t, name in ((a, "a"), (w, "w"), (out, "out")):
         if not t.is_cuda or t.dtype != torch.float32 or t.dim() != 2 or t.stride(1) != 1:
@@ -988,8 +1035,12 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
     n, k2 = w.shape
     if k != k2 or out.shape != (m, n):
         raise KernelError(f"gemm_f32 shapes do not agree: a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)}")
+    tile, groups = f32_plan(m, n, k, chip().units)
+    parts = torch.empty((8, m, n), dtype=torch.float32, device=a.device) if groups > 1 else None
     _ok(
-        core().rl_gemm_f32(_p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(0), _stream()),
+        core().rl_gemm_f32(
+            _p(a), _p(w), _p(out), _p(parts), m, n, k, a.stride(0), w.stride(0), out.stride(0), tile, groups, _stream()
+        ),
         "rl_gemm_f32",
     )
 

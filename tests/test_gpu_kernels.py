@@ -638,6 +638,57 @@ def test_gemm_f32_keeps_what_bfloat16_would_lose():
     assert out.item() == k + 2.0 ** -12
 
 
+@pytest.mark.parametrize("shape", [(1, 16, 32), (16, 33, 1000), (17, 64, 32), (32, 70, 290), (33, 130, 1056),
+                                   (65, 127, 96), (129, 260, 4128), (257, 513, 72), (300, 1028, 8)])
+def test_gemm_f32_every_tile_and_sharing(shape):
+    """Every kernel of the float32 product (streamed weights, tiles of 32, 64 and 128 rows, their runs of K
+    shared or not) gives the same bits, within the rounding of the sums they are defined by."""
+    ops = _ops()
+    m, n, k = shape
+    gen = torch.Generator().manual_seed(m)
+    # magnitudes over ten powers of two, so that the operands' lower pieces count
+    a, w = (torch.randn(r, k, generator=gen) * torch.exp2(torch.randint(-5, 6, (r, k), generator=gen)) for r in (m, n))
+    want = a.double() @ w.double().T
+    # a chunk of 32 k is six additions, a run an eighth of the chunks, the runs are eight more; an
+    # addition rounds by at most half a unit in the last place of a partial sum (the instruction's own
+    # sum of 32 products is allowed as much again), and the three partial products left out are 2^-25
+    steps = 6 * -(--(-k // 32) // 8) + 8
+    bound = (a.double().abs() @ w.double().abs().T) * (2 * steps + 2) * 2.0**-24
+    ad, wd, first = a.to(DEV), w.to(DEV), None
+    plans = [(1, 1), (2, 1)] if m <= 16 else []
+    plans += [(tile, groups) for tile in (32, 64, 128) for groups in (1, 2, 4, 8)]
+    for tile, groups in plans:
+        out = torch.full((m, n + 1), float("nan"), device=DEV)
+        parts = torch.empty((8, m, n), device=DEV)
+        code = ops.core().rl_gemm_f32(ops._p(ad), ops._p(wd), ops._p(out), ops._p(parts), m, n, k, k, k, n + 1, tile,
+                                      groups, ops._stream())
+        assert code == 0
+        assert bool(out[:, n].isnan().all())
+        first = out[:, :n] if first is None else first
+        assert torch.equal(out[:, :n], first), (tile, groups)
+    assert bool(((first.cpu().double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m", [3, 40, 200])
+def test_gemm_f32_of_infinite_and_largest_operands(m):
+    """Operands that three bfloat16 numbers cannot stand for give what the float32 sum gives: an infinity
+    times a number, an infinity times zero, and numbers that bfloat16 would round to infinity."""
+    ops = _ops()
+    n, k = 70, 96
+    gen = torch.Generator().manual_seed(m)
+    a, w = torch.randn(m, k, generator=gen), torch.randn(n, k, generator=gen)
+    a[0, 5], w[3, 5], w[4, 5] = float("inf"), 1.0, 0.0
+    a[1, 7] = 3.4e38
+    w[:, 7] *= 2.0**-20
+    w[9, 11] = -float("inf")
+    a[2, 60] = float("nan")
+    out = torch.empty(m, n, device=DEV)
+    ops.gemm_f32(a.to(DEV), w.to(DEV), out)
+    want = (a.double() @ w.double().T).float()
+    torch.testing.assert_close(out.cpu(), want, rtol=1e-5, atol=1e-4, equal_nan=True)
+    assert out[0, 3].item() == float("inf") and bool(out[0, 4].isnan()) and bool(out[2].isnan().all())
+
+
 @pytest.mark.parametrize("shape", [(1, 503, 96), (8, 4096, 4096), (16, 300, 1000), (64, 1000, 12288), (17, 6144, 4096), (200, 331, 80), (3, 24, 48),
                                    (8, 6144, 4096), (1, 5000, 256), (16, 4618, 1160), (11, 6120, 96)])  # the last four: workgroups of 24 weight rows
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32], ids=["bf16out", "f32out"])
