@@ -13,9 +13,13 @@
 //
 // A row's result does not depend on the tile it falls in, on the other rows there, or on how
 // a prompt was cut into steps: keys are taken in tiles of 16 at absolute positions 0, 16, ..,
-// each wave takes its tiles in ascending order; within a tile the order of every sum is fixed
-// by the key's position; a tile that holds no visible key of a row leaves that row's state as
-// it is, exactly (factor 1, terms 0), and so does a wave without visible keys in the fold.  Masked keys contribute exactly zero
+// in spans of SPAN keys at absolute positions.  Within a span each wave takes its tiles in ascending
+// order, beginning with an empty state; a wave's states of the spans are folded in their order, and then
+// the waves'.  Within a tile the order of every sum is fixed by the key's position; a tile that holds
+// no visible key of a row leaves that row's state as it is, exactly (factor 1, terms 0), and so does
+// a span or a wave without visible keys in the fold.  A launch of few tiles (decoding) may therefore
+// give every span to a workgroup of its own, which leaves its waves' states to a second kernel that
+// folds them in the same order: the same bits.  Masked keys contribute exactly zero
 // (rapid_llm/kernels/ops/attention/flashdecoding.py:223-237); scores are (q . k) / sqrt(d)
 // (rapid_llm/modules/attention.py:62), softmax over keys in float32
 // (rapid_llm/kernels/ops/attention/flashattention2_nopad.py:138-168).
@@ -30,6 +34,12 @@ namespace f32attn {
 constexpr int D = RL_HEAD_DIM;
 constexpr int DB = D / 16;  // 16-channel chunks of the first product = blocks of the output
 constexpr int AW = 4;       // waves per workgroup: key tile i belongs to wave i % AW
+// Keys a span: 256 workgroups for eight requests of 2,048 keys and eight kv heads; eight tiles a wave
+// between two folds.  Eight requests of 512 to 1,536 keys of the 8B shape: 64 workgroups that walked
+// whole contexts took 65 us a layer, the latency of their chain of tiles, the step 8.95 ms; spans in
+// workgroups of their own leave it at 7.80 ms.
+constexpr int SPAN = 512;
+constexpr int STATE = D + 2;  // floats a (row, wave, span) state takes in memory: sums, maximum, sum of weights
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ inline f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
@@ -44,11 +54,29 @@ __device__ inline float row_sum(float v) {
     return v + __shfl_xor(v, 32, RL_WAVE);
 }
 
+// (m, l, acc) folded with the state of later keys, (m2, l2, acc2); written out so that every kernel
+// rounds alike.  `none`: neither has seen a key.
+struct Fold {
+    float m, fa, fb;
+    bool none;
+};
+__device__ inline Fold fold_of(float m, float m2) {
+    Fold f;
+    f.m = fmaxf(m, m2);
+    f.none = f.m == -INFINITY;
+    f.fa = f.none ? 1.f : expf(m - f.m);
+    f.fb = f.none ? 0.f : expf(m2 - f.m);
+    return f;
+}
+__device__ inline float fold_sum(float x, float x2, const Fold& f) { return fmaf(x2, f.fb, x * f.fa); }
+
 // tile_info: [tiles][3] = index of the request's first token in the step, its tokens in the
 // step, first row of the tile.  The request's first position is read from `positions`.
+// SPLIT: blockIdx.z is the span; states[tile][kv head][span][wave][row][STATE] take the place of `out`.
+template <bool SPLIT>
 __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache,
-    const float* __restrict__ v_cache, float* __restrict__ out,
+    const float* __restrict__ v_cache, float* __restrict__ out, float* __restrict__ states,
     const int* __restrict__ tile_info, const int* __restrict__ positions,
     const int* __restrict__ token_slot, const int* __restrict__ block_table, int table_stride,
     int page_size, int nq, int nkv, int window, float scale) {
@@ -81,6 +109,10 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
     const int first_key = (window > 0 && first_pos - window + 1 > 0) ? first_pos - window + 1 : 0;
     const int lo = first_key & ~15;
     const int hi = last_pos + 1;  // keys below hi are in the cache
+    // the keys this workgroup walks
+    const int from = SPLIT ? max(lo, (int)blockIdx.z * SPAN) : lo;
+    const int upto = SPLIT ? min(hi, ((int)blockIdx.z + 1) * SPAN) : hi;
+    if (SPLIT && from >= upto) return;  // the fold knows which spans there are
 
     // Q^T: lane (row r16, g) holds channels 16c + 4g .. + 3 of its row
     f32x4 qf[DB];
@@ -97,26 +129,25 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
 
     // operands of one tile of 16 keys: lane (key r16, g) reads channels 16c + 4g .. + 3 of its
     // key; lane (channel r16, g) reads keys kb + 4g .. + 3 of its channel in every block
-    struct Frags {
-        f32x4 k[DB], v[DB];
-    };
-    auto load = [&](int kb, Frags& f) {
+    auto load_keys = [&](int kb, f32x4 (&f)[DB]) {
         const int key = min(kb + r16, hi - 1);  // beyond the cache: any real key, masked below
         const float* krow =
             k_cache + (((size_t)table[key / page_size] * nkv + hk) * page_size + key % page_size) * D + 4 * g;
 #pragma unroll
-        for (int c = 0; c < DB; ++c) f.k[c] = ld4(krow + 16 * c);
+        for (int c = 0; c < DB; ++c) f[c] = ld4(krow + 16 * c);
+    };
+    auto load_values = [&](int kb, f32x4 (&f)[DB]) {
         const int key4 = min(kb + 4 * g, (hi - 1) & ~3);
         const float* vrow = v_cache +
                             (((size_t)table[key4 / page_size] * nkv + hk) * D + r16) * page_size +
                             key4 % page_size;
 #pragma unroll
-        for (int b = 0; b < DB; ++b) f.v[b] = ld4(vrow + (size_t)16 * b * page_size);
+        for (int b = 0; b < DB; ++b) f[b] = ld4(vrow + (size_t)16 * b * page_size);
     };
 
     // S^T = K Q^T of one tile, the chunks dealt to four accumulators that are added at the
     // end (one chain of dependent instructions would leave the matrix core idle)
-    auto scores = [&](const Frags& f) -> f32x4 {
+    auto scores = [&](const f32x4 (&f)[DB]) -> f32x4 {
         f32x4 part[4];
 #pragma unroll
         for (int a4 = 0; a4 < 4; ++a4) part[a4] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -125,7 +156,7 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 part[c & 3] =
-                    __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[c][j], qf[c][j], part[c & 3], 0, 0, 0);
+                    __builtin_amdgcn_mfma_f32_16x16x4f32(f[c][j], qf[c][j], part[c & 3], 0, 0, 0);
         return (part[0] + part[1]) + (part[2] + part[3]);
     };
 
@@ -149,7 +180,7 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) p[i] = expf(s[i] - m_new);  // masked: exactly 0
         }
-        l = l * alpha + row_sum((p[0] + p[1]) + (p[2] + p[3]));
+        l = fmaf(l, alpha, row_sum((p[0] + p[1]) + (p[2] + p[3])));
         m = m_new;
         // ---- O^T = O^T alpha + V^T P^T --------------------------------------------------------
 #pragma unroll
@@ -170,29 +201,48 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
         }
     };
 
+    // a span is over: its state joins the wave's (a launch that walks whole contexts)
+    float m_all = -INFINITY, l_all = 0.f;
+    f32x4 acc_all[DB];
+    if (!SPLIT) {
+#pragma unroll
+        for (int b = 0; b < DB; ++b) acc_all[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    auto finish_span = [&]() {
+        const Fold f = fold_of(m_all, m);
+        l_all = fold_sum(l_all, l, f);
+        m_all = f.m;
+        m = -INFINITY;
+        l = 0.f;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc_all[b][i] = fold_sum(acc_all[b][i], acc[b][i], f);
+            acc[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
+    };
+
     // Software pipeline over the wave's tiles: while a tile goes through softmax and the second
-    // product, the scores of the next have been multiplied and the operands of the one after
-    // are in flight.  The last two tiles stand outside the loop, so that inside it the loads
-    // are issued without a condition and stay where they are written (behind a condition the
+    // product, the scores of the next have been multiplied, and that tile's values and the keys of
+    // the one after are in flight (values travel a tile later than their keys: 32 registers fewer at 128
+    // channels, which keeps two waves a SIMD).  The last two tiles stand outside the loop, so that inside
+    // it the loads are issued without a condition and stay where they are written (behind a condition the
     // compiler counts a load as absent and makes every older operand wait for it; left to
     // itself the scheduler moves loads down to their use).
     constexpr int STEP = 16 * AW;
-    const int mine = lo + 16 * ((wave - lo / 16) & (AW - 1));  // first tile >= lo with index % AW == wave
-    if (mine < hi) {
-        int left = (hi - mine + STEP - 1) / STEP;  // tiles of this wave, the current one included
+    const int mine = from + 16 * ((wave - from / 16) & (AW - 1));  // first tile >= from with index % AW == wave
+    if (mine < upto) {
+        int left = (upto - mine + STEP - 1) / STEP;  // tiles of this wave, the current one included
         int kb = mine;
-        Frags nxt;
-        f32x4 vcur[DB], vnext[DB];
-        load(kb, nxt);
-        f32x4 sc = scores(nxt);
-#pragma unroll
-        for (int b = 0; b < DB; ++b) vcur[b] = nxt.v[b];
-        if (left > 1) load(kb + STEP, nxt);
+        f32x4 keys[DB], vcur[DB], vnext[DB];
+        load_keys(kb, keys);
+        load_values(kb, vcur);
+        f32x4 sc = scores(keys);
+        if (left > 1) load_keys(kb + STEP, keys);
         while (left > 2) {
-            const f32x4 s_next = scores(nxt);
-#pragma unroll
-            for (int b = 0; b < DB; ++b) vnext[b] = nxt.v[b];
-            load(kb + 2 * STEP, nxt);
+            const f32x4 s_next = scores(keys);
+            load_values(kb + STEP, vnext);
+            load_keys(kb + 2 * STEP, keys);
             __builtin_amdgcn_sched_barrier(0);
             finish_tile(kb, sc, vcur);
             sc = s_next;
@@ -200,63 +250,139 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
             for (int b = 0; b < DB; ++b) vcur[b] = vnext[b];
             kb += STEP;
             --left;
+            if (!SPLIT && kb % SPAN < STEP) finish_span();
         }
         if (left == 2) {
-            const f32x4 s_next = scores(nxt);
+            const f32x4 s_next = scores(keys);
+            load_values(kb + STEP, vnext);
             finish_tile(kb, sc, vcur);
-            finish_tile(kb + STEP, s_next, nxt.v);
+            if (!SPLIT && (kb + STEP) % SPAN < STEP) finish_span();
+            finish_tile(kb + STEP, s_next, vnext);
         } else {
             finish_tile(kb, sc, vcur);
         }
     }
-    // ---- fold the waves' states in their order (a wave without visible keys has m = -inf,
-    // l = 0 and zero sums: it changes nothing, exactly) ----------------------------------------
-    if (wave > 0) {
-        fold_ml[wave - 1][0][lane] = m;
-        fold_ml[wave - 1][1][lane] = l;
+    if (SPLIT) {
+        float* to = states + ((((size_t)tile * nkv + hk) * gridDim.z + blockIdx.z) * AW + wave) * 16 * STATE + r16 * STATE;
 #pragma unroll
         for (int b = 0; b < DB; ++b)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) fold_acc[wave - 1][4 * b + i][lane] = acc[b][i];
+            for (int i = 0; i < 4; ++i) to[16 * b + 4 * g + i] = acc[b][i];
+        if (g == 0) {
+            to[D] = m;
+            to[D + 1] = l;
+        }
+        return;
+    }
+    finish_span();
+    // ---- fold the waves' states in their order (a wave without visible keys has m = -inf,
+    // l = 0 and zero sums: it changes nothing, exactly) ----------------------------------------
+    if (wave > 0) {
+        fold_ml[wave - 1][0][lane] = m_all;
+        fold_ml[wave - 1][1][lane] = l_all;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) fold_acc[wave - 1][4 * b + i][lane] = acc_all[b][i];
     }
     __syncthreads();
     if (wave > 0) return;
 #pragma unroll
     for (int w = 0; w < AW - 1; ++w) {
-        const float m_w = fold_ml[w][0][lane], l_w = fold_ml[w][1][lane];
-        const float m_new = fmaxf(m, m_w);
-        if (m_new == -INFINITY) continue;
-        const float fa = expf(m - m_new), fb = expf(m_w - m_new);
-        l = l * fa + l_w * fb;
+        const Fold f = fold_of(m_all, fold_ml[w][0][lane]);
+        l_all = fold_sum(l_all, fold_ml[w][1][lane], f);
+        m_all = f.m;
 #pragma unroll
         for (int b = 0; b < DB; ++b)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[b][i] = acc[b][i] * fa + fold_acc[w][4 * b + i][lane] * fb;
-        m = m_new;
+            for (int i = 0; i < 4; ++i) acc_all[b][i] = fold_sum(acc_all[b][i], fold_acc[w][4 * b + i][lane], f);
     }
     if (!row_ok) return;
-    // acc[b][i] is channel 16b + 4g + i of the lane's row
+    // acc_all[b][i] is channel 16b + 4g + i of the lane's row
     float* orow = out + ((size_t)(at + tok) * nq + head) * D + 4 * g;
-    const float inv = 1.f / l;
+    const float inv = 1.f / l_all;
 #pragma unroll
     for (int b = 0; b < DB; ++b)
-        *reinterpret_cast<f32x4*>(orow + 16 * b) =
-            (f32x4){acc[b][0] * inv, acc[b][1] * inv, acc[b][2] * inv, acc[b][3] * inv};
+        *reinterpret_cast<f32x4*>(orow + 16 * b) = (f32x4){acc_all[b][0] * inv, acc_all[b][1] * inv,
+                                                           acc_all[b][2] * inv, acc_all[b][3] * inv};
+}
+
+// The states of a split launch folded as the other launch folds them: a workgroup per (tile, kv head),
+// 16 lanes a row, D / 16 channels a lane.  Bound by its start: the states of the next span are asked for
+// together with this one's.
+__global__ __launch_bounds__(256) void attn_f32_fold_kernel(const float* __restrict__ states, float* __restrict__ out,
+                                                            const int* __restrict__ tile_info,
+                                                            const int* __restrict__ positions, int spans, int nq,
+                                                            int nkv, int window) {
+    const int tile = blockIdx.x, hk = blockIdx.y;
+    const int G = nq / nkv;
+    const int at = tile_info[3 * tile], n = tile_info[3 * tile + 1], row0 = tile_info[3 * tile + 2];
+    const int rows = n * G;
+    const int r16 = threadIdx.x >> 4, part = threadIdx.x & 15;
+    const int row = row0 + r16;
+    if (row >= rows) return;
+    const int start = positions[at];
+    const int first_pos = start + row0 / G;
+    const int last_pos = start + (min(rows, row0 + 16) - 1) / G;
+    const int first_key = (window > 0 && first_pos - window + 1 > 0) ? first_pos - window + 1 : 0;
+    const int s_lo = first_key / SPAN, s_hi = min(last_pos / SPAN + 1, spans);  // the spans that were walked
+
+    float m_out = -INFINITY, l_out = 0.f, acc_out[DB];
+#pragma unroll
+    for (int b = 0; b < DB; ++b) acc_out[b] = 0.f;
+    for (int w = 0; w < AW; ++w) {
+        float m = -INFINITY, l = 0.f, acc[DB];
+#pragma unroll
+        for (int b = 0; b < DB; ++b) acc[b] = 0.f;
+#pragma unroll 2
+        for (int s = s_lo; s < s_hi; ++s) {
+            const float* from = states + ((((size_t)tile * nkv + hk) * spans + s) * AW + w) * 16 * STATE + r16 * STATE;
+            const Fold f = fold_of(m, from[D]);
+            l = fold_sum(l, from[D + 1], f);
+            m = f.m;
+#pragma unroll
+            for (int b = 0; b < DB; ++b) acc[b] = fold_sum(acc[b], from[16 * b + part], f);
+        }
+        const Fold f = fold_of(m_out, m);
+        l_out = fold_sum(l_out, l, f);
+        m_out = f.m;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) acc_out[b] = fold_sum(acc_out[b], acc[b], f);
+    }
+    float* orow = out + ((size_t)(at + row / G) * nq + hk * G + row % G) * D;
+    const float inv = 1.f / l_out;
+#pragma unroll
+    for (int b = 0; b < DB; ++b) orow[16 * b + part] = acc_out[b] * inv;
 }
 
 }  // namespace f32attn
 
 // Every token of the step, single tokens and portions alike.  page_size must be a multiple
-// of 4 (the four keys of a lane lie in one page).
-extern "C" int rl_attn_f32(const float* q, const float* k_cache, const float* v_cache, float* out,
+// of 4 (the four keys of a lane lie in one page).  `spans` > 0 gives every span of keys to workgroups of
+// its own, with `states` [tiles, nkv, spans, 4, 16, D + 2]; it must cover the longest context.
+extern "C" int rl_attn_f32(const float* q, const float* k_cache, const float* v_cache, float* out, float* states,
                            const int* tile_info, int num_tiles, const int* positions,
                            const int* token_slot, const int* block_table, int table_stride,
-                           int page_size, int nq, int nkv, int window, float scale,
+                           int page_size, int nq, int nkv, int window, float scale, int spans,
                            hipStream_t stream) {
+    using namespace f32attn;
     if (num_tiles <= 0) return RL_OK;
     if (nkv < 1 || nq % nkv || page_size < 4 || page_size % 4 || nkv > 65535) return RL_ERR_ARG;
-    hipLaunchKernelGGL(f32attn::attn_f32_kernel, dim3(num_tiles, nkv), dim3(f32attn::AW * RL_WAVE), 0, stream, q,
-                       k_cache, v_cache, out, tile_info, positions, token_slot, block_table,
-                       table_stride, page_size, nq, nkv, window, scale);
+    if (spans < 0 || spans > 65535 || (spans && !states)) return RL_ERR_ARG;
+    const dim3 block(AW * RL_WAVE);
+    if (!spans) {
+        hipLaunchKernelGGL(attn_f32_kernel<false>, dim3(num_tiles, nkv), block, 0, stream, q, k_cache, v_cache, out,
+                           states, tile_info, positions, token_slot, block_table, table_stride, page_size, nq, nkv,
+                           window, scale);
+        return rl_launch_status();
+    }
+    hipLaunchKernelGGL(attn_f32_kernel<true>, dim3(num_tiles, nkv, spans), block, 0, stream, q, k_cache, v_cache, out,
+                       states, tile_info, positions, token_slot, block_table, table_stride, page_size, nq, nkv, window,
+                       scale);
+    if (int code = rl_launch_status()) return code;
+    hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(num_tiles, nkv), dim3(256), 0, stream, states, out, tile_info,
+                       positions, spans, nq, nkv, window);
     return rl_launch_status();
 }
+
+extern "C" int rl_attn_f32_span() { return f32attn::SPAN; }

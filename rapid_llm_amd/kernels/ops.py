@@ -79,6 +79,8 @@ def attention_lib(head_dim: int) -> ctypes.CDLL:
         lib = build.load(build.attention_library(head_dim))
         if lib.rl_attn_head_dim() != head_dim:
             raise KernelError(f"attention library for head size {head_dim} reports {lib.rl_attn_head_dim()}")
+        if lib.rl_attn_f32_span() != _F32_SPAN:
+            raise KernelError(f"the float32 attention walks spans of {lib.rl_attn_f32_span()} keys, the launch rules expect {_F32_SPAN}")
         _attn[head_dim] = lib
     return lib
 
@@ -1752,6 +1754,27 @@ def _f32_tiles(ctx, group: int, tile_rows: int = 16, chunk: int = 0) -> tuple[to
     return made
 
 
+_F32_SPAN = 512  # keys of a span of the float32 attention
+_F32_SPLIT_BYTES = 1 << 28  # what a launch may take for the states of its spans
+
+
+def f32_spans(tiles: int, nkv: int, d: int, longest: int, window: int, units: int | None = None) -> int:
+    """Spans of keys that get workgroups of their own in a float32 launch of ``tiles`` tiles over contexts of up
+    to ``longest`` keys; 0: a workgroup walks a tile's whole context, which is the faster way where there is
+    one for every compute unit (no states are written and folded) and where a window spans too little."""
+    units = chip().units if units is None else units
+    spans = -(-longest // _F32_SPAN)
+    if spans < 2 or tiles * nkv >= units or 0 < window < 2 * _F32_SPAN:
+        return 0
+    return spans if tiles * nkv * spans * 64 * (d + 2) * 4 <= _F32_SPLIT_BYTES else 0
+
+
+def f32_states_bytes(rows: int, nq: int, nkv: int, d: int, longest: int, window: int) -> int:
+    """Bytes of a float32 launch's states for ``rows`` single tokens."""
+    tiles = rows * -(-(nq // nkv) // 16)
+    return tiles * nkv * f32_spans(tiles, nkv, d, longest, window) * 64 * (d + 2) * 4
+
+
 def attention_f32(
     q: torch.Tensor,
     k_cache: torch.Tensor,
@@ -1787,11 +1810,17 @@ def attention_f32(
     if nkv > 65535:
         raise KernelError(f"{nkv} kv heads exceed the launch grid")
     tiles, num_tiles = _f32_tiles(ctx, nq // nkv)
+    # under a graph the launch is laid out for the longest context of the graph's bucket
+    longest = _static(ctx).get("context_bound", ctx.max_position + 1)
+    spans = f32_spans(num_tiles, nkv, d, longest, window)
+    states = None
+    if spans:
+        states = torch.empty((num_tiles, nkv, spans, 4, 16, d + 2), dtype=torch.float32, device=q.device)
     _ok(
         attention_lib(d).rl_attn_f32(
-            _p(q), _p(k_cache), _p(v_cache), _p(out), _p(tiles), num_tiles, _p(ctx.positions),
+            _p(q), _p(k_cache), _p(v_cache), _p(out), _p(states), _p(tiles), num_tiles, _p(ctx.positions),
             _p(ctx.token_slot), _p(block_table), block_table.stride(0), page_size, nq, nkv, window,
-            ctypes.c_float(scale), _stream(),
+            ctypes.c_float(scale), spans, _stream(),
         ),
         "rl_attn_f32",
     )

@@ -310,6 +310,8 @@ class GQAAttention(PackedMixer):
             # the shares of a tile's keys that several workgroups leave for the merge kernel
             splits = ops.tile_splits(rows * self.nkv, context_bound, self.window, self.keep_first)
             return 0 if splits == 1 else rows * self.nq * splits * (self.dv + 2) * 4
+        if self.runtime.dtype == torch.float32:
+            return ops.f32_states_bytes(rows, self.nq, self.nkv, self.d, context_bound, self.window)
         return ops.decode_scratch_bytes(rows, self.nq, self.nkv, self.d, context_bound, page_size, self.window)
 
     # ---- step ------------------------------------------------------------------

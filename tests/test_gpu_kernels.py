@@ -175,6 +175,24 @@ def test_order_by_length_names_the_longest_first():
         assert rc == 0 and order.cpu().tolist() == want, (n, spread, "scattered")
 
 
+@pytest.mark.parametrize("window", [0, 1024, 1100], ids=lambda w: f"w{w}")
+@pytest.mark.parametrize("d,nq,nkv,page", [(128, 8, 2, 16), (48, 20, 1, 12)], ids=["d128", "d48"])
+def test_attention_f32_spans_in_workgroups_of_their_own(d, nq, nkv, page, window, monkeypatch):
+    """A float32 launch whose spans of keys go to workgroups of their own gives the bits of one that walks
+    whole contexts: contexts that end at a span's edge and one key on either side, a portion across one."""
+    ops = _ops()
+    seqs = [(510, 1), (511, 1), (512, 1), (0, 1), (1023, 1), (1024, 1), (2100, 1), (500, 30), (1530, 7)]
+    q, kc, vc, table, ctx, want = _paged_problem(seqs, nq, nkv, d, page, torch.float32, d + window, window)
+    outs = []
+    for spans in (0, 5, 8):  # 8: laid out for a longer context than there is
+        monkeypatch.setattr(ops, "f32_spans", lambda *args: spans)
+        out = torch.full_like(q, float("nan"))
+        ops.attention_f32(q, kc, vc, out, ctx, table, page, nq, nkv, d, window, 1.0 / math.sqrt(d))
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    torch.testing.assert_close(outs[0].cpu(), want, rtol=2e-5, atol=3e-6)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 def test_decode_attention_of_many_requests_of_mixed_lengths(dtype):
     """More workgroups than the chip holds at a time: the decode kernel then takes the requests
