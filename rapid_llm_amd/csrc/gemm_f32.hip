@@ -99,7 +99,8 @@ __device__ inline f32x4 load_k4(const float* p, int limit) {
 }
 
 // ---- up to 16 rows: the weights are streamed once -----------------------------------------------
-// One workgroup per NT tiles of 16 rows of W, one wave per run of K.  Bound by the weights' bytes.
+// One workgroup per NT tiles of 16 rows of W, one wave per run of K.  Bound by the weights' bytes, and from a
+// few rows on by the rows of A beside them, which every workgroup reads whole (f32_plan says when NT is 2 or 3).
 template <int NT, bool VEC>
 __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_stream_kernel(
     const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
@@ -126,8 +127,9 @@ __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_stream_kernel(
     const int per = (chunks + FRUNS - 1) / FRUNS;
     const int c_lo = min(chunks, wave * per), c_hi = min(chunks, c_lo + per);
 
-    // two chunks are asked for together: 256 contiguous bytes of every row
-    constexpr int U = 2;
+    // two chunks are asked for together: 256 contiguous bytes of every row (with many tiles one, whose
+    // loads are as many)
+    constexpr int U = NT > 2 ? 1 : 2;
     struct Rows {
         f32x4 w[U][NT][2], a[U][2];
     };
@@ -147,14 +149,19 @@ __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_stream_kernel(
     };
     auto products = [&](const f32x4 (&w)[NT][2], const f32x4 (&a)[2]) {
         const Split as = split8(a[0], a[1], (wave & 1u) << 31);
-        Split ws[NT];
+        constexpr int NB = NT % 2 ? 1 : 2;  // tiles whose instructions alternate
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) ws[nt] = split8(w[nt][0], w[nt][1]);
+        for (int n0 = 0; n0 < NT; n0 += NB) {
+            Split ws[NB];
 #pragma unroll
-        for (int s = 0; s < 6; ++s)
+            for (int j = 0; j < NB; ++j) ws[j] = split8(w[n0 + j][0], w[n0 + j][1]);
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[nt].p[PIECE_W[s]], as.p[PIECE_A[s]], acc[nt], 0, 0, 0);
+            for (int s = 0; s < 6; ++s)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    acc[n0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[j].p[PIECE_W[s]], as.p[PIECE_A[s]],
+                                                                         acc[n0 + j], 0, 0, 0);
+        }
     };
     auto group_products = [&](const Rows& r) {
 #pragma unroll
@@ -489,8 +496,8 @@ static int launch_tile(const float* A, const float* W, float* C, float* parts, i
     return rl_launch_status();
 }
 
-// Rows of A and W may be strided; the inner dimension is contiguous.  `tile`: 1 and 2 stream the weights
-// (up to 16 rows; so many tiles of 16 weight rows a workgroup), 32, 64 and 128 are the rows of A a tile takes;
+// Rows of A and W may be strided; the inner dimension is contiguous.  `tile`: 1, 2 and 3 stream the
+// weights (up to 16 rows; so many tiles of 16 weight rows a workgroup), 32, 64 and 128 are the rows of A a tile takes;
 // `groups` (1, 2, 4, 8): workgroups that share a tile's runs, with `parts` [8, M, N] for the runs' results
 // where there is more than one.
 extern "C" int rl_gemm_f32(const float* A, const float* W, float* C, float* parts, int M, int N, int K, int lda,
@@ -502,10 +509,11 @@ extern "C" int rl_gemm_f32(const float* A, const float* W, float* C, float* part
                      (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(W) & 15) == 0;
     const bool full = vec && K % FCH == 0;
-    if (tile <= 2) {
+    if (tile <= 3) {
         if (M > 16 || groups != 1) return RL_ERR_ARG;
         if (tile == 1) return launch_stream<1>(A, W, C, M, N, K, lda, ldw, ldc, vec, stream);
         if (tile == 2) return launch_stream<2>(A, W, C, M, N, K, lda, ldw, ldc, vec, stream);
+        if (tile == 3) return launch_stream<3>(A, W, C, M, N, K, lda, ldw, ldc, vec, stream);
         return RL_ERR_ARG;
     }
     if (tile == 32) return launch_tile<1, 2>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, full, stream);

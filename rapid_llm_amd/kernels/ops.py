@@ -997,15 +997,21 @@ _F32_MOST_SCRATCH = 1 << 27  # bytes of partial results a product may take
 @functools.lru_cache(maxsize=4096)
 def f32_plan(m: int, n: int, k: int, units: int) -> tuple[int, int]:
     """(tile, workgroups that share a tile's runs of K) of the float32 product.  Up to 16 rows the kernel that
-    streams the weights: one tile of 16 weight rows a workgroup, or two (tile 1 or 2) where that makes one
-    round of what would be a round and a half (6,144 weight rows on 256 units, 8 rows: 25.2 against 26.3 us;
-    a single row, whose time is the first loads': 23.3 against 22.1), and, from 13 rows on, where the rows read
-    again by every workgroup weigh as much as its weights (24,576 x 4,096, 16 rows: 92 against 98 us; 8 rows:
-    87 against 76).  More rows: the tile and the sharing for which the estimate is lowest; sharing fills
+    streams the weights, with one, two or three tiles of 16 weight rows a workgroup (tile 1, 2, 3).  Two where that
+    makes one round of what would be a round and a half (6,144 weight rows on 256 units, K = 4,096, 8 and 16
+    rows: 25.3 against 27.0 and 27.4 against 32.4 us; up to 4 rows only for short rows, whose time is not the
+    first loads': K = 4,096, one row 23.6 against 22.5).  Three for wide matrices from 5 rows on, because the rows
+    of A, read again by every workgroup, weigh as much as its weights (24,576 x 4,096 at 1, 8 and 16 rows: 69.0,
+    69.6 and 71.4 us against 65.7, 77.8 and 96.0 with one; 151,936 x 4,096 at 16 rows 445 against 574; the
+    three tiles also keep one chunk in flight instead of two, so two workgroups fit a unit).  More rows: the tile and the sharing for which the estimate is lowest; sharing fills
     the chip where the tiles do not, and writes and reads eight partial results for it."""
     if m <= 16:
         tiles = -(-n // 16)
-        return (2 if (units < tiles <= 2 * units and m > 4) or (tiles > 2 * units and m > 12) else 1), 1
+        if tiles <= units:
+            return 1, 1
+        if tiles <= 2 * units:
+            return (2 if m > 4 or k < 4096 else 1), 1
+        return (3 if m > 4 else 1), 1
     best = None
     for tile in (32,) if m <= 32 else (64,) if m <= 64 else (64, 128):
         width, costs = _F32_TILES[tile]

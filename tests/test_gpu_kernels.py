@@ -673,7 +673,7 @@ def test_gemm_f32_every_tile_and_sharing(shape):
     steps = 6 * -(--(-k // 32) // 8) + 8
     bound = (a.double().abs() @ w.double().abs().T) * (2 * steps + 2) * 2.0**-24
     ad, wd, first = a.to(DEV), w.to(DEV), None
-    plans = [(1, 1), (2, 1)] if m <= 16 else []
+    plans = [(1, 1), (2, 1), (3, 1)] if m <= 16 else []
     plans += [(tile, groups) for tile in (32, 64, 128) for groups in (1, 2, 4, 8)]
     for tile, groups in plans:
         out = torch.full((m, n + 1), float("nan"), device=DEV)
