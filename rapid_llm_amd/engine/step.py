@@ -156,12 +156,14 @@ class ModelRunner:
         self.device_cache = DeviceCache(self.cache, needs, group_of, self.dtype, self.device)
         self.computed: dict[str, int] = {}
         self.vocab_size = self.spec.vocab_size
-        self._graphs: dict[tuple[int, int], tuple] = {}
+        # (rows, context bound) -> whether the contexts are of unlike length -> the recorded step
+        self._graphs: dict[tuple[int, int], dict[bool, tuple]] = {}
         # (rows, context bound) -> products of the library that the recorded step holds; a key
         # whose step is not replayed because of them (library_in_graph="eager") is listed too
         self.graph_library_products: dict[tuple[int, int], int] = {}
         # a part that does not promise to be replayable keeps every step eager
         self.graphs_allowed = self.model.replayable()
+        self.ragged_matters = any(getattr(p, "deals_ragged_contexts", False) for p in self.model.all_parts())
         # where the sampling kernels leave their choices, one row per sampled request of a
         # step; the next step's embedding reads fed tokens from here
         self.sampled = torch.zeros(max(1, self.engine.max_num_seqs), dtype=torch.int32, device=self.device)
@@ -240,7 +242,9 @@ class ModelRunner:
             total += len(bounds) * scratch
             for bound in bounds:
                 kept = max((p.recorded_step_bytes(rows, bound, e.page_size) for p in parts), default=0)
-                total += rows * 4 * (self.spec.vocab_size + 8 * widest) + 2 * kept
+                # steps over contexts of unlike length may be recorded beside those of like ones
+                both = 2 if 8 <= rows <= 64 and bound > 512 and any(getattr(p, "deals_ragged_contexts", False) for p in parts) else 1
+                total += both * (rows * 4 * (self.spec.vocab_size + 8 * widest) + 2 * kept)
         return total
 
     # ------------------------------------------------------------------ requests
@@ -417,8 +421,10 @@ class ModelRunner:
         while bound <= meta["max_position"]:
             bound *= 2
         bound = min(bound, self.engine.max_seq_len)
+        # a step whose requests are of unlike length is laid out otherwise where a part says so
+        ragged = self.ragged_matters and ops.ragged_contexts([start + 1 for start in meta["h_seq_starts"][:batch]])
         key = (rows, bound)
-        entry = self._graphs.get(key)
+        entry = self._graphs.get(key, {}).get(ragged)
         if entry is None and self.engine.library_in_graph == "eager" and self.graph_library_products.get(key):
             return None  # found out at the first try: this shape's step holds a library product
         if entry is None:
@@ -435,6 +441,7 @@ class ModelRunner:
             )
             ctx.static["decode_only_tokens"] = torch.arange(rows, dtype=torch.int32, device=self.device)
             ctx.static["context_bound"] = bound
+            ctx.static["ragged_contexts"] = ragged
             library_before = ops.library_products
             current = torch.cuda.current_stream()
             side = torch.cuda.Stream()
@@ -467,7 +474,7 @@ class ModelRunner:
             # allocated outside the capture (the static inputs, what ctx.static holds) must
             # live as long as the graph does, so the context is kept with it
             entry = (graph, static, logits, ctx)
-            self._graphs[key] = entry
+            self._graphs.setdefault(key, {})[ragged] = entry
         graph, static, logits, _ctx = entry
         upload(host, self.device, into=static)
         graph.replay()

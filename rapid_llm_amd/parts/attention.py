@@ -293,6 +293,8 @@ class GQAAttention(PackedMixer):
             h = torch.arange(1, self.nq + 1, dtype=torch.float64)
             self.slopes = torch.exp2(-self.slope_exponent * h / self.nq).to(torch.float32).to(runtime.device)
         self.runtime = runtime
+        # the bfloat16 kernel that splits single tokens' keys
+        self.deals_ragged_contexts = not self.extended and runtime.dtype == torch.bfloat16 and self.d % 16 == 0 and not self.window
 
     # ---- cache -----------------------------------------------------------------
     def cache_need(self) -> CacheNeed:

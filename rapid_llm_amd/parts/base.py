@@ -212,6 +212,9 @@ class Part:
     #: emptied between the two.  A model with a part that does not declare it runs every step
     #: eagerly.
     replayable = False
+    #: Whether the part lays its launches out otherwise where ``ctx.static["ragged_contexts"]`` says that the
+    #: requests of a recorded step have contexts of unlike length: such steps are then recorded for themselves.
+    deals_ragged_contexts = False
 
     def param_specs(self) -> list[ParamSpec]:
         return []

@@ -192,6 +192,45 @@ def test_graph_of_more_requests_than_the_chip_holds_workgroups(tmp_path):
         r.cache.check_invariants()
 
 
+@pytest.mark.parametrize("batch", [8, 20, 40])  # 32, 80 and 160 workgroups unsplit: both of the rule's shares
+def test_graphs_of_like_and_unlike_contexts(tmp_path, batch):
+    """Requests of unlike length are recorded apart from those of like length, with finer splits of the
+    keys; one engine replays both kinds in turn, each against eager steps and the plain implementation."""
+    from rapid_llm_amd import EngineConfig, ModelRunner, StepEntry, write_random_model
+    from rapid_llm_amd.kernels import ops
+
+    page, seed, longest = 8, 17, 1100
+    config = dict(MANY_HEADS, max_position_embeddings=2048)
+    model_dir = tmp_path / "many_heads"
+    write_random_model(config, seed, model_dir, dtype="bfloat16", norm_std=0.1)
+    make = lambda graph: ModelRunner(
+        model_dir,
+        EngineConfig(dtype="bfloat16", max_seq_len=2048, page_size=page, num_pages=2 * batch * 150 + 8,
+                     max_num_seqs=2 * batch, use_graph=graph),
+    )
+    eager, graph = make(False), make(True)
+    pcfg, pw = plain_load(model_dir)
+    # the unlike ones: a few long, the rest short; the like ones all about as long as the longest
+    lengths = {f"u{i}": longest if i % 7 == 0 else 5 + 13 * i for i in range(batch)}
+    lengths |= {f"l{i}": longest - i for i in range(batch)}
+    seqs = {rid: random_tokens(n + 3, config["vocab_size"], seed + k) for k, (rid, n) in enumerate(lengths.items())}
+    for rid, n in lengths.items():
+        for r in (eager, graph):
+            r.step([StepEntry(rid, seqs[rid][:n])])
+    for step in range(3):
+        for kind in "ul":
+            rids = [rid for rid in lengths if rid[0] == kind]
+            starts = [lengths[rid] + step for rid in rids]
+            assert ops.ragged_contexts([s + 1 for s in starts]) == (kind == "u")
+            entries = [StepEntry(rid, [seqs[rid][s]], [0]) for rid, s in zip(rids, starts)]
+            a, b = eager.step(entries).clone(), graph.step(entries).clone()
+            parity.assert_bf16_close(b.cpu(), a.cpu(), f"graph of {batch} {kind} against eager/step {step}")
+            if step == 2:
+                want = torch.stack([plain_forward(pcfg, pw, seqs[rid][: s + 1], rows=[s])[0] for rid, s in zip(rids[:9], starts)])
+                parity.assert_bf16_close(b.cpu()[:9], want, f"graph of {batch} {kind}/step {step}")
+    assert [set(kinds) for kinds in graph._graphs.values()] == [{False, True}]
+
+
 def test_ragged_batches_share_a_few_graphs(tmp_path):
     """Requests that end at different times walk the batch size down one by one: the steps are
     padded with filler rows to a ladder of sizes, so few graphs are captured; with and without

@@ -197,6 +197,23 @@ def test_launch_rules_follow_the_number_of_compute_units():
     assert ops._prefill_shape(tile, 8, 0, 128, units=8) == (1, 1)
 
 
+def test_decode_splits_of_unlike_contexts():
+    """Requests of unlike length get more splits of their keys, whatever that would be for fewer than eight
+    and more than 64, and never splits that hold no whole step; the bytes reserved cover both."""
+    from rapid_llm_amd.kernels import ops
+
+    assert ops.ragged_contexts([64] * 7 + [4000]) and not ops.ragged_contexts([64] * 6 + [4000])
+    assert not ops.ragged_contexts([2000, 2400] * 6) and not ops.ragged_contexts([64] * 64 + [4000])
+    assert not ops.ragged_contexts([])
+    for rows in (8, 12, 16, 17, 24, 32, 64):
+        for span in (512, 1024, 4096, 40000):
+            pairs, chunk, like = ops._decode_split(rows, 32, 8, span, 16, 0, units=256)
+            _, fine, unlike = ops._decode_split(rows, 32, 8, span, 16, 0, units=256, ragged=True)
+            assert unlike >= like and fine <= chunk and fine % 32 == 0 and fine * unlike >= span
+            assert unlike == 1 or fine >= 128
+            assert ops.decode_scratch_bytes(rows, 32, 8, 128, span, 16, 0) >= (0 if unlike == 1 else rows * 32 * unlike * 130 * 4)
+
+
 def test_weight_rows_a_workgroup_of_the_few_row_product():
     """The host's rule: 24 rows (code 3) only for a product that just stores its result, on a
     matrix of 257 to 1,023 tiles, where that puts the fewest rows on a compute unit."""
