@@ -496,6 +496,44 @@ def test_rope_table_matches_plain():
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("nq,nkv,d,dv,col0", [(4, 3, 64, 64, 0), (2, 5, 128, 128, 8), (3, 1, 32, 20, 0), (1, 2, 256, 256, 16)])
+@pytest.mark.parametrize("tokens", [8, 17, 50])
+def test_keys_and_values_alone(dtype, nq, nkv, d, dv, col0, tokens):
+    """A step whose queries the attention finishes writes the same keys, bit for bit, as one that writes
+    queries too, (token, key head) pairs packed across tokens, and the values as they are: rows read 16
+    bytes at a time and rows that cannot be."""
+    ops = _ops()
+    page, width = 8, -(-(col0 + (nq + nkv) * d + nkv * dv) // 8) * 8
+    gen = torch.Generator().manual_seed(tokens + d)
+    qkv = torch.randn(tokens, width, generator=gen).to(dtype)
+    qw, kw = (1 + 0.1 * torch.randn(d, generator=gen) for _ in range(2))
+    start = 3  # pages and the kernel's groups of 16 tokens do not line up
+    table = torch.randperm((start + tokens) // page + 1, generator=gen).to(torch.int32)[None] + 1
+    pages = int(table.max()) + 1
+    cos, sin = ops.rope_table(plain_inv_freq(d, 1e4).to(DEV), 64)
+    caches = []
+    for queries in (True, False):
+        kc = torch.full((pages, nkv, page, d), float("nan"), dtype=dtype, device=DEV)
+        vc = torch.full((pages, nkv, dv, page), float("nan"), dtype=dtype, device=DEV)
+        q_out = torch.empty(tokens, nq * d, dtype=dtype, device=DEV) if queries else None
+        ops.qknorm_rope_kvwrite(
+            qkv.to(DEV), q_out, kc, vc, qw.to(DEV), kw.to(DEV), cos, sin,
+            torch.arange(start, start + tokens, dtype=torch.int32, device=DEV),
+            torch.zeros(tokens, dtype=torch.int32, device=DEV), table.to(DEV), page, nq, nkv, d, 1e-5,
+            start + tokens - 1, value_dim=dv, col0=col0,
+        )
+        caches.append((kc, vc))
+    for a, b in zip(*caches):
+        assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0))
+    vc = caches[0][1].cpu()
+    v = qkv[:, col0 + (nq + nkv) * d :][:, : nkv * dv].view(tokens, nkv, dv)
+    for t in range(tokens):
+        p = start + t
+        assert torch.equal(vc[int(table[0, p // page]), :, :, p % page], v[t])
+    assert int((~vc.isnan()).sum()) == v.numel() and int((~caches[0][0].isnan()).sum()) == tokens * nkv * d
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("shape", [(5, 5, 48, 8), (6, 2, 128, 16), (3, 1, 16, 4), (4, 4, 256, 4)])
 @pytest.mark.parametrize("many", [False, True], ids=["few", "many"])
 def test_qknorm_rope_kvwrite(dtype, shape, many):
