@@ -34,11 +34,12 @@ namespace f32attn {
 constexpr int D = RL_HEAD_DIM;
 constexpr int DB = D / 16;  // 16-channel chunks of the first product = blocks of the output
 constexpr int AW = 4;       // waves per workgroup: key tile i belongs to wave i % AW
-// Keys a span: 256 workgroups for eight requests of 2,048 keys and eight kv heads; eight tiles a wave
-// between two folds.  Eight requests of 512 to 1,536 keys of the 8B shape: 64 workgroups that walked
-// whole contexts took 65 us a layer, the latency of their chain of tiles, the step 8.95 ms; spans in
-// workgroups of their own leave it at 7.80 ms.
-constexpr int SPAN = 512;
+// Keys a span.  Eight requests of 512 to 1,536 keys of the 8B shape: 64 workgroups that walked whole
+// contexts took 65 us a layer, the latency of their chain of tiles, the step 8.95 ms; spans in workgroups
+// of their own leave it at 7.80 ms.  Spans of 256 keys rather than 512 take a single request of 1,000 keys
+// of the 0.6B shape from 2.19 to 1.97 ms a step and cost a prompt of 2,048 tokens 0.3%, for a fold every
+// four tiles of a wave; of 128 they cost it 4%.
+constexpr int SPAN = 256;
 constexpr int STATE = D + 2;  // floats a (row, wave, span) state takes in memory: sums, maximum, sum of weights
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -72,14 +73,14 @@ __device__ inline float fold_sum(float x, float x2, const Fold& f) { return fmaf
 
 // tile_info: [tiles][3] = index of the request's first token in the step, its tokens in the
 // step, first row of the tile.  The request's first position is read from `positions`.
-// SPLIT: blockIdx.z is the span; states[tile][kv head][span][wave][row][STATE] take the place of `out`.
+// SPLIT: blockIdx.z takes `per` spans; states[tile][kv head][span][wave][row][STATE] take the place of `out`.
 template <bool SPLIT>
 __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache,
     const float* __restrict__ v_cache, float* __restrict__ out, float* __restrict__ states,
     const int* __restrict__ tile_info, const int* __restrict__ positions,
     const int* __restrict__ token_slot, const int* __restrict__ block_table, int table_stride,
-    int page_size, int nq, int nkv, int window, float scale) {
+    int page_size, int nq, int nkv, int window, float scale, int spans, int per) {
     const int tile = blockIdx.x;
     const int hk = blockIdx.y;
     const int G = nq / nkv;
@@ -110,8 +111,8 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
     const int lo = first_key & ~15;
     const int hi = last_pos + 1;  // keys below hi are in the cache
     // the keys this workgroup walks
-    const int from = SPLIT ? max(lo, (int)blockIdx.z * SPAN) : lo;
-    const int upto = SPLIT ? min(hi, ((int)blockIdx.z + 1) * SPAN) : hi;
+    const int from = SPLIT ? max(lo, (int)blockIdx.z * per * SPAN) : lo;
+    const int upto = SPLIT ? min(min(hi, spans * SPAN), ((int)blockIdx.z + 1) * per * SPAN) : hi;
     if (SPLIT && from >= upto) return;  // the fold knows which spans there are
 
     // Q^T: lane (row r16, g) holds channels 16c + 4g .. + 3 of its row
@@ -201,25 +202,42 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
         }
     };
 
-    // a span is over: its state joins the wave's (a launch that walks whole contexts)
+    // a span is over: its state joins the wave's (a launch that walks whole contexts), or goes to memory
     float m_all = -INFINITY, l_all = 0.f;
     f32x4 acc_all[DB];
     if (!SPLIT) {
 #pragma unroll
         for (int b = 0; b < DB; ++b) acc_all[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
+    int span = from / SPAN;
     auto finish_span = [&]() {
-        const Fold f = fold_of(m_all, m);
-        l_all = fold_sum(l_all, l, f);
-        m_all = f.m;
+        if (SPLIT) {
+            // (a single token's tile holds no more rows than its kv head has query heads)
+            if (row_ok) {
+                float* to = states + ((((size_t)tile * nkv + hk) * spans + span) * AW + wave) * 16 * STATE + r16 * STATE;
+#pragma unroll
+                for (int b = 0; b < DB; ++b)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) to[16 * b + 4 * g + i] = acc[b][i];
+                if (g == 0) {
+                    to[D] = m;
+                    to[D + 1] = l;
+                }
+            }
+            ++span;
+        } else {
+            const Fold f = fold_of(m_all, m);
+            l_all = fold_sum(l_all, l, f);
+            m_all = f.m;
+#pragma unroll
+            for (int b = 0; b < DB; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc_all[b][i] = fold_sum(acc_all[b][i], acc[b][i], f);
+        }
         m = -INFINITY;
         l = 0.f;
 #pragma unroll
-        for (int b = 0; b < DB; ++b) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc_all[b][i] = fold_sum(acc_all[b][i], acc[b][i], f);
-            acc[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        }
+        for (int b = 0; b < DB; ++b) acc[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
     };
 
     // Software pipeline over the wave's tiles: while a tile goes through softmax and the second
@@ -231,6 +249,7 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
     // itself the scheduler moves loads down to their use).
     constexpr int STEP = 16 * AW;
     const int mine = from + 16 * ((wave - from / 16) & (AW - 1));  // first tile >= from with index % AW == wave
+    if (SPLIT && mine < upto && mine / SPAN > span) finish_span();  // no tile of this wave in the first span
     if (mine < upto) {
         int left = (upto - mine + STEP - 1) / STEP;  // tiles of this wave, the current one included
         int kb = mine;
@@ -250,28 +269,21 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
             for (int b = 0; b < DB; ++b) vcur[b] = vnext[b];
             kb += STEP;
             --left;
-            if (!SPLIT && kb % SPAN < STEP) finish_span();
+            if (kb % SPAN < STEP) finish_span();
         }
         if (left == 2) {
             const f32x4 s_next = scores(keys);
             load_values(kb + STEP, vnext);
             finish_tile(kb, sc, vcur);
-            if (!SPLIT && (kb + STEP) % SPAN < STEP) finish_span();
+            if ((kb + STEP) % SPAN < STEP) finish_span();
             finish_tile(kb + STEP, s_next, vnext);
         } else {
             finish_tile(kb, sc, vcur);
         }
     }
     if (SPLIT) {
-        float* to = states + ((((size_t)tile * nkv + hk) * gridDim.z + blockIdx.z) * AW + wave) * 16 * STATE + r16 * STATE;
-#pragma unroll
-        for (int b = 0; b < DB; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) to[16 * b + 4 * g + i] = acc[b][i];
-        if (g == 0) {
-            to[D] = m;
-            to[D + 1] = l;
-        }
+        // the last span, and one that holds no tile of this wave
+        while (span <= (upto - 1) / SPAN) finish_span();
         return;
     }
     finish_span();
@@ -360,25 +372,26 @@ __global__ __launch_bounds__(256) void attn_f32_fold_kernel(const float* __restr
 // Every token of the step, single tokens and portions alike.  page_size must be a multiple
 // of 4 (the four keys of a lane lie in one page).  `spans` > 0 gives every span of keys to workgroups of
 // its own, with `states` [tiles, nkv, spans, 4, 16, D + 2]; it must cover the longest context.
+// `per`: spans a workgroup takes.
 extern "C" int rl_attn_f32(const float* q, const float* k_cache, const float* v_cache, float* out, float* states,
                            const int* tile_info, int num_tiles, const int* positions,
                            const int* token_slot, const int* block_table, int table_stride,
-                           int page_size, int nq, int nkv, int window, float scale, int spans,
+                           int page_size, int nq, int nkv, int window, float scale, int spans, int per,
                            hipStream_t stream) {
     using namespace f32attn;
     if (num_tiles <= 0) return RL_OK;
     if (nkv < 1 || nq % nkv || page_size < 4 || page_size % 4 || nkv > 65535) return RL_ERR_ARG;
-    if (spans < 0 || spans > 65535 || (spans && !states)) return RL_ERR_ARG;
+    if (spans < 0 || spans > 65535 || per < 1 || (spans && !states)) return RL_ERR_ARG;
     const dim3 block(AW * RL_WAVE);
     if (!spans) {
         hipLaunchKernelGGL(attn_f32_kernel<false>, dim3(num_tiles, nkv), block, 0, stream, q, k_cache, v_cache, out,
                            states, tile_info, positions, token_slot, block_table, table_stride, page_size, nq, nkv,
-                           window, scale);
+                           window, scale, 0, 1);
         return rl_launch_status();
     }
-    hipLaunchKernelGGL(attn_f32_kernel<true>, dim3(num_tiles, nkv, spans), block, 0, stream, q, k_cache, v_cache, out,
-                       states, tile_info, positions, token_slot, block_table, table_stride, page_size, nq, nkv, window,
-                       scale);
+    hipLaunchKernelGGL(attn_f32_kernel<true>, dim3(num_tiles, nkv, (spans + per - 1) / per), block, 0, stream, q, k_cache,
+                       v_cache, out, states, tile_info, positions, token_slot, block_table, table_stride, page_size, nq,
+                       nkv, window, scale, spans, per);
     if (int code = rl_launch_status()) return code;
     hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(num_tiles, nkv), dim3(256), 0, stream, states, out, tile_info,
                        positions, spans, nq, nkv, window);

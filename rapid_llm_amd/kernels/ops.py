@@ -1781,7 +1781,7 @@ def _f32_tiles(ctx, group: int, tile_rows: int = 16, chunk: int = 0) -> tuple[to
     return made
 
 
-_F32_SPAN = 512  # keys of a span of the float32 attention
+_F32_SPAN = 256  # keys of a span of the float32 attention
 _F32_SPLIT_BYTES = 1 << 28  # what a launch may take for the states of its spans
 
 
@@ -1791,7 +1791,7 @@ def f32_spans(tiles: int, nkv: int, d: int, longest: int, window: int, units: in
     one for every compute unit (no states are written and folded) and where a window spans too little."""
     units = chip().units if units is None else units
     spans = -(-longest // _F32_SPAN)
-    if spans < 2 or tiles * nkv >= units or 0 < window < 2 * _F32_SPAN:
+    if spans < 3 or tiles * nkv >= units or 0 < window < 4 * _F32_SPAN:
         return 0
     return spans if tiles * nkv * spans * 64 * (d + 2) * 4 <= _F32_SPLIT_BYTES else 0
 
@@ -1840,14 +1840,17 @@ def attention_f32(
     # under a graph the launch is laid out for the longest context of the graph's bucket
     longest = _static(ctx).get("context_bound", ctx.max_position + 1)
     spans = f32_spans(num_tiles, nkv, d, longest, window)
-    states = None
+    states, per = None, 1
     if spans:
+        # as many workgroups as a unit takes in two rounds: more of them only begin more often (16 requests of
+        # 300 to 2,500 keys, 8 kv heads: 3.78 ms a step with one span each)
+        per = -(-num_tiles * nkv * spans // (4 * chip().units))
         states = torch.empty((num_tiles, nkv, spans, 4, 16, d + 2), dtype=torch.float32, device=q.device)
     _ok(
         attention_lib(d).rl_attn_f32(
             _p(q), _p(k_cache), _p(v_cache), _p(out), _p(states), _p(tiles), num_tiles, _p(ctx.positions),
             _p(ctx.token_slot), _p(block_table), block_table.stride(0), page_size, nq, nkv, window,
-            ctypes.c_float(scale), spans, _stream(),
+            ctypes.c_float(scale), spans, per, _stream(),
         ),
         "rl_attn_f32",
     )

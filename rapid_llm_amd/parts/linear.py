@@ -5,8 +5,8 @@ kernel of its own after the product.
 
 Which product runs is decided by the weight's storage type:
 
-* float32 weight: the hand-written float32 FMA kernel (true 32-bit; the only product of
-  the float32 engine).  A bfloat16 activation is widened first, so a matrix that the
+* float32 weight: the hand-written float32 product (operands split into three bfloat16 numbers that add
+  up to them, so that no bit of them is lost; the only product of the float32 engine).  A bfloat16 activation is widened first, so a matrix that the
   checkpoint stores in 32-bit is used at full precision in a bfloat16 engine too.
 * bfloat16 weight: few rows (decode) go to the hand-written bandwidth-bound matrix-core
   kernel; many rows go to the library product, as in the reference, whose dense products

@@ -181,15 +181,17 @@ def test_attention_f32_spans_in_workgroups_of_their_own(d, nq, nkv, page, window
     """A float32 launch whose spans of keys go to workgroups of their own gives the bits of one that walks
     whole contexts: contexts that end at a span's edge and one key on either side, a portion across one."""
     ops = _ops()
-    seqs = [(510, 1), (511, 1), (512, 1), (0, 1), (1023, 1), (1024, 1), (2100, 1), (500, 30), (1530, 7)]
+    seqs = [(254, 1), (255, 1), (256, 1), (270, 1), (0, 1), (1023, 1), (1024, 1), (2100, 1), (500, 30), (1530, 7)]
     q, kc, vc, table, ctx, want = _paged_problem(seqs, nq, nkv, d, page, torch.float32, d + window, window)
     outs = []
-    for spans in (0, 5, 8):  # 8: laid out for a longer context than there is
+    # 9 spans and laid out for a longer context than there is, one and several spans a workgroup
+    for spans, units in ((0, 256), (9, 256), (13, 256), (9, 40), (13, 16)):
         monkeypatch.setattr(ops, "f32_spans", lambda *args: spans)
+        monkeypatch.setattr(ops, "chip", lambda: ops.Chip(units))
         out = torch.full_like(q, float("nan"))
         ops.attention_f32(q, kc, vc, out, ctx, table, page, nq, nkv, d, window, 1.0 / math.sqrt(d))
         outs.append(out)
-    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
     torch.testing.assert_close(outs[0].cpu(), want, rtol=2e-5, atol=3e-6)
 
 
