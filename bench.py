@@ -1228,7 +1228,8 @@ def main() -> int:
             "value": round(prompt_len / sec, 1),
             "tokens": prompt_len,
             "ms": round(sec * 1e3, 3),
-            "frac": round(flops / sec / (PEAK_TFLOPS[args.dtype] * 1e12), 4),
+            # a float32 product is six bfloat16 ones (of operands split in three)
+            "frac": round(flops / sec / (PEAK_TFLOPS["bfloat16"] / (6 if args.dtype == "float32" else 1) * 1e12), 4),
         }
         print(f"[bench] prefill {prefill}", file=sys.stderr, flush=True)
 
