@@ -320,33 +320,34 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
 }
 
 // The states of a split launch folded as the other launch folds them: a workgroup per (tile, kv head),
-// 16 lanes a row, D / 16 channels a lane.  Bound by its start: the states of the next span are asked for
-// together with this one's.
-__global__ __launch_bounds__(256) void attn_f32_fold_kernel(const float* __restrict__ states, float* __restrict__ out,
-                                                            const int* __restrict__ tile_info,
-                                                            const int* __restrict__ positions, int spans, int nq,
-                                                            int nkv, int window) {
+// 16 lanes a row, D / 16 channels a lane.  Bound by the chain of its loads: a quarter of the threads
+// folds the spans of one wave of the launch before (all four in turn took 14 us at nine spans), the first
+// quarter then folds the waves.
+__global__ __launch_bounds__(256 * AW) void attn_f32_fold_kernel(const float* __restrict__ states, float* __restrict__ out,
+                                                                 const int* __restrict__ tile_info,
+                                                                 const int* __restrict__ positions, int spans, int nq,
+                                                                 int nkv, int window) {
+    __shared__ float part_ml[AW][2][256];
+    __shared__ float part_acc[AW][DB][256];
     const int tile = blockIdx.x, hk = blockIdx.y;
     const int G = nq / nkv;
     const int at = tile_info[3 * tile], n = tile_info[3 * tile + 1], row0 = tile_info[3 * tile + 2];
     const int rows = n * G;
-    const int r16 = threadIdx.x >> 4, part = threadIdx.x & 15;
+    const int w = threadIdx.x >> 8, thread = threadIdx.x & 255;
+    const int r16 = thread >> 4, part = thread & 15;
     const int row = row0 + r16;
-    if (row >= rows) return;
+    const bool row_ok = row < rows;
     const int start = positions[at];
     const int first_pos = start + row0 / G;
     const int last_pos = start + (min(rows, row0 + 16) - 1) / G;
     const int first_key = (window > 0 && first_pos - window + 1 > 0) ? first_pos - window + 1 : 0;
     const int s_lo = first_key / SPAN, s_hi = min(last_pos / SPAN + 1, spans);  // the spans that were walked
 
-    float m_out = -INFINITY, l_out = 0.f, acc_out[DB];
+    float m = -INFINITY, l = 0.f, acc[DB];
 #pragma unroll
-    for (int b = 0; b < DB; ++b) acc_out[b] = 0.f;
-    for (int w = 0; w < AW; ++w) {
-        float m = -INFINITY, l = 0.f, acc[DB];
-#pragma unroll
-        for (int b = 0; b < DB; ++b) acc[b] = 0.f;
-#pragma unroll 2
+    for (int b = 0; b < DB; ++b) acc[b] = 0.f;
+    if (row_ok) {
+#pragma unroll 4
         for (int s = s_lo; s < s_hi; ++s) {
             const float* from = states + ((((size_t)tile * nkv + hk) * spans + s) * AW + w) * 16 * STATE + r16 * STATE;
             const Fold f = fold_of(m, from[D]);
@@ -355,16 +356,25 @@ __global__ __launch_bounds__(256) void attn_f32_fold_kernel(const float* __restr
 #pragma unroll
             for (int b = 0; b < DB; ++b) acc[b] = fold_sum(acc[b], from[16 * b + part], f);
         }
-        const Fold f = fold_of(m_out, m);
-        l_out = fold_sum(l_out, l, f);
-        m_out = f.m;
+        part_ml[w][0][thread] = m;
+        part_ml[w][1][thread] = l;
 #pragma unroll
-        for (int b = 0; b < DB; ++b) acc_out[b] = fold_sum(acc_out[b], acc[b], f);
+        for (int b = 0; b < DB; ++b) part_acc[w][b][thread] = acc[b];
+    }
+    __syncthreads();
+    if (w > 0 || !row_ok) return;
+#pragma unroll
+    for (int v = 1; v < AW; ++v) {
+        const Fold f = fold_of(m, part_ml[v][0][thread]);
+        l = fold_sum(l, part_ml[v][1][thread], f);
+        m = f.m;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) acc[b] = fold_sum(acc[b], part_acc[v][b][thread], f);
     }
     float* orow = out + ((size_t)(at + row / G) * nq + hk * G + row % G) * D;
-    const float inv = 1.f / l_out;
+    const float inv = 1.f / l;
 #pragma unroll
-    for (int b = 0; b < DB; ++b) orow[16 * b + part] = acc_out[b] * inv;
+    for (int b = 0; b < DB; ++b) orow[16 * b + part] = acc[b] * inv;
 }
 
 }  // namespace f32attn
@@ -393,7 +403,7 @@ extern "C" int rl_attn_f32(const float* q, const float* k_cache, const float* v_
                        v_cache, out, states, tile_info, positions, token_slot, block_table, table_stride, page_size, nq,
                        nkv, window, scale, spans, per);
     if (int code = rl_launch_status()) return code;
-    hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(num_tiles, nkv), dim3(256), 0, stream, states, out, tile_info,
+    hipLaunchKernelGGL(attn_f32_fold_kernel, dim3(num_tiles, nkv), dim3(256 * AW), 0, stream, states, out, tile_info,
                        positions, spans, nq, nkv, window);
     return rl_launch_status();
 }
