@@ -47,6 +47,7 @@ CORE_SOURCES = (
     "sampling.hip",
     "gemm_bf16.hip",
     "gemm_rows.hip",
+    "gemm_block.hip",
     "latent.hip",
     "router.hip",
     "sublayer_sum.hip",

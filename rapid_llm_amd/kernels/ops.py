@@ -1467,6 +1467,7 @@ def gemm_bf16_residual(
 
 
 TILE_MAX_ROWS = 512  # rows up to which small matrices run the one-launch tile product
+TILE_GATED_MAX_ROWS = 128  # and the packed gate and up matrices, which the many-row product takes from there on
 _TILE_MAX_WEIGHTS = 7 << 20  # elements of a matrix (14 MB) up to which it is used
 _TILE_MIN_COLS = 2048  # fewer columns leave too few workgroups
 
@@ -1485,7 +1486,9 @@ def _tile_applies(m: int, weight_rows: int, k: int, cols: int) -> bool:
     are the faster ones on the device (512 rows: 10.6 / 12.2, with the activation 20.1 / 19.1;
     1,024 rows: 13.5 / 21.3 and 25.7 / 32.6), but a step of a few hundred tokens of so small a
     model is bound by the host, where a call of the library costs 18 us and one of this kernel
-    6: a 512-token prompt of the Qwen3-0.6B shape 5.4 -> 4.2 ms.  Hence up to 512 rows."""
+    6: a 512-token prompt of the Qwen3-0.6B shape 5.4 -> 4.2 ms.  Hence up to 512 rows.  The packed gate and up
+    matrices go on to the many-row product from 129 rows on (6,144 x 1,024 at 64 / 128 / 160 / 256 / 512 rows, the tile
+    product first: 10.7 / 11.8, 11.7 / 12.3, 14.7 / 11.9, 15.3 / 12.3, 19.3 / 12.5)."""
     return (
         SKINNY_MAX_ROWS < m <= TILE_MAX_ROWS
         and k % 128 == 0
@@ -1493,6 +1496,84 @@ def _tile_applies(m: int, weight_rows: int, k: int, cols: int) -> bool:
         and cols * (weight_rows // cols) >= _TILE_MIN_COLS
         and weight_rows * k <= _TILE_MAX_WEIGHTS
     )
+
+
+# The many-row product's tiles (pieces of 64 weight rows x pieces of 64 rows of X) and what a launch of each
+# takes: microseconds a chunk of 64 k with next to no compute unit busy, what full occupancy adds (the clock falls,
+# memory is shared), and microseconds a round of workgroups beyond its chunks (the first chunks' way from memory, the
+# results' way back).  Fitted to 39 row counts from 72 to 8,192 over the four matrices of the family's 0.6B to 8B
+# members; the tile they pick is the fastest or within 3% of it at all of them (gated), 12% at worst and 0.5% on
+# average (runs of K, where an element of a run costs another _BLOCK_RUN_ELEMENT microseconds to write and to add).
+_BLOCK_TILES = ((4, 4), (3, 4), (2, 4), (4, 2), (3, 2), (2, 2))
+_BLOCK_COSTS = {
+    "gated": ((0.86, 0.49, 7.4), (0.74, 0.36, 5.9), (0.59, 0.24, 3.9), (0.745, 0.153, 2.5), (0.663, 0.068, 2.3), (0.518, 0.044, 1.9)),
+    "runs": ((0.85, 0.47, 9.8), (0.73, 0.34, 6.2), (0.56, 0.25, 3.5), (0.64, 0.25, 4.0), (0.525, 0.19, 3.0), (0.42, 0.14, 2.3)),
+}
+_BLOCK_RUN_ELEMENT = 1.1e-6
+
+
+def block_plan(m: int, n: int, k: int, kind: str, units: int | None = None) -> tuple[int, int, int] | None:
+    """(pieces of weight rows, pieces of rows of X, runs of K) of the many-row product for ``m`` rows and ``n``
+    result columns, ``None`` where it does not apply.
+
+    ``"gated"``: the packed gate and up matrices with the activation in the epilogue, from 65 rows on.  Against the
+    library's product and the activation kernel, microseconds at 128 / 512 / 2,048 / 8,192 rows (the library first):
+    8B 55.6 / 54.1, 93.5 / 80.5, 303 / 286, 1,176 / 1,106; 4B 35.8 / 33.9, 63.5 / 49.6, 218 / 172, 756 / 587; 1.7B
+    21.3 / 21.0, 35.6 / 27.9, 105 / 82.7, 337 / 302; 0.6B 14.7 / 12.4, 20.0 / 12.8, 37.3 / 25.8, 113 / 91.2.
+
+    ``"runs"``: a product whose result feeds the residual, as float32 runs of K that the norm adds: long sums of few
+    columns, which leave the library's kernels for 65 to some 2,000 rows without work for the whole chip.  With the
+    norm, at 128 / 512 / 1,024 / 2,048 rows: 8B (K = 12,288) 70.0 / 35.0, 86.1 / 64.2, 126 / 99.3, 187 / 171; 4B (9,728)
+    48.7 / 24.0, 51.8 / 42.0, 82.4 / 64.3, 115 / 101; 1.7B (6,144) 18.6 / 18.3, 28.7 / 28.1, 43.5 / 41.4, and slower from
+    there (1,500 rows 50.4 / 54.4).  Against the blocks of 64 rows of the mid-size product, at 65 / 128 / 192 rows:
+    8B 42.4 / 30.2, 41.0 / 34.1, 54.6 / 38.9; 4B 23.7 / 21.8, 25.3 / 25.7, 32.3 / 26.2; 1.7B, which stays there up to
+    128 rows, 15.3 / 16.1, 16.6 / 17.9, 20.6 / 19.3.  Sums of 4,096 and less are level or the library's (8B output projection 33.6 / 32.9,
+    48.2 / 48.4, 74.9 / 73.7; 0.6B down 16.7 / 16.9, 19.8 / 21.4, 27.4 / 28.9)."""
+    return _block_plan(m, n, k, kind, chip().units if units is None else units)
+
+
+@functools.lru_cache(maxsize=4096)
+def _block_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int, int] | None:
+    if m <= ROWS_MAX_ROWS or n % 8 or k % 64 or k < 64:
+        return None
+    # offsets inside an operand are 32-bit in the kernel, those of rows beyond it too
+    if max((m + 256) * k, ((2 if kind == "gated" else 1) * n + 256) * k) * 2 > 0x7FFFFFFF:
+        return None
+    chunks = k // 64
+    runs = (1,)
+    if kind == "runs":
+        squares = -(-m // 256) * -(-n // 256)
+        if k < 6144 or (k < 8192 and (m <= 128 or squares > 32)) or squares > 128:
+            return None
+        runs = (1, 2, 3, 4, 6, 8)
+    best = None
+    for (nw, nx), (chunk, full, round_) in zip(_BLOCK_TILES, _BLOCK_COSTS[kind]):
+        tiles = -(-n // ((32 if kind == "gated" else 64) * nw)) * -(-m // (64 * nx))
+        for ks in runs:
+            per = -(-chunks // ks)
+            if ks > 1 and (per < 4 or per * (ks - 1) >= chunks):  # every run holds a chunk
+                continue
+            rounds = -(-tiles * ks // units)
+            cost = rounds * (per * (chunk + full * tiles * ks / (rounds * units)) + round_)
+            if kind == "runs":
+                cost += m * n * ks * _BLOCK_RUN_ELEMENT
+            if best is None or cost < best[0]:
+                best = (cost, (nw, nx, ks))
+    return best[1]
+
+
+_BLOCK_KINDS = {"runs": 1, "gated": 2}  # as the kernel's entry point counts them
+
+
+def _aligned(*tensors: torch.Tensor) -> bool:
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _block(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str, plan: tuple[int, int, int]) -> torch.Tensor:
+    m, k = x.shape
+    n = out.shape[-1]
+    _ok(core().rl_gemm_block(_p(x), _p(w), _p(out), m, n, k, k, k, n, _BLOCK_KINDS[kind], *plan, _stream()), "rl_gemm_block")
+    return out
 
 
 # Rows up to which a product's runs of K may be left to the norm that follows.  Beyond 64 rows the
@@ -1528,13 +1609,18 @@ def _mid_runs(n: int, k: int, units: int) -> int:
 
 
 def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x[M,K] @ w[N,K]^T`` for 17 to 192 rows as float32 runs of K, ``[runs, M, N]``: their sum
-    is the product.  For products whose result goes into the residual: the norm that follows
-    adds the runs (``add_rmsnorm_parts``)."""
+    """``x[M,K] @ w[N,K]^T`` for 17 to 192 rows, or as many as :func:`block_plan` says, as float32 runs of K,
+    ``[runs, M, N]``: their sum is the product.  For products whose result goes into the residual: the norm that
+    follows adds the runs (``add_rmsnorm_parts``)."""
     _need(x, "x", torch.bfloat16)
     _need(w, "w", torch.bfloat16)
     m, k = x.shape
     n = w.shape[0]
+    plan = block_plan(m, n, k, "runs") if k == w.shape[1] else None
+    if plan is not None and not _aligned(x, w):  # (a view that begins inside a unit of 16 bytes)
+        x, w = (t if _aligned(t) else t.clone() for t in (x, w))
+    if plan is not None:
+        return _block(x, w, torch.empty((plan[2], m, n), dtype=torch.float32, device=x.device), "runs", plan)
     ks = mid_runs(n, k)
     if k != w.shape[1] or m > MID_MAX_ROWS or ks < 1:
         raise KernelError(f"gemm_bf16_parts does not take x {tuple(x.shape)}, w {tuple(w.shape)}")
@@ -1567,8 +1653,8 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
                      alpha: float = GLU_ALPHA, activation: str = "silu",
                      bias: Optional[torch.Tensor] = None) -> torch.Tensor | None:
     """``act(x Wg^T, x Wu^T)`` for the packed ``[gate | up]`` matrix in one kernel: for few rows,
-    and for up to 512 rows over a small matrix; ``None`` when the shape is not one a fused kernel
-    takes.  ``act`` is ``silu(g) * u``, or with a ``limit`` the clamped variant of :func:`swiglu`;
+    for up to 512 rows over a small matrix, and with ``silu(g) * u`` for many; ``None`` when the shape is not one a
+    fused kernel takes.  ``act`` is ``silu(g) * u``, or with a ``limit`` the clamped variant of :func:`swiglu`;
     ``activation`` and ``bias`` (float32, gate entries first) as there.
     ``scaled``: as in ``gemm_bf16``."""
     m, k = x.shape
@@ -1584,7 +1670,12 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
             return None
         _need(x, "x", torch.bfloat16)
         _need(w_gate_up, "w_gate_up", torch.bfloat16, (two_i, k))
-        if _tile_applies(m, two_i, k, inter):
+        tile = _tile_applies(m, two_i, k, inter)
+        if (not tile or m > TILE_GATED_MAX_ROWS) and activation == "silu" and limit <= 0 and bias is None:
+            plan = block_plan(m, inter, k, "gated")
+            if plan is not None and _aligned(x, w_gate_up):
+                return _block(x, w_gate_up, torch.empty((m, inter), dtype=torch.bfloat16, device=x.device), "gated", plan)
+        if tile:
             out = torch.empty((m, inter), dtype=torch.bfloat16, device=x.device)
             _ok(core().rl_gemm_tile(_p(x), _p(w_gate_up), _p(out), m, inter, k, k, k, inter, 1, *glu, _stream()), "rl_gemm_tile")
             return out

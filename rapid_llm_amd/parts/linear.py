@@ -12,8 +12,8 @@ Which product runs is decided by the weight's storage type:
   its bits in a bfloat16 engine too.
 * bfloat16 weight: few rows (decode) go to the hand-written bandwidth-bound matrix-core
   kernel; many rows go to the library product, as in the reference, whose dense products
-  are ``F.linear`` (rapid_llm/kernels/ops/gemm/linear.py:17-40).  In between (17 to 192 rows) a
-  narrow matrix whose result a norm adds to the residual may hand that norm float32 runs of
+  are ``F.linear`` (rapid_llm/kernels/ops/gemm/linear.py:17-40).  In between (17 to 192 rows, more where K is
+  long) a narrow matrix whose result a norm adds to the residual may hand that norm float32 runs of
   K instead (``partial_sums``).
 """
 
@@ -63,11 +63,12 @@ class Linear:
     def midsize(self, x) -> bool:
         """Whether ``x`` (more rows than the few-row kernel takes) may run as float32 runs of K
         that a norm adds (narrow matrices only: the wide ones are faster in the library)."""
-        return (
-            self.weight.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
-            and ops.SKINNY_MAX_ROWS < x.shape[0] <= ops.MID_MAX_ROWS
-            and ops.mid_runs(self.out_features, self.in_features) > 0
-        )
+        rows = x.shape[0]
+        if self.weight.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or rows <= ops.SKINNY_MAX_ROWS:
+            return False
+        if rows <= ops.MID_MAX_ROWS and ops.mid_runs(self.out_features, self.in_features) > 0:
+            return True
+        return ops.block_plan(rows, self.out_features, self.in_features, "runs") is not None
 
     def partial_sums(self, x: torch.Tensor) -> torch.Tensor:
         """``[runs, M, out]`` float32 whose sum over the runs is ``x W^T`` (without the bias)."""
@@ -75,8 +76,8 @@ class Linear:
 
     def deferred(self, x: torch.Tensor, ctx=None):
         """The product, or a :class:`DeferredProduct` of it where one of this product's kernels
-        could fold a neighbouring norm into itself (bfloat16, up to 16 rows, or 17 to 192 rows of a
-        narrow matrix), or where it has a bias, which the kernel that adds the product to the
+        could fold a neighbouring norm into itself (bfloat16, up to 16 rows, or more of a
+        narrow matrix, see :meth:`midsize`), or where it has a bias, which the kernel that adds the product to the
         residual can add.  Whoever receives it and has no use for that simply materialises it."""
         if isinstance(x, torch.Tensor) and (self.bias is not None or self.folds(x)):
             return DeferredProduct(self, x)

@@ -1112,6 +1112,88 @@ def test_product_in_runs_of_k_and_the_norm_that_adds_them(shape):
     assert torch.equal(res2, got_res) and torch.equal(out2, out)
 
 
+# rows, result columns, K: one chunk of 64 k and fewer chunks than a tile has buffers for, an odd number of them and
+# many; rows and columns that end inside a piece of 64, inside a tile and at its edge; more tiles than dies, and counts
+# that the dies do not share evenly
+BLOCK_SHAPES = [(1, 8, 64), (65, 72, 128), (128, 256, 192), (257, 520, 320), (300, 1032, 1024), (700, 264, 4160)]
+
+
+@pytest.mark.parametrize("shape", BLOCK_SHAPES)
+@pytest.mark.parametrize("nw,nx", [(4, 4), (3, 4), (2, 4), (4, 2), (3, 2), (2, 2)])
+def test_many_row_product_every_tile(nw, nx, shape):
+    """Every tile of the many-row product, called directly: float32 runs of K, whole and cut, and the gated form;
+    rows and columns behind the result stay as they were, and a row that is not finite stays alone."""
+    ops = _ops()
+    m, n, k = shape
+    gen = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn((m, k), generator=gen).bfloat16()
+    w = (torch.randn((2 * n, k), generator=gen) / math.sqrt(k)).bfloat16()
+    x[m - 1], w[n - 1], w[2 * n - 1] = 1.0, 3.0 / math.sqrt(k), -2.0 / math.sqrt(k)  # clamped or dropped edges show
+    exact = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    xd, wd = x.to(DEV), w.to(DEV)
+
+    def run(kind, rows, cols, splits, x=xd):
+        dtype = torch.bfloat16 if kind == 2 else torch.float32
+        out = torch.full((splits * rows + 3, n + 8), 7.0, dtype=dtype, device=DEV)
+        code = ops.core().rl_gemm_block(ops._p(x), ops._p(wd), ops._p(out), rows, cols, k, k, k, n + 8, kind, nw, nx, splits, ops._stream())
+        assert code == 0
+        assert torch.all(out[splits * rows:] == 7.0) and torch.all(out[:, cols:] == 7.0)
+        return out[: splits * rows, :cols]
+
+    for splits in (1, 2, 3):
+        chunks = k // 64
+        if -(-chunks // splits) * (splits - 1) >= chunks:
+            continue
+        got = run(1, m, n, splits).view(splits, m, n).double().sum(0).cpu()
+        # k additions, each rounded once, of partial sums of at most the operands' sizes
+        assert torch.all((got - exact[:, :n]).abs() <= k * 2.0**-24 * size[:, :n])
+    gate, up = exact[:, :n].bfloat16().double(), exact[:, n:].bfloat16().double()
+    want = gate * torch.sigmoid(gate) * up
+    got = run(2, m, n, 1)
+    # gate and up may each be rounded the other way (a step of 2^-8; silu grows by at most 1.1 a unit), the result is rounded
+    bound = 2.0**-8 * (1.1 * (gate * up).abs() + 2 * want.abs()) + 1e-6
+    assert torch.all((got.double().cpu() - want).abs() <= bound)
+    assert torch.equal(run(2, m, n, 1), got)
+    if m > 1:
+        bad = xd.clone()
+        bad[0] = float("inf")
+        other = run(2, m, n, 1, bad)
+        assert not torch.isfinite(other[0]).any() or n < 64
+        assert torch.equal(other[1:], got[1:])
+
+
+@pytest.mark.parametrize("m,n,k,kind", [(65, 4096, 12288, "runs"), (520, 2560, 9728, "runs"), (129, 2048, 6144, "runs"),
+                                        (65, 4096, 512, "gated"), (129, 3072, 1024, "gated"), (1100, 1032, 320, "gated")])
+def test_many_row_product_through_its_rule(m, n, k, kind):
+    """What the launch rule gives the many-row product, through the entry points that the layers call; a weight that begins inside
+    a unit of 16 bytes gives the same."""
+    ops = _ops()
+    plan = ops.block_plan(m, n, k, kind)
+    assert plan is not None
+    gen = torch.Generator().manual_seed(m)
+    x = torch.randn((m, k), generator=gen).bfloat16().to(DEV)
+    rows = 2 * n if kind == "gated" else n
+    room = (torch.randn(rows * k + 1, generator=gen) / math.sqrt(k)).bfloat16().to(DEV)
+    w, odd = room[:-1].view(rows, k), torch.cat([room[:1], room])[1:-1].view(rows, k)
+    odd.copy_(w)
+    assert odd.data_ptr() % 16
+    if kind == "runs":
+        parts = ops.gemm_bf16_parts(x, w)
+        assert parts.shape == (plan[2], m, n) and torch.equal(ops.gemm_bf16_parts(x, odd), parts)
+        got, want = parts.sum(0), x.float() @ w.float().T
+        torch.testing.assert_close(got, want, rtol=0, atol=k * 2.0**-24 * float((x.float().abs() @ w.float().abs().T).max()))
+        return
+    before = ops.library_products
+    got = ops.gemm_bf16_swiglu(x, w)
+    assert got is not None and ops.library_products == before
+    assert ops.gemm_bf16_swiglu(x, odd) is None or ops._tile_applies(m, rows, k, n)
+    gu = x.float() @ w.float().T
+    gate, up = gu[:, :n].bfloat16().float(), gu[:, n:].bfloat16().float()
+    want = torch.nn.functional.silu(gate) * up
+    assert torch.all((got.float() - want).abs() <= 2.0**-8 * (1.1 * (gate * up).abs() + 2 * want.abs()) + 1e-6)
+
+
 # rows, result columns, K, SwiGLU, float32 result: every number of tiles a workgroup may hold
 # (1, 2, 3, 6 tiles; 2, 3, 5 pairs), shares that leave some workgroups a tile short, more tiles
 # than one round of workgroups holds (the vocabulary), 17 to 64 rows around the blocks of 16,

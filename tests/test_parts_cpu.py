@@ -174,6 +174,32 @@ def test_which_products_run_in_one_launch_of_this_package():
     assert not ops._tile_applies(64, 4098, 1024, 4098)    # four result columns a lane
 
 
+def test_where_the_many_row_product_applies():
+    """The rule of the many-row product on the chip it was measured on: what it takes, the tiles at both ends
+    of its range, runs of K that all hold a chunk, and what stays where it was."""
+    from rapid_llm_amd.kernels import ops
+
+    plan = lambda *a: ops.block_plan(*a, units=256)
+    assert plan(512, 12288, 4096, "gated") == (3, 4, 1)    # 256 tiles of 192 x 256: one a compute unit
+    assert plan(2048, 12288, 4096, "gated") == (4, 4, 1)
+    assert plan(160, 3072, 1024, "gated") == (2, 2, 1)     # few rows: as many workgroups as there can be
+    assert plan(64, 12288, 4096, "gated") is None          # the kernel for up to 64 rows
+    assert plan(512, 12288, 4100, "gated") is None and plan(512, 12290, 4096, "gated") is None
+    assert plan(90000, 12288, 12288, "gated") is None      # offsets beyond 31 bits
+    assert plan(2048, 4096, 4096, "runs") is None          # short sums: the library's
+    assert plan(2049, 4096, 12288, "runs") is None and plan(2048, 4096, 12288, "runs") == (4, 4, 2)
+    assert plan(128, 2048, 6144, "runs") is None and plan(129, 2048, 6144, "runs") is not None
+    assert plan(1025, 2048, 6144, "runs") is None
+    for m in (65, 100, 300, 777, 1024):
+        for n, k in ((4096, 12288), (2560, 9728), (2048, 6144), (8, 8192)):
+            found = plan(m, n, k, "runs")
+            if found is None:
+                assert k < 8192
+                continue
+            per = -(-(k // 64) // found[2])
+            assert per * (found[2] - 1) < k // 64
+
+
 def test_launch_rules_follow_the_number_of_compute_units():
     """Every launch rule takes the chip's geometry from one place on the host
     (``ops.chip()``; without a device the chip the rules were measured on), so that a part
