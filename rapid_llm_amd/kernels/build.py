@@ -48,6 +48,7 @@ CORE_SOURCES = (
     "gemm_bf16.hip",
     "gemm_rows.hip",
     "gemm_block.hip",
+    "repeat.hip",
     "latent.hip",
     "router.hip",
     "sublayer_sum.hip",

@@ -1,0 +1,119 @@
+"""The launches of a piece of a step, noted while they are made, so that they can be made again for
+layers that differ in nothing but their tensors (``ops.repeat_launches``).
+
+Notes are a thread's own and live for the piece alone.  They keep every tensor that a noted launch was
+given: the launches are made again with the same temporary tensors, which must not have gone to
+somebody else meanwhile."""
+
+from __future__ import annotations
+
+import bisect
+import contextlib
+import ctypes
+import threading
+
+import numpy as np
+import torch
+
+# as csrc/repeat.hip lays them out
+MAX_INTS, MAX_FLOATS = 32, 8
+_CALL = np.dtype([("entry", "<i8"), ("ints", "<i8", (MAX_INTS,)), ("floats", "<f4", (MAX_FLOATS,))], align=True)
+
+
+class _Thread(threading.local):
+    notes: "Notes | None" = None
+
+
+noting = _Thread()
+
+
+class _Library:
+    """A compiled library whose calls are noted."""
+
+    def __init__(self, notes: "Notes", lib: ctypes.CDLL) -> None:
+        self._notes, self._lib = notes, lib
+
+    def __getattr__(self, name: str):
+        entry = getattr(self._lib, name)
+
+        def call(*args):
+            self._notes.last = (entry, args)
+            return entry(*args)
+
+        return call
+
+
+class Notes:
+    def __init__(self) -> None:
+        self.calls: list[tuple] = []  # (the library's function, its arguments), as made
+        self.tensors: list[torch.Tensor | None] = []
+        self.last: tuple | None = None
+        self.complete = True
+
+    def library(self, lib: ctypes.CDLL) -> _Library:
+        return _Library(self, lib)
+
+    def made(self, what: str) -> None:
+        """The call just made was a launch (calls that only ask a library something are not reported)."""
+        if self.last is None:
+            self.complete = False  # of a library whose calls are not noted
+        else:
+            self.calls.append(self.last)
+            self.last = None
+
+    def plan(self, tables, carried):
+        """(calls, slots, table of pointers) for ``rl_repeat_calls``, or ``None`` where a call does not fit."""
+        if not self.complete or not self.calls:
+            return None
+        table = np.array([[t.data_ptr() for t in row] for row in tables], dtype=np.int64)
+        column: dict[int, tuple[int, int]] = {}
+        spans = []
+        for back, row in ((1, tables[0]), (0, tables[1])):
+            for j, t in enumerate(row):
+                at = int(table[1 - back, j])
+                if at in column:
+                    return None  # two layers share it: a pointer does not say whose it is
+                column[at] = (j, back)
+                spans.append((at, at + t.numel() * t.element_size()))
+        spans.sort()
+        starts = [s for s, _ in spans]
+        before, after = (t.data_ptr() for t in carried)
+        calls = np.zeros(len(self.calls), dtype=_CALL)
+        slots = []
+        for c, (entry, args) in enumerate(self.calls):
+            ints, floats = [], []
+            for arg in args:
+                if arg is None or isinstance(arg, ctypes.c_void_p):
+                    value = 0 if arg is None else arg.value or 0
+                    if value in column:
+                        slots.append((c, len(ints), *column[value]))
+                    elif value == before:
+                        value = after
+                    elif value:
+                        i = bisect.bisect_right(starts, value) - 1
+                        if i >= 0 and value < spans[i][1]:
+                            return None
+                    ints.append(value)
+                elif isinstance(arg, ctypes.c_float):
+                    floats.append(arg.value)
+                elif isinstance(arg, int):
+                    ints.append(int(arg))
+                else:
+                    return None
+            if len(ints) > MAX_INTS or len(floats) > MAX_FLOATS:
+                return None
+            calls[c]["entry"] = ctypes.cast(entry, ctypes.c_void_p).value
+            calls[c]["ints"][: len(ints)] = ints
+            calls[c]["floats"][: len(floats)] = floats
+        return calls, np.array(slots, dtype=np.int32).reshape(-1, 4), table
+
+
+@contextlib.contextmanager
+def taking_notes():
+    """Note the launches that this thread makes inside the block."""
+    outer, notes = noting.notes, Notes()
+    noting.notes = notes
+    try:
+        yield notes
+    finally:
+        noting.notes = outer

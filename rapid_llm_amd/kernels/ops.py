@@ -15,6 +15,7 @@ from typing import Optional
 import torch
 
 from . import build
+from .notes import Notes, noting
 from .upload import upload_ints
 
 F32, BF16 = 0, 1
@@ -72,7 +73,8 @@ def core() -> ctypes.CDLL:
     global _core
     if _core is None:
         _core = build.load(build.core_library())
-    return _core
+    notes = noting.notes
+    return _core if notes is None else notes.library(_core)
 
 
 def attention_lib(head_dim: int) -> ctypes.CDLL:
@@ -84,7 +86,8 @@ def attention_lib(head_dim: int) -> ctypes.CDLL:
         if lib.rl_attn_f32_span() != _F32_SPAN:
             raise KernelError(f"the float32 attention walks spans of {lib.rl_attn_f32_span()} keys, the launch rules expect {_F32_SPAN}")
         _attn[head_dim] = lib
-    return lib
+    notes = noting.notes
+    return lib if notes is None else notes.library(lib)
 
 
 _attn_tile: dict[tuple[int, int], ctypes.CDLL] = {}
@@ -145,6 +148,9 @@ def _stream() -> ctypes.c_void_p:
 
 
 def _p(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
+    notes = noting.notes
+    if notes is not None:
+        notes.tensors.append(t)
     return ctypes.c_void_p(0 if t is None else t.data_ptr())
 
 
@@ -172,9 +178,31 @@ def _need(t: torch.Tensor, name: str, dtype: torch.dtype | None = None, shape=No
 
 
 def _ok(code: int, what: str) -> None:
+    if noting.notes is not None:
+        noting.notes.made(what)
     if code != 0:
         reason = {1: "an argument the kernel refuses", 2: "the launch failed"}.get(code, "unknown")
         raise KernelError(f"{what}: error {code} ({reason})")
+
+
+def repeat_launches(notes: Notes, tables: list[list[torch.Tensor]], carried: tuple[torch.Tensor, torch.Tensor]) -> bool:
+    """Make the launches that ``notes`` holds, those of place 1 of a run order, again for the places behind it, from
+    native code.  ``tables``: every place's own tensors (weights, pages), one row a place, alike in shape and type;
+    what place 1 took from place 0's row, place i takes from place i - 1's.  ``carried``: the tensor that place 1
+    read of what place 0 left, and the one in its stead that it left itself.  False, with nothing launched, where the
+    launches do not say which layer they are of (a pointer into the middle of a tensor)."""
+    plan = notes.plan(tables, carried)
+    if plan is None:
+        return False
+    calls, slots, table = plan
+    _ok(
+        core().rl_repeat_calls(
+            ctypes.c_void_p(calls.ctypes.data), len(calls), ctypes.c_void_p(slots.ctypes.data), len(slots),
+            ctypes.c_void_p(table.ctypes.data), table.shape[1], 2, len(tables),
+        ),
+        "a repeated launch",
+    )
+    return True
 
 
 # --------------------------------------------------------------------------- #
@@ -694,7 +722,7 @@ def qknorm_rope_kvwrite(
         raise KernelError(f"a query temperature needs written queries and a positive step, got {query_temperature}")
     _ok(
         core().rl_qknorm_rope_kvwrite(
-            ctypes.c_void_p(qkv.data_ptr() + col0 * qkv.element_size()), _p(q_out), _p(k_cache), _p(v_cache), _p(q_norm_w), _p(k_norm_w), _p(cos),
+            _column(qkv, col0), _p(q_out), _p(k_cache), _p(v_cache), _p(q_norm_w), _p(k_norm_w), _p(cos),
             _p(sin), _p(positions), _p(token_slot), _p(block_table), block_table.stride(0),
             page_size, tokens, nq, nkv, d, half, ROTARY_PAIRINGS[pairing], ctypes.c_float(eps), int(write),
             row_width, value_col0, dv, _p(bias), ctypes.c_float(coef), ctypes.c_float(every), int(bool(norm_values)),
@@ -734,7 +762,7 @@ def _out_columns(out: torch.Tensor, dtype: torch.dtype, tokens: int, width: int,
 
 
 def _column(t: torch.Tensor, col: int) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr() + col * t.element_size())
+    return ctypes.c_void_p(_p(t).value + col * t.element_size())
 
 
 def attention_generic(

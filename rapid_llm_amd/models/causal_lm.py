@@ -13,6 +13,7 @@ from dataclasses import replace
 import torch
 
 from ..kernels import ops
+from ..kernels.notes import taking_notes
 from ..parts.base import (
     BLOCKS,
     EMBEDDINGS,
@@ -25,9 +26,14 @@ from ..parts.base import (
     ParamSpec,
 )
 from ..parts.inject import StreamMix
-from ..parts.lazy import plain, run_norm, settle
+from ..parts.lazy import DeferredProduct, plain, run_norm, settle
 from ..parts.offsets import StreamOffsetTable
 from .spec import ModelSpec
+
+
+# Tokens up to which a step's layers behind the second are launched from what the second launched: beyond, the device has
+# more to do than the host in any model, and the noted layer keeps its temporary tensors until all are launched
+REPEAT_MAX_TOKENS = 2048
 
 
 class CausalLM:
@@ -161,6 +167,33 @@ class CausalLM:
         return needs
 
     # ---- step ------------------------------------------------------------------
+    def _alike(self, ctx, caches) -> bool:
+        """Whether every layer's launches of this step are the second one's with the layer's own tensors."""
+        if ctx.num_tokens > REPEAT_MAX_TOKENS or len(self.order) < 4 or "decode_only_tokens" in ctx.static:
+            return False
+        if self.offsets is not None or self.mixes is not None or self.returns:
+            return False
+        first = self.blocks[self.order[0]].launch_signature()
+        if first is None or any(self.blocks[li].launch_signature() != first for li in self.order[1:]):
+            return False
+        kinds = {(c.group_id, c.page_size, c.owns_pages, len(c.pages), len(c.states)) for c in caches}
+        return len(kinds) == 1 and all(c.owns_pages and not c.states for c in caches)
+
+    def _repeat(self, notes, delta, left, caches):
+        """The layers behind the second, launched from the notes of the second's launches; ``delta`` is what the first
+        left for it, ``left`` what it left itself.  Returns what the last layer leaves, ``None`` if nothing was launched."""
+        lazy = isinstance(left, DeferredProduct)
+        if type(left) is not type(delta) or not (lazy or isinstance(left, torch.Tensor)):
+            return None
+        before, after = (delta.x, left.x) if lazy else (delta, left)
+        if before.shape != after.shape or before.dtype != after.dtype:
+            return None
+        tables = [self.blocks[li].own_tensors() + list(cache.pages.values()) for li, cache in zip(self.order, caches)]
+        kinds = [[(t.shape, t.dtype) for t in row] for row in tables]
+        if any(k != kinds[0] for k in kinds[1:]) or not ops.repeat_launches(notes, tables, (before, after)):
+            return None
+        return DeferredProduct(self.blocks[self.order[-1]].feed_forward.last_product, after) if lazy else after
+
     def forward(self, ctx, caches) -> torch.Tensor:
         """Run the tokens of ``ctx`` through every layer (which writes their keys and values)
         and return float32 logits ``[len(ctx.logit_rows), vocab]``."""
@@ -169,8 +202,19 @@ class CausalLM:
         # in place)
         first = residual.clone() if self.mixes is not None or self.returns else None
         delta = None
+        alike = self._alike(ctx, caches)
         for place, li in enumerate(self.order):
             block = self.blocks[li]
+            if alike and place == 1:
+                products = ops.library_products
+                with taking_notes() as notes:
+                    left = block.forward(residual, delta, ctx, caches[1])
+                    last = self._repeat(notes, delta, left, caches) if ops.library_products == products else None
+                if last is not None:
+                    delta = last
+                    break
+                delta = left
+                continue
             if self.mixes is not None and self.mixes.at(place):
                 delta = settle(residual, delta)
                 if delta is not None:

@@ -322,6 +322,19 @@ class GQAAttention(PackedMixer):
     def accepts_scaled_rows(self) -> bool:
         return self.qkv.takes_scaled_rows()
 
+    def launch_signature(self):
+        # plain attention alone: the other forms, and kinds derived from this one, may do more
+        if type(self) is not GQAAttention or not self.plain_row:
+            return None
+        return (self.hidden_size, self.nq, self.nkv, self.d, self.window, self.scale, self.qk_norm_eps,
+                self.qkv_bias, self.o_bias, id(self.position))
+
+    def own_tensors(self) -> list[torch.Tensor]:
+        norms = [w for w in (self.q_norm_w, self.k_norm_w) if w is not None]
+        if not self.qk_norm_weights:
+            norms = norms[:1]  # one vector of ones for both
+        return self.qkv.own_tensors() + self.o.own_tensors() + norms
+
     def run(self, packed, col0, out, out_col, out_scale, ctx, cache):
         """The heads between the two products (layers with one of the options beyond plain attention)."""
         pos_enc = self.position

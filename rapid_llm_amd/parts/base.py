@@ -217,6 +217,17 @@ class Part:
     #: of unlike length (such steps are then recorded for themselves); 0: it does not.
     deals_ragged_contexts = 0
 
+    def launch_signature(self) -> "tuple | None":
+        """What two parts of different layers have in common if their ``forward`` makes the same launches in every step,
+        with nothing but their :meth:`own_tensors` (and a cache's pages) in the place of one another's, and does
+        nothing else on the device: the launches of one are then made again for the other without running its
+        ``forward``.  ``None``: no such promise."""
+        return None
+
+    def own_tensors(self) -> "list[torch.Tensor]":
+        """The tensors of this part alone that its launches point at, each at its beginning."""
+        return []
+
     def param_specs(self) -> list[ParamSpec]:
         return []
 

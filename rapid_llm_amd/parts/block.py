@@ -30,6 +30,15 @@ class PreNormBlock(Block):
             return (self.mixer_norm, self.mixer)
         return (self.mixer_norm, self.mixer, self.feed_forward_norm, self.feed_forward)
 
+    def launch_signature(self):
+        if type(self) is not PreNormBlock or self.feed_forward is None or not hasattr(self.feed_forward, "last_product"):
+            return None
+        signatures = tuple(p.launch_signature() for p in self.parts())
+        return None if None in signatures else signatures
+
+    def own_tensors(self):
+        return [t for p in self.parts() for t in p.own_tensors()]
+
     def forward(self, residual, delta, ctx, cache):
         x = run_norm(self.mixer_norm, residual, delta, ctx, consumer=self.mixer)
         a = self.mixer.forward(x, ctx, cache)

@@ -42,6 +42,10 @@ class Linear:
         self.weight = weight
         self.bias = bias
 
+    def own_tensors(self) -> list[torch.Tensor]:
+        """What a launch of this product may point at that is its own."""
+        return [t for t in (self.weight, self.bias) if t is not None]
+
     # ---- folding a neighbouring norm into the product (decode steps, bfloat16) ----------
     def skinny(self, x) -> bool:
         """Whether ``x`` runs through the hand-written few-row kernel, which has the epilogues."""

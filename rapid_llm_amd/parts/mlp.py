@@ -81,6 +81,20 @@ class SwiGLU(FeedForward):
     def accepts_scaled_rows(self) -> bool:
         return self.gate_up.takes_scaled_rows()
 
+    def launch_signature(self):
+        if type(self) is not SwiGLU:  # a kind derived from this one may do more
+            return None
+        return (self.hidden_size, self.intermediate_size, self.limit, self.alpha, self.activation, self.has_bias)
+
+    def own_tensors(self) -> list[torch.Tensor]:
+        # the bias of gate and up is added by the activation
+        bias = [self.gate_up_bias] if self.has_bias else []
+        return self.gate_up.own_tensors() + self.down.own_tensors() + bias
+
+    @property
+    def last_product(self) -> Linear:
+        return self.down
+
     def forward(self, x, ctx):
         w = self.gate_up.weight
         if w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16:

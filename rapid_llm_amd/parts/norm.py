@@ -53,6 +53,14 @@ class RMSNorm(Norm):
             self.weight = self.weight.reshape(1).expand(self.size).contiguous()
         self.dtype = runtime.dtype
 
+    def launch_signature(self):
+        if type(self) is not RMSNorm:  # a kind derived from this one may do more
+            return None
+        return (self.size, self.eps, self.dtype)
+
+    def own_tensors(self) -> list[torch.Tensor]:
+        return [self.weight]
+
     def forward(self, residual, delta, ctx, rows=None, scaled_ok=False):
         if isinstance(delta, NormedDelta):
             # the sub-layer's own norm, the add and this norm in one kernel

@@ -1,0 +1,78 @@
+"""Steps whose layers behind the second are launched from the second's notes: bit for bit what the layers'
+own code launches, in every kind of step, and only where the layers are alike."""
+
+import pytest
+import torch
+
+from tiny_configs import random_tokens
+
+pytestmark = pytest.mark.gpu
+
+BASE = dict(
+    architectures=["Qwen3ForCausalLM"], model_type="qwen3", num_hidden_layers=5, hidden_size=256, num_attention_heads=4,
+    num_key_value_heads=2, head_dim=64, intermediate_size=512, vocab_size=277, rope_theta=30000.0, rms_norm_eps=1e-5,
+    tie_word_embeddings=False, max_position_embeddings=1024, hidden_act="silu", attention_bias=False,
+)
+# request -> its portions: single tokens eager and few rows of a prompt (norms inside the products), tens of rows (runs
+# of K), a hundred and more, single tokens beside portions, a portion of a long prompt (its keys in runs)
+STEPS = [{"a": 5}, {"a": 1, "b": 11}, {"a": 1, "b": 1}, {"c": 40, "a": 1}, {"d": 150, "b": 30, "c": 1},
+         {"e": 640}, {"e": 130, "a": 1, "b": 1}]
+
+
+def _run(runner, most, monkeypatch):
+    from rapid_llm_amd import StepEntry
+    from rapid_llm_amd.kernels import ops
+    from rapid_llm_amd.models import causal_lm
+
+    ran = []
+    real = ops.repeat_launches
+    monkeypatch.setattr(causal_lm, "REPEAT_MAX_TOKENS", most)
+    monkeypatch.setattr(ops, "repeat_launches", lambda *a: ran.append(real(*a)) or ran[-1])
+    done, logits = {}, []
+    for i, step in enumerate(STEPS):
+        entries = []
+        for rid, n in step.items():
+            tokens = random_tokens(n, runner.vocab_size, 100 * i + ord(rid))
+            entries.append(StepEntry(rid, tokens, [n - 1]))
+            done[rid] = done.get(rid, 0) + n
+        logits.append(runner.step(entries, use_graph=False).clone())
+    for rid in done:
+        runner.finish(rid)
+    monkeypatch.setattr(ops, "repeat_launches", real)
+    return logits, ran
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("change", [{}, {"head_dim": 48, "num_attention_heads": 6, "hidden_size": 200},
+                                    {"head_dim": 128, "num_hidden_layers": 4, "num_attention_heads": 12, "intermediate_size": 2048}],
+                         ids=["d64", "d48", "d128"])
+def test_repeated_layers_are_the_layers(dtype, change, monkeypatch):
+    from rapid_llm_amd import EngineConfig, ModelRunner
+
+    engine = EngineConfig(dtype=dtype, max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8)
+    runner = ModelRunner({**BASE, **change}, engine, load_format="random", weight_norm_std=0.1)
+    want, none = _run(runner, 0, monkeypatch)
+    got, ran = _run(runner, 2048, monkeypatch)
+    # (a step with a product of the library's is launched by the layers; float32 has none, and the widths of the
+    # last shape keep to this package's products up to 192 rows)
+    least = 7 if dtype == "float32" else 6 if runner.config.head_dim == 128 else 3
+    assert not none and ran == [True] * len(ran) and len(ran) >= least
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    # weights that are other tensors now are the ones that are read
+    runner.model.blocks[3].feed_forward.down.weight = torch.zeros_like(runner.model.blocks[3].feed_forward.down.weight)
+    want, got = _run(runner, 0, monkeypatch)[0], _run(runner, 2048, monkeypatch)[0]
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+def test_layers_that_differ_are_not_repeated(monkeypatch):
+    from rapid_llm_amd import EngineConfig, ModelRunner
+
+    body = {**BASE, "sliding_window": 40, "layer_types": ["full_attention"] * 4 + ["sliding_attention"]}
+    runner = ModelRunner(body, EngineConfig(dtype="bfloat16", max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
+                         load_format="random")
+    assert _run(runner, 2048, monkeypatch)[1] == []
+    few = ModelRunner({**BASE, "num_hidden_layers": 3}, EngineConfig(dtype="bfloat16", max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
+                      load_format="random")
+    assert _run(few, 2048, monkeypatch)[1] == []

@@ -1,0 +1,101 @@
+"""Calls noted and made again from native code: arguments of every kind in any order, pointers out of the table."""
+
+import ctypes
+
+import pytest
+import torch
+
+from rapid_llm_amd.kernels import notes as notes_module
+from rapid_llm_amd.kernels import ops
+
+I, F, P = ctypes.c_int, ctypes.c_float, ctypes.c_void_p
+
+
+def _entry(log, kinds):
+    def body(*args):
+        log.append(args)
+        return 0
+
+    return ctypes.CFUNCTYPE(I, *kinds)(body)
+
+
+class _Lib:
+    def __init__(self, **entries):
+        self.__dict__.update(entries)
+
+
+def _noted(lib, name, *args):
+    with notes_module.taking_notes() as notes:
+        getattr(notes.library(lib), name)(*args)
+        ops._ok(0, name)
+    return notes
+
+
+def _again(notes, tables, carried):
+    plan = notes.plan(tables, carried)
+    assert plan is not None
+    calls, slots, table = plan
+    at = lambda a: P(a.ctypes.data)
+    return ops.core().rl_repeat_calls(at(calls), len(calls), at(slots), len(slots), at(table), table.shape[1], 2, len(tables))
+
+
+def test_calls_are_made_again_with_every_layers_tensors():
+    # more integers than there are registers, floats between them, and as many of each as there may be
+    kinds = [P, I, F, P, P, I, F, I, P, I, I, F, I, I, I, I, F, P, I, F, F, F, I, I, I, I, I, I, I, I, I, I, I, I, I, F, I, I, I, P]
+    assert sum(k is not F for k in kinds) == notes_module.MAX_INTS and sum(k is F for k in kinds) == notes_module.MAX_FLOATS
+    log = []
+    lib = _Lib(rl_x=_entry(log, kinds))
+    layers = [[torch.zeros(8), torch.zeros(3)] for _ in range(5)]
+    x0, x1, other = torch.zeros(4), torch.zeros(4), torch.zeros(9)
+    values = []
+    for n, k in enumerate(kinds):
+        values.append(F(n + 0.5) if k is F else P(other.data_ptr()) if k is P else -n if n % 2 else n)
+    values[0], values[3], values[4], values[8] = (P(t.data_ptr()) for t in (layers[1][0], layers[0][1], x0, layers[1][1]))
+    values[17] = None
+    notes = _noted(lib, "rl_x", *values)
+    assert _again(notes, layers, (x0, x1)) == 0
+    assert len(log) == 4
+    for place, args in enumerate(log[1:], start=2):
+        want = list(log[0])
+        want[0], want[3], want[4], want[8] = (t.data_ptr() for t in (layers[place][0], layers[place - 1][1], x1, layers[place][1]))
+        assert list(args) == want
+
+
+def test_a_call_that_fails_ends_it():
+    log = []
+    fail = ctypes.CFUNCTYPE(I, I)(lambda n: log.append(n) or (7 if len(log) > 2 else 0))
+    notes = _noted(_Lib(rl_x=fail), "rl_x", 5)
+    layers = [[torch.zeros(2)] for _ in range(9)]
+    assert _again(notes, layers, (torch.zeros(1), torch.zeros(1))) == 7 and log == [5, 5, 5]
+
+
+@pytest.mark.parametrize("why", ["inside", "shared", "argument", "many", "unknown"])
+def test_what_cannot_be_made_again(why):
+    layers = [[torch.zeros(8)] for _ in range(4)]
+    lib = _Lib(rl_x=lambda *a: 0)
+    args = [P(layers[1][0].data_ptr())]
+    if why == "inside":
+        args = [P(layers[0][0].data_ptr() + 4)]  # the middle of a layer's tensor
+    if why == "shared":
+        layers[1][0] = layers[0][0]
+    if why == "argument":
+        args.append(1.5)  # neither a pointer nor an integer nor a float of the kernels' width
+    if why == "many":
+        args += [1] * notes_module.MAX_INTS
+    notes = _noted(lib, "rl_x", *args)
+    if why == "unknown":
+        with notes_module.taking_notes() as notes:
+            ops._ok(0, "a launch of a library that is not noted")
+    assert notes.plan(layers, (torch.zeros(1), torch.zeros(1))) is None
+
+
+def test_notes_end_with_their_block_and_are_the_threads_own():
+    import threading
+
+    seen = []
+    with notes_module.taking_notes():
+        t = threading.Thread(target=lambda: seen.append(notes_module.noting.notes))
+        t.start()
+        t.join()
+        assert notes_module.noting.notes is not None
+    assert seen == [None] and notes_module.noting.notes is None
