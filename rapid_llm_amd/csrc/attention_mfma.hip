@@ -261,8 +261,12 @@ __device__ inline void prepared_query(bf16x8 (&qf)[DC], const bf16_t* qrow, bool
 // before anyone reads them (rapid_llm/modules/attention.py:126-138), so that a decode step
 // needs no separate kernel for that.  Needs D % 64 == 0: a lane then holds both channels of
 // every rotation pair.
-template <bool V16, bool FUSED>
-__global__ __launch_bounds__(DEC_WAVES* RL_WAVE) void attn_decode_kernel(
+//
+// WAVES: four, or two where contexts are so short and requests so few that units would be idle (ops._decode_short has
+// the figures).  More than four lose: a unit takes keys only so fast, and one request of 300 keys of the Qwen3-0.6B shape in
+// one workgroup a kv head of eight or twelve waves, without a merge, took 1,066 and 1,095 us a step against 1,003.
+template <bool V16, bool FUSED, int WAVES>
+__global__ __launch_bounds__(WAVES* RL_WAVE) void attn_decode_kernel(
     const bf16_t* __restrict__ q, const bf16_t* k_cache, const bf16_t* v_cache,
     bf16_t* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, const int* __restrict__ seq_token,
@@ -270,9 +274,9 @@ __global__ __launch_bounds__(DEC_WAVES* RL_WAVE) void attn_decode_kernel(
     const int* __restrict__ token_slot, const int* __restrict__ block_table, int table_stride,
     int page_size, int nq, int nkv, int window, float scale_log2, int split_chunk, int nsplit,
     DecodeExtra ex) {
-    __shared__ float lds_o[DEC_WAVES / 2][D * 16];
-    __shared__ float lds_m[DEC_WAVES / 2][16];
-    __shared__ float lds_l[DEC_WAVES / 2][16];
+    __shared__ float lds_o[WAVES / 2][D * 16];
+    __shared__ float lds_m[WAVES / 2][16];
+    __shared__ float lds_l[WAVES / 2][16];
     __shared__ int lds_pages[DEC_MAX_PAGES + 2];
 
     const int G = nq / nkv;
@@ -301,12 +305,12 @@ __global__ __launch_bounds__(DEC_WAVES* RL_WAVE) void attn_decode_kernel(
     const int kstart = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
     // The launch has nsplit splits of at most split_chunk keys, laid out for the longest context
     // it may meet (a recorded step serves every context of its bucket).  This request's keys are
-    // dealt to the splits evenly: runs of a multiple of 32 keys, at least 128 (shorter runs only
-    // add merge work), never more than split_chunk (the page ids of a run are staged in LDS).
+    // dealt to the splits evenly: runs of a multiple of 32 keys, at least one step of every wave (shorter
+    // runs only add merge work), never more than split_chunk (the page ids of a run are staged in LDS).
     // nsplit * split_chunk covers the longest context, so the runs cover this one.
     const int first = kstart & ~31;
     int run = ((kend - first + nsplit - 1) / nsplit + 31) & ~31;
-    run = min(max(run, 128), split_chunk);
+    run = min(max(run, 32 * WAVES), split_chunk);
     const int lo = first + split * run;
     const int hi = min(kend, lo + run);
 
@@ -326,7 +330,7 @@ __global__ __launch_bounds__(DEC_WAVES* RL_WAVE) void attn_decode_kernel(
         const int page0 = lo / page_size;
         {
             const int npages = last_key / page_size - page0 + 1;
-            for (int i = threadIdx.x; i < npages && i < DEC_MAX_PAGES + 2; i += DEC_WAVES * RL_WAVE)
+            for (int i = threadIdx.x; i < npages && i < DEC_MAX_PAGES + 2; i += WAVES * RL_WAVE)
                 lds_pages[i] = table[page0 + i];
         }
         const bf16_t* qrow = q + (size_t)t * ex.qkv_stride + (size_t)head * D;
@@ -403,7 +407,7 @@ __global__ __launch_bounds__(DEC_WAVES* RL_WAVE) void attn_decode_kernel(
         // 16,000 keys 95.5 -> 94.0); forcing four waves a SIMD spills and loses again.
         DecodeFrags cur;
         int base = lo + 32 * wave;
-        for (; base < hi; base += 32 * DEC_WAVES) {
+        for (; base < hi; base += 32 * WAVES) {
             decode_load<V16>(cur, k_cache, v_cache, lds_pages, page0, page_size, nkv, hk, base,
                              last_key, col, g);
             // ---- S^T = K Q^T for two blocks of 16 keys --------------------------------
@@ -470,9 +474,9 @@ __global__ __launch_bounds__(DEC_WAVES* RL_WAVE) void attn_decode_kernel(
             l = l * f1 + l_o * f2;
             m = mm;
         };
-        // waves [s, 2s) hand their state to waves [0, s), for s = DEC_WAVES / 2, .., 1
+        // waves [s, 2s) hand their state to waves [0, s), for s = WAVES / 2, .., 1
 #pragma unroll
-        for (int s = DEC_WAVES / 2; s >= 1; s >>= 1) {
+        for (int s = WAVES / 2; s >= 1; s >>= 1) {
             if (wave >= s && wave < 2 * s) put(wave - s);
             __syncthreads();
             if (wave < s) take(wave);
@@ -565,7 +569,7 @@ extern "C" int rl_attn_decode(const void* q, const void* k_cache, const void* v_
                               const int* seq_order, const int* positions, const int* token_slot,
                               const int* block_table, int table_stride, int page_size,
                               int num_seqs, int nq, int nkv, int window, float scale,
-                              int split_chunk, int nsplit, int fused, const float* q_norm_w,
+                              int split_chunk, int nsplit, int waves, int fused, const float* q_norm_w,
                               const float* k_norm_w, const float* cos_tab, const float* sin_tab,
                               void* k_write, void* v_write, float eps, hipStream_t stream) {
     if (num_seqs <= 0) return RL_OK;
@@ -575,6 +579,7 @@ extern "C" int rl_attn_decode(const void* q, const void* k_cache, const void* v_
     // a split's pages are staged in LDS (its keys may start up to 31 before a page's first)
     if ((split_chunk + 31) / page_size + 1 > DEC_MAX_PAGES) return RL_ERR_ARG;
     if (nsplit > 1 && (!part_o || !part_ml)) return RL_ERR_ARG;
+    if (waves != DEC_WAVES && waves != 2) return RL_ERR_ARG;
     if (fused && (D % 64 != 0 || (cos_tab && !sin_tab) || (k_write && !v_write))) return RL_ERR_ARG;
     const int G = nq / nkv;
     const int head_chunks = (G + 15) / 16;
@@ -589,28 +594,36 @@ extern "C" int rl_attn_decode(const void* q, const void* k_cache, const void* v_
     ex.v_write = fused ? (bf16_t*)v_write : nullptr;
     ex.eps = eps;
     ex.qkv_stride = fused ? (nq + 2 * nkv) * D : nq * D;
-    dim3 grid(nkv * head_chunks, num_seqs, nsplit), block(DEC_WAVES * RL_WAVE);
-#define RL_DECODE(V16, FUSED)                                                                  \
-    hipLaunchKernelGGL((attn_decode_kernel<V16, FUSED>), grid, block, 0, stream,               \
+    dim3 grid(nkv * head_chunks, num_seqs, nsplit), block(waves * RL_WAVE);
+#define RL_DECODE_BY(V16, FUSED, WAVES)                                                        \
+    hipLaunchKernelGGL((attn_decode_kernel<V16, FUSED, WAVES>), grid, block, 0, stream,        \
                        (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache,       \
                        (bf16_t*)out, part_o, part_ml, seq_token, seq_order, positions,         \
                        token_slot,                                                             \
                        block_table, table_stride, page_size, nq, nkv, window, scale_log2,      \
                        split_chunk, nsplit, ex)
+#define RL_DECODE(V16, FUSED)                    \
+    if (waves == 2)                              \
+        RL_DECODE_BY(V16, FUSED, 2);             \
+    else                                         \
+        RL_DECODE_BY(V16, FUSED, DEC_WAVES)
     if (fused) {
         if constexpr (D % 64 == 0) {
-            if (page_size % 8 == 0)
+            if (page_size % 8 == 0) {
                 RL_DECODE(true, true);
-            else
+            } else {
                 RL_DECODE(false, true);
+            }
         }
     } else {
-        if (page_size % 8 == 0)
+        if (page_size % 8 == 0) {
             RL_DECODE(true, false);
-        else
+        } else {
             RL_DECODE(false, false);
+        }
     }
 #undef RL_DECODE
+#undef RL_DECODE_BY
     if (hipGetLastError() != hipSuccess) return RL_ERR_LAUNCH;
     if (nsplit > 1) {
         hipLaunchKernelGGL(attn_merge_kernel, dim3(num_seqs, nq), dim3(D < 64 ? 64 : D), 0,

@@ -2303,6 +2303,10 @@ def _decode_launch(lib, plan, ctx, q, k_cache, v_cache, out, block_table, page_s
                                          ragged=window <= 0 and plan.ragged(decode_workgroups(nq, nkv)))
     if plan.num_decode > 65535:
         raise KernelError(f"{plan.num_decode} single-token requests exceed the decode kernel's launch grid")
+    waves = 4
+    short = _decode_short(pairs, chunk, span, window)
+    if short is not None:
+        (chunk, nsplit), waves = short, 2
     # with more workgroups than start at once, the longest requests go first
     order = plan.decode_order(ctx) if pairs * nsplit > chip().decode_resident else None
     part_o = part_ml = None
@@ -2318,7 +2322,7 @@ def _decode_launch(lib, plan, ctx, q, k_cache, v_cache, out, block_table, page_s
             _p(q), _p(k_cache), _p(v_cache), _p(out), _p(part_o), _p(part_ml),
             _p(plan.seq_token), _p(order), _p(ctx.positions), _p(ctx.token_slot), _p(block_table),
             block_table.stride(0), page_size, plan.num_decode, nq, nkv, window,
-            ctypes.c_float(scale), chunk, nsplit, int(fused is not None), _p(qn), _p(kn), _p(cos),
+            ctypes.c_float(scale), chunk, nsplit, waves, int(fused is not None), _p(qn), _p(kn), _p(cos),
             _p(sin), _p(kw), _p(vw), ctypes.c_float(eps), _stream(),
         ),
         "rl_attn_decode",
@@ -2390,12 +2394,34 @@ def _decode_split(num_decode: int, nq: int, nkv: int, span: int, page_size: int,
     return pairs, chunk, -(-span // chunk)
 
 
+_SHORT_KEYS = 512  # keys up to which few requests get splits of half the size
+
+
+def _decode_short(pairs: int, chunk: int, span: int, window: int, units: int | None = None) -> tuple[int, int] | None:
+    """(keys a split, splits) of two waves where ``pairs`` workgroups before splitting over at most ``span`` keys leave
+    units idle with splits of 128 keys, ``None`` where they do not.
+
+    A unit takes a split's keys one wave's 32 at a time, so half as many keys a unit are the shorter chain: a step of
+    the Qwen3-0.6B shape with one request of 100 / 300 / 500 keys 1,015 / 1,002 / 1,020 -> 981 / 986 / 991 us, four of
+    400 1,031 -> 1,015, of the 8B shape one of 300 3,328 -> 3,304.  The merge's share grows with the splits: one request
+    of 1,000 keys 1,025 -> 1,020, of 2,000 1,049 -> 1,071, hence up to 512 keys."""
+    units = chip().units if units is None else units
+    if window > 0:
+        span = min(span, window + 31)
+    if chunk != _MIN_SPLIT_KEYS or span > _SHORT_KEYS:
+        return None
+    keys = max(64, -(-(-(-span // max(1, units // pairs))) // 64) * 64)
+    return (keys, -(-span // keys)) if keys < chunk else None
+
+
 def decode_scratch_bytes(rows: int, nq: int, nkv: int, d: int, span: int, page_size: int, window: int) -> int:
     """Bytes of split results (float32 outputs, maxima and sums) that a decode launch of
     ``rows`` single tokens over at most ``span`` keys keeps between its two kernels."""
     unlike = window <= 0 and 4 * rows * decode_workgroups(nq, nkv) >= chip().units
     nsplit = max(_decode_split(rows, nq, nkv, span, page_size, window, ragged=ragged)[2]
                  for ragged in ((False, True) if unlike else (False,)))
+    pairs, chunk, _ = _decode_split(rows, nq, nkv, span, page_size, window)
+    nsplit = max(nsplit, (_decode_short(pairs, chunk, span, window) or (0, 0))[1])
     return 0 if nsplit == 1 else rows * nq * nsplit * (d + 2) * 4
 
 

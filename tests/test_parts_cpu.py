@@ -307,6 +307,25 @@ def test_decode_splits_of_unlike_contexts():
             assert ops.decode_scratch_bytes(rows, 32, 8, 128, span, 16, 0) >= (0 if unlike == 1 else rows * 32 * unlike * 130 * 4)
 
 
+def test_decode_splits_of_few_short_contexts():
+    """Half-sized splits only where units would be idle and contexts are short; they cover the span, and the bytes
+    reserved cover them."""
+    from rapid_llm_amd.kernels import ops
+
+    for rows in (1, 2, 4, 5, 8, 32):
+        for span in (1, 64, 65, 128, 300, 512, 513, 4096):
+            for window in (0, 100):
+                pairs, chunk, nsplit = ops._decode_split(rows, 32, 8, span, 16, window, units=256)
+                short = ops._decode_short(pairs, chunk, span, window, units=256)
+                assert short is None or (short[0] == 64 and span <= 512 or window)
+                if short is not None:
+                    seen = min(span, window + 31) if window else span
+                    assert short[0] * short[1] >= seen and short[0] % 64 == 0 and short[0] < chunk
+                    assert pairs * short[1] <= 256 or pairs >= 256
+                    assert ops.decode_scratch_bytes(rows, 32, 8, 128, span, 16, window) >= (short[1] > 1) * rows * 32 * short[1] * 130 * 4
+    assert ops._decode_short(8, 128, 300, 0, units=256) == (64, 5) and ops._decode_short(256, 128, 100, 0, units=256) is None
+
+
 def test_weight_rows_a_workgroup_of_the_few_row_product():
     """The host's rule: 24 rows (code 3) only for a product that just stores its result, on a
     matrix of 257 to 1,023 tiles, where that puts the fewest rows on a compute unit."""
