@@ -7,9 +7,9 @@
 // most, half a unit in its last place (|mid| <= 2^-8, |lo| <= 2^-17 of the operand's power of two: mid lo and
 // lo mid are 2^-25 each), and far less on the average.  The float32 instruction (v_mfma_f32_16x16x4_f32) has 157
 // TFLOP/s at most, and the kernel on it that this one replaces reached 101; six bfloat16 instructions
-// come to a sixth of 2.5 PFLOP/s, of which the library's bfloat16 products reach half.  Measured at 2,048
-// rows: 6,144 x 4,096 1,018 -> 530 us, 24,576 x 4,096 4,259 -> 2,000 us, 4,096 x 12,288 2,007 -> 985 us
-// (200 to 210 TFLOP/s); at 225 rows of a small model 6,144 x 1,024 53 -> 36 us and 1,024 x 3,072 68 -> 20
+// come to a sixth of 2.5 PFLOP/s, of which bfloat16 products of real operands reach 0.6.  Measured at 2,048
+// rows: 6,144 x 4,096 1,018 -> 453 us, 24,576 x 4,096 4,259 -> 1,624 us, 4,096 x 12,288 2,007 -> 817 us
+// (227 to 254 TFLOP/s); at 225 rows of a small model 6,144 x 1,024 53 -> 36 us and 1,024 x 3,072 68 -> 20
 // us.  Error against 64 bits over normal operands, relative to the result: K = 4,096 4.1e-7 -> 3.4e-7,
 // K = 12,288 7.0e-7 -> 6.0e-7.
 //
@@ -42,6 +42,8 @@
 // The transposed product is computed (W supplies the A operand, the rows of A the B operand),
 // so a lane's four results are four consecutive n of one row of C.
 #include "common.h"
+
+#include <type_traits>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -521,6 +523,255 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(
     }
 }
 
+// ---- many rows: the pieces of A laid out before, eight waves in two halves ----------------------
+// One kernel splits A once, instead of every workgroup that reads its rows, and lays the pieces down as the matrix
+// instruction reads them (bound by memory, 10 bytes an element: 10 us for 2,048 x 4,096): [16 rows][chunk][hi, mid, lo][64 lanes][8 k], 1 KB a piece.  Rows behind the last are zeros.
+__global__ __launch_bounds__(256) void gemm_f32_pieces_kernel(const float* __restrict__ A, __bf16* __restrict__ P, int M,
+                                                              int chunks, int lda, int per) {
+    const int lane = threadIdx.x & (RL_WAVE - 1), r16 = lane & 15, g = lane >> 4;
+    const int block = blockIdx.y, c = blockIdx.x * 4 + threadIdx.x / RL_WAVE;
+    if (c >= chunks) return;
+    const int row = block * 16 + r16;
+    f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
+    if (row < M) {
+        const float* p = A + (size_t)row * lda + c * FCH + 8 * g;
+        x = load4(p), y = load4(p + 4);
+    }
+    const Split s = split8(x, y, c / per & 1 ? -UP : UP);
+    __bf16* out = P + ((size_t)block * chunks + c) * 1536 + lane * 8;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(out + p * 512) = s.p[p];
+}
+
+typedef __attribute__((address_space(3))) void* rl_lds_ptr;
+#define WIDE_A (256 * FCH * 6)  // bytes of a chunk's pieces of A
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void turn() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+}
+// operand reads wait in the block that asks, so that the compiler adds no wait for loads that are on their way into LDS
+__device__ __forceinline__ void read_w(bf16x8 (&w)[4][3], uint32_t at) {
+    asm volatile(
+        "ds_read_b128 %0, %12\n ds_read_b128 %1, %12 offset:8192\n ds_read_b128 %2, %12 offset:16384\n"
+        "ds_read_b128 %3, %12 offset:1024\n ds_read_b128 %4, %12 offset:9216\n ds_read_b128 %5, %12 offset:17408\n"
+        "ds_read_b128 %6, %12 offset:2048\n ds_read_b128 %7, %12 offset:10240\n ds_read_b128 %8, %12 offset:18432\n"
+        "ds_read_b128 %9, %12 offset:3072\n ds_read_b128 %10, %12 offset:11264\n ds_read_b128 %11, %12 offset:19456\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(w[0][0]), "=&v"(w[0][1]), "=&v"(w[0][2]), "=&v"(w[1][0]), "=&v"(w[1][1]), "=&v"(w[1][2]),
+          "=&v"(w[2][0]), "=&v"(w[2][1]), "=&v"(w[2][2]), "=&v"(w[3][0]), "=&v"(w[3][1]), "=&v"(w[3][2])
+        : "v"(at)
+        : "memory");
+}
+__device__ __forceinline__ void read_w(bf16x8 (&w)[3][3], uint32_t at) {
+    asm volatile(
+        "ds_read_b128 %0, %9\n ds_read_b128 %1, %9 offset:6144\n ds_read_b128 %2, %9 offset:12288\n"
+        "ds_read_b128 %3, %9 offset:1024\n ds_read_b128 %4, %9 offset:7168\n ds_read_b128 %5, %9 offset:13312\n"
+        "ds_read_b128 %6, %9 offset:2048\n ds_read_b128 %7, %9 offset:8192\n ds_read_b128 %8, %9 offset:14336\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(w[0][0]), "=&v"(w[0][1]), "=&v"(w[0][2]), "=&v"(w[1][0]), "=&v"(w[1][1]), "=&v"(w[1][2]),
+          "=&v"(w[2][0]), "=&v"(w[2][1]), "=&v"(w[2][2])
+        : "v"(at)
+        : "memory");
+}
+__device__ __forceinline__ void read_a2(bf16x8 (&a)[2][3], uint32_t at) {
+    asm volatile(
+        "ds_read_b128 %0, %6\n ds_read_b128 %1, %6 offset:1024\n ds_read_b128 %2, %6 offset:2048\n"
+        "ds_read_b128 %3, %6 offset:3072\n ds_read_b128 %4, %6 offset:4096\n ds_read_b128 %5, %6 offset:5120\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[0][2]), "=&v"(a[1][0]), "=&v"(a[1][1]), "=&v"(a[1][2])
+        : "v"(at)
+        : "memory");
+}
+
+// The tiles above with 256 rows of A and 32 TN of W a workgroup, 64 x 16 TN a wave; the same sums in the same order.  What
+// bounds it: the matrix cores at the clock they hold with real operands (2,048 rows of 24,576 x 4,096 run at 1.51
+// PFLOP/s of bfloat16, a large bfloat16 product at 1.54), so everything else is kept out of their way:
+//   * A's pieces go from memory straight into LDS, no wave splits a row of A; W, whose pieces would be half as many bytes
+//     again as it, is split by the workgroup, 8 k of a row a thread: 60 vector instructions a chunk beside 96 products.
+//   * The waves are two halves that take turns: while one multiplies (48 products), the other reads its next operands,
+//     splits and stores W's next chunk and asks memory for later ones.  A barrier ends each turn, the second half begins
+//     one barrier later.
+//   * A chunk is two turns, each with half of the wave's rows of A, so every half has a place of its own in LDS and is
+//     asked for one and a half chunks ahead; W one chunk ahead, through registers.  Nothing waits for all loads.
+//   * No bank is met twice: A lies as it is read, W's rows are permuted as in the kernel above.
+// Microseconds at 2,048 rows, the tiles of 128 x 128 / this with A's pieces made: 6,144 x 4,096 521 / 453, 4,096 x 4,096
+// 326 / 279, 24,576 x 4,096 1,957 / 1,624, 4,096 x 12,288 1,006 / 817.  TN = 3 is for matrices whose tiles of
+// 128 columns leave a short last round (ops.f32_wide has the rule).
+template <int TN>
+__global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restrict__ A, const __bf16* __restrict__ P,
+                                                            const float* __restrict__ W, float* __restrict__ C, int M,
+                                                            int N, int K, int lda, int ldw, int ldc, int tiles_m,
+                                                            int tiles_n) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the host pass does not know the LDS loads)
+    constexpr int BN = 32 * TN, PLANE_W = BN * FCH * 2, WIDE_W = 3 * PLANE_W;
+    // [2][16 blocks][3 pieces][1 KB] of A, [2][3 pieces][2 TN blocks][1 KB] of W
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * WIDE_A + 2 * WIDE_W];
+    const int tid = threadIdx.x, lane = tid & (RL_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / RL_WAVE);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int wm = wave >> 1, wn = wave & 1;  // the wave's rows of A, of W
+
+    // the order of the tiles: as in gemm_f32_tile_kernel
+    const int tiles = tiles_m * tiles_n;
+    int t = blockIdx.x;
+    {
+        const int share = tiles / 8, rest = tiles % 8, die = t % 8;
+        t = die * share + min(die, rest) + t / 8;
+    }
+    const int band = t / (8 * tiles_n), first = band * 8, high = min(8, tiles_m - first);
+    const int tm = first + t % (8 * tiles_n) % high, m0 = tm * 256;
+    const int n0 = t % (8 * tiles_n) / high * BN;
+
+    const int chunks = K / FCH, per = (chunks + FRUNS - 1) / FRUNS;
+
+    // A: 48 pieces a chunk, three loads a wave and turn: blocks 2 j and 2 j + 1 of every wave's four (j: turn)
+    const int blocks = min(16, (M + 15) / 16 - tm * 16);  // that exist
+    const uint32_t block_bytes = (uint32_t)chunks * 3072;
+    auto rs_a = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)P + (size_t)tm * 16 * block_bytes), 0, blocks * block_bytes, 0x00020000);
+    uint32_t a_from[3], a_to[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int j = wave * 3 + i, block = j / 6 * 4 + j % 6 / 3, piece = j % 3;  // of turn 0; turn 1: two blocks on
+        a_from[i] = block * block_bytes + piece * 1024 + lane * 16;
+        a_to[i] = block * 3072 + piece * 1024;
+    }
+    auto load_a = [&](int c, int j) {  // (behind the last chunk: that again, nobody reads it)
+        const uint32_t off = (uint32_t)min(c, chunks - 1) * 3072 + 2 * j * block_bytes;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (rl_lds_ptr)(lds + (c & 1) * WIDE_A + a_to[i] + 2 * j * 3072), 16, a_from[i] + off, 0, 0, 0);
+    };
+    // W: 8 k of a row a thread, through registers (where the rows are fewer, the last threads carry what others do:
+    // every wave has the same loads on their way)
+    const int piece = tid & 3, row = (tid >> 2) < BN ? tid >> 2 : (tid >> 2) - 32;
+    const float* from_w = W + (size_t)min(n0 + row, N - 1) * ldw + 8 * piece;
+    unsigned char* to_w = lds + 2 * WIDE_A + (row >> 4) * 1024 + (piece * 16 + ((row & 15) ^ (2 * piece))) * 16;
+    f32x4 raw[2];
+    auto load_w = [&](int c) {
+        const float* p = from_w + min(c, chunks - 1) * FCH;
+        raw[0] = load4(p), raw[1] = load4(p + 4);
+    };
+    auto store_w = [&](int c) {
+        const Split s = split8(raw[0], raw[1]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const uint32_t at = (uint32_t)(uintptr_t)(rl_lds_ptr)(to_w + (c & 1) * WIDE_W);
+            asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(at), "v"(s.p[p]), "n"(p * PLANE_W) : "memory");
+        }
+    };
+
+    const uint32_t l0 = (uint32_t)(uintptr_t)(rl_lds_ptr)lds;
+    const uint32_t w_at = l0 + 2 * WIDE_A + wn * TN * 1024 + (g * 16 + (r16 ^ (2 * g))) * 16;
+    const uint32_t a_at = l0 + wm * 4 * 3072 + lane * 16;
+
+    f32x4 acc[TN][4], total[TN][4];
+    bf16x8 w[TN][3], a[2][3];
+    auto products = [&](auto y0c) {
+        constexpr int y0 = decltype(y0c)::value;
+        turn();
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int s = 0; s < 6; ++s)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int x = 0; x < TN; ++x)
+                    acc[x][y0 + y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[x][PIECE_W[s]], a[y][PIECE_A[s]], acc[x][y0 + y], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        turn();
+    };
+#pragma unroll
+    for (int x = 0; x < TN; ++x)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) acc[x][y] = total[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    load_w(0);
+    load_a(0, 0);
+    load_a(0, 1);
+    store_w(0);
+    load_w(1);
+    load_a(1, 0);
+    wait_loads<5>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    turn();
+    if (wave >= 4) __builtin_amdgcn_s_barrier();  // the second half is one turn behind
+    __builtin_amdgcn_sched_barrier(0);
+
+    int run = 0, left = per;  // chunks until the run is over
+    auto finish_run = [&]() {
+        const float sign = run & 1 ? -1.f : 1.f;
+#pragma unroll
+        for (int x = 0; x < TN; ++x)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) total[x][y][i] = fmaf(acc[x][y][i], sign, total[x][y][i]);
+                acc[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            }
+        ++run;
+        left = per;
+    };
+#pragma unroll 1
+    for (int c = 0; c < chunks; ++c) {
+        // all of W, half of A; the other half's place for the next chunk has been read
+        load_a(c + 1, 1);
+        read_w(w, w_at + (c & 1) * WIDE_W);
+        read_a2(a, a_at + (c & 1) * WIDE_A);
+        wait_loads<8>();  // this chunk's second half of A is there
+        products(std::integral_constant<int, 0>{});
+        // the other half of A; W's next chunk goes to LDS
+        read_a2(a, a_at + (c & 1) * WIDE_A + 2 * 3072);
+        store_w(c + 1);
+        load_w(c + 2);
+        load_a(c + 2, 0);
+        wait_loads<8>();  // the next chunk's first half of A
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        products(std::integral_constant<int, 2>{});
+        if (--left == 0 || c + 1 == chunks) finish_run();
+    }
+    while (run < FRUNS) finish_run();  // runs without a chunk: zeros
+    wait_loads<0>();  // nothing may still be on its way into LDS when it is given back
+    if (wave < 4) __builtin_amdgcn_s_barrier();
+
+    uint64_t wide = 0;
+    const bool whole = (ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+#pragma unroll
+    for (int x = 0; x < TN; ++x)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const int m = m0 + wm * 64 + y * 16 + r16, n = n0 + (wn * TN + x) * 16 + 4 * g;
+            if (m >= M) continue;
+            f32x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (!__builtin_isfinite(total[x][y][i])) wide |= 1ull << ((x * 4 + y) * 4 + i);
+                v[i] = total[x][y][i] * DOWN;
+            }
+            float* out = C + (size_t)m * ldc + n;
+            if (whole && n + 3 < N) {
+                *reinterpret_cast<f32x4*>(out) = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < N) out[i] = v[i];
+            }
+        }
+    while (wide) {
+        const int e = __ffsll((unsigned long long)wide) - 1;
+        wide &= wide - 1;
+        const int m = m0 + wm * 64 + (e >> 2) % 4 * 16 + r16, n = n0 + (wn * TN + (e >> 4)) * 16 + 4 * g + (e & 3);
+        if (n < N) C[(size_t)m * ldc + n] = wide_sum(A + (size_t)m * lda, W + (size_t)n * ldw, K);
+    }
+#endif
+}
+
 // the runs of the tile kernel added in their order
 __global__ __launch_bounds__(256) void gemm_f32_add_runs_kernel(
     const float* __restrict__ parts, const float* __restrict__ A, const float* __restrict__ W,
@@ -623,4 +874,27 @@ extern "C" int rl_gemm_f32(const float* A, const float* W, float* C, float* part
     if (tile == 64) return launch_tile<2, 2>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
     if (tile == 128) return launch_tile<4, 4>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
     return RL_ERR_ARG;
+}
+
+// The same for many rows and K a multiple of 32: `pieces` holds 96 K bytes for every 16 rows of A; `cols` (128 or 96) are
+// the rows of W a tile takes.
+extern "C" int rl_gemm_f32_wide(const float* A, const float* W, float* C, void* pieces, int M, int N, int K, int lda,
+                                int ldw, int ldc, int cols, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return RL_OK;
+    const int chunks = K / FCH, blocks = (M + 15) / 16;
+    if (!pieces || (uintptr_t)pieces % 16 || K <= 0 || K % FCH || lda < K || ldw < K || ldc < N || (cols != 128 && cols != 96))
+        return RL_ERR_ARG;
+    const int tm = (M + 255) / 256, tn = (N + cols - 1) / cols;
+    // the pieces of a tile are addressed with 32 bits
+    if (K > 1 << 20 || blocks > 65535 || (long long)tm * tn > 0x7fffffffLL / 16) return RL_ERR_ARG;
+    hipLaunchKernelGGL(gemm_f32_pieces_kernel, dim3((chunks + 3) / 4, blocks), dim3(256), 0, stream, A, (__bf16*)pieces, M,
+                       chunks, lda, (chunks + FRUNS - 1) / FRUNS);
+    if (int code = rl_launch_status()) return code;
+    if (cols == 128)
+        hipLaunchKernelGGL(gemm_f32_wide_kernel<4>, dim3(tm * tn), dim3(512), 0, stream, A, (const __bf16*)pieces, W, C, M, N,
+                           K, lda, ldw, ldc, tm, tn);
+    else
+        hipLaunchKernelGGL(gemm_f32_wide_kernel<3>, dim3(tm * tn), dim3(512), 0, stream, A, (const __bf16*)pieces, W, C, M, N,
+                           K, lda, ldw, ldc, tm, tn);
+    return rl_launch_status();
 }

@@ -239,8 +239,8 @@ class ModelRunner:
         wide = [tuple(p.shape) for p in self.params.values() if p.dim() == 2 and p.dtype == torch.float32]
         total = 0
         for fewer, rows in zip([0, *sizes], sizes):
-            # a float32 product's partial results, given back behind it
-            scratch = max((ops.f32_scratch_bytes(rows, *shape) for shape in wide), default=0)
+            # a float32 product's partial results or pieces, given back behind it
+            scratch = max((ops.f32_product_bytes(rows, *shape) for shape in wide), default=0)
             total += len(bounds) * scratch
             for bound in bounds:
                 kept = max((p.recorded_step_bytes(rows, bound, e.page_size) for p in parts), default=0)

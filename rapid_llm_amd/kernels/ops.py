@@ -1065,6 +1065,11 @@ def f32_plan(m: int, n: int, k: int, units: int) -> tuple[int, int]:
             return 1, 1
         if -(-tiles // 2) * blocks <= 2 * units:
             return 2, 1
+    return _f32_tile_plan(m, n, k, units)[1:]
+
+
+def _f32_tile_plan(m: int, n: int, k: int, units: int) -> tuple[float, int, int]:
+    """(estimated microseconds, rows of A a tile takes, workgroups that share its runs)."""
     best = None
     for tile in (32,) if m <= 32 else (64,) if m <= 64 else (64, 128):
         width, costs = _F32_TILES[tile]
@@ -1080,7 +1085,50 @@ def f32_plan(m: int, n: int, k: int, units: int) -> tuple[int, int]:
                 time += _F32_SHARED + 64.0 * m * n / _F32_RUN_BYTES
             if best is None or time < best[0]:
                 best = (time, tile, groups)
-    return best[1], best[2]
+    return best
+
+
+# The many-row product's tiles (rows of W a workgroup takes, of A it takes 256): microseconds a chunk of 32 k takes with
+# few units busy and with all (the clock falls), fitted to 60 shapes of 512 to 4,096 rows: the estimate is within 8%.
+_F32_WIDE = {128: (1.54, 2.03), 96: (1.33, 1.63)}
+_F32_WIDE_ROUND = 9.0  # microseconds a round of workgroups takes beyond its chunks
+_F32_PIECE_BYTES = 1e7  # bytes a microsecond at which A is read and its pieces are written
+_F32_MOST_PIECES = 1 << 28  # bytes of pieces beyond which a product is cut into launches of fewer rows
+
+
+@functools.lru_cache(maxsize=4096)
+def f32_wide(m: int, n: int, k: int, units: int) -> int:
+    """Rows of W a tile of the float32 product for many rows takes, 0 where the tiles of ``f32_plan`` are the faster
+    ones.  The bits are the same either way.
+
+    Its tiles are two and one and a half times the largest there and a unit holds one, so they pay where they fill the
+    chip; the narrower ones where the others would leave a short last round.  Microseconds at 1,024 / 2,048 / 4,096 rows, ``f32_plan``'s tiles
+    first: 6,144 x 4,096 290 / 222, 521 / 453, 954 / 816; 4,096 x 4,096 208 / 191, 326 / 279, 651 / 558;
+    24,576 x 4,096 988 / 814, 1,957 / 1,624, 3,890 / 3,190; 4,096 x 12,288 535 / 557, 1,006 / 817, 1,956 / 1,640;
+    4,096 x 1,024 67 / 61, 90 / 81, 175 / 159; 1,024 x 3,072 48 / 143, 85 / 149, 156 / 161."""
+    if m <= 64 or k % 32 or k > 1 << 20:
+        return 0
+    best, cols = 0.97 * (_f32_tile_plan(m, n, k, units)[0] + _F32_WIDE_ROUND), 0
+    for width, (few, full) in _F32_WIDE.items():
+        rounds, rest = divmod(-(-m // 256) * -(-n // width), units)
+        chunk = rounds * full + (max(few, full * rest / units) if rest else 0.0)
+        time = chunk * (k // 32) + _F32_WIDE_ROUND * (rounds + (rest > 0)) + 2.0 + 10.0 * m * k / _F32_PIECE_BYTES
+        if time < best:
+            best, cols = time, width
+    return cols
+
+
+def _f32_piece_rows(m: int, k: int) -> int:
+    """Rows a launch of that product takes: all, or even shares of whole tiles."""
+    launches = -(-96 * k * -(-m // 16) // _F32_MOST_PIECES)
+    return -(-(-(-m // launches)) // 256) * 256
+
+
+def f32_product_bytes(m: int, n: int, k: int) -> int:
+    """What a float32 product of ``m`` rows over ``[n, k]`` weights takes beside its result."""
+    if f32_wide(m, n, k, chip().units):
+        return 96 * k * -(-min(m, _f32_piece_rows(m, k)) // 16)
+    return f32_scratch_bytes(m, n, k)
 
 
 def f32_scratch_bytes(m: int, n: int, k: int) -> int:
@@ -1098,6 +1146,19 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
     n, k2 = w.shape
     if k != k2 or out.shape != (m, n):
         raise KernelError(f"gemm_f32 shapes do not agree: a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)}")
+    cols = f32_wide(m, n, k, chip().units)
+    if cols:
+        rows = _f32_piece_rows(m, k)
+        pieces = torch.empty(96 * k * -(-min(m, rows) // 16), dtype=torch.uint8, device=a.device)
+        for lo in range(0, m, rows):
+            _ok(
+                core().rl_gemm_f32_wide(
+                    _p(a[lo:]), _p(w), _p(out[lo:]), _p(pieces), min(rows, m - lo), n, k, a.stride(0), w.stride(0), out.stride(0), cols,
+                    _stream()
+                ),
+                "rl_gemm_f32_wide",
+            )
+        return
     tile, groups = f32_plan(m, n, k, chip().units)
     parts = torch.empty((8, m, n), dtype=torch.float32, device=a.device) if groups > 1 else None
     _ok(

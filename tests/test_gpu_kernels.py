@@ -732,6 +732,41 @@ def test_gemm_f32_keeps_what_bfloat16_would_lose():
     assert out.item() == k + 2.0 ** -12
 
 
+@pytest.mark.parametrize("cols", [128, 96])
+@pytest.mark.parametrize("shape", [(1, 1, 32), (17, 97, 64), (255, 129, 96), (257, 193, 288), (300, 260, 1056), (513, 520, 4128)])
+def test_gemm_f32_for_many_rows(shape, cols):
+    """The many-row kernel called directly gives the tile kernel's bits: rows that end inside a piece, a block and a tile,
+    runs without a chunk, one chunk, strided and odd rows; nothing behind the results; elements that the pieces cannot hold."""
+    ops = _ops()
+    m, n, k = shape
+    gen = torch.Generator().manual_seed(m)
+    a, w = (torch.randn(r, k + 3, generator=gen) * torch.exp2(torch.randint(-5, 6, (r, k + 3), generator=gen)) for r in (m, n))
+    a[m // 2, k // 2], w[n - 1, k - 1] = float("inf"), 2.0**104
+    ad, wd = a.to(DEV)[:, 1 : k + 1], w.to(DEV)[:, 2 : k + 2]
+    out, want = torch.full((m, n + 1), 7.0, device=DEV), torch.empty((m, n), device=DEV)
+    parts, pieces = torch.empty((8, m, n), device=DEV), torch.empty(96 * k * -(-m // 16), dtype=torch.uint8, device=DEV)
+    lib, p = ops.core(), ops._p
+    assert lib.rl_gemm_f32(p(ad), p(wd), p(want), p(parts), m, n, k, k + 3, k + 3, n, 128, 1, ops._stream()) == 0
+    assert lib.rl_gemm_f32_wide(p(ad), p(wd), p(out), p(pieces), m, n, k, k + 3, k + 3, n + 1, cols, ops._stream()) == 0
+    assert bool((out[:, n] == 7.0).all())
+    torch.testing.assert_close(out[:, :n], want, rtol=0, atol=0, equal_nan=True)
+
+
+def test_gemm_f32_many_rows_in_several_launches(monkeypatch):
+    """Pieces beyond their limit: launches of fewer rows, the same bits."""
+    ops = _ops()
+    m, n, k = 1100, 3072, 256
+    gen = torch.Generator().manual_seed(1)
+    a, w = torch.randn(m, k, generator=gen).to(DEV), torch.randn(n, k, generator=gen).to(DEV)
+    monkeypatch.setattr(ops, "f32_wide", lambda *_: 96)
+    one, more = torch.empty((m, n), device=DEV), torch.full((m, n), 7.0, device=DEV)
+    ops.gemm_f32(a, w, one)
+    monkeypatch.setattr(ops, "_F32_MOST_PIECES", 1 << 20)
+    assert ops._f32_piece_rows(m, k) == 768  # two launches, the first of whole tiles
+    ops.gemm_f32(a, w, more)
+    assert torch.equal(one, more)
+
+
 @pytest.mark.parametrize("shape", [(1, 16, 32), (16, 33, 1000), (17, 64, 32), (32, 70, 290), (33, 130, 1056),
                                    (65, 127, 96), (129, 260, 4128), (257, 513, 72), (300, 1028, 8)])
 def test_gemm_f32_every_tile_and_sharing(shape):

@@ -290,6 +290,24 @@ def test_plans_of_the_float32_product():
     assert ops.f32_plan(8, 8192, 4096, 256)[0] == 1 and ops.f32_plan(9, 8192, 4096, 256)[0] == 2
 
 
+def test_plans_of_the_float32_product_for_many_rows():
+    """Large tiles only for whole chunks and more than 64 rows, where they fill the chip; launches hold whole tiles and
+    what they take is what is reserved."""
+    from rapid_llm_amd.kernels import ops
+
+    for units in (1, 40, 256, 304):
+        for m in (1, 64, 65, 225, 2048, 8192, 70000):
+            for n in (1, 333, 4096, 24576):
+                for k in (32, 1000, 1024, 4096, 12288):
+                    cols = ops.f32_wide(m, n, k, units)
+                    assert cols in (0, 96, 128) and (not cols or (m > 64 and k % 32 == 0))
+                    rows = ops._f32_piece_rows(m, k)
+                    assert rows % 256 == 0 and 96 * k * (rows // 16 - 16) <= ops._F32_MOST_PIECES
+    assert ops.f32_wide(2048, 24576, 4096, 256) == 128 and ops.f32_wide(2048, 6144, 4096, 256) == 96
+    assert ops.f32_wide(2048, 1024, 3072, 256) == 0 and ops.f32_wide(225, 4096, 1024, 256) == 0
+    assert ops._f32_piece_rows(2048, 12288) == 2048 and ops._f32_piece_rows(8192, 12288) == 2816
+
+
 def test_decode_splits_of_unlike_contexts():
     """Requests of unlike length get more splits of their keys, whatever that would be for fewer than eight
     and more than 64, and never splits that hold no whole step; the bytes reserved cover both."""
