@@ -1397,7 +1397,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
 
     Up to 16 rows (decode) run the hand-written bandwidth-bound kernel, which can write
     float32 directly; so does the kernel for 17 to 64 rows over wide matrices.  Small matrices
-    run the one-launch tile product up to 512 rows.  Everything else goes to the library
+    run the one-launch tile product beyond, up to 512 rows.  Everything else goes to the library
     product, as the reference's dense products do (``F.linear``).  A float32 result is written by the
     product itself, save the one-launch tile product's, which is bfloat16 and widened by the caller.
     ``x`` may be columns of a wider row."""
@@ -1430,7 +1430,8 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
     x = x.contiguous()
     if scaled is not None:
         raise KernelError(f"scaled rows need the few-row product: {m} rows over {k}")
-    if _tile_applies(m, n, k, n):
+    plan = rows_plan(m, n, k, swiglu=False)
+    if _tile_applies(m, n, k, n) and not (plan is not None and k >= 512 and out_dtype == torch.bfloat16 and _aligned(x, w)):
         out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
         _ok(
             core().rl_gemm_tile(_p(x), _p(w), _p(out), m, n, k, k, k, n, 0, ctypes.c_float(0.0), ctypes.c_float(0.0),
@@ -1438,7 +1439,6 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
             "rl_gemm_tile",
         )
         return out
-    plan = rows_plan(m, n, k, swiglu=False)
     if plan is not None:
         wide = torch.float32 if out_dtype == torch.float32 else torch.bfloat16
         out = torch.empty((m, n), dtype=wide, device=x.device)
@@ -1577,7 +1577,12 @@ def _tile_applies(m: int, weight_rows: int, k: int, cols: int) -> bool:
     model is bound by the host, where a call of the library costs 18 us and one of this kernel
     6: a 512-token prompt of the Qwen3-0.6B shape 5.4 -> 4.2 ms.  Hence up to 512 rows.  The packed gate and up
     matrices go on to the many-row product from 129 rows on (6,144 x 1,024 at 64 / 128 / 160 / 256 / 512 rows, the tile
-    product first: 10.7 / 11.8, 11.7 / 12.3, 14.7 / 11.9, 15.3 / 12.3, 19.3 / 12.5)."""
+    product first: 10.7 / 11.8, 11.7 / 12.3, 14.7 / 11.9, 15.3 / 12.3, 19.3 / 12.5).  Up to 64 rows, where
+    :func:`rows_plan` has a plan, operands are aligned and the result is bfloat16, the kernel that keeps X in registers comes
+    first (over weights from memory at 17 / 37 / 64 rows, the tile product first: 4,096 x 1,024 7.1 / 4.9, 8.0 / 5.9, 8.9 / 6.5;
+    2,048 x 1,024 5.7 / 4.1, 6.6 / 4.7, 7.5 / 5.6; at 17 and 64 rows 2,048 x 3,072 16.1 / 7.7, 20.2 / 12.0; 4,096 x 512 4.2 / 3.7,
+    5.3 / 4.5; 8,192 x 128 3.1 / 3.4, 3.7 / 4.1; gate and up of 6,144 x 1,024 9.2 / 8.1, 10.9 / 9.2, 12.6 / 10.4, of 12,288
+    x 512 7.3 / 7.7, 10.1 / 9.8), hence from 512 k on, gate and up from 1,024."""
     return (
         SKINNY_MAX_ROWS < m <= TILE_MAX_ROWS
         and k % 128 == 0
@@ -1759,16 +1764,16 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
             return None
         _need(x, "x", torch.bfloat16)
         _need(w_gate_up, "w_gate_up", torch.bfloat16, (two_i, k))
-        tile = _tile_applies(m, two_i, k, inter)
+        plan = rows_plan(m, inter, k, swiglu=True)
+        tile = _tile_applies(m, two_i, k, inter) and not (plan is not None and k >= 1024 and _aligned(x, w_gate_up))
         if (not tile or m > TILE_GATED_MAX_ROWS) and activation == "silu" and limit <= 0 and bias is None:
-            plan = block_plan(m, inter, k, "gated")
-            if plan is not None and _aligned(x, w_gate_up):
-                return _block(x, w_gate_up, torch.empty((m, inter), dtype=torch.bfloat16, device=x.device), "gated", plan)
+            block = block_plan(m, inter, k, "gated")
+            if block is not None and _aligned(x, w_gate_up):
+                return _block(x, w_gate_up, torch.empty((m, inter), dtype=torch.bfloat16, device=x.device), "gated", block)
         if tile:
             out = torch.empty((m, inter), dtype=torch.bfloat16, device=x.device)
             _ok(core().rl_gemm_tile(_p(x), _p(w_gate_up), _p(out), m, inter, k, k, k, inter, 1, *glu, _stream()), "rl_gemm_tile")
             return out
-        plan = rows_plan(m, inter, k, swiglu=True)
         if plan is None:
             return None
         out = torch.empty((m, inter), dtype=torch.bfloat16, device=x.device)

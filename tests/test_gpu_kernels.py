@@ -1166,6 +1166,29 @@ def test_product_in_runs_of_k_and_the_norm_that_adds_them(shape):
     assert torch.equal(res2, got_res) and torch.equal(out2, out)
 
 
+@pytest.mark.parametrize("m", [17, 48, 49, 64, 65])
+def test_small_matrices_up_to_64_rows_keep_x_in_registers(m):
+    """17 to 64 rows over the matrices of a small model go to the kernel that keeps X in registers, more and weights that
+    begin inside a unit of 16 bytes to the tile product: either gives the product."""
+    ops = _ops()
+    k, gen = 1024, torch.Generator().manual_seed(m)
+    x = torch.randn((m, k), generator=gen).bfloat16().to(DEV)
+    room = (torch.randn(6144 * k + 1, generator=gen) / 32).bfloat16().to(DEV)
+    w, odd = room[:-1].view(6144, k), torch.cat([room[:1], room])[1:-1].view(6144, k)
+    odd.copy_(w)
+    exact = x.float() @ w.float().T
+    size = x.float().abs() @ w.float().abs().T
+    for weights in (w, odd):
+        got = ops.gemm_bf16(x, weights[:4096], torch.bfloat16).float()
+        # the result is rounded to bfloat16, its sum of k products to float32
+        assert torch.all((got - exact[:, :4096]).abs() <= 2.0**-8 * exact[:, :4096].abs() + k * 2.0**-24 * size[:, :4096])
+        got = ops.gemm_bf16_swiglu(x, weights).float()
+        gate, up = (t.bfloat16().float() for t in (exact[:, :3072], exact[:, 3072:]))
+        want = torch.nn.functional.silu(gate) * up
+        # gate and up may each be rounded the other way, as in test_many_row_product_every_tile
+        assert torch.all((got - want).abs() <= 2.0**-8 * (1.1 * (gate * up).abs() + 2 * want.abs()) + 1e-6)
+
+
 # rows, result columns, K: one chunk of 64 k and fewer chunks than a tile has buffers for, an odd number of them and
 # many; rows and columns that end inside a piece of 64, inside a tile and at its edge; more tiles than dies, and counts
 # that the dies do not share evenly
