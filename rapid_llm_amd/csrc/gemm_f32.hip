@@ -788,6 +788,63 @@ __global__ __launch_bounds__(256) void gemm_f32_add_runs_kernel(
     C[(size_t)m * ldc + n] = finite_or_wide(v, A + (size_t)m * lda, W + (size_t)n * ldw, K);
 }
 
+// The same sums where a norm follows: added to the residual in place (with the product's bias, where it has one), whose rows
+// are normed as add_rmsnorm does, bit for bit, in one kernel instead of two and without the product's way through
+// memory.  Bound by its start and the runs' bytes.  Microseconds of product and norm at 17 / 64 / 225 / 1,024 rows, as
+// kernels of their own / so: 1,024 x 3,072 15.5 / 14.0, 18.1 / 16.2, 24.0 / 21.3, 54.2 / 48.8; 1,024 x 2,048 13.2 / 11.6,
+// 15.2 / 13.3, 21.5 / 18.8, 41.9 / 38.7; 2,560 x 9,728 43.6 / 42.1, 47.9 / 45.8, 107 / 98, 301 / 294.
+template <int CHUNKS>
+__global__ void gemm_f32_add_runs_rmsnorm_kernel(const float* __restrict__ parts, const float* __restrict__ A,
+                                                 const float* __restrict__ W, int M, int K, int lda, int ldw,
+                                                 float* __restrict__ residual, const float* __restrict__ weight,
+                                                 float* __restrict__ out, int hidden, float eps,
+                                                 const float* __restrict__ bias) {
+    __shared__ float scratch[16];
+    const int m = blockIdx.x, nvec = hidden >> 2;
+    const size_t stride = (size_t)M * hidden;
+    f32x4* res = reinterpret_cast<f32x4*>(residual + (size_t)m * hidden);
+    f32x4 val[CHUNKS], wt[CHUNKS];
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const int i = threadIdx.x + c * blockDim.x;
+        if (i < nvec) wt[c] = reinterpret_cast<const f32x4*>(weight)[i];
+    }
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const int i = threadIdx.x + c * blockDim.x;
+        if (i < nvec) {
+            const float* p = parts + (size_t)m * hidden + 4 * i;
+            f32x4 run[FRUNS];
+#pragma unroll
+            for (int r = 0; r < FRUNS; ++r) run[r] = *reinterpret_cast<const f32x4*>(p + r * stride);
+            f32x4 v = res[i], d = run[0];
+#pragma unroll
+            for (int r = 1; r < FRUNS; ++r) d = r & 1 ? d - run[r] : d + run[r];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] += finite_or_wide(d[j], A + (size_t)m * lda, W + (size_t)(4 * i + j) * ldw, K);
+                if (bias) v[j] += bias[4 * i + j];
+            }
+            res[i] = v;
+            val[c] = v;
+            ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+        }
+    }
+    ss = block_sum(ss, scratch);
+    const float rrms = rsqrtf(ss / (float)hidden + eps);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const int i = threadIdx.x + c * blockDim.x;
+        if (i < nvec) {
+            f32x4 y;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[j] = val[c][j] * rrms * wt[c][j];
+            reinterpret_cast<f32x4*>(out + (size_t)m * hidden)[i] = y;
+        }
+    }
+}
+
 // Up to FEW k: a thread a result, bound by the results (2,048 x 6,144 of 1 and 3 k 15 and 19 us; the kernel on the
 // float32 instruction took 40 and 39).
 __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W,
@@ -836,6 +893,7 @@ static int launch_tile_of(const float* A, const float* W, float* C, float* parts
     hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TN, L, true>), dim3(tm * tn, groups), block, 0, stream, A, W, parts,
                        M, N, K, lda, ldw, ldc, tm, tn, FRUNS / groups);
     if (int code = rl_launch_status()) return code;
+    if (!C) return RL_OK;  // (rl_gemm_f32_add_rmsnorm adds them)
     hipLaunchKernelGGL(gemm_f32_add_runs_kernel, dim3((N + 255) / 256, M), block, 0, stream, parts, A, W, C, M, N,
                        K, lda, ldw, ldc);
     return rl_launch_status();
@@ -856,7 +914,7 @@ static int launch_tile(const float* A, const float* W, float* C, float* parts, i
 extern "C" int rl_gemm_f32(const float* A, const float* W, float* C, float* parts, int M, int N, int K, int lda,
                            int ldw, int ldc, int tile, int groups, hipStream_t stream) {
     if (M <= 0 || N <= 0) return RL_OK;
-    if (K <= 0 || lda < K || ldw < K || ldc < N) return RL_ERR_ARG;
+    if (K <= 0 || lda < K || ldw < K || ldc < N || !C) return RL_ERR_ARG;
     if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return RL_ERR_ARG;
     if (K <= FEW) {  // whatever the tile
         hipLaunchKernelGGL(gemm_f32_few_kernel, dim3((N + 255) / 256, M < 1024 ? M : 1024), dim3(256), 0, stream, A, W,
@@ -896,5 +954,29 @@ extern "C" int rl_gemm_f32_wide(const float* A, const float* W, float* C, void* 
     else
         hipLaunchKernelGGL(gemm_f32_wide_kernel<3>, dim3(tm * tn), dim3(512), 0, stream, A, (const __bf16*)pieces, W, C, M, N,
                            K, lda, ldw, ldc, tm, tn);
+    return rl_launch_status();
+}
+
+// residual[M, N] += A W^T (+ bias) in place and out[M, N] = rmsnorm(residual) * weight, where f32_plan cuts the product into
+// runs (`tile` 32, 64 or 128, `groups` 2, 4 or 8); N a multiple of 4 up to 16 K.
+extern "C" int rl_gemm_f32_add_rmsnorm(const float* A, const float* W, float* parts, int M, int N, int K, int lda, int ldw,
+                                       int tile, int groups, float* residual, const float* weight, float* out, float eps,
+                                       const float* bias, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return RL_OK;
+    if (K <= FEW || lda < K || ldw < K || N % 4 || N > 16 * 1024 || !parts || !residual || !weight || !out) return RL_ERR_ARG;
+    if (groups != 2 && groups != 4 && groups != 8) return RL_ERR_ARG;
+    int code = RL_ERR_ARG;
+    if (tile == 32) code = launch_tile<1, 2>(A, W, nullptr, parts, M, N, K, lda, ldw, N, groups, stream);
+    if (tile == 64) code = launch_tile<2, 2>(A, W, nullptr, parts, M, N, K, lda, ldw, N, groups, stream);
+    if (tile == 128) code = launch_tile<4, 4>(A, W, nullptr, parts, M, N, K, lda, ldw, N, groups, stream);
+    if (code != RL_OK) return code;
+    // threads as for add_rmsnorm: the order of the row's sum
+    const int threads = (N / 4 + RL_WAVE - 1) / RL_WAVE * RL_WAVE;
+    if (threads <= 1024)
+        hipLaunchKernelGGL(gemm_f32_add_runs_rmsnorm_kernel<1>, dim3(M), dim3(threads), 0, stream, parts, A, W, M, K, lda, ldw,
+                           residual, weight, out, N, eps, bias);
+    else
+        hipLaunchKernelGGL(gemm_f32_add_runs_rmsnorm_kernel<4>, dim3(M), dim3(1024), 0, stream, parts, A, W, M, K, lda, ldw,
+                           residual, weight, out, N, eps, bias);
     return rl_launch_status();
 }

@@ -1169,6 +1169,38 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
     )
 
 
+def f32_runs(m: int, n: int, k: int) -> bool:
+    """Whether a float32 product leaves runs of K that a kernel behind it adds: the norm that follows can be that one."""
+    return not f32_wide(m, n, k, chip().units) and f32_plan(m, n, k, chip().units)[1] > 1
+
+
+def gemm_f32_add_rmsnorm(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
+                         eps: float, bias: Optional[torch.Tensor] = None) -> None:
+    """``residual += a w^T (+ bias)`` in place, ``out = norm(residual) * weight``, for products of :func:`f32_runs`: the bits
+    of :func:`gemm_f32` and :func:`add_rmsnorm`."""
+    for t, name in ((a, "a"), (w, "w")):
+        if not t.is_cuda or t.dtype != torch.float32 or t.dim() != 2 or t.stride(1) != 1:
+            raise KernelError(f"gemm_f32 operand {name} must be a float32 GPU matrix with unit inner stride")
+    m, k = a.shape
+    n = w.shape[0]
+    if k != w.shape[1]:
+        raise KernelError(f"gemm_f32 shapes do not agree: a {tuple(a.shape)}, w {tuple(w.shape)}")
+    _need(residual, "residual", torch.float32, (m, n))
+    _need(weight, "norm weight", torch.float32, (n,))
+    _need(out, "out", torch.float32, (m, n))
+    if bias is not None:
+        _need(bias, "bias", torch.float32, (n,))
+    tile, groups = f32_plan(m, n, k, chip().units)
+    parts = torch.empty((8, m, n), dtype=torch.float32, device=a.device)
+    _ok(
+        core().rl_gemm_f32_add_rmsnorm(
+            _p(a), _p(w), _p(parts), m, n, k, a.stride(0), w.stride(0), tile, groups, _p(residual), _p(weight), _p(out),
+            ctypes.c_float(eps), _p(bias), _stream()
+        ),
+        "rl_gemm_f32_add_rmsnorm",
+    )
+
+
 def _row_index(row_index: Optional[torch.Tensor]) -> None:
     if row_index is not None:
         _need(row_index, "row_index", torch.int32)

@@ -57,7 +57,14 @@ class Linear:
     def folds(self, x) -> bool:
         """Whether this product may absorb the residual add and norm that follow it: one of the
         two kernels with that epilogue runs it."""
-        return self.skinny(x) or self.midsize(x)
+        return self.skinny(x) or self.midsize(x) or self.f32_runs(x)
+
+    def f32_runs(self, x) -> bool:
+        """Whether ``x`` runs as a float32 product whose runs of K a norm can add."""
+        return (
+            self.weight.dtype == torch.float32 and x.dtype == torch.float32
+            and ops.f32_runs(x.shape[0], self.out_features, self.in_features)
+        )
 
     def takes_scaled_rows(self) -> bool:
         """Whether this product can finish a norm whose rows arrive unscaled (whatever the
@@ -81,7 +88,7 @@ class Linear:
     def deferred(self, x: torch.Tensor, ctx=None):
         """The product, or a :class:`DeferredProduct` of it where one of this product's kernels
         could fold a neighbouring norm into itself (bfloat16, up to 16 rows, or more of a
-        narrow matrix, see :meth:`midsize`), or where it has a bias, which the kernel that adds the product to the
+        narrow matrix, see :meth:`midsize`; float32 where it is cut into runs), or where it has a bias, which the kernel that adds the product to the
         residual can add.  Whoever receives it and has no use for that simply materialises it."""
         if isinstance(x, torch.Tensor) and (self.bias is not None or self.folds(x)):
             return DeferredProduct(self, x)

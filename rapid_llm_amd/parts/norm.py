@@ -97,6 +97,13 @@ class RMSNorm(Norm):
                 out = torch.empty((residual.shape[0], self.size), dtype=self.dtype, device=residual.device)
                 ops.add_rmsnorm_parts(residual, delta.linear.partial_sums(delta.x), self.weight, out, self.eps, bias)
                 return out
+            if (
+                rows is None and delta.linear.out_features == self.size and self.dtype == torch.float32
+                and self.size % 4 == 0 and self.size <= 16 * 1024 and delta.linear.f32_runs(delta.x)
+            ):
+                out = torch.empty((residual.shape[0], self.size), dtype=self.dtype, device=residual.device)
+                ops.gemm_f32_add_rmsnorm(delta.x, delta.linear.weight, residual, self.weight, out, self.eps, bias)
+                return out
             delta = delta.linear.product(delta.x)
         n = residual.shape[0] if rows is None else rows.numel()
         out = torch.empty((n, self.size), dtype=self.dtype, device=residual.device)

@@ -1,5 +1,6 @@
 """Each HIP kernel alone against its plain reference, at sizes other than the tiny models'."""
 
+import ctypes
 import math
 import random
 from types import SimpleNamespace
@@ -750,6 +751,27 @@ def test_gemm_f32_for_many_rows(shape, cols):
     assert lib.rl_gemm_f32_wide(p(ad), p(wd), p(out), p(pieces), m, n, k, k + 3, k + 3, n + 1, cols, ops._stream()) == 0
     assert bool((out[:, n] == 7.0).all())
     torch.testing.assert_close(out[:, :n], want, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 1024, 1000), (64, 4096, 288), (225, 1024, 3072), (300, 2052, 2048), (130, 4100, 4096)])
+def test_gemm_f32_whose_runs_the_norm_adds(m, n, k):
+    """Every tile and sharing: the bits of the product, its bias and the norm as kernels of their own, an infinite row too."""
+    ops = _ops()
+    gen = torch.Generator().manual_seed(m)
+    a, w, res, nw, bias = (torch.randn(s, generator=gen).to(DEV) for s in ((m, k), (n, k), (m, n), (n,), (n,)))
+    a[m // 2, 3] = float("inf")
+    for b in (None, bias):
+        want_res, want = res.clone(), torch.empty_like(res)
+        y = torch.empty((m, n), device=DEV)
+        ops.gemm_f32(a, w, y)
+        ops.add_rmsnorm(want_res, y, nw, want, 1e-6, None, b)
+        for tile, groups in [(t, g) for t in (32, 64, 128) for g in (2, 4, 8)]:
+            got_res, got, parts = res.clone(), torch.empty_like(res), torch.empty((8, m, n), device=DEV)
+            code = ops.core().rl_gemm_f32_add_rmsnorm(ops._p(a), ops._p(w), ops._p(parts), m, n, k, k, k, tile, groups, ops._p(got_res),
+                                                      ops._p(nw), ops._p(got), ctypes.c_float(1e-6), ops._p(b), ops._stream())
+            assert code == 0
+            torch.testing.assert_close(got_res, want_res, rtol=0, atol=0, equal_nan=True)
+            torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True)
 
 
 def test_gemm_f32_many_rows_in_several_launches(monkeypatch):
