@@ -563,7 +563,9 @@ extern "C" int rl_attn_head_dim() { return D; }
 // tables may be null, `k_write` / `v_write` null for a layer that writes no cache.  The splits
 // are merged by a second kernel: letting the split that finishes last merge (a counter and
 // device-wide fences) was measured and lost, 226 us against 108 us at 64 requests of 2,048
-// keys in four splits, because every workgroup's fence writes the L2 back.
+// keys in four splits, because every workgroup's fence writes the L2 back.  With stores and loads that pass by the L2 and
+// no fence the step of the 0.6B shape with one request of 300 keys went from 989 to 974 us, that of 8B with one of 2,048
+// from 3,402 to 3,427, 30 requests of 500 to 3,000 keys from 2,567 to 2,590: not kept.
 extern "C" int rl_attn_decode(const void* q, const void* k_cache, const void* v_cache, void* out,
                               float* part_o, float* part_ml, const int* seq_token,
                               const int* seq_order, const int* positions, const int* token_slot,
