@@ -2502,11 +2502,12 @@ def _decode_short(pairs: int, chunk: int, span: int, window: int, units: int | N
     A unit takes a split's keys one wave's 32 at a time, so half as many keys a unit are the shorter chain: a step of
     the Qwen3-0.6B shape with one request of 100 / 300 / 500 keys 1,015 / 1,002 / 1,020 -> 981 / 986 / 991 us, four of
     400 1,031 -> 1,015, of the 8B shape one of 300 3,328 -> 3,304.  The merge's share grows with the splits: one request
-    of 1,000 keys 1,025 -> 1,020, of 2,000 1,049 -> 1,071, hence up to 512 keys."""
+    of 1,000 keys 1,025 -> 1,020, of 2,000 1,049 -> 1,071, hence up to 512 keys.  Launches for at most 128 keys have one split and no
+    merge."""
     units = chip().units if units is None else units
     if window > 0:
         span = min(span, window + 31)
-    if chunk != _MIN_SPLIT_KEYS or span > _SHORT_KEYS:
+    if chunk != _MIN_SPLIT_KEYS or not _MIN_SPLIT_KEYS < span <= _SHORT_KEYS:
         return None
     keys = max(64, -(-(-(-span // max(1, units // pairs))) // 64) * 64)
     return (keys, -(-span // keys)) if keys < chunk else None
