@@ -19,6 +19,8 @@
 //     1 KB takes 4 cycles).
 //   * A wave's results are neighbouring columns (128 to 256 bytes of a row), stored 16 bytes a lane: with 32 and
 //     64 bytes a wave 2,048 rows of 24,576 x 4,096 took 294 us, so 289, 8,926 rows of 6,144 x 1,024 119 and 112.
+// With one piece of X (49 to 64 rows) the weights' bytes bound it: five chunks, 120 KB, are on their way, and a workgroup
+// of 64 columns reads X where the kernel that keeps X in registers has 48 (8B gate and up 52.2 -> 48.1 us at 64 rows).
 // A workgroup has one tile.  Workgroups that walk several, with the next tile's loads on their way during the
 // epilogue, were slower (2,048 rows of 24,576 x 4,096: 316 us): stores and loads share a counter, in order, so the next
 // tile's operands waited for this one's results to reach memory.  A new workgroup does not.
@@ -122,6 +124,19 @@ __device__ __forceinline__ void read_a(bf16x8 (&w)[NA][2][2], bf16x8 (&x)[NX][2]
               "=&v"(w[2][0][0]), "=&v"(w[2][0][1]), "=&v"(w[2][1][0]), "=&v"(w[2][1][1]),
               "=&v"(w[3][0][0]), "=&v"(w[3][0][1]), "=&v"(w[3][1][0]), "=&v"(w[3][1][1]),
               "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1])
+            : "v"(a0), "v"(a1), "v"(b0), "v"(b1)
+            : "memory");
+    } else if constexpr (NA == 2 && NX == 1) {
+        asm volatile(
+            "ds_read_b128 %0, %10\n ds_read_b128 %1, %11\n"
+            "ds_read_b128 %2, %10 offset:2048\n ds_read_b128 %3, %11 offset:2048\n"
+            "ds_read_b128 %4, %10 offset:8192\n ds_read_b128 %5, %11 offset:8192\n"
+            "ds_read_b128 %6, %10 offset:10240\n ds_read_b128 %7, %11 offset:10240\n"
+            "ds_read_b128 %8, %12\n ds_read_b128 %9, %13\n"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(w[0][0][0]), "=&v"(w[0][0][1]), "=&v"(w[0][1][0]), "=&v"(w[0][1][1]),
+              "=&v"(w[1][0][0]), "=&v"(w[1][0][1]), "=&v"(w[1][1][0]), "=&v"(w[1][1][1]),
+              "=&v"(x[0][0]), "=&v"(x[0][1])
             : "v"(a0), "v"(a1), "v"(b0), "v"(b1)
             : "memory");
     } else {
@@ -376,7 +391,7 @@ static int launch_block(const BlockArgs& a, int kind, hipStream_t stream) {
 
 // kind 1: out float32 [splits, M, N], run r of K's chunks in part r.  Kind 2: W = [gate | up] stacked, [2N, K], out
 // bfloat16 [M, N] = silu(gate) * up of the products rounded to bfloat16.
-// nw, nx: pieces of 64 rows of a tile (2 to 4, 2 or 4).  K a multiple of 64, N of 8.
+// nw, nx: pieces of 64 rows of a tile (2 to 4, 2 or 4; 2, 1).  K a multiple of 64, N of 8.
 extern "C" int rl_gemm_block(const void* X, const void* W, void* out, int M, int N, int K, int ldx, int ldw, int ldo,
                              int kind, int nw, int nx, int splits, hipStream_t stream) {
     if (M <= 0 || N <= 0) return RL_OK;
@@ -405,6 +420,7 @@ extern "C" int rl_gemm_block(const void* X, const void* W, void* out, int M, int
     RL_BLOCK(4, 2);
     RL_BLOCK(3, 2);
     RL_BLOCK(2, 2);
+    RL_BLOCK(2, 1);
 #undef RL_BLOCK
     return RL_ERR_ARG;
 }

@@ -1688,6 +1688,20 @@ def _block_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int
     return best[1]
 
 
+def block_few_plan(m: int, n: int, k: int, units: int | None = None) -> tuple[int, int, int] | None:
+    """The plan of the same product for the gate and up matrices at 49 to 64 rows, ``None`` where the kernel that keeps X in
+    registers is the faster one.
+
+    That one holds at most three pairs of tiles there, so 256 workgroups of the 8B shape read all of X; here 192 do.
+    Microseconds at 64 rows, that kernel first: 8B 52.2 / 48.1, 4B 29.6 / 28.6, 1.7B 20.3 / 19.8, 0.6B 10.3 / 11.2; at 48 rows
+    45.3 / 47.7, 28.2 / 26.8, 17.6 / 19.0.  Hence from 6,144 columns of 2,048 k on, as long as a round of
+    workgroups holds them."""
+    units = chip().units if units is None else units
+    if not 48 < m <= ROWS_MAX_ROWS or k < 2048 or k % 64 or n % 8 or n < 6144 or -(-n // 64) > units:
+        return None
+    return (2, 1, 1) if (2 * n + 256) * k * 2 <= 0x7FFFFFFF else None
+
+
 _BLOCK_KINDS = {"runs": 1, "gated": 2}  # as the kernel's entry point counts them
 
 
@@ -1799,7 +1813,7 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
         plan = rows_plan(m, inter, k, swiglu=True)
         tile = _tile_applies(m, two_i, k, inter) and not (plan is not None and k >= 1024 and _aligned(x, w_gate_up))
         if (not tile or m > TILE_GATED_MAX_ROWS) and activation == "silu" and limit <= 0 and bias is None:
-            block = block_plan(m, inter, k, "gated")
+            block = block_plan(m, inter, k, "gated") or block_few_plan(m, inter, k)
             if block is not None and _aligned(x, w_gate_up):
                 return _block(x, w_gate_up, torch.empty((m, inter), dtype=torch.bfloat16, device=x.device), "gated", block)
         if tile:

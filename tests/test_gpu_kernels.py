@@ -1218,7 +1218,7 @@ BLOCK_SHAPES = [(1, 8, 64), (65, 72, 128), (128, 256, 192), (257, 520, 320), (30
 
 
 @pytest.mark.parametrize("shape", BLOCK_SHAPES)
-@pytest.mark.parametrize("nw,nx", [(4, 4), (3, 4), (2, 4), (4, 2), (3, 2), (2, 2)])
+@pytest.mark.parametrize("nw,nx", [(4, 4), (3, 4), (2, 4), (4, 2), (3, 2), (2, 2), (2, 1)])
 def test_many_row_product_every_tile(nw, nx, shape):
     """Every tile of the many-row product, called directly: float32 runs of K, whole and cut, and the gated form;
     rows and columns behind the result stay as they were, and a row that is not finite stays alone."""
@@ -1260,6 +1260,24 @@ def test_many_row_product_every_tile(nw, nx, shape):
         other = run(2, m, n, 1, bad)
         assert not torch.isfinite(other[0]).any() or n < 64
         assert torch.equal(other[1:], got[1:])
+
+
+@pytest.mark.parametrize("m", [49, 64])
+def test_gate_and_up_of_49_to_64_rows(m):
+    """Where a round of the many-row product's workgroups holds the columns: the gated product of the gate and up matrices."""
+    ops = _ops()
+    inter, k = 6152, 2048
+    assert ops.block_few_plan(m, inter, k) == (2, 1, 1) and ops.block_few_plan(48, inter, k) is None
+    gen = torch.Generator().manual_seed(m)
+    x = torch.randn((m, k), generator=gen).bfloat16().to(DEV)
+    w = (torch.randn((2 * inter, k), generator=gen) / math.sqrt(k)).bfloat16().to(DEV)
+    before = ops.library_products
+    got = ops.gemm_bf16_swiglu(x, w)
+    assert got is not None and ops.library_products == before
+    gu = x.float() @ w.float().T
+    gate, up = gu[:, :inter].bfloat16().float(), gu[:, inter:].bfloat16().float()
+    want = torch.nn.functional.silu(gate) * up
+    assert torch.all((got.float() - want).abs() <= 2.0**-8 * (1.1 * (gate * up).abs() + 2 * want.abs()) + 1e-6)
 
 
 @pytest.mark.parametrize("m,n,k,kind", [(65, 4096, 12288, "runs"), (520, 2560, 9728, "runs"), (129, 2048, 6144, "runs"),

@@ -190,6 +190,10 @@ def test_where_the_many_row_product_applies():
     assert plan(2049, 4096, 12288, "runs") is None and plan(2048, 4096, 12288, "runs") == (4, 4, 2)
     assert plan(128, 2048, 6144, "runs") is None and plan(129, 2048, 6144, "runs") is not None
     assert plan(1025, 2048, 6144, "runs") is None
+    few = lambda *a: ops.block_few_plan(*a, units=256)
+    assert few(49, 12288, 4096) == few(64, 6144, 2048) == (2, 1, 1)
+    assert few(48, 12288, 4096) is None and few(65, 12288, 4096) is None and few(64, 3072, 1024) is None
+    assert few(64, 17408, 5120) is None and few(64, 6148, 2048) is None and few(64, 12288, 4100) is None
     for m in (65, 100, 300, 777, 1024):
         for n, k in ((4096, 12288), (2560, 9728), (2048, 6144), (8, 8192)):
             found = plan(m, n, k, "runs")
