@@ -1089,7 +1089,7 @@ def _f32_tile_plan(m: int, n: int, k: int, units: int) -> tuple[float, int, int]
 
 
 # The many-row product's tiles (rows of W a workgroup takes, of A it takes 256): microseconds a chunk of 32 k takes with
-# few units busy and with all (the clock falls), fitted to 60 shapes of 512 to 4,096 rows: the estimate is within 8%.
+# few units busy and with all (the clock falls), fitted to 72 shapes of 250 to 4,096 rows: the estimate is 13% low to 8% high.
 _F32_WIDE = {128: (1.54, 2.03), 96: (1.33, 1.63)}
 _F32_WIDE_ROUND = 9.0  # microseconds a round of workgroups takes beyond its chunks
 _F32_PIECE_BYTES = 1e7  # bytes a microsecond at which A is read and its pieces are written
