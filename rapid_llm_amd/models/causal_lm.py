@@ -173,8 +173,12 @@ class CausalLM:
             return False
         if self.offsets is not None or self.mixes is not None or self.returns:
             return False
-        first = self.blocks[self.order[0]].launch_signature()
-        if first is None or any(self.blocks[li].launch_signature() != first for li in self.order[1:]):
+        blocks = [self.blocks[li] for li in self.order]
+        first = blocks[0].launch_signature()
+        # (a signature says that a block and its parts are of known classes, the same ones in every layer)
+        if first is None or not all(p.forward_as_written() for p in (blocks[0], *blocks[0].parts())):
+            return False
+        if any(b.launch_signature() != first for b in blocks):
             return False
         kinds = {(c.group_id, c.page_size, c.owns_pages, len(c.pages), len(c.states)) for c in caches}
         return len(kinds) == 1 and all(c.owns_pages and not c.states for c in caches)

@@ -48,12 +48,13 @@ a product that another mixer shares (``packs``).
 from __future__ import annotations
 
 import math
+import operator
 
 import torch
 
 from ..kernels import ops
 from .base import MIXERS, CacheNeed, PackedMixer, ParamSpec, Source, StateSpec
-from .linear import Linear
+from .linear import Linear, plain_products
 
 
 class GQAAttention(PackedMixer):
@@ -324,10 +325,9 @@ class GQAAttention(PackedMixer):
 
     def launch_signature(self):
         # plain attention alone: the other forms, and kinds derived from this one, may do more
-        if type(self) is not GQAAttention or not self.plain_row:
+        if type(self) is not GQAAttention or not self.plain_row or "forward" in self.__dict__ or not plain_products(self.qkv, self.o):
             return None
-        return (self.hidden_size, self.nq, self.nkv, self.d, self.window, self.scale, self.qk_norm_eps,
-                self.qkv_bias, self.o_bias, id(self.position))
+        return _FIXED(self)
 
     def own_tensors(self) -> list[torch.Tensor]:
         norms = [w for w in (self.q_norm_w, self.k_norm_w) if w is not None]
@@ -412,5 +412,8 @@ class GQAAttention(PackedMixer):
             ops.head_gate(out, qkv, self.qkv_rows, self.nq, self.d)
         return self.o.deferred(out, ctx)
 
+
+# what the launches of a plain layer depend on beside its tensors
+_FIXED = operator.attrgetter("hidden_size", "nq", "nkv", "d", "window", "scale", "qk_norm_eps", "qkv_bias", "o_bias", "position")
 
 MIXERS.register("gqa_attention", GQAAttention)

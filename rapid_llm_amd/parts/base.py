@@ -217,11 +217,21 @@ class Part:
     #: of unlike length (such steps are then recorded for themselves); 0: it does not.
     deals_ragged_contexts = 0
 
+    def __init_subclass__(cls, **kwargs) -> None:
+        super().__init_subclass__(**kwargs)
+        cls._forward_as_written = getattr(cls, "forward", None)
+
+    @classmethod
+    def forward_as_written(cls) -> bool:
+        """Whether the class's ``forward`` is the one it was written with, not something put in its place since."""
+        return cls.forward is cls._forward_as_written
+
     def launch_signature(self) -> "tuple | None":
         """What two parts of different layers have in common if their ``forward`` makes the same launches in every step,
         with nothing but their :meth:`own_tensors` (and a cache's pages) in the place of one another's, and does
         nothing else on the device: the launches of one are then made again for the other without running its
-        ``forward``.  ``None``: no such promise."""
+        ``forward``.  ``None``: no such promise, as where the part has a ``forward`` (or a product a method) of its own on
+        the instance: a timer or a hook that somebody put there is to be called in every layer."""
         return None
 
     def own_tensors(self) -> "list[torch.Tensor]":

@@ -33,7 +33,10 @@ class PreNormBlock(Block):
     def launch_signature(self):
         if type(self) is not PreNormBlock or self.feed_forward is None or not hasattr(self.feed_forward, "last_product"):
             return None
-        signatures = tuple(p.launch_signature() for p in self.parts())
+        if "forward" in self.__dict__:
+            return None
+        signatures = (self.mixer_norm.launch_signature(), self.mixer.launch_signature(),
+                      self.feed_forward_norm.launch_signature(), self.feed_forward.launch_signature())
         return None if None in signatures else signatures
 
     def own_tensors(self):

@@ -144,3 +144,8 @@ class Linear:
             ops.cast(y, narrow)
             y = narrow
         return y
+
+
+def plain_products(first, second) -> bool:
+    """Whether both are this class's products, with nothing of the instance's own in the place of a method."""
+    return type(first) is Linear and type(second) is Linear and len(first.__dict__) == 4 and len(second.__dict__) == 4

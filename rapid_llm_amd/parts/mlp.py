@@ -15,12 +15,14 @@ experts behind a softmax router.
 
 from __future__ import annotations
 
+import operator
+
 import torch
 
 from ..kernels import ops
 from .base import FEED_FORWARDS, FeedForward, ParamSpec, Source
 from .lazy import LayerSum, Returned, ScaledRows, Term, plain
-from .linear import Linear
+from .linear import Linear, plain_products
 
 
 class SwiGLU(FeedForward):
@@ -82,9 +84,10 @@ class SwiGLU(FeedForward):
         return self.gate_up.takes_scaled_rows()
 
     def launch_signature(self):
-        if type(self) is not SwiGLU:  # a kind derived from this one may do more
+        # a kind derived from this one may do more
+        if type(self) is not SwiGLU or "forward" in self.__dict__ or not plain_products(self.gate_up, self.down):
             return None
-        return (self.hidden_size, self.intermediate_size, self.limit, self.alpha, self.activation, self.has_bias)
+        return _FIXED(self)
 
     def own_tensors(self) -> list[torch.Tensor]:
         # the bias of gate and up is added by the activation
@@ -108,6 +111,10 @@ class SwiGLU(FeedForward):
         act = torch.empty((x.shape[0], self.intermediate_size), dtype=gu.dtype, device=x.device)
         ops.swiglu(gu, act, self.limit, self.alpha, activation=self.activation, bias=self.gate_up_bias)
         return self.down.deferred(act, ctx)
+
+
+# what the launches of a SwiGLU depend on beside its tensors
+_FIXED = operator.attrgetter("hidden_size", "intermediate_size", "limit", "alpha", "activation", "has_bias")
 
 
 class TwoLayer(FeedForward):

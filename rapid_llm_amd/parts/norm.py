@@ -54,7 +54,7 @@ class RMSNorm(Norm):
         self.dtype = runtime.dtype
 
     def launch_signature(self):
-        if type(self) is not RMSNorm:  # a kind derived from this one may do more
+        if type(self) is not RMSNorm or "forward" in self.__dict__:  # a kind derived from this one may do more
             return None
         return (self.size, self.eps, self.dtype)
 

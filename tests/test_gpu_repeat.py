@@ -76,3 +76,41 @@ def test_layers_that_differ_are_not_repeated(monkeypatch):
     few = ModelRunner({**BASE, "num_hidden_layers": 3}, EngineConfig(dtype="bfloat16", max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
                       load_format="random")
     assert _run(few, 2048, monkeypatch)[1] == []
+
+
+@pytest.mark.parametrize("where", ["mixer", "mixer_norm", "feed_forward_norm", "feed_forward", "block", "class", "product"])
+def test_a_forward_put_in_the_place_of_a_layers_own_is_called(where, monkeypatch):
+    """A timer or a hook around one layer's part, its block, its product or a part's class: called in every step."""
+    from rapid_llm_amd import EngineConfig, ModelRunner, StepEntry
+    from rapid_llm_amd.parts.mlp import SwiGLU
+
+    runner = ModelRunner(BASE, EngineConfig(dtype="bfloat16", max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
+                         load_format="random", weight_norm_std=0.1)
+    block, calls = runner.model.blocks[3], []
+    target, name = {"block": (block, "forward"), "class": (SwiGLU, "forward"), "product": (block.feed_forward.down, "deferred")}.get(
+        where, (getattr(block, where, None), "forward"))
+    inner = getattr(target, name)
+    step = lambda: runner.step([StepEntry("a", [5, 6, 7, 8, 9], [4])], use_graph=False).clone()
+    want = step()
+    runner.finish("a")
+    monkeypatch.setattr(target, name, lambda *args, **kw: calls.append(0) or inner(*args, **kw))
+    assert torch.equal(step(), want) and len(calls) == (5 if where == "class" else 1)
+
+
+def test_every_layer_is_timed(monkeypatch):
+    """Regions around parts count every layer of every step, prompts and single tokens."""
+    from collections import Counter
+
+    from rapid_llm_amd import EngineConfig, ModelRunner, StepEntry
+    from rapid_llm_amd.engine.timeline import Timeline, instrument
+
+    runner = ModelRunner(BASE, EngineConfig(dtype="bfloat16", max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
+                         load_format="random")
+    timeline = Timeline()
+    instrument(runner, timeline)
+    runner.step([StepEntry("a", [5, 6, 7, 8, 9], [4])])
+    for token in (3, 4, 5):
+        runner.step([StepEntry("a", [token], [0])])
+    seen = Counter((r.phase, r.name) for r in timeline.collect())
+    for name in ("mixer norm (RMSNorm)", "mixer (GQAAttention)", "feed-forward norm (RMSNorm)", "feed-forward (SwiGLU)"):
+        assert seen["steps with prompt portions", name] == 5 and seen["decode steps", name] == 15

@@ -1,0 +1,61 @@
+"""Which steps are launched by making the second layer's launches again: the rule, without a device."""
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from rapid_llm_amd.config.qwen3 import Qwen3Config
+from rapid_llm_amd.models.causal_lm import CausalLM
+from rapid_llm_amd.models.qwen3 import build_qwen3_spec
+
+BODY = dict(
+    architectures=["Qwen3ForCausalLM"], model_type="qwen3", num_hidden_layers=5, hidden_size=64, num_attention_heads=4,
+    num_key_value_heads=2, head_dim=16, intermediate_size=128, vocab_size=97, rope_theta=10000.0, rms_norm_eps=1e-6,
+    tie_word_embeddings=True, max_position_embeddings=128, hidden_act="silu", attention_bias=False,
+)
+
+
+def _model():
+    model = CausalLM(build_qwen3_spec(Qwen3Config.from_dict(BODY)))
+    for block in model.blocks:
+        block.mixer_norm.dtype = block.feed_forward_norm.dtype = torch.bfloat16
+    caches = [SimpleNamespace(group_id=0, page_size=16, owns_pages=True, pages={"k": None, "v": None}, states={}) for _ in range(5)]
+    return model, caches
+
+
+def _alike(model, caches, tokens=37, static=()):
+    return model._alike(SimpleNamespace(num_tokens=tokens, static=dict(static)), caches)
+
+
+def test_layers_of_one_model_are_alike():
+    model, caches = _model()
+    assert _alike(model, caches)
+    assert not _alike(model, caches, static={"decode_only_tokens": 1}) and not _alike(model, caches, tokens=1 << 20)
+    model.blocks[4].feed_forward.limit = 7.0
+    assert not _alike(model, caches)
+
+
+@pytest.mark.parametrize("layer", [0, 1, 4])
+@pytest.mark.parametrize("where", ["mixer", "mixer_norm", "feed_forward_norm", "feed_forward", "block", "product", "kind"])
+def test_a_layer_with_a_function_of_its_own_is_called(where, layer):
+    """What somebody puts in the place of a part's or a product's own method runs in every step."""
+    model, caches = _model()
+    block = model.blocks[layer]
+    if where == "product":
+        block.mixer.qkv.product = lambda x, out_dtype=None: x
+    elif where == "kind":
+        block.feed_forward.down = SimpleNamespace(weight=None, bias=None)
+    else:
+        target = block if where == "block" else getattr(block, where)
+        target.forward = target.forward
+    assert not _alike(model, caches)
+
+
+@pytest.mark.parametrize("where", ["mixer", "mixer_norm", "feed_forward", "block"])
+def test_a_class_whose_forward_was_replaced_is_called(where, monkeypatch):
+    model, caches = _model()
+    kind = type(model.blocks[0] if where == "block" else getattr(model.blocks[0], where))
+    inner = kind.forward
+    monkeypatch.setattr(kind, "forward", lambda self, *args: inner(self, *args))
+    assert not _alike(model, caches)
