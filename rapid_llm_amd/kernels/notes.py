@@ -43,6 +43,11 @@ class _Library:
         return call
 
 
+def _extent(t: torch.Tensor) -> int:
+    """Bytes from a tensor's first element to behind its last."""
+    return t.element_size() * (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride()))) if t.numel() else 0
+
+
 class Notes:
     def __init__(self) -> None:
         self.calls: list[tuple] = []  # (the library's function, its arguments), as made
@@ -74,10 +79,13 @@ class Notes:
                 if at in column:
                     return None  # two layers share it: a pointer does not say whose it is
                 column[at] = (j, back)
-                spans.append((at, at + t.numel() * t.element_size()))
+                spans.append((at, at + _extent(t)))
         spans.sort()
         starts = [s for s, _ in spans]
         before, after = (t.data_ptr() for t in carried)
+        if carried[0].stride() != carried[1].stride() or carried[0].shape != carried[1].shape:
+            return None
+        behind = before + _extent(carried[0])
         calls = np.zeros(len(self.calls), dtype=_CALL)
         slots = []
         for c, (entry, args) in enumerate(self.calls):
@@ -87,8 +95,8 @@ class Notes:
                     value = 0 if arg is None else arg.value or 0
                     if value in column:
                         slots.append((c, len(ints), *column[value]))
-                    elif value == before:
-                        value = after
+                    elif before <= value < behind:
+                        value += after - before  # (a launch may begin at any of its rows)
                     elif value:
                         i = bisect.bisect_right(starts, value) - 1
                         if i >= 0 and value < spans[i][1]:

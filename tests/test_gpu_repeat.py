@@ -114,3 +114,46 @@ def test_every_layer_is_timed(monkeypatch):
     seen = Counter((r.phase, r.name) for r in timeline.collect())
     for name in ("mixer norm (RMSNorm)", "mixer (GQAAttention)", "feed-forward norm (RMSNorm)", "feed-forward (SwiGLU)"):
         assert seen["steps with prompt portions", name] == 5 and seen["decode steps", name] == 15
+
+
+@pytest.fixture
+def biased():
+    """BASE with biases on every projection: a down projection's is added by the norm behind, float32 too."""
+    import dataclasses
+
+    from rapid_llm_amd.config.qwen3 import Qwen3Config
+    from rapid_llm_amd.config.registry import register_architecture, unregister_architecture
+    from rapid_llm_amd.models.qwen3 import build_qwen3_spec
+
+    def spec(cfg):
+        whole = build_qwen3_spec(cfg)
+        more = lambda part, **kw: dataclasses.replace(part, params={**part.params, **kw})
+        return dataclasses.replace(whole, layers=tuple(
+            dataclasses.replace(layer, mixer=more(layer.mixer, qkv_bias=True, o_bias=True),
+                                feed_forward=more(layer.feed_forward, bias=True)) for layer in whole.layers))
+
+    register_architecture("BiasedQwen3", Qwen3Config, spec)
+    yield {**BASE, "architectures": ["BiasedQwen3"], "model_type": "BiasedQwen3"}
+    unregister_architecture("BiasedQwen3")
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_repeated_layers_with_biases_and_products_cut_into_launches(biased, dtype, monkeypatch):
+    """What a layer leaves is then read from several of its rows on."""
+    from rapid_llm_amd import EngineConfig, ModelRunner
+    from rapid_llm_amd.kernels import ops
+
+    runner = ModelRunner(biased, EngineConfig(dtype=dtype, max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
+                         load_format="random", weight_norm_std=0.1)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    for name, t in runner.params.items():
+        if "bias" in name:
+            t.normal_(0.0, 0.1, generator=gen)
+    monkeypatch.setattr(ops, "f32_wide", lambda m, n, k, units: 96 if m > 64 and k % 32 == 0 else 0)
+    monkeypatch.setattr(ops, "_F32_MOST_PIECES", 1 << 20)
+    assert ops._f32_piece_rows(640, 512) == 512  # the long portion's down projection: two launches
+    want, _ = _run(runner, 0, monkeypatch)
+    got, ran = _run(runner, 2048, monkeypatch)
+    assert len(ran) >= (7 if dtype == "float32" else 3) and all(ran)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

@@ -61,6 +61,21 @@ def test_calls_are_made_again_with_every_layers_tensors():
         assert list(args) == want
 
 
+def test_pointers_into_the_carried_tensor_move_with_it():
+    """A product cut into launches of fewer rows points at rows of what the layer before left, a view with rows apart too."""
+    for wide, cols in ((torch.zeros(2, 6, 4), 4), (torch.zeros(2, 6, 9), 4)):
+        x0, x1 = wide[0][:, :cols], wide[1][:, :cols]
+        layers, log = [[torch.zeros(8)] for _ in range(4)], []
+        behind = x0.data_ptr() + 4 * (5 * x0.stride(0) + cols)
+        places = [x0.data_ptr(), x0[2:].data_ptr(), x0[5:].data_ptr() + 4]
+        notes = _noted(_Lib(rl_x=_entry(log, [P, P, P, P])), "rl_x", *(P(p) for p in places), P(behind))
+        assert _again(notes, layers, (x0, x1)) == 0
+        step = x1.data_ptr() - x0.data_ptr()
+        assert log[1:] == [(*(p + step for p in places), behind)] * 2
+    x2 = torch.zeros(6, 8)[:, :4]  # rows elsewhere
+    assert notes.plan(layers, (x0, x2)) is None
+
+
 def test_a_call_that_fails_ends_it():
     log = []
     fail = ctypes.CFUNCTYPE(I, I)(lambda n: log.append(n) or (7 if len(log) > 2 else 0))
