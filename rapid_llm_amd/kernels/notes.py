@@ -37,7 +37,7 @@ class _Library:
         entry = getattr(self._lib, name)
 
         def call(*args):
-            self._notes.last = (entry, args)
+            self._notes.last = (name, entry, args)
             return entry(*args)
 
         return call
@@ -59,12 +59,13 @@ class Notes:
         return _Library(self, lib)
 
     def made(self, what: str) -> None:
-        """The call just made was a launch (calls that only ask a library something are not reported)."""
-        if self.last is None:
-            self.complete = False  # of a library whose calls are not noted
+        """The call of the entry point ``what`` just made was a launch (calls that only ask a library something are not
+        reported)."""
+        if self.last is None or self.last[0] != what:
+            self.complete = False  # of a library whose calls are not noted: the last noted call is another one
         else:
-            self.calls.append(self.last)
-            self.last = None
+            self.calls.append(self.last[1:])
+        self.last = None
 
     def plan(self, tables, carried):
         """(calls, slots, table of pointers) for ``rl_repeat_calls``, or ``None`` where a call does not fit."""

@@ -200,7 +200,7 @@ def repeat_launches(notes: Notes, tables: list[list[torch.Tensor]], carried: tup
             ctypes.c_void_p(calls.ctypes.data), len(calls), ctypes.c_void_p(slots.ctypes.data), len(slots),
             ctypes.c_void_p(table.ctypes.data), table.shape[1], 2, len(tables),
         ),
-        "a repeated launch",
+        "rl_repeat_calls",
     )
     return True
 

@@ -84,7 +84,7 @@ def test_a_call_that_fails_ends_it():
     assert _again(notes, layers, (torch.zeros(1), torch.zeros(1))) == 7 and log == [5, 5, 5]
 
 
-@pytest.mark.parametrize("why", ["inside", "shared", "argument", "many", "unknown"])
+@pytest.mark.parametrize("why", ["inside", "shared", "argument", "many", "unknown", "asked"])
 def test_what_cannot_be_made_again(why):
     layers = [[torch.zeros(8)] for _ in range(4)]
     lib = _Lib(rl_x=lambda *a: 0)
@@ -101,7 +101,21 @@ def test_what_cannot_be_made_again(why):
     if why == "unknown":
         with notes_module.taking_notes() as notes:
             ops._ok(0, "a launch of a library that is not noted")
+    if why == "asked":  # a question to a noted library, then a launch of one that is not
+        with notes_module.taking_notes() as notes:
+            notes.library(_Lib(rl_rows=lambda: 16)).rl_rows()
+            ops._ok(0, "rl_x")
     assert notes.plan(layers, (torch.zeros(1), torch.zeros(1))) is None
+
+
+def test_every_launch_is_reported_under_its_entry_points_name():
+    """What tells a launch from a question: a check's text is the name of the entry point whose code it checks."""
+    import ast
+    import inspect
+
+    checks = [n for n in ast.walk(ast.parse(inspect.getsource(ops))) if isinstance(n, ast.Call) and getattr(n.func, "id", "") == "_ok"]
+    named = [(n.args[0].func.attr, n.args[1].value) for n in checks]
+    assert len(named) > 50 and all(entry == text for entry, text in named)
 
 
 def test_notes_end_with_their_block_and_are_the_threads_own():
