@@ -67,6 +67,13 @@ class Notes:
             self.calls.append(self.last[1:])
         self.last = None
 
+    def give_up(self) -> None:
+        """Something was launched that cannot be noted: nothing will be made again, and no tensor is kept for it."""
+        self.complete = False
+        self.last = None
+        self.calls.clear()
+        self.tensors.clear()
+
     def plan(self, tables, carried):
         """(calls, slots, table of pointers) for ``rl_repeat_calls``, or ``None`` where a call does not fit."""
         if not self.complete or not self.calls:
@@ -115,6 +122,13 @@ class Notes:
             calls[c]["ints"][: len(ints)] = ints
             calls[c]["floats"][: len(floats)] = floats
         return calls, np.array(slots, dtype=np.int32).reshape(-1, 4), table
+
+
+def unnoted() -> None:
+    """To be called beside every kernel on a step's way that is not this package's (a product or a copy of torch's)."""
+    if noting.notes is not None:
+        noting.notes.give_up()
+        noting.notes = None
 
 
 @contextlib.contextmanager

@@ -15,7 +15,7 @@ from typing import Optional
 import torch
 
 from . import build
-from .notes import Notes, noting
+from .notes import Notes, noting, unnoted
 from .upload import upload_ints
 
 F32, BF16 = 0, 1
@@ -183,6 +183,14 @@ def _ok(code: int, what: str) -> None:
     if code != 0:
         reason = {1: "an argument the kernel refuses", 2: "the launch failed"}.get(code, "unknown")
         raise KernelError(f"{what}: error {code} ({reason})")
+
+
+def whole_rows(x: torch.Tensor) -> torch.Tensor:
+    """``x`` with its rows side by side: itself, or a copy."""
+    if x.is_contiguous():
+        return x
+    unnoted()
+    return x.contiguous()
 
 
 def repeat_launches(notes: Notes, tables: list[list[torch.Tensor]], carried: tuple[torch.Tensor, torch.Tensor]) -> bool:
@@ -1436,7 +1444,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
     if x.dim() == 2 and not x.is_contiguous() and not (
         x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and x.shape[0] <= SKINNY_MAX_ROWS
     ):
-        x = x.contiguous()
+        x = whole_rows(x)
     if x.is_contiguous():
         _need(x, "x", torch.bfloat16)
     elif not x.is_cuda or x.dtype != torch.bfloat16:
@@ -1459,7 +1467,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
             "rl_gemm_skinny",
         )
         return out
-    x = x.contiguous()
+    x = whole_rows(x)
     if scaled is not None:
         raise KernelError(f"scaled rows need the few-row product: {m} rows over {k}")
     plan = rows_plan(m, n, k, swiglu=False)
@@ -1512,6 +1520,7 @@ def library_product(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = t
     1,024 channels and 429 of 4,096, the one product takes 137 and 351 (65 rows: 99 / 88 and 294 / 275)."""
     global library_products
     library_products += 1
+    unnoted()
     if out_dtype == torch.float32:
         return torch.mm(x, w.t(), out_dtype=torch.float32)
     return torch.matmul(x, w.t())
@@ -1758,6 +1767,7 @@ def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     n = w.shape[0]
     plan = block_plan(m, n, k, "runs") if k == w.shape[1] else None
     if plan is not None and not _aligned(x, w):  # (a view that begins inside a unit of 16 bytes)
+        unnoted()
         x, w = (t if _aligned(t) else t.clone() for t in (x, w))
     if plan is not None:
         return _block(x, w, torch.empty((plan[2], m, n), dtype=torch.float32, device=x.device), "runs", plan)

@@ -210,10 +210,9 @@ class CausalLM:
         for place, li in enumerate(self.order):
             block = self.blocks[li]
             if alike and place == 1:
-                products = ops.library_products
                 with taking_notes() as notes:
                     left = block.forward(residual, delta, ctx, caches[1])
-                    last = self._repeat(notes, delta, left, caches) if ops.library_products == products else None
+                last = self._repeat(notes, delta, left, caches) if notes.complete else None
                 if last is not None:
                     delta = last
                     break

@@ -133,7 +133,7 @@ class Linear:
         if w.dtype == torch.float32:
             if x.dtype != torch.float32:
                 wide = torch.empty(x.shape, dtype=torch.float32, device=x.device)
-                ops.cast(x.contiguous(), wide)
+                ops.cast(ops.whole_rows(x), wide)
                 x = wide
             y = torch.empty((rows, self.out_features), dtype=torch.float32, device=x.device)
             ops.gemm_f32(x, w, y)

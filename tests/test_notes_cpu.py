@@ -128,3 +128,21 @@ def test_notes_end_with_their_block_and_are_the_threads_own():
         t.join()
         assert notes_module.noting.notes is not None
     assert seen == [None] and notes_module.noting.notes is None
+
+
+@pytest.mark.parametrize("what", ["library", "copy", "nothing"])
+def test_what_is_not_this_packages_ends_the_notes(what):
+    """A product or a copy of torch's between the launches: nothing is made again, and no tensor is kept for it."""
+    layers = [[torch.zeros(8)] for _ in range(4)]
+    lib, x = _Lib(rl_x=_entry([], [P])), torch.zeros(4, 8)
+    with notes_module.taking_notes() as notes:
+        notes.library(lib).rl_x(ops._p(layers[1][0]))
+        ops._ok(0, "rl_x")
+        if what == "library":
+            ops.library_product(x, x)
+        ops.whole_rows(x[:, :4] if what == "copy" else x)
+        notes.library(lib).rl_x(ops._p(x))
+        ops._ok(0, "rl_x")
+    left = what == "nothing"
+    assert (notes.plan(layers, (torch.zeros(1), torch.zeros(1))) is not None) == left
+    assert notes.complete == left and bool(notes.tensors) == left
