@@ -79,6 +79,8 @@ class Notes:
         if not self.complete or not self.calls:
             return None
         table = np.array([[t.data_ptr() for t in row] for row in tables], dtype=np.int64)
+        if ((table ^ table[0]) & 15).any():
+            return None  # which kernel runs may depend on where a tensor begins
         column: dict[int, tuple[int, int]] = {}
         spans = []
         for back, row in ((1, tables[0]), (0, tables[1])):
@@ -91,7 +93,7 @@ class Notes:
         spans.sort()
         starts = [s for s, _ in spans]
         before, after = (t.data_ptr() for t in carried)
-        if carried[0].stride() != carried[1].stride() or carried[0].shape != carried[1].shape:
+        if carried[0].stride() != carried[1].stride() or carried[0].shape != carried[1].shape or (before ^ after) & 15:
             return None
         behind = before + _extent(carried[0])
         calls = np.zeros(len(self.calls), dtype=_CALL)

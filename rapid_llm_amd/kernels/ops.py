@@ -195,10 +195,11 @@ def whole_rows(x: torch.Tensor) -> torch.Tensor:
 
 def repeat_launches(notes: Notes, tables: list[list[torch.Tensor]], carried: tuple[torch.Tensor, torch.Tensor]) -> bool:
     """Make the launches that ``notes`` holds, those of place 1 of a run order, again for the places behind it, from
-    native code.  ``tables``: every place's own tensors (weights, pages), one row a place, alike in shape and type;
+    native code.  ``tables``: every place's own tensors (weights, pages), one row a place, alike in shape and type, rows side by side;
     what place 1 took from place 0's row, place i takes from place i - 1's.  ``carried``: the tensor that place 1
     read (from any of its rows on) of what place 0 left, and the one in its stead that it left itself.  False, with nothing launched, where the
-    launches do not say which layer they are of (a pointer into the middle of a tensor)."""
+    launches do not say which layer they are of (a pointer into the middle of a tensor), or where the tensors do not
+    begin alike inside a unit of 16 bytes."""
     plan = notes.plan(tables, carried)
     if plan is None:
         return False

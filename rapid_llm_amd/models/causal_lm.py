@@ -193,8 +193,8 @@ class CausalLM:
         if before.shape != after.shape or before.dtype != after.dtype:
             return None
         tables = [self.blocks[li].own_tensors() + list(cache.pages.values()) for li, cache in zip(self.order, caches)]
-        kinds = [[(t.shape, t.dtype) for t in row] for row in tables]
-        if any(k != kinds[0] for k in kinds[1:]) or not ops.repeat_launches(notes, tables, (before, after)):
+        kinds = [[(t.shape, t.dtype, t.is_contiguous()) for t in row] for row in tables]
+        if not all(k[2] for k in kinds[0]) or any(k != kinds[0] for k in kinds[1:]) or not ops.repeat_launches(notes, tables, (before, after)):
             return None
         return DeferredProduct(self.blocks[self.order[-1]].feed_forward.last_product, after) if lazy else after
 

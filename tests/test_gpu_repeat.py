@@ -178,3 +178,23 @@ def test_weights_that_are_copied_are_every_layers_own(monkeypatch):
     got, _ = _run(runner, 2048, monkeypatch)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("how,dtype", [("odd", "bfloat16"), ("odd", "float32"), ("apart", "float32")])
+def test_a_layer_whose_weight_lies_otherwise(how, dtype, monkeypatch):
+    """One layer's product begins inside a unit of 16 bytes (float32: or has its rows apart): its launches are its own."""
+    from rapid_llm_amd import EngineConfig, ModelRunner
+
+    runner = ModelRunner({**BASE, "hidden_size": 1024, "intermediate_size": 3072},
+                         EngineConfig(dtype=dtype, max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
+                         load_format="random", weight_norm_std=0.1)
+    gate_up = runner.model.blocks[3].feed_forward.gate_up
+    rows, k = gate_up.weight.shape
+    room = torch.empty((rows + 1) * (k + 4), dtype=gate_up.weight.dtype, device="cuda")
+    other = room[1 : 1 + rows * k].view(rows, k) if how == "odd" else room.view(rows + 1, k + 4)[:rows, :k]
+    gate_up.weight = other.copy_(gate_up.weight)
+    want, _ = _run(runner, 0, monkeypatch)
+    got, ran = _run(runner, 2048, monkeypatch)
+    assert not any(ran)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

@@ -63,7 +63,7 @@ def test_calls_are_made_again_with_every_layers_tensors():
 
 def test_pointers_into_the_carried_tensor_move_with_it():
     """A product cut into launches of fewer rows points at rows of what the layer before left, a view with rows apart too."""
-    for wide, cols in ((torch.zeros(2, 6, 4), 4), (torch.zeros(2, 6, 9), 4)):
+    for wide, cols in ((torch.zeros(2, 6, 4), 4), (torch.zeros(2, 6, 10), 4)):
         x0, x1 = wide[0][:, :cols], wide[1][:, :cols]
         layers, log = [[torch.zeros(8)] for _ in range(4)], []
         behind = x0.data_ptr() + 4 * (5 * x0.stride(0) + cols)
@@ -84,7 +84,7 @@ def test_a_call_that_fails_ends_it():
     assert _again(notes, layers, (torch.zeros(1), torch.zeros(1))) == 7 and log == [5, 5, 5]
 
 
-@pytest.mark.parametrize("why", ["inside", "shared", "argument", "many", "unknown", "asked"])
+@pytest.mark.parametrize("why", ["inside", "shared", "argument", "many", "unknown", "asked", "address", "carried"])
 def test_what_cannot_be_made_again(why):
     layers = [[torch.zeros(8)] for _ in range(4)]
     lib = _Lib(rl_x=lambda *a: 0)
@@ -105,7 +105,15 @@ def test_what_cannot_be_made_again(why):
         with notes_module.taking_notes() as notes:
             notes.library(_Lib(rl_rows=lambda: 16)).rl_rows()
             ops._ok(0, "rl_x")
-    assert notes.plan(layers, (torch.zeros(1), torch.zeros(1))) is None
+    carried = (torch.zeros(1), torch.zeros(1))
+    if why == "address":  # a layer's tensor begins inside a unit of 16 bytes, the second's does not
+        notes = _noted(_Lib(rl_x=_entry([], [P])), "rl_x", *args)
+        assert notes.plan(layers, carried) is not None
+        layers[3][0] = torch.zeros(9)[1:]
+    if why == "carried":
+        notes = _noted(_Lib(rl_x=_entry([], [P])), "rl_x", *args)
+        carried = (torch.zeros(1), torch.zeros(2)[1:])
+    assert notes.plan(layers, carried) is None
 
 
 def test_every_launch_is_reported_under_its_entry_points_name():
