@@ -1501,7 +1501,7 @@ def gemm_bf16_wide(x: torch.Tensor, w: torch.Tensor, scaled=None) -> torch.Tenso
     if scaled is not None:
         raise KernelError(f"scaled rows need the few-row product: {m} rows over {k}")
     if m <= MID_MAX_ROWS and mid_runs(w.shape[0], k) == 1:
-        return gemm_bf16_parts(x, w)[0]
+        return _mid_parts(x, w, 1)[0]
     _need(x, "x", torch.bfloat16)
     _need(w, "w", torch.bfloat16, (None, k))
     return library_product(x, w, torch.float32)
@@ -1762,19 +1762,28 @@ def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x[M,K] @ w[N,K]^T`` for 17 to 192 rows, or as many as :func:`block_plan` says, as float32 runs of K,
     ``[runs, M, N]``: their sum is the product.  For products whose result goes into the residual: the norm that
     follows adds the runs (``add_rmsnorm_parts``)."""
-    _need(x, "x", torch.bfloat16)
-    _need(w, "w", torch.bfloat16)
     m, k = x.shape
     n = w.shape[0]
     plan = block_plan(m, n, k, "runs") if k == w.shape[1] else None
-    if plan is not None and not _aligned(x, w):  # (a view that begins inside a unit of 16 bytes)
-        unnoted()
-        x, w = (t if _aligned(t) else t.clone() for t in (x, w))
     if plan is not None:
+        _need(x, "x", torch.bfloat16)
+        _need(w, "w", torch.bfloat16)
+        if not _aligned(x, w):  # (a view that begins inside a unit of 16 bytes)
+            unnoted()
+            x, w = (t if _aligned(t) else t.clone() for t in (x, w))
         return _block(x, w, torch.empty((plan[2], m, n), dtype=torch.float32, device=x.device), "runs", plan)
     ks = mid_runs(n, k)
     if k != w.shape[1] or m > MID_MAX_ROWS or ks < 1:
         raise KernelError(f"gemm_bf16_parts does not take x {tuple(x.shape)}, w {tuple(w.shape)}")
+    return _mid_parts(x, w, ks)
+
+
+def _mid_parts(x: torch.Tensor, w: torch.Tensor, ks: int) -> torch.Tensor:
+    """The mid-size product of up to 192 rows in ``ks`` runs of K (:func:`mid_runs`)."""
+    _need(x, "x", torch.bfloat16)
+    m, k = x.shape
+    _need(w, "w", torch.bfloat16, (None, k))
+    n = w.shape[0]
     parts = torch.empty((ks, m, n), dtype=torch.float32, device=x.device)
     _ok(core().rl_gemm_mid_parts(_p(x), _p(w), _p(parts), m, n, k, k, k, ks, _stream()), "rl_gemm_mid_parts")
     return parts

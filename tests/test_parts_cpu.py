@@ -1,5 +1,6 @@
 """What parts decide on the host, without a device."""
 
+import pytest
 import torch
 
 from rapid_llm_amd.parts.linear import Linear
@@ -270,6 +271,39 @@ def test_spans_of_the_float32_attention():
                 tiles, held = rows * -(-group // 16), min(16, group)
                 n = ops.f32_spans(tiles, nkv, 128, longest, 0, held)
                 assert ops.f32_states_bytes(rows, nq, nkv, 128, longest, 0) == tiles * nkv * n * 4 * -(-held * 130 // 32) * 128
+
+
+@pytest.mark.parametrize("units", [40, 64, 128, 256, 304])
+def test_a_product_left_in_float32_is_one_run_of_k(units, monkeypatch):
+    """What enters a recurrence in 32 bits is a whole sum, whatever the rule for products that a norm adds cuts K into."""
+    from types import SimpleNamespace
+
+    from rapid_llm_amd.kernels import ops
+
+    asked = []
+
+    class Library:
+        def __getattr__(self, name):
+            return lambda *args: asked.append((name, args)) or 0
+
+    monkeypatch.setattr(ops, "chip", lambda: SimpleNamespace(units=units))
+    monkeypatch.setattr(ops, "core", Library)
+    monkeypatch.setattr(ops, "_stream", lambda: None)
+    monkeypatch.setattr(ops, "_need", lambda *args: None)
+    cut = 0
+    for m, n, k in ((129, 4160, 6144), (129, 2112, 6144), (65, 1088, 8192), (192, 8192, 9728), (100, 512, 512)):
+        x, w = (torch.empty((rows, k), dtype=torch.bfloat16, device="meta") for rows in (m, n))
+        w.data_ptr = x.data_ptr = lambda: 0
+        if ops.mid_runs(n, k) != 1:
+            continue
+        found = ops.block_plan(m, n, k, "runs")
+        cut += found is not None and found[2] > 1
+        monkeypatch.setattr(ops, "_p", lambda t: t)
+        got = ops.gemm_bf16_wide(x, w)
+        assert got.shape == (m, n) and got.dtype == torch.float32
+        name, args = asked.pop()
+        assert name == "rl_gemm_mid_parts" and args[8] == 1 and not asked
+    assert cut > 0 or units >= 256  # (there the two rules meet nowhere)
 
 
 def test_plans_of_the_float32_product():
