@@ -1719,6 +1719,13 @@ def _aligned(*tensors: torch.Tensor) -> bool:
     return all(t.data_ptr() % 16 == 0 for t in tensors)
 
 
+def block_reads(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the many-row product takes the operands of its ``"runs"`` form as they are: a plan, rows side by side,
+    whole units of 16 bytes."""
+    return (block_plan(x.shape[0], w.shape[0], w.shape[1], "runs") is not None and _aligned(x, w)
+            and x.is_contiguous() and w.is_contiguous())
+
+
 def _block(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str, plan: tuple[int, int, int]) -> torch.Tensor:
     m, k = x.shape
     n = out.shape[-1]
@@ -1758,13 +1765,14 @@ def _mid_runs(n: int, k: int, units: int) -> int:
     return ks
 
 
-def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor, copies: bool = True) -> torch.Tensor:
     """``x[M,K] @ w[N,K]^T`` for 17 to 192 rows, or as many as :func:`block_plan` says, as float32 runs of K,
     ``[runs, M, N]``: their sum is the product.  For products whose result goes into the residual: the norm that
-    follows adds the runs (``add_rmsnorm_parts``)."""
+    follows adds the runs (``add_rmsnorm_parts``).  Operands that begin inside a unit of 16 bytes are copied where
+    the many-row product takes them; without ``copies`` the mid-size product reads them as they are."""
     m, k = x.shape
     n = w.shape[0]
-    plan = block_plan(m, n, k, "runs") if k == w.shape[1] else None
+    plan = block_plan(m, n, k, "runs") if k == w.shape[1] and (copies or _aligned(x, w)) else None
     if plan is not None:
         _need(x, "x", torch.bfloat16)
         _need(w, "w", torch.bfloat16)

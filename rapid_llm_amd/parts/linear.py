@@ -79,11 +79,11 @@ class Linear:
             return False
         if rows <= ops.MID_MAX_ROWS and ops.mid_runs(self.out_features, self.in_features) > 0:
             return True
-        return ops.block_plan(rows, self.out_features, self.in_features, "runs") is not None
+        return ops.block_reads(x, self.weight)
 
     def partial_sums(self, x: torch.Tensor) -> torch.Tensor:
         """``[runs, M, out]`` float32 whose sum over the runs is ``x W^T`` (without the bias)."""
-        return ops.gemm_bf16_parts(x, self.weight)
+        return ops.gemm_bf16_parts(x, self.weight, copies=False)
 
     def deferred(self, x: torch.Tensor, ctx=None):
         """The product, or a :class:`DeferredProduct` of it where one of this product's kernels

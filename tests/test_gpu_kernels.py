@@ -1311,6 +1311,31 @@ def test_many_row_product_through_its_rule(m, n, k, kind):
     assert torch.all((got.float() - want).abs() <= 2.0**-8 * (1.1 * (gate * up).abs() + 2 * want.abs()) + 1e-6)
 
 
+def test_operands_inside_a_unit_of_16_bytes_are_not_copied_by_a_layers_product():
+    """A product over long sums whose weight or rows the many-row product does not take as they are: the mid-size one up
+    to 192 rows, a plain product beyond; rows apart as well."""
+    from rapid_llm_amd.parts.lazy import DeferredProduct
+    from rapid_llm_amd.parts.linear import Linear
+
+    ops = _ops()
+    n, k, gen = 2560, 9728, torch.Generator().manual_seed(5)
+    room = (torch.randn(n * k + 8, generator=gen) / math.sqrt(k)).bfloat16().to(DEV)
+    x = torch.randn((520, k + 8), generator=gen).bfloat16().to(DEV)
+    even, odd = Linear(k, n), Linear(k, n)
+    even.bind(room[: n * k].view(n, k))
+    odd.bind(room[1 : 1 + n * k].view(n, k))
+    assert odd.weight.data_ptr() % 16 and not even.weight.data_ptr() % 16
+    few, many, apart = x[:150, :k].contiguous(), x[:, :k].contiguous(), x[:, :k]
+    assert isinstance(even.deferred(many), DeferredProduct) and ops.block_plan(150, n, k, "runs") is not None
+    assert torch.equal(odd.partial_sums(few), ops._mid_parts(few, odd.weight, ops.mid_runs(n, k)))
+    want = many.float() @ odd.weight.float().T
+    bound = k * 2.0**-24 * float((many.float().abs() @ odd.weight.float().abs().T).max())
+    for linear, rows, exact in ((odd, many, want), (even, apart, many.float() @ even.weight.float().T)):
+        got = linear.deferred(rows)
+        assert isinstance(got, torch.Tensor)  # rounded to bfloat16 once more
+        assert torch.all((got.float() - exact).abs() <= 2.0**-8 * exact.abs() + bound)
+
+
 # rows, result columns, K, SwiGLU, float32 result: every number of tiles a workgroup may hold
 # (1, 2, 3, 6 tiles; 2, 3, 5 pairs), shares that leave some workgroups a tile short, more tiles
 # than one round of workgroups holds (the vocabulary), 17 to 64 rows around the blocks of 16,
