@@ -29,7 +29,8 @@
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32;
 typedef u32 u32x2 __attribute__((ext_vector_type(2)));
@@ -170,15 +171,33 @@ __device__ __forceinline__ void read_b(bf16x8 (&w)[NA][2][2], u32 a0, u32 a1) {
     }
 }
 
-// silu(g) * u: exp(-g) as a power of two whose argument's rounding is put back (the argument is cut at
-// +-90, where the power is already 0 or infinite), so that what is left are the roundings of the
-// power, the sum, the reciprocal and the products: an ulp each
+// silu(g) * u of bfloat16 numbers below SILU_WIDE in magnitude.  Their product is exact and comes first; exp(-g) is a
+// power of two whose argument's rounding is put back; the quotient is by a reciprocal and one Newton step.  No step
+// leaves the normal range (87 log2(e) < 126).  Over all gates and eight factors, in ulp of float32, worst and root mean
+// square: 2.4 and 0.20; g / (1 + expf(-g)) * u, the other kernels' form, 2.5 and 0.22.  That form in its place, microseconds at
+// 8,192 rows: 24,576 x 4,096 1,158 against 1,117, 6,144 x 1,024 99 against 90.
+#define SILU_WIDE 87.f
+#define SILU_WIDE_BITS 0x42ae  // as bfloat16
 __device__ __forceinline__ float silu_times(float g, float u) {
-    const float c = __builtin_amdgcn_fmed3f(g, -90.f, 90.f);
-    const float t = c * -1.44269502162933349609375f;                        // -log2(e), its high part
-    const float r = fmaf(c, -1.925963033500011079e-8f, fmaf(c, -1.44269502162933349609375f, -t));
+    const float t = g * -1.44269502162933349609375f;  // -log2(e), its high part
+    const float r = fmaf(g, -1.925963033500011079e-8f, fmaf(g, -1.44269502162933349609375f, -t));
     const float p = __builtin_amdgcn_exp2f(t);
-    return g * __builtin_amdgcn_rcpf(1.f + fmaf(p, r * 0.693147182464599609375f, p)) * u;
+    const float d = 1.f + fmaf(p, r * 0.693147182464599609375f, p);
+    const float y = __builtin_amdgcn_rcpf(d), n = g * u, q = n * y;
+    return fmaf(fmaf(-d, q, n), y, q);
+}
+// the same for any two, by the numbers alone (never by what stands beside them)
+__device__ __forceinline__ float silu_times_any(float g, float u) {
+    return fmaxf(fabsf(g), fabsf(u)) < SILU_WIDE ? silu_times(g, u) : g / (1.f + expf(-g)) * u;
+}
+
+// four numbers rounded to bfloat16, two an instruction; `most` keeps the largest magnitudes' bits (NaN above infinity)
+__device__ __forceinline__ f32x4 rounded(f32x4 v, u16x2& most) {
+    const u32 a = __builtin_bit_cast(u32, __builtin_convertvector(__builtin_shufflevector(v, v, 0, 1), bf16x2));
+    const u32 b = __builtin_bit_cast(u32, __builtin_convertvector(__builtin_shufflevector(v, v, 2, 3), bf16x2));
+    most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, a & 0x7fff7fffu));
+    most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, b & 0x7fff7fffu));
+    return __builtin_bit_cast(f32x4, (u32x4){a << 16, a & 0xffff0000u, b << 16, b & 0xffff0000u});
 }
 
 enum BlockOut { OUT_RUNS = 1, OUT_GLU = 2 };
@@ -344,22 +363,20 @@ __global__ __launch_bounds__(BT) void gemm_block_kernel(BlockArgs a) {
     char* base = (char*)a.out + ((GLU ? 0 : (size_t)split * a.M * a.ldo) + (size_t)m0 * a.ldo + n0) * elem;
     const int rows = min(64 * NX, a.M - m0), cols = a.N - n0;
     auto rs = __builtin_amdgcn_make_buffer_rsrc(base, 0, (u32)rows * (u32)a.ldo * elem, 0x00020000);
-#pragma unroll
-    for (int x = 0; x < NX; ++x) {
+    // rows and columns that do not exist fall off the records
+    auto finish = [&](int x, auto any_c) {
         const int row = 64 * x + 16 * xi + r16;
         bf16x8 o;
 #pragma unroll
         for (int u = 0; u < NW; ++u) {
-            // rows and columns that do not exist fall off the records
             if constexpr (GLU) {
                 const bool pair = (u | 1) < NW;
                 const int col = 16 * NW * wi + (pair ? 16 * (u & ~1) + 8 * g + 4 * (u & 1) : 16 * u + 4 * g);
                 const bool in = row < rows && col < cols;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    // the activation reads its operands rounded to bfloat16, as where the product's result is stored first
-                    const float gate = (float)(__bf16)acc[u][0][x][i], up = (float)(__bf16)acc[u][1][x][i];
-                    o[4 * (u & 1) + i] = (__bf16)silu_times(gate, up);
+                    const float gate = acc[u][0][x][i], up = acc[u][1][x][i];
+                    o[4 * (u & 1) + i] = (__bf16)(decltype(any_c)::value ? silu_times_any(gate, up) : silu_times(gate, up));
                 }
                 if (pair && (u & 1))
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rs, in ? (row * a.ldo + col - 4) * 2 : -1, 0, 0);
@@ -375,6 +392,23 @@ __global__ __launch_bounds__(BT) void gemm_block_kernel(BlockArgs a) {
                                                            in ? (row * a.ldo + col + 4 * t) * 4 : -1, 0, 0);
             }
         }
+    };
+    u16x2 most = {0, 0};
+    if constexpr (GLU) {
+        // the activation reads its operands rounded to bfloat16, as where the product's result is stored first
+#pragma unroll
+        for (int x = 0; x < NX; ++x)
+#pragma unroll
+            for (int u = 0; u < NW; ++u)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) acc[u][t][x] = rounded(acc[u][t][x], most);
+    }
+    if (__builtin_expect(!GLU || !__any(max(most[0], most[1]) >= SILU_WIDE_BITS), 1)) {
+#pragma unroll
+        for (int x = 0; x < NX; ++x) finish(x, Int<0>{});
+    } else {
+#pragma unroll
+        for (int x = 0; x < NX; ++x) finish(x, Int<1>{});
     }
 #endif
 }

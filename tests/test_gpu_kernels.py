@@ -1262,6 +1262,44 @@ def test_many_row_product_every_tile(nw, nx, shape):
         assert torch.equal(other[1:], got[1:])
 
 
+def test_many_row_products_activation_over_every_gate():
+    """silu(gate) * up of every normal bfloat16 gate against 64 bits: the result is rounded to bfloat16 once, from float32
+    numbers 2.6 ulp off at most.  What one element is does not depend on what stands beside it."""
+    ops = _ops()
+    bits = torch.arange(65536, dtype=torch.int32).to(torch.uint16)
+    gates = bits.view(torch.bfloat16)
+    gates = gates[(gates.abs() >= 2.0**-126) & gates.isfinite()]
+    ups = torch.tensor([1.0, -1.3359375, 0.01953125, 86.5, 100.0], dtype=torch.bfloat16)
+
+    def run(gates, ups):
+        n, m = -(-gates.numel() // 8) * 8, ups.numel()
+        x, w = torch.zeros(m, 64, dtype=torch.bfloat16), torch.zeros(2 * n, 64, dtype=torch.bfloat16)
+        x[:, 0], x[:, 1], w[: gates.numel(), 0], w[n:, 1] = 1.0, ups, gates, 1.0
+        out = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+        xd, wd = x.to(DEV), w.to(DEV)
+        assert ops.core().rl_gemm_block(ops._p(xd), ops._p(wd), ops._p(out), m, n, 64, 64, 64, n, 2, 4, 4, 1, ops._stream()) == 0
+        return out[:, : gates.numel()].cpu()
+
+    got, g, u = run(gates, ups), gates.double(), ups.double()[:, None]
+    exact = g / (1.0 + torch.exp(-g)) * u
+    binade = torch.exp2(torch.floor(torch.log2(exact.abs().clamp_min(2.0**-126))))
+    # where exp(-g) is beyond float32 (g < -88.7) the result is a zero
+    lost = torch.where(g < -88.7, exact.abs(), 0.0)
+    fits = exact.abs() < 3.38e38
+    assert torch.all(((got.double() - exact).abs() <= binade * (2.0**-8 + 2.6 * 2.0**-23) + lost)[fits])
+    assert torch.all(got[~fits].isinf() | (got[~fits].abs() > 3.37e38))
+    few = (gates.abs() < 87.0).nonzero()[:, 0]  # no element that is not: the other path of the epilogue
+    assert torch.equal(run(gates[few], ups[:4]), got[:4][:, few])
+    odd = torch.tensor([float("inf"), -float("inf"), float("nan"), 1.0], dtype=torch.bfloat16)
+    for gate in odd:
+        gu, plain = torch.stack([gate, odd[3]])[None].to(DEV), torch.empty((1, 1), dtype=torch.bfloat16, device=DEV)
+        ops.swiglu(gu, plain)
+        x, w = torch.zeros(1, 64, dtype=torch.bfloat16, device=DEV), torch.ones(16, 64, dtype=torch.bfloat16, device=DEV)
+        x[0, 0], w[:8, 0], out = 1.0, gate, torch.empty((1, 8), dtype=torch.bfloat16, device=DEV)
+        assert ops.core().rl_gemm_block(ops._p(x), ops._p(w), ops._p(out), 1, 8, 64, 64, 64, 8, 2, 2, 2, 1, ops._stream()) == 0
+        torch.testing.assert_close(out, plain.expand(1, 8), rtol=0, atol=0, equal_nan=True)
+
+
 @pytest.mark.parametrize("m", [49, 64])
 def test_gate_and_up_of_49_to_64_rows(m):
     """Where a round of the many-row product's workgroups holds the columns: the gated product of the gate and up matrices."""
