@@ -25,6 +25,9 @@ class _Thread(threading.local):
 
 
 noting = _Thread()
+#: The notes that threads are taking, none of them most of the time: a launch asks for its thread's own only where this is
+#: not empty (a dozen questions a launch, 50 ns each for a thread's own, 10 for this).
+taking: "list[Notes]" = []
 
 
 class _Library:
@@ -128,7 +131,7 @@ class Notes:
 
 def unnoted() -> None:
     """To be called beside every kernel on a step's way that is not this package's (a product or a copy of torch's)."""
-    if noting.notes is not None:
+    if taking and noting.notes is not None:
         noting.notes.give_up()
         noting.notes = None
 
@@ -137,8 +140,10 @@ def unnoted() -> None:
 def taking_notes():
     """Note the launches that this thread makes inside the block."""
     outer, notes = noting.notes, Notes()
+    taking.append(notes)
     noting.notes = notes
     try:
         yield notes
     finally:
         noting.notes = outer
+        taking.remove(notes)

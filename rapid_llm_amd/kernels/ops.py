@@ -15,7 +15,7 @@ from typing import Optional
 import torch
 
 from . import build
-from .notes import Notes, noting, unnoted
+from .notes import Notes, noting, taking, unnoted
 from .upload import upload_ints
 
 F32, BF16 = 0, 1
@@ -73,8 +73,7 @@ def core() -> ctypes.CDLL:
     global _core
     if _core is None:
         _core = build.load(build.core_library())
-    notes = noting.notes
-    return _core if notes is None else notes.library(_core)
+    return noting.notes.library(_core) if taking and noting.notes is not None else _core
 
 
 def attention_lib(head_dim: int) -> ctypes.CDLL:
@@ -86,8 +85,7 @@ def attention_lib(head_dim: int) -> ctypes.CDLL:
         if lib.rl_attn_f32_span() != _F32_SPAN:
             raise KernelError(f"the float32 attention walks spans of {lib.rl_attn_f32_span()} keys, the launch rules expect {_F32_SPAN}")
         _attn[head_dim] = lib
-    notes = noting.notes
-    return lib if notes is None else notes.library(lib)
+    return noting.notes.library(lib) if taking and noting.notes is not None else lib
 
 
 _attn_tile: dict[tuple[int, int], ctypes.CDLL] = {}
@@ -148,9 +146,8 @@ def _stream() -> ctypes.c_void_p:
 
 
 def _p(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    notes = noting.notes
-    if notes is not None:
-        notes.tensors.append(t)
+    if taking and noting.notes is not None:
+        noting.notes.tensors.append(t)
     return ctypes.c_void_p(0 if t is None else t.data_ptr())
 
 
@@ -178,7 +175,7 @@ def _need(t: torch.Tensor, name: str, dtype: torch.dtype | None = None, shape=No
 
 
 def _ok(code: int, what: str) -> None:
-    if noting.notes is not None:
+    if taking and noting.notes is not None:
         noting.notes.made(what)
     if code != 0:
         reason = {1: "an argument the kernel refuses", 2: "the launch failed"}.get(code, "unknown")

@@ -154,3 +154,16 @@ def test_what_is_not_this_packages_ends_the_notes(what):
     left = what == "nothing"
     assert (notes.plan(layers, (torch.zeros(1), torch.zeros(1))) is not None) == left
     assert notes.complete == left and bool(notes.tensors) == left
+
+
+def test_launches_outside_of_notes_do_not_look_for_a_threads_own(monkeypatch):
+    class Nobody:
+        @property
+        def notes(self):
+            raise AssertionError("looked for")
+
+    with notes_module.taking_notes():
+        pass
+    monkeypatch.setattr(ops, "noting", Nobody())
+    assert not notes_module.taking
+    ops.core(), ops._p(torch.zeros(1)), ops._ok(0, "rl_x"), ops.library_product(torch.zeros(2, 2), torch.zeros(2, 2))
