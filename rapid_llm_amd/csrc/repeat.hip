@@ -20,9 +20,6 @@ struct RlSlot {
     int call, arg, column, back;
 };
 
-extern "C" int rl_repeat_max_ints() { return RL_CALL_INTS; }
-extern "C" int rl_repeat_max_floats() { return RL_CALL_FLOATS; }
-
 #if defined(__x86_64__) && defined(__linux__)
 // System V AMD64 calling convention: integers and pointers go to six registers and then, eight bytes each, to the
 // stack in their order, floats to eight registers of their own (no more are passed here); the callee reads as many
@@ -30,6 +27,10 @@ extern "C" int rl_repeat_max_floats() { return RL_CALL_FLOATS; }
 typedef long long I;
 typedef int (*RlEntry)(I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, float, float,
                        float, float, float, float, float, float);
+
+// what a call holds at most, 0 on hosts whose calls are not known here
+extern "C" int rl_repeat_max_ints() { return RL_CALL_INTS; }
+extern "C" int rl_repeat_max_floats() { return RL_CALL_FLOATS; }
 
 static int make_call(const RlCall& c) {
     const long long* i = c.ints;
@@ -39,6 +40,9 @@ static int make_call(const RlCall& c) {
                               i[29], i[30], i[31], f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]);
 }
 #else
+extern "C" int rl_repeat_max_ints() { return 0; }
+extern "C" int rl_repeat_max_floats() { return 0; }
+
 static int make_call(const RlCall&) { return RL_ERR_ARG; }
 #endif
 

@@ -15,7 +15,7 @@ from typing import Optional
 import torch
 
 from . import build
-from .notes import Notes, noting, taking, unnoted
+from .notes import MAX_FLOATS, MAX_INTS, Notes, noting, taking, unnoted
 from .upload import upload_ints
 
 F32, BF16 = 0, 1
@@ -195,14 +195,17 @@ def repeat_launches(notes: Notes, tables: list[list[torch.Tensor]], carried: tup
     native code.  ``tables``: every place's own tensors (weights, pages), one row a place, alike in shape and type, rows side by side;
     what place 1 took from place 0's row, place i takes from place i - 1's.  ``carried``: the tensor that place 1
     read (from any of its rows on) of what place 0 left, and the one in its stead that it left itself.  False, with nothing launched, where the
-    launches do not say which layer they are of (a pointer into the middle of a tensor), or where the tensors do not
-    begin alike inside a unit of 16 bytes."""
+    launches do not say which layer they are of (a pointer into the middle of a tensor), where the tensors do not
+    begin alike inside a unit of 16 bytes, and on hosts whose calls the library does not know how to make."""
+    lib = core()
+    if (lib.rl_repeat_max_ints(), lib.rl_repeat_max_floats()) != (MAX_INTS, MAX_FLOATS):
+        return False
     plan = notes.plan(tables, carried)
     if plan is None:
         return False
     calls, slots, table = plan
     _ok(
-        core().rl_repeat_calls(
+        lib.rl_repeat_calls(
             ctypes.c_void_p(calls.ctypes.data), len(calls), ctypes.c_void_p(slots.ctypes.data), len(slots),
             ctypes.c_void_p(table.ctypes.data), table.shape[1], 2, len(tables),
         ),

@@ -167,3 +167,15 @@ def test_launches_outside_of_notes_do_not_look_for_a_threads_own(monkeypatch):
     monkeypatch.setattr(ops, "noting", Nobody())
     assert not notes_module.taking
     ops.core(), ops._p(torch.zeros(1)), ops._ok(0, "rl_x"), ops.library_product(torch.zeros(2, 2), torch.zeros(2, 2))
+
+
+def test_a_host_whose_calls_are_not_known_repeats_nothing(monkeypatch):
+    """The library then says that a call holds nothing: the layers make their own launches."""
+    layers = [[torch.zeros(8)] for _ in range(4)]
+    log = []
+    notes = _noted(_Lib(rl_x=_entry(log, [P])), "rl_x", P(layers[1][0].data_ptr()))
+    carried = (torch.zeros(1), torch.zeros(1))
+    assert ops.repeat_launches(notes, layers, carried) and len(log) == 3
+    nowhere = _Lib(rl_repeat_max_ints=lambda: 0, rl_repeat_max_floats=lambda: 0, rl_repeat_calls=lambda *args: 1)
+    monkeypatch.setattr(ops, "core", lambda: nowhere)
+    assert not ops.repeat_launches(notes, layers, carried) and len(log) == 3
