@@ -1698,6 +1698,16 @@ def _block_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int
     return best[1]
 
 
+def product_bytes(m: int, w: torch.Tensor) -> int:
+    """About what ``m`` rows times a weight take: the rows, the result, and what the product keeps beside it."""
+    n, k = w.shape
+    if w.dtype == torch.float32:
+        return 4 * m * (n + k) + f32_product_bytes(m, n, k)
+    plan = block_plan(m, n, k, "runs")
+    runs = plan[2] if plan is not None else mid_runs(n, k) if SKINNY_MAX_ROWS < m <= MID_MAX_ROWS else 0
+    return 2 * m * (n + k) + 4 * m * n * runs
+
+
 def block_few_plan(m: int, n: int, k: int, units: int | None = None) -> tuple[int, int, int] | None:
     """The plan of the same product for the gate and up matrices at 49 to 64 rows, ``None`` where the kernel that keeps X in
     registers is the faster one.

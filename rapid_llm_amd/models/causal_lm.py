@@ -32,8 +32,12 @@ from .spec import ModelSpec
 
 
 # Tokens up to which a step's layers behind the second are launched from what the second launched: beyond, the device has
-# more to do than the host in any model, and the noted layer keeps its temporary tensors until all are launched
+# more to do than the host in any model.
 REPEAT_MAX_TOKENS = 2048
+# The noted layer keeps its temporary tensors until all layers are launched, where a layer alone gives each back
+# behind its last use: bytes of them, as estimated, up to which that is done.  A quarter of what the engine leaves for a step's
+# activations, so that no step comes to need more than there is; steps that are this large are not bound by the host.
+REPEAT_MAX_BYTES = 1 << 28
 
 
 class CausalLM:
@@ -180,8 +184,18 @@ class CausalLM:
             return False
         if any(b.launch_signature() != first for b in blocks):
             return False
+        if sum(ops.product_bytes(ctx.num_tokens, t) for t in blocks[0].own_tensors() if t.dim() == 2) > REPEAT_MAX_BYTES:
+            return False
         kinds = {(c.group_id, c.page_size, c.owns_pages, len(c.pages), len(c.states)) for c in caches}
         return len(kinds) == 1 and all(c.owns_pages and not c.states for c in caches)
+
+    def _second(self, residual, delta, ctx, caches):
+        """The second layer of a step whose layers are alike, and those behind it where its launches say enough: what is
+        left to add, and whether that is the last layer's.  What its notes kept is given back here."""
+        with taking_notes() as notes:
+            left = self.blocks[self.order[1]].forward(residual, delta, ctx, caches[1])
+        last = self._repeat(notes, delta, left, caches) if notes.complete else None
+        return (left, False) if last is None else (last, True)
 
     def _repeat(self, notes, delta, left, caches):
         """The layers behind the second, launched from the notes of the second's launches; ``delta`` is what the first
@@ -208,16 +222,12 @@ class CausalLM:
         delta = None
         alike = self._alike(ctx, caches)
         for place, li in enumerate(self.order):
-            block = self.blocks[li]
             if alike and place == 1:
-                with taking_notes() as notes:
-                    left = block.forward(residual, delta, ctx, caches[1])
-                last = self._repeat(notes, delta, left, caches) if notes.complete else None
-                if last is not None:
-                    delta = last
+                delta, whole = self._second(residual, delta, ctx, caches)
+                if whole:
                     break
-                delta = left
                 continue
+            block = self.blocks[li]
             if self.mixes is not None and self.mixes.at(place):
                 delta = settle(residual, delta)
                 if delta is not None:

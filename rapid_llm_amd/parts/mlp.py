@@ -110,6 +110,7 @@ class SwiGLU(FeedForward):
         gu = self.gate_up(x)
         act = torch.empty((x.shape[0], self.intermediate_size), dtype=gu.dtype, device=x.device)
         ops.swiglu(gu, act, self.limit, self.alpha, activation=self.activation, bias=self.gate_up_bias)
+        del gu  # the widest tensor of a layer: what the down product keeps beside it may lie there
         return self.down.deferred(act, ctx)
 
 
@@ -339,6 +340,7 @@ class RoutedExperts(FeedForward):
             act = torch.empty((x.shape[0], self.inner), dtype=hidden.dtype, device=x.device)
             ops.swiglu(hidden, act, self.limit, self.alpha, route=weights, expert_ff=self.expert_size,
                        route_input=self.scale_input)
+            del hidden
             return self.down.deferred(act, ctx)
         ops.unary_act(hidden, hidden, self.activation, weights, self.expert_size)
         return self.down.deferred(hidden, ctx)

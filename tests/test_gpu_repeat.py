@@ -198,3 +198,30 @@ def test_a_layer_whose_weight_lies_otherwise(how, dtype, monkeypatch):
     assert not any(ran)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_what_a_noted_layer_kept_is_given_back_before_the_end_of_the_step(dtype, monkeypatch):
+    """Behind the last layer no more is allocated than where every layer makes its own launches, and the step's most is
+    what the estimate says beyond that."""
+    from rapid_llm_amd import EngineConfig, ModelRunner, StepEntry
+    from rapid_llm_amd.kernels import ops
+    from rapid_llm_amd.models import causal_lm
+
+    body = {**BASE, "hidden_size": 1024, "num_attention_heads": 16, "num_key_value_heads": 8, "head_dim": 128, "intermediate_size": 3072}
+    runner = ModelRunner(body, EngineConfig(dtype=dtype, max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
+                         load_format="random")
+    norm, at_end = runner.model.final_norm, []
+    inner = norm.forward
+    monkeypatch.setattr(norm, "forward", lambda *args, **kw: at_end.append(torch.cuda.memory_allocated()) or inner(*args, **kw))
+    tokens, most = random_tokens(180, runner.vocab_size, 1), []
+    for limit in (0, 2048):
+        monkeypatch.setattr(causal_lm, "REPEAT_MAX_TOKENS", limit)
+        for _ in range(2):
+            torch.cuda.reset_peak_memory_stats()
+            runner.step([StepEntry("a", tokens, [179])])
+            runner.finish("a")
+        most.append(torch.cuda.max_memory_allocated())
+    assert at_end[3] <= at_end[1]
+    weights = [t for t in runner.model.blocks[0].own_tensors() if t.dim() == 2]
+    assert most[1] - most[0] <= 1.5 * sum(ops.product_bytes(180, w) for w in weights)

@@ -16,10 +16,13 @@ BODY = dict(
 )
 
 
-def _model():
-    model = CausalLM(build_qwen3_spec(Qwen3Config.from_dict(BODY)))
+def _model(dtype=torch.bfloat16, **change):
+    model = CausalLM(build_qwen3_spec(Qwen3Config.from_dict({**BODY, **change})))
     for block in model.blocks:
-        block.mixer_norm.dtype = block.feed_forward_norm.dtype = torch.bfloat16
+        for norm in (block.mixer_norm, block.feed_forward_norm):
+            norm.dtype, norm.weight = dtype, torch.empty(norm.size, device="meta")
+        for linear in (block.mixer.qkv, block.mixer.o, block.feed_forward.gate_up, block.feed_forward.down):
+            linear.weight = torch.empty((linear.out_features, linear.in_features), dtype=dtype, device="meta")
     caches = [SimpleNamespace(group_id=0, page_size=16, owns_pages=True, pages={"k": None, "v": None}, states={}) for _ in range(5)]
     return model, caches
 
@@ -59,3 +62,18 @@ def test_a_class_whose_forward_was_replaced_is_called(where, monkeypatch):
     inner = kind.forward
     monkeypatch.setattr(kind, "forward", lambda self, *args: inner(self, *args))
     assert not _alike(model, caches)
+
+
+def test_steps_whose_temporary_tensors_are_large_are_not_repeated():
+    """The noted layer keeps them all: a float32 step of a large model lets its layers give them back one by one."""
+    from rapid_llm_amd.models.causal_lm import REPEAT_MAX_BYTES, REPEAT_MAX_TOKENS
+
+    large = dict(hidden_size=5120, num_attention_heads=64, num_key_value_heads=8, head_dim=128, intermediate_size=25600)
+    model, caches = _model(torch.float32, **large)
+    assert _alike(model, caches, 17) and not _alike(model, caches, REPEAT_MAX_TOKENS)
+    small = dict(hidden_size=1024, num_attention_heads=16, num_key_value_heads=8, head_dim=128, intermediate_size=3072)
+    for dtype, tokens in ((torch.float32, 512), (torch.bfloat16, 1024)):
+        assert _alike(*_model(dtype, **small), tokens)
+    # gate and up, the widest, is the most that is left alive: its result alone is within the bound
+    rows = max(m for m in range(1, REPEAT_MAX_TOKENS) if _alike(model, caches, m))
+    assert 4 * rows * 2 * 25600 < REPEAT_MAX_BYTES
