@@ -81,30 +81,31 @@ class Notes:
         """(calls, slots, table of pointers) for ``rl_repeat_calls``, or ``None`` where a call does not fit."""
         if not self.complete or not self.calls:
             return None
-        table = np.array([[t.data_ptr() for t in row] for row in tables], dtype=np.int64)
+        pointers = [[t.data_ptr() for t in row] for row in tables]
+        table = np.array(pointers, dtype=np.int64)
         if ((table ^ table[0]) & 15).any():
             return None  # which kernel runs may depend on where a tensor begins
         column: dict[int, tuple[int, int]] = {}
         spans = []
         for back, row in ((1, tables[0]), (0, tables[1])):
             for j, t in enumerate(row):
-                at = int(table[1 - back, j])
+                at = pointers[1 - back][j]
                 if at in column:
                     return None  # two layers share it: a pointer does not say whose it is
                 column[at] = (j, back)
-                spans.append((at, at + _extent(t)))
+                spans.append((at, at + t.nbytes))
         spans.sort()
         starts = [s for s, _ in spans]
         before, after = (t.data_ptr() for t in carried)
         if carried[0].stride() != carried[1].stride() or carried[0].shape != carried[1].shape or (before ^ after) & 15:
             return None
         behind = before + _extent(carried[0])
-        calls = np.zeros(len(self.calls), dtype=_CALL)
-        slots = []
+        entries, all_ints, all_floats, slots = [], [], [], []
         for c, (entry, args) in enumerate(self.calls):
             ints, floats = [], []
             for arg in args:
-                if arg is None or isinstance(arg, ctypes.c_void_p):
+                kind = type(arg)
+                if kind is ctypes.c_void_p or arg is None:
                     value = 0 if arg is None else arg.value or 0
                     if value in column:
                         slots.append((c, len(ints), *column[value]))
@@ -115,17 +116,19 @@ class Notes:
                         if i >= 0 and value < spans[i][1]:
                             return None
                     ints.append(value)
-                elif isinstance(arg, ctypes.c_float):
+                elif kind is int or kind is bool:
+                    ints.append(arg)
+                elif kind is ctypes.c_float:
                     floats.append(arg.value)
-                elif isinstance(arg, int):
-                    ints.append(int(arg))
                 else:
                     return None
             if len(ints) > MAX_INTS or len(floats) > MAX_FLOATS:
                 return None
-            calls[c]["entry"] = ctypes.cast(entry, ctypes.c_void_p).value
-            calls[c]["ints"][: len(ints)] = ints
-            calls[c]["floats"][: len(floats)] = floats
+            entries.append(ctypes.cast(entry, ctypes.c_void_p).value)
+            all_ints.append(ints + [0] * (MAX_INTS - len(ints)))
+            all_floats.append(floats + [0.0] * (MAX_FLOATS - len(floats)))
+        calls = np.zeros(len(entries), dtype=_CALL)
+        calls["entry"], calls["ints"], calls["floats"] = entries, all_ints, all_floats
         return calls, np.array(slots, dtype=np.int32).reshape(-1, 4), table
 
 

@@ -220,9 +220,8 @@ class CausalLM:
         # in place)
         first = residual.clone() if self.mixes is not None or self.returns else None
         delta = None
-        alike = self._alike(ctx, caches)
         for place, li in enumerate(self.order):
-            if alike and place == 1:
+            if place == 1 and self._alike(ctx, caches):  # (asked while the device has the first layer to do)
                 delta, whole = self._second(residual, delta, ctx, caches)
                 if whole:
                     break

@@ -330,10 +330,12 @@ class GQAAttention(PackedMixer):
         return _FIXED(self)
 
     def own_tensors(self) -> list[torch.Tensor]:
-        norms = [w for w in (self.q_norm_w, self.k_norm_w) if w is not None]
-        if not self.qk_norm_weights:
-            norms = norms[:1]  # one vector of ones for both
-        return self.qkv.own_tensors() + self.o.own_tensors() + norms
+        own = self.qkv.own_tensors() + self.o.own_tensors()
+        if self.q_norm_w is not None:
+            own.append(self.q_norm_w)
+        if self.k_norm_w is not None and self.k_norm_w is not self.q_norm_w:  # (one vector of ones may serve both)
+            own.append(self.k_norm_w)
+        return own
 
     def run(self, packed, col0, out, out_col, out_scale, ctx, cache):
         """The heads between the two products (layers with one of the options beyond plain attention)."""

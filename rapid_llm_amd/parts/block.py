@@ -40,7 +40,8 @@ class PreNormBlock(Block):
         return None if None in signatures else signatures
 
     def own_tensors(self):
-        return [t for p in self.parts() for t in p.own_tensors()]
+        return [*self.mixer_norm.own_tensors(), *self.mixer.own_tensors(),
+                *self.feed_forward_norm.own_tensors(), *self.feed_forward.own_tensors()]
 
     def forward(self, residual, delta, ctx, cache):
         x = run_norm(self.mixer_norm, residual, delta, ctx, consumer=self.mixer)

@@ -44,7 +44,7 @@ class Linear:
 
     def own_tensors(self) -> list[torch.Tensor]:
         """What a launch of this product may point at that is its own."""
-        return [t for t in (self.weight, self.bias) if t is not None]
+        return [self.weight] if self.bias is None else [self.weight, self.bias]
 
     # ---- folding a neighbouring norm into the product (decode steps, bfloat16) ----------
     def skinny(self, x) -> bool:

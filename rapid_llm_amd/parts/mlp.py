@@ -90,9 +90,10 @@ class SwiGLU(FeedForward):
         return _FIXED(self)
 
     def own_tensors(self) -> list[torch.Tensor]:
-        # the bias of gate and up is added by the activation
-        bias = [self.gate_up_bias] if self.has_bias else []
-        return self.gate_up.own_tensors() + self.down.own_tensors() + bias
+        own = self.gate_up.own_tensors() + self.down.own_tensors()
+        if self.has_bias:
+            own.append(self.gate_up_bias)  # (added by the activation)
+        return own
 
     @property
     def last_product(self) -> Linear:
