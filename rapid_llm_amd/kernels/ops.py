@@ -1618,7 +1618,7 @@ def _tile_applies(m: int, weight_rows: int, k: int, cols: int) -> bool:
     1,024 rows: 13.5 / 21.3 and 25.7 / 32.6), but a step of a few hundred tokens of so small a
     model is bound by the host, where a call of the library costs 18 us and one of this kernel
     6: a 512-token prompt of the Qwen3-0.6B shape 5.4 -> 4.2 ms.  Hence up to 512 rows.  The packed gate and up
-    matrices go on to the many-row product from 129 rows on (6,144 x 1,024 at 64 / 128 / 160 / 256 / 512 rows, the tile
+    matrices may go on to the many-row product from 129 rows on (:func:`_tile_gives_way`; 6,144 x 1,024 at 64 / 128 / 160 / 256 / 512 rows, the tile
     product first: 10.7 / 11.8, 11.7 / 12.3, 14.7 / 11.9, 15.3 / 12.3, 19.3 / 12.5).  Up to 64 rows, where
     :func:`rows_plan` has a plan, operands are aligned and the result is bfloat16, the kernel that keeps X in registers comes
     first (over weights from memory at 17 / 37 / 64 rows, the tile product first: 4,096 x 1,024 7.1 / 4.9, 8.0 / 5.9, 8.9 / 6.5;
@@ -1632,6 +1632,21 @@ def _tile_applies(m: int, weight_rows: int, k: int, cols: int) -> bool:
         and cols * (weight_rows // cols) >= _TILE_MIN_COLS
         and weight_rows * k <= _TILE_MAX_WEIGHTS
     )
+
+
+@functools.lru_cache(maxsize=4096)
+def _tile_gives_way(m: int, inter: int, k: int, units: int) -> bool:
+    """Whether packed gate and up matrices that the one-launch tile product takes go to the many-row product: from 129 rows
+    on, where that has tiles for three eighths of the units (weights from memory, the tile product first: 3,072 columns
+    of 1,024 k at 129 / 256 / 512 rows, 96 to 192 tiles, 13.3 / 12.8, 15.9 / 13.9, 20.4 / 14.2; 2,048 columns, 64 to 128
+    tiles, 10.7 / 12.4, 12.2 / 13.6, 16.2 / 13.6; 1,024 columns, 32 to 64 tiles, 9.5 / 11.6, 11.3 / 11.6, 11.4 / 11.6)."""
+    plan = _block_plan(m, inter, k, "gated", units) if m > TILE_GATED_MAX_ROWS else None
+    return plan is not None and 8 * _block_tiles(m, inter, "gated", plan) >= 3 * units
+
+
+def _block_tiles(m: int, n: int, kind: str, plan: tuple[int, int, int]) -> int:
+    """Workgroups a run of K has under a plan of :func:`block_plan`."""
+    return -(-n // ((32 if kind == "gated" else 64) * plan[0])) * -(-m // (64 * plan[1]))
 
 
 # The many-row product's tiles (pieces of 64 weight rows x pieces of 64 rows of X) and what a launch of each
@@ -1857,7 +1872,7 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
         _need(w_gate_up, "w_gate_up", torch.bfloat16, (two_i, k))
         plan = rows_plan(m, inter, k, swiglu=True)
         tile = _tile_applies(m, two_i, k, inter) and not (plan is not None and k >= 1024 and _aligned(x, w_gate_up))
-        if (not tile or m > TILE_GATED_MAX_ROWS) and activation == "silu" and limit <= 0 and bias is None:
+        if (not tile or _tile_gives_way(m, inter, k, chip().units)) and activation == "silu" and limit <= 0 and bias is None:
             block = block_plan(m, inter, k, "gated") or block_few_plan(m, inter, k)
             if block is not None and _aligned(x, w_gate_up):
                 return _block(x, w_gate_up, torch.empty((m, inter), dtype=torch.bfloat16, device=x.device), "gated", block)

@@ -211,6 +211,18 @@ def test_where_the_many_row_product_applies():
             assert per * (found[2] - 1) < k // 64
 
 
+def test_small_gate_and_up_matrices_leave_the_tile_product_for_a_filled_chip():
+    from rapid_llm_amd.kernels import ops
+
+    goes = lambda *a: ops._tile_gives_way(*a, 256)
+    assert goes(129, 3072, 1024) and goes(512, 2048, 1024) and goes(400, 1536, 512)
+    assert not goes(128, 3072, 1024) and not goes(256, 2048, 1024) and not goes(512, 1024, 1024) and not goes(129, 1536, 1024)
+    for inter in range(512, 3585, 64):
+        for m in (129, 200, 300, 512):
+            plan = ops.block_plan(m, inter, 1024, "gated", units=256)
+            assert goes(m, inter, 1024) == (8 * ops._block_tiles(m, inter, "gated", plan) >= 3 * 256)
+
+
 def test_launch_rules_follow_the_number_of_compute_units():
     """Every launch rule takes the chip's geometry from one place on the host
     (``ops.chip()``; without a device the chip the rules were measured on), so that a part
