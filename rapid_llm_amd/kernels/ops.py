@@ -1735,11 +1735,16 @@ def block_few_plan(m: int, n: int, k: int, units: int | None = None) -> tuple[in
     registers is the faster one.
 
     That one holds at most three pairs of tiles there, so 256 workgroups of the 8B shape read all of X; here 192 do.
-    Microseconds at 64 rows, that kernel first: 8B 52.2 / 48.1, 4B 29.6 / 28.6, 1.7B 20.3 / 19.8, 0.6B 10.3 / 11.2; at 48 rows
-    45.3 / 47.7, 28.2 / 26.8, 17.6 / 19.0.  Hence from 6,144 columns of 2,048 k on, as long as a round of
-    workgroups holds them."""
+    A round of workgroups has to hold them, and enough of them to be at work: five eighths of the units up to 4,096 k and
+    seven eighths beyond.  Microseconds at 64 rows over weights from memory, that kernel first: 12,288 columns of 4,096 k
+    50.7 / 47.9, 11,008 of 2,048 28.7 / 26.1, 14,336 of 5,120 93.8 / 63.1; with fewer 9,728 of 2,560 31.4 / 32.3, 8,192 of
+    4,096 38.0 / 43.7, 7,168 of 2,048 21.7 / 23.3, 12,288 of 5,120 58.4 / 61.4.  At 6,144 columns of 2,048 k that kernel has
+    as few (20.4 / 20.1); at 48 rows it holds more (8B 45.3 / 47.7)."""
     units = chip().units if units is None else units
-    if not 48 < m <= ROWS_MAX_ROWS or k < 2048 or k % 64 or n % 8 or n < 6144 or -(-n // 64) > units:
+    tiles = -(-n // 64)
+    if not 48 < m <= ROWS_MAX_ROWS or k < 2048 or k % 64 or n % 8 or n < 6144 or tiles > units:
+        return None
+    if 8 * tiles < (5 if k <= 4096 else 7) * units and (k > 2048 or 5 * tiles > 2 * units):
         return None
     return (2, 1, 1) if (2 * n + 256) * k * 2 <= 0x7FFFFFFF else None
 

@@ -200,6 +200,8 @@ def test_where_the_many_row_product_applies():
     few = lambda *a: ops.block_few_plan(*a, units=256)
     assert few(49, 12288, 4096) == few(64, 6144, 2048) == (2, 1, 1)
     assert few(48, 12288, 4096) is None and few(65, 12288, 4096) is None and few(64, 3072, 1024) is None
+    assert few(64, 9728, 2560) is None and few(49, 8192, 4096) is None and few(64, 7168, 2048) is None and few(64, 12288, 5120) is None
+    assert few(64, 11008, 4096) and few(49, 14336, 5120) and few(64, 16384, 8192) and few(64, 6152, 2048)
     assert few(64, 17408, 5120) is None and few(64, 6148, 2048) is None and few(64, 12288, 4100) is None
     for m in (65, 100, 300, 777, 1024):
         for n, k in ((4096, 12288), (2560, 9728), (2048, 6144), (8, 8192)):
