@@ -1757,10 +1757,27 @@ def _aligned(*tensors: torch.Tensor) -> bool:
 
 
 def block_reads(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether the many-row product takes the operands of its ``"runs"`` form as they are: a plan, rows side by side,
-    whole units of 16 bytes."""
-    return (block_plan(x.shape[0], w.shape[0], w.shape[1], "runs") is not None and _aligned(x, w)
+    """Whether a layer's product goes to the many-row product's ``"runs"`` form: it is the faster one (:func:`block_pays`)
+    and takes the operands as they are, rows side by side in whole units of 16 bytes."""
+    return (block_pays(x.shape[0], w.shape[0], w.shape[1], chip().units) and _aligned(x, w)
             and x.is_contiguous() and w.is_contiguous())
+
+
+@functools.lru_cache(maxsize=4096)
+def block_pays(m: int, n: int, k: int, units: int) -> bool:
+    """Whether the ``"runs"`` form is faster, with the norm, than what else there is: the mid-size product up to 192 rows,
+    where its workgroups (tiles times runs) have to cover five eighths of the units, the library's beyond, where three
+    eighths do.  Microseconds over weights from memory at 65 / 128 / 192 rows, the mid-size product first: 512 columns of
+    12,288 k (32, 32 and 64 workgroups) 14.9 / 19.7, 15.3 / 20.7, 16.3 / 20.7; 1,536 of 9,728 (96, 96 and 192) 21.4 / 21.2,
+    22.3 / 24.1, 26.7 / 23.4; 3,072 of 8,192 (192, 192 and 256) 25.8 / 22.1, 26.9 / 25.5, 33.9 / 29.1.  At 224 / 384 rows, the
+    library's first: 512 columns of 12,288 k (64 and 96) 20.6 / 21.7, 26.0 / 22.1.  Beyond 1,280 rows sums of less than 9,216 k
+    are 12% slower to 23% faster than the library's, as its kernels happen to fit (8,192 k at 1,500 rows: 2,048 columns 0.89
+    of its speed, 1,536 1.23), and stay there.  Of 352 sizes, 512 to 8,192 columns at 65 to 2,048 rows, 3 are left slower, by 4%."""
+    plan = _block_plan(m, n, k, "runs", units)
+    if plan is None or (k < 9216 and m > 1280):
+        return False
+    share = 5 if m <= MID_MAX_ROWS and _mid_runs(n, k, units) > 0 else 3
+    return 8 * plan[2] * _block_tiles(m, n, "runs", plan) >= share * units
 
 
 def _block(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str, plan: tuple[int, int, int]) -> torch.Tensor:
@@ -1805,11 +1822,11 @@ def _mid_runs(n: int, k: int, units: int) -> int:
 def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor, copies: bool = True) -> torch.Tensor:
     """``x[M,K] @ w[N,K]^T`` for 17 to 192 rows, or as many as :func:`block_plan` says, as float32 runs of K,
     ``[runs, M, N]``: their sum is the product.  For products whose result goes into the residual: the norm that
-    follows adds the runs (``add_rmsnorm_parts``).  Operands that begin inside a unit of 16 bytes are copied where
-    the many-row product takes them; without ``copies`` the mid-size product reads them as they are."""
+    follows adds the runs (``add_rmsnorm_parts``).  The many-row product runs wherever it can, over copies of operands that
+    begin inside a unit of 16 bytes; without ``copies`` only where :func:`block_reads` says so."""
     m, k = x.shape
     n = w.shape[0]
-    plan = block_plan(m, n, k, "runs") if k == w.shape[1] and (copies or _aligned(x, w)) else None
+    plan = block_plan(m, n, k, "runs") if k == w.shape[1] and (copies or block_reads(x, w)) else None
     if plan is not None:
         _need(x, "x", torch.bfloat16)
         _need(w, "w", torch.bfloat16)

@@ -159,15 +159,13 @@ def test_repeated_layers_with_biases_and_products_cut_into_launches(biased, dtyp
         assert torch.equal(a, b)
 
 
-def test_weights_that_are_copied_are_every_layers_own(monkeypatch):
-    """Down projections whose rows begin inside a unit of 16 bytes, in steps whose kernel wants whole units."""
+def test_weights_inside_a_unit_of_16_bytes_are_every_layers_own(monkeypatch):
+    """Down projections over long sums whose rows begin inside a unit of 16 bytes."""
     from rapid_llm_amd import EngineConfig, ModelRunner
-    from rapid_llm_amd.kernels import ops
 
     runner = ModelRunner({**BASE, "intermediate_size": 8192},
                          EngineConfig(dtype="bfloat16", max_seq_len=1024, page_size=16, num_pages=200, max_num_seqs=8),
                          load_format="random", weight_norm_std=0.1)
-    assert ops.block_plan(150, 256, 8192, "runs") is not None
     for block in runner.model.blocks:
         down = block.feed_forward.down
         room = torch.empty(down.weight.numel() + 1, dtype=down.weight.dtype, device="cuda")

@@ -213,6 +213,24 @@ def test_where_the_many_row_product_applies():
             assert per * (found[2] - 1) < k // 64
 
 
+def test_products_over_long_sums_leave_the_others_for_a_filled_chip():
+    """What a layer asks for, as against what the many-row product can do: it is to be the faster one."""
+    from rapid_llm_amd.kernels import ops
+
+    pays = lambda *a: ops.block_pays(*a, 256)
+    # the mid-size product's range and the library's
+    assert pays(65, 4096, 12288) and pays(128, 2560, 9728) and pays(160, 1536, 9728) and pays(384, 512, 12288)
+    assert not pays(65, 512, 12288) and not pays(192, 1024, 12288) and not pays(128, 1536, 9728) and not pays(224, 512, 12288)
+    assert pays(2048, 4096, 12288) and pays(1280, 2048, 8192) and not pays(1281, 2048, 8192) and not pays(300, 4096, 4096)
+    for units in (64, 256, 304):
+        for m in (65, 192, 193, 700, 2000):
+            for n in (8, 512, 2056, 4096):
+                for k in (6144, 8192, 12288):
+                    if ops.block_pays(m, n, k, units):
+                        plan = ops.block_plan(m, n, k, "runs", units=units)
+                        assert 8 * plan[2] * ops._block_tiles(m, n, "runs", plan) >= 3 * units
+
+
 def test_small_gate_and_up_matrices_leave_the_tile_product_for_a_filled_chip():
     from rapid_llm_amd.kernels import ops
 
