@@ -1114,10 +1114,12 @@ def f32_wide(m: int, n: int, k: int, units: int) -> int:
     chip; the narrower ones where the others would leave a short last round.  Microseconds at 1,024 / 2,048 / 4,096 rows, ``f32_plan``'s tiles
     first: 6,144 x 4,096 290 / 222, 521 / 453, 954 / 816; 4,096 x 4,096 208 / 191, 326 / 279, 651 / 558;
     24,576 x 4,096 988 / 814, 1,957 / 1,624, 3,890 / 3,190; 4,096 x 12,288 535 / 557, 1,006 / 817, 1,956 / 1,640;
-    4,096 x 1,024 67 / 61, 90 / 81, 175 / 159; 1,024 x 3,072 48 / 143, 85 / 149, 156 / 161."""
-    if m <= 64 or k % 32 or k > 1 << 20:
+    4,096 x 1,024 67 / 61, 90 / 81, 175 / 159; 1,024 x 3,072 48 / 143, 85 / 149, 156 / 161.  Up to 512 k the making of A's
+    pieces is not paid back (256 k: 3,120 weight rows at 1,982 rows, 11,272 at 259, 0.92 of the other tiles' speed), and the
+    estimate has to be lower by 8%: of 289 sizes drawn, 34 go here, 1.04 to 1.41 times as fast."""
+    if m <= 64 or k % 32 or k <= 512 or k > 1 << 20:
         return 0
-    best, cols = 0.97 * (_f32_tile_plan(m, n, k, units)[0] + _F32_WIDE_ROUND), 0
+    best, cols = 0.92 * (_f32_tile_plan(m, n, k, units)[0] + _F32_WIDE_ROUND), 0
     for width, (few, full) in _F32_WIDE.items():
         rounds, rest = divmod(-(-m // 256) * -(-n // width), units)
         chunk = rounds * full + (max(few, full * rest / units) if rest else 0.0)

@@ -220,6 +220,8 @@ def test_what_a_noted_layer_kept_is_given_back_before_the_end_of_the_step(dtype,
             runner.step([StepEntry("a", tokens, [179])])
             runner.finish("a")
         most.append(torch.cuda.max_memory_allocated())
-    assert at_end[3] <= at_end[1]
     weights = [t for t in runner.model.blocks[0].own_tensors() if t.dim() == 2]
-    assert most[1] - most[0] <= 1.5 * sum(ops.product_bytes(180, w) for w in weights)
+    kept = sum(ops.product_bytes(180, w) for w in weights)
+    # (a block may be up to 1 MB larger than what lies in it, and a few are alive at the end)
+    assert at_end[3] - at_end[1] <= 4 << 20 < kept / 2
+    assert most[1] - most[0] <= 1.5 * kept

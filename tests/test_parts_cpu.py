@@ -380,6 +380,8 @@ def test_plans_of_the_float32_product_for_many_rows():
                     rows = ops._f32_piece_rows(m, k)
                     assert rows % 256 == 0 and 96 * k * (rows // 16 - 16) <= ops._F32_MOST_PIECES
     assert ops.f32_wide(2048, 24576, 4096, 256) == 128 and ops.f32_wide(2048, 6144, 4096, 256) == 96
+    # short sums, and sizes at which the two are level
+    assert ops.f32_wide(1982, 3120, 256, 256) == 0 and ops.f32_wide(269, 12032, 512, 256) == 0 and ops.f32_wide(247, 12784, 3296, 256) == 0
     assert ops.f32_wide(2048, 1024, 3072, 256) == 0 and ops.f32_wide(225, 4096, 1024, 256) == 0
     assert ops._f32_piece_rows(2048, 12288) == 2048 and ops._f32_piece_rows(8192, 12288) == 2816
 
