@@ -1674,10 +1674,11 @@ def block_plan(m: int, n: int, k: int, kind: str, units: int | None = None) -> t
     8B 55.6 / 54.1, 93.5 / 80.5, 303 / 286, 1,176 / 1,106; 4B 35.8 / 33.9, 63.5 / 49.6, 218 / 172, 756 / 587; 1.7B
     21.3 / 21.0, 35.6 / 27.9, 105 / 82.7, 337 / 302; 0.6B 14.7 / 12.4, 20.0 / 12.8, 37.3 / 25.8, 113 / 91.2; 14B at 65 /
     256 / 1,024 rows 93.9 / 78.9, 119 / 103, 411 / 292; 32B 108 / 103, 164 / 142, 509 / 440 (slower at most: 777 rows 383 / 401).
-    A tile walks K alone, so beyond 1,024 k its product needs tiles for a share of the units that grows with K, from half
-    at 2,048 k to seven eighths at 5,120 (weights from memory: 2,048 columns of 5,120 k at 65 rows in 32 tiles 24.1 / 49.8,
-    6,144 of 4,096 at 96 rows in 96 tiles 38.0 / 42.2; up to 1,024 k 1.2 times as fast from 64 tiles on).  Of 393 sizes that
-    pass, 1,536 to 14,336 columns of 512 to 8,192 k at 65 to 512 rows, 20 are slower than the library's, by 16% at most.
+    A tile walks K alone, so beyond 1,024 k its product needs tiles for a share of the units that grows with K, three
+    eighths up to 2,048 k (there the two are level, and this one is a launch of 6 us for the host, not two of 25) to seven
+    eighths at 5,120 (weights from memory: 2,048 columns of 5,120 k at 65 rows in 32 tiles 24.1 / 49.8,
+    6,144 of 4,096 at 96 rows in 96 tiles 38.0 / 42.2; up to 1,024 k 1.2 times as fast from 64 tiles on).  Of 404 sizes that
+    pass, 1,536 to 14,336 columns of 512 to 8,192 k at 65 to 512 rows, 22 are slower than the library's, by 16% at most.
 
     ``"runs"``: a product whose result feeds the residual, as float32 runs of K that the norm adds: long sums of few
     columns, which leave the library's kernels for 65 to some 2,000 rows without work for the whole chip.  With the
@@ -1717,7 +1718,7 @@ def _block_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int
                 cost += m * n * ks * _BLOCK_RUN_ELEMENT
             if best is None or cost < best[0]:
                 best = (cost, (nw, nx, ks), tiles)
-    if kind == "gated" and k > 1024 and 8192 * best[2] < units * min(2048 + k, 7168):
+    if kind == "gated" and k > 1024 and 8192 * best[2] < units * (3072 if k <= 2048 else min(2048 + k, 7168)):
         return None
     return best[1]
 

@@ -186,11 +186,12 @@ def test_where_the_many_row_product_applies():
     assert plan(160, 3072, 1024, "gated") == (2, 2, 1)     # few rows: as many workgroups as there can be
     assert plan(64, 12288, 4096, "gated") is None          # the kernel for up to 64 rows
     # tiles for too few units, each of which would walk a long K alone
-    assert plan(65, 2048, 5120, "gated") is None and plan(128, 6144, 2048, "gated") is None and plan(96, 6144, 4096, "gated") is None
-    assert plan(129, 6144, 2048, "gated") and plan(65, 9728, 2560, "gated") and plan(65, 12288, 4096, "gated") and plan(65, 4096, 512, "gated")
+    assert plan(65, 2048, 5120, "gated") is None and plan(128, 5120, 2048, "gated") is None and plan(96, 6144, 4096, "gated") is None
+    assert plan(128, 6144, 2048, "gated") and plan(129, 6144, 2048, "gated") and plan(65, 9728, 2560, "gated") and plan(65, 12288, 4096, "gated") and plan(65, 4096, 512, "gated")
     for units in (64, 128, 304):  # (as a share of the units that there are)
         for tiles in range(1, units + 1):
-            assert (ops.block_plan(65, 64 * tiles, 2048, "gated", units=units) is None) == (2 * tiles < units)
+            assert (ops.block_plan(65, 64 * tiles, 2048, "gated", units=units) is None) == (8 * tiles < 3 * units)
+            assert (ops.block_plan(65, 64 * tiles, 4096, "gated", units=units) is None) == (4 * tiles < 3 * units)
     assert plan(512, 12288, 4100, "gated") is None and plan(512, 12290, 4096, "gated") is None
     assert plan(90000, 12288, 12288, "gated") is None      # offsets beyond 31 bits
     assert plan(2048, 4096, 4096, "runs") is None          # short sums: the library's
