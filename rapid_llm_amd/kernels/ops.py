@@ -1473,7 +1473,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
     x = whole_rows(x)
     if scaled is not None:
         raise KernelError(f"scaled rows need the few-row product: {m} rows over {k}")
-    plan = rows_plan(m, n, k, swiglu=False)
+    plan = rows_plan(m, n, k, swiglu=False) if m <= ROWS_MAX_ROWS else None
     if _tile_applies(m, n, k, n) and not (plan is not None and k >= 512 and out_dtype == torch.bfloat16 and _aligned(x, w)):
         out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
         _ok(
@@ -1492,6 +1492,15 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
         )
         return out
     return library_product(x, w, out_dtype)
+
+
+def library_takes(m: int, n: int, k: int) -> bool:
+    """Whether :func:`gemm_bf16` gives ``m`` rows over an ``[n, k]`` matrix to the library."""
+    if m <= SKINNY_MAX_ROWS and k % 8 == 0:
+        return False
+    if m <= ROWS_MAX_ROWS and rows_plan(m, n, k, swiglu=False) is not None:
+        return False
+    return not _tile_applies(m, n, k, n)
 
 
 def gemm_bf16_wide(x: torch.Tensor, w: torch.Tensor, scaled=None) -> torch.Tensor:
@@ -1646,6 +1655,14 @@ def _tile_gives_way(m: int, inter: int, k: int, units: int) -> bool:
     return plan is not None and 8 * _block_tiles(m, inter, "gated", plan) >= 3 * units
 
 
+@functools.lru_cache(maxsize=4096)
+def _gated_block(m: int, inter: int, k: int, tile: bool, units: int) -> tuple[int, int, int] | None:
+    """The many-row product's plan for gate and up, ``None`` where another kernel takes them (``tile``: the tile product can)."""
+    if tile and not _tile_gives_way(m, inter, k, units):
+        return None
+    return _block_plan(m, inter, k, "gated", units) or block_few_plan(m, inter, k, units)
+
+
 def _block_tiles(m: int, n: int, kind: str, plan: tuple[int, int, int]) -> int:
     """Workgroups a run of K has under a plan of :func:`block_plan`."""
     return -(-n // ((32 if kind == "gated" else 64) * plan[0])) * -(-m // (64 * plan[1]))
@@ -1663,6 +1680,7 @@ _BLOCK_COSTS = {
     "runs": ((0.85, 0.47, 9.8), (0.73, 0.34, 6.2), (0.56, 0.25, 3.5), (0.64, 0.25, 4.0), (0.525, 0.19, 3.0), (0.42, 0.14, 2.3)),
 }
 _BLOCK_RUN_ELEMENT = 1.1e-6
+BLOCK_RUNS_MIN_K = 6144  # shorter sums than this are never cut into its runs
 
 
 def block_plan(m: int, n: int, k: int, kind: str, units: int | None = None) -> tuple[int, int, int] | None:
@@ -1702,7 +1720,7 @@ def _block_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int
     runs = (1,)
     if kind == "runs":
         squares = -(-m // 256) * -(-n // 256)
-        if k < 6144 or (k < 8192 and (m <= 128 or squares > 32)) or squares > 128:
+        if k < BLOCK_RUNS_MIN_K or (k < 8192 and (m <= 128 or squares > 32)) or squares > 128:
             return None
         runs = (1, 2, 3, 4, 6, 8)
     best = None
@@ -1755,8 +1773,8 @@ def block_few_plan(m: int, n: int, k: int, units: int | None = None) -> tuple[in
 _BLOCK_KINDS = {"runs": 1, "gated": 2}  # as the kernel's entry point counts them
 
 
-def _aligned(*tensors: torch.Tensor) -> bool:
-    return all(t.data_ptr() % 16 == 0 for t in tensors)
+def _aligned(a: torch.Tensor, b: torch.Tensor) -> bool:
+    return not (a.data_ptr() | b.data_ptr()) & 15
 
 
 def block_reads(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -1835,7 +1853,7 @@ def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor, copies: bool = True) -> to
         _need(w, "w", torch.bfloat16)
         if not _aligned(x, w):  # (a view that begins inside a unit of 16 bytes)
             unnoted()
-            x, w = (t if _aligned(t) else t.clone() for t in (x, w))
+            x, w = (t.clone() if t.data_ptr() & 15 else t for t in (x, w))
         return _block(x, w, torch.empty((plan[2], m, n), dtype=torch.float32, device=x.device), "runs", plan)
     ks = mid_runs(n, k)
     if k != w.shape[1] or m > MID_MAX_ROWS or ks < 1:
@@ -1886,7 +1904,7 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
     two_i = w_gate_up.shape[0]
     if bias is not None:
         _need(bias, "bias of gate and up", torch.float32, (two_i,))
-    glu = (ctypes.c_float(limit), ctypes.c_float(alpha), _gate_kind(activation, limit), _p(bias))
+    kind = _gate_kind(activation, limit)
     if k % 8 or two_i % 2 or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16:
         return None
     if m > SKINNY_MAX_ROWS:
@@ -1895,12 +1913,13 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
             return None
         _need(x, "x", torch.bfloat16)
         _need(w_gate_up, "w_gate_up", torch.bfloat16, (two_i, k))
-        plan = rows_plan(m, inter, k, swiglu=True)
+        plan = rows_plan(m, inter, k, swiglu=True) if m <= ROWS_MAX_ROWS else None
         tile = _tile_applies(m, two_i, k, inter) and not (plan is not None and k >= 1024 and _aligned(x, w_gate_up))
-        if (not tile or _tile_gives_way(m, inter, k, chip().units)) and activation == "silu" and limit <= 0 and bias is None:
-            block = block_plan(m, inter, k, "gated") or block_few_plan(m, inter, k)
+        if activation == "silu" and limit <= 0 and bias is None:
+            block = _gated_block(m, inter, k, tile, chip().units)
             if block is not None and _aligned(x, w_gate_up):
                 return _block(x, w_gate_up, torch.empty((m, inter), dtype=torch.bfloat16, device=x.device), "gated", block)
+        glu = (ctypes.c_float(limit), ctypes.c_float(alpha), kind, _p(bias))
         if tile:
             out = torch.empty((m, inter), dtype=torch.bfloat16, device=x.device)
             _ok(core().rl_gemm_tile(_p(x), _p(w_gate_up), _p(out), m, inter, k, k, k, inter, 1, *glu, _stream()), "rl_gemm_tile")
@@ -1918,6 +1937,7 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
     inter = two_i // 2
     out = torch.empty((m, inter), dtype=torch.bfloat16, device=x.device)
     nt = 2  # one (gate, up) pair of tiles per workgroup
+    glu = (ctypes.c_float(limit), ctypes.c_float(alpha), kind, _p(bias))
     _ok(
         core().rl_gemm_skinny_swiglu(
             _p(x), _p(w_gate_up), _p(out), m, inter, k, k, k, inter, nt, chip().units,

@@ -182,7 +182,7 @@ class CausalLM:
         # (a signature says that a block and its parts are of known classes, the same ones in every layer)
         if first is None or not all(p.forward_as_written() for p in (blocks[0], *blocks[0].parts())):
             return False
-        if any(b.launch_signature() != first for b in blocks):
+        if blocks[0].calls_library(ctx.num_tokens) or any(b.launch_signature() != first for b in blocks):
             return False
         if sum(ops.product_bytes(ctx.num_tokens, t) for t in blocks[0].own_tensors() if t.dim() == 2) > REPEAT_MAX_BYTES:
             return False

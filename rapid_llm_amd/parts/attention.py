@@ -329,6 +329,9 @@ class GQAAttention(PackedMixer):
             return None
         return _FIXED(self)
 
+    def calls_library(self, rows: int) -> bool:
+        return self.o.calls_library(rows, folded=True) or self.qkv.calls_library(rows)
+
     def own_tensors(self) -> list[torch.Tensor]:
         own = self.qkv.own_tensors() + self.o.own_tensors()
         if self.q_norm_w is not None:

@@ -234,6 +234,11 @@ class Part:
         the instance: a timer or a hook that somebody put there is to be called in every layer."""
         return None
 
+    def calls_library(self, rows: int) -> bool:
+        """Whether ``forward`` calls the library's product in a step of ``rows`` tokens, so that its launches cannot be made
+        again: saves looking at the layers.  (False promises nothing: such a call is seen when it is made.)"""
+        return False
+
     def own_tensors(self) -> "list[torch.Tensor]":
         """The tensors of this part alone that its launches point at, each at its beginning."""
         return []

@@ -39,6 +39,9 @@ class PreNormBlock(Block):
                       self.feed_forward_norm.launch_signature(), self.feed_forward.launch_signature())
         return None if None in signatures else signatures
 
+    def calls_library(self, rows):
+        return self.mixer.calls_library(rows) or (self.feed_forward is not None and self.feed_forward.calls_library(rows))
+
     def own_tensors(self):
         return [*self.mixer_norm.own_tensors(), *self.mixer.own_tensors(),
                 *self.feed_forward_norm.own_tensors(), *self.feed_forward.own_tensors()]

@@ -55,9 +55,8 @@ class Linear:
         )
 
     def folds(self, x) -> bool:
-        """Whether this product may absorb the residual add and norm that follow it: one of the
-        two kernels with that epilogue runs it."""
-        return self.skinny(x) or self.midsize(x) or self.f32_runs(x)
+        """Whether this product may absorb the residual add and norm that follow it, or leave the norm runs of K to add."""
+        return self.f32_runs(x) if self.weight.dtype == torch.float32 else self.skinny(x) or self.midsize(x)
 
     def f32_runs(self, x) -> bool:
         """Whether ``x`` runs as a float32 product whose runs of K a norm can add."""
@@ -65,6 +64,16 @@ class Linear:
             self.weight.dtype == torch.float32 and x.dtype == torch.float32
             and ops.f32_runs(x.shape[0], self.out_features, self.in_features)
         )
+
+    def calls_library(self, rows: int, folded: bool = False) -> bool:
+        """Whether so many bfloat16 rows go to the library's product; ``folded``: a norm behind it may add runs of K."""
+        n, k = self.out_features, self.in_features
+        if self.weight.dtype != torch.bfloat16:
+            return False
+        if folded and ((rows <= ops.MID_MAX_ROWS and ops.mid_runs(n, k) > 0)
+                       or (k >= ops.BLOCK_RUNS_MIN_K and ops.block_pays(rows, n, k, ops.chip().units))):
+            return False
+        return ops.library_takes(rows, n, k)
 
     def takes_scaled_rows(self) -> bool:
         """Whether this product can finish a norm whose rows arrive unscaled (whatever the
@@ -79,7 +88,7 @@ class Linear:
             return False
         if rows <= ops.MID_MAX_ROWS and ops.mid_runs(self.out_features, self.in_features) > 0:
             return True
-        return ops.block_reads(x, self.weight)
+        return self.in_features >= ops.BLOCK_RUNS_MIN_K and ops.block_reads(x, self.weight)
 
     def partial_sums(self, x: torch.Tensor) -> torch.Tensor:
         """``[runs, M, out]`` float32 whose sum over the runs is ``x W^T`` (without the bias)."""

@@ -89,6 +89,9 @@ class SwiGLU(FeedForward):
             return None
         return _FIXED(self)
 
+    def calls_library(self, rows: int) -> bool:
+        return self.down.calls_library(rows, folded=True)
+
     def own_tensors(self) -> list[torch.Tensor]:
         own = self.gate_up.own_tensors() + self.down.own_tensors()
         if self.has_bias:

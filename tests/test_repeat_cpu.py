@@ -27,7 +27,7 @@ def _model(dtype=torch.bfloat16, **change):
     return model, caches
 
 
-def _alike(model, caches, tokens=37, static=()):
+def _alike(model, caches, tokens=5, static=()):
     return model._alike(SimpleNamespace(num_tokens=tokens, static=dict(static)), caches)
 
 
@@ -72,8 +72,20 @@ def test_steps_whose_temporary_tensors_are_large_are_not_repeated():
     model, caches = _model(torch.float32, **large)
     assert _alike(model, caches, 17) and not _alike(model, caches, REPEAT_MAX_TOKENS)
     small = dict(hidden_size=1024, num_attention_heads=16, num_key_value_heads=8, head_dim=128, intermediate_size=3072)
-    for dtype, tokens in ((torch.float32, 512), (torch.bfloat16, 1024)):
+    for dtype, tokens in ((torch.float32, 512), (torch.bfloat16, 192)):
         assert _alike(*_model(dtype, **small), tokens)
     # gate and up, the widest, is the most that is left alive: its result alone is within the bound
     rows = max(m for m in range(1, REPEAT_MAX_TOKENS) if _alike(model, caches, m))
     assert 4 * rows * 2 * 25600 < REPEAT_MAX_BYTES
+
+
+def test_steps_with_library_products_are_told_beforehand():
+    """Their layers are not looked at; what float32 layers and few rows launch is all this package's."""
+    small = dict(hidden_size=1024, num_attention_heads=16, num_key_value_heads=8, head_dim=128, intermediate_size=3072)
+    model, caches = _model(**small)
+    for tokens, library in ((1, False), (16, False), (17, False), (64, False), (192, False), (193, True), (512, True), (2048, True)):
+        assert model.blocks[0].calls_library(tokens) == library and _alike(model, caches, tokens) != library
+    assert not _model(torch.float32, **small)[0].blocks[0].calls_library(2048)
+    wide = dict(hidden_size=4096, num_attention_heads=32, num_key_value_heads=8, head_dim=128, intermediate_size=12288)
+    model, _ = _model(**wide)
+    assert not model.blocks[0].calls_library(64) and model.blocks[0].calls_library(65)  # (queries, keys and values)
