@@ -173,9 +173,9 @@ __device__ __forceinline__ void read_b(bf16x8 (&w)[NA][2][2], u32 a0, u32 a1) {
 
 // silu(g) * u of bfloat16 numbers below SILU_WIDE in magnitude.  Their product is exact and comes first; exp(-g) is a
 // power of two whose argument's rounding is put back; the quotient is by a reciprocal and one Newton step.  No step
-// leaves the normal range (87 log2(e) < 126).  Over all gates and eight factors, in ulp of float32, worst and root mean
-// square: 2.4 and 0.20; g / (1 + expf(-g)) * u, the other kernels' form, 2.5 and 0.22.  That form in its place, microseconds at
-// 8,192 rows: 24,576 x 4,096 1,158 against 1,117, 6,144 x 1,024 99 against 90.
+// leaves the normal range (87 log2(e) < 126).  Over all gates and eight factors, in ulp of float32, root mean square
+// 0.204; g / (1 + expf(-g)) * u, the other kernels' form, 0.222; neither is further off than 2.5 at worst.  That form in its
+// place, microseconds at 8,192 rows: 24,576 x 4,096 1,158 against 1,117, 6,144 x 1,024 99 against 90.
 #define SILU_WIDE 87.f
 #define SILU_WIDE_BITS 0x42ae  // as bfloat16
 __device__ __forceinline__ float silu_times(float g, float u) {

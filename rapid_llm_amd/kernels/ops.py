@@ -1609,7 +1609,7 @@ def gemm_bf16_residual(
 
 
 TILE_MAX_ROWS = 512  # rows up to which small matrices run the one-launch tile product
-TILE_GATED_MAX_ROWS = 128  # and the packed gate and up matrices, which the many-row product takes from there on
+TILE_GATED_MAX_ROWS = 128  # and the packed gate and up matrices always; beyond see _tile_gives_way
 _TILE_MAX_WEIGHTS = 7 << 20  # elements of a matrix (14 MB) up to which it is used
 _TILE_MIN_COLS = 2048  # fewer columns leave too few workgroups
 
@@ -2619,7 +2619,7 @@ def _decode_short(pairs: int, chunk: int, span: int, window: int, units: int | N
     units idle with splits of 128 keys, ``None`` where they do not.
 
     A unit takes a split's keys one wave's 32 at a time, so half as many keys a unit are the shorter chain: a step of
-    the Qwen3-0.6B shape with one request of 100 / 300 / 500 keys 1,015 / 1,002 / 1,020 -> 981 / 986 / 991 us, four of
+    the Qwen3-0.6B shape with one request of 300 / 500 keys 1,002 / 1,020 -> 986 / 991 us, four of
     400 1,031 -> 1,015, of the 8B shape one of 300 3,328 -> 3,304.  The merge's share grows with the splits: one request
     of 1,000 keys 1,025 -> 1,020, of 2,000 1,049 -> 1,071, hence up to 512 keys.  Launches for at most 128 keys have one split and no
     merge."""

@@ -11,10 +11,11 @@ Which product runs is decided by the weight's storage type:
   engine).  A bfloat16 activation is widened first, so a matrix that the checkpoint stores in 32-bit keeps
   its bits in a bfloat16 engine too.
 * bfloat16 weight: few rows (decode) go to the hand-written bandwidth-bound matrix-core
-  kernel; many rows go to the library product, as in the reference, whose dense products
-  are ``F.linear`` (rapid_llm/kernels/ops/gemm/linear.py:17-40).  In between (17 to 192 rows, more where K is
-  long) a narrow matrix whose result a norm adds to the residual may hand that norm float32 runs of
-  K instead (``partial_sums``).
+  kernel, more to kernels of this package for small and for wide matrices; a matrix whose result a norm adds
+  to the residual may hand that norm float32 runs of K instead (``partial_sums``: 17 to 192 rows of a
+  narrow one, more where K is long).  What none of them takes goes to the library product, as in the reference, whose dense
+  products are ``F.linear`` (rapid_llm/kernels/ops/gemm/linear.py:17-40).  The packed gate and up matrices have kernels of
+  their own (``ops.gemm_bf16_swiglu``).
 """
 
 from __future__ import annotations
@@ -81,8 +82,9 @@ class Linear:
         return self.weight is not None and self.weight.dtype == torch.bfloat16 and self.in_features % 8 == 0
 
     def midsize(self, x) -> bool:
-        """Whether ``x`` (more rows than the few-row kernel takes) may run as float32 runs of K
-        that a norm adds (narrow matrices only: the wide ones are faster in the library)."""
+        """Whether ``x`` (more rows than the few-row kernel takes) may run as float32 runs of K that a norm adds: up to
+        192 rows over a narrow matrix (wide ones have nothing to gain), any number of them over long sums where the many-row
+        product is the faster one (``ops.block_reads``)."""
         rows = x.shape[0]
         if self.weight.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or rows <= ops.SKINNY_MAX_ROWS:
             return False
