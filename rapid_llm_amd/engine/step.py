@@ -237,7 +237,7 @@ class ModelRunner:
         parts = list(self.model.all_parts())
         each_of = {getattr(p, "deals_ragged_contexts", 0) for p in parts} - {0}
         wide = [tuple(p.shape) for p in self.params.values() if p.dim() == 2 and p.dtype == torch.float32]
-        total = 0
+        total = self.model.chain_bytes(e.max_seq_len) if self.dtype == torch.bfloat16 else 0
         for fewer, rows in zip([0, *sizes], sizes):
             # a float32 product's partial results or pieces, given back behind it
             scratch = max((ops.f32_product_bytes(rows, *shape) for shape in wide), default=0)

@@ -16,6 +16,7 @@ Two kinds of library exist:
   (scans, short convolutions, head and grouped norms), compiled when a model has such a mixer.
 * ``linear_attention``: linear attention with decays a channel or a head (chunked walk, single tokens,
   gated norm of its outputs), compiled when a model has such a mixer.
+* ``decode_chain``: all layers of a decode step of few tokens in one launch, for heads of 128 channels.
 * ``attn_tile_d<D>_v<DV>``: the tile attention for key heads of ``D`` and value heads of ``DV``
   channels, compiled when a model has a mixer that needs it.
 
@@ -59,6 +60,7 @@ MLSTM_SOURCES = ("mlstm.hip",)
 RECURRENT_SOURCES = ("recurrent.hip",)
 LINEAR_ATTENTION_SOURCES = ("linear_attention.hip",)
 ATTENTION_TILE_SOURCES = ("attention_tile.hip",)
+DECODE_CHAIN_SOURCES = ("decode_chain.hip",)
 HEADERS = ("common.h", "static_entry.h")
 
 # head sizes built ahead of time by build_all(): every one the kernels take.  A fresh
@@ -247,6 +249,11 @@ def linear_attention_library(force: bool = False) -> Path:
     return compile_library("linear_attention", LINEAR_ATTENTION_SOURCES, ("-mllvm", "-amdgpu-mfma-vgpr-form=1"), force=force)
 
 
+def decode_chain_library(force: bool = False) -> Path:
+    # (as the attention kernels: the softmax rescales its accumulators)
+    return compile_library("decode_chain", DECODE_CHAIN_SOURCES, ("-mllvm", "-amdgpu-mfma-vgpr-form=1"), force=force)
+
+
 def attention_tile_library(head_dim: int, value_dim: int, force: bool = False) -> Path:
     # beyond 320 / 256 channels a lane's operands no longer fit its registers: the compiler
     # parks some in scratch memory, which is slower and as exact
@@ -260,7 +267,7 @@ def attention_tile_library(head_dim: int, value_dim: int, force: bool = False) -
 def build_all(head_dims: tuple[int, ...] = DEFAULT_HEAD_DIMS, force: bool = True) -> list[Path]:
     """Compile every library (what ``__graft_entry__.build`` calls)."""
     out = [core_library(force=force), mlstm_library(force=force), recurrent_library(force=force),
-           linear_attention_library(force=force)]
+           linear_attention_library(force=force), decode_chain_library(force=force)]
     with ThreadPoolExecutor(8) as pool:
         out += list(pool.map(lambda pair: attention_tile_library(*pair, force=force), DEFAULT_TILE_HEAD_DIMS))
     if not all((CSRC / s).is_file() for s in ATTENTION_SOURCES):

@@ -12,7 +12,7 @@ from dataclasses import replace
 
 import torch
 
-from ..kernels import ops
+from ..kernels import decode_chain, ops
 from ..kernels.notes import taking_notes
 from ..parts.base import (
     BLOCKS,
@@ -72,6 +72,7 @@ class CausalLM:
             for place in self.returns:
                 if not 0 <= place < len(self.order):
                     raise ValueError(f"the embedding returns at place {place} of a run order of {len(self.order)}")
+        self._chain_space: decode_chain.Space | None = None  # of the recorded steps that run all layers in one launch
         self._positions: dict[str, object] = {}
         self.blocks = []
         for i, layer in enumerate(spec.layers):
@@ -171,6 +172,70 @@ class CausalLM:
         return needs
 
     # ---- step ------------------------------------------------------------------
+    def _chain(self, ctx, caches) -> "decode_chain.DecodeChain | None":
+        """The launch of all layers of a recorded step of few tokens, where they are plain dense layers of sizes that it
+        takes; made by the eager run in front of the recording and kept with the graph."""
+        if "decode_only_tokens" not in ctx.static or ctx.num_tokens > decode_chain.MAX_ROWS:
+            return None
+        if "decode_chain" not in ctx.static:
+            ctx.static["decode_chain"] = self._new_chain(ctx, caches)
+        return ctx.static["decode_chain"]
+
+    def chainable(self) -> bool:
+        """Whether the layers are such that one launch may run them all (``decode_chain``), whatever a step's rows are."""
+        if self.offsets is not None or self.mixes is not None or self.returns or len(self.order) < 2:
+            return False
+        blocks = [self.blocks[li] for li in self.order]
+        first = blocks[0].launch_signature()
+        # (a signature says that a block and its parts are of known classes, the same ones in every layer)
+        if first is None or any(b.launch_signature() != first for b in blocks):
+            return False
+        if not all(p.forward_as_written() for p in (blocks[0], *blocks[0].parts())):
+            return False
+        mixer, ff, norms = blocks[0].mixer, blocks[0].feed_forward, (blocks[0].mixer_norm, blocks[0].feed_forward_norm)
+        if not hasattr(mixer, "qkv") or not hasattr(ff, "gate_up") or not all(hasattr(n, "eps") for n in norms):
+            return False
+        cos = mixer.position.cos if mixer.position is not None else None
+        tensors = [t for b in blocks for t in (b.mixer.qkv.weight, b.mixer.o.weight, b.feed_forward.gate_up.weight, b.feed_forward.down.weight)]
+        return (
+            mixer.window <= 0 and not mixer.qkv_bias and not mixer.o_bias and not ff.has_bias and not ff.limit and ff.activation == "silu"
+            and (mixer.q_norm_w is None) == (mixer.k_norm_w is None)
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+            and ops.attention_prepares_queries(torch.bfloat16, mixer.d, 0 if cos is None else cos.shape[1],
+                                               getattr(mixer.position, "pairing", "half_split") if cos is not None else "half_split")
+            and decode_chain.fits(1, mixer.hidden_size, mixer.nq, mixer.nkv, mixer.d, ff.intermediate_size, 8)
+        )
+
+    def chain_bytes(self, span: int) -> int:
+        """Bytes that the recorded steps of few tokens share for their launches (contexts of at most ``span`` keys)."""
+        if not self.chainable():
+            return 0
+        mixer, ff = self.blocks[self.order[0]].mixer, self.blocks[self.order[0]].feed_forward
+        return sum(decode_chain.space_bytes(len(self.order), mixer.hidden_size, mixer.nq, mixer.nkv, ff.intermediate_size, span))
+
+    def _new_chain(self, ctx, caches):
+        kinds = {(c.group_id, c.page_size, c.owns_pages, len(c.pages), len(c.states)) for c in caches}
+        if len(kinds) != 1 or not all(c.owns_pages and not c.states and c.k is not None and c.v is not None for c in caches) or not self.chainable():
+            return None
+        blocks = [self.blocks[li] for li in self.order]
+        mixer, ff = blocks[0].mixer, blocks[0].feed_forward
+        sizes = (mixer.hidden_size, mixer.nq, mixer.nkv)
+        if not decode_chain.fits(ctx.num_tokens, *sizes, mixer.d, ff.intermediate_size, caches[0].page_size):
+            return None
+        layers = [
+            (b.mixer.qkv.weight, b.mixer.o.weight, b.feed_forward.gate_up.weight, b.feed_forward.down.weight, b.mixer.q_norm_w,
+             b.mixer.k_norm_w, b.feed_forward_norm.weight, behind.mixer_norm.weight if behind is not None else None, c.k, c.v)
+            for b, behind, c in zip(blocks, [*blocks[1:], None], caches)
+        ]
+        if any(t is not None and t.data_ptr() % 16 for layer in layers for t in layer):
+            return None
+        if self._chain_space is None:  # (one step of a runner runs at a time)
+            self._chain_space = decode_chain.Space(len(layers), *sizes, ff.intermediate_size, ctx.runtime.max_seq_len, mixer.qkv.weight.device)
+        return decode_chain.DecodeChain(
+            layers, self._chain_space, ctx.num_tokens, *sizes, ff.intermediate_size, ctx.static["context_bound"], mixer.scale,
+            (mixer.qk_norm_eps or 0.0, blocks[0].mixer_norm.eps, blocks[0].feed_forward_norm.eps),
+        )
+
     def _alike(self, ctx, caches) -> bool:
         """Whether every layer's launches of this step are the second one's with the layer's own tensors."""
         if ctx.num_tokens > REPEAT_MAX_TOKENS or len(self.order) < 4 or "decode_only_tokens" in ctx.static:
@@ -220,7 +285,14 @@ class CausalLM:
         # in place)
         first = residual.clone() if self.mixes is not None or self.returns else None
         delta = None
-        for place, li in enumerate(self.order):
+        chain = self._chain(ctx, caches)
+        if chain is not None:
+            first_block = self.blocks[self.order[0]]
+            position = first_block.mixer.position
+            x = run_norm(first_block.mixer_norm, residual, None, ctx)
+            delta = chain.run(x, residual, ctx.positions, ctx.token_slot, ctx.block_tables[caches[0].group_id],
+                              position.cos if position is not None else None, position.sin if position is not None else None, ctx.max_position)
+        for place, li in enumerate(self.order if chain is None else ()):
             if place == 1 and self._alike(ctx, caches):  # (asked while the device has the first layer to do)
                 delta, whole = self._second(residual, delta, ctx, caches)
                 if whole:

@@ -1,0 +1,179 @@
+"""All layers of a recorded step of few tokens in one launch: as close to the plain implementation as any other way of
+running the step, at the edges of its sizes, with any number of workgroups, and beside another launch of its kind."""
+
+import threading
+
+import pytest
+import torch
+
+import parity
+from plain_model import plain_forward, plain_load
+from tiny_configs import random_tokens
+
+pytestmark = pytest.mark.gpu
+
+BASE = dict(
+    architectures=["Qwen3ForCausalLM"], model_type="qwen3", num_hidden_layers=3, hidden_size=256, num_attention_heads=4,
+    num_key_value_heads=2, head_dim=128, intermediate_size=384, vocab_size=277, rope_theta=30000.0, rms_norm_eps=1e-5,
+    tie_word_embeddings=False, max_position_embeddings=2048, hidden_act="silu", attention_bias=False,
+)
+# contractions of 1 chunk of 128 (waves without one), of 9 (more for one wave) and of 33 (more than the ring holds; gate and
+# up in pairs), one to four query heads a kv head, one kv head, fewer items than workgroups
+SHAPES = {
+    "small": dict(hidden_size=128, intermediate_size=128, num_attention_heads=1, num_key_value_heads=1, num_hidden_layers=2),
+    "base": {},
+    "uneven": dict(hidden_size=1152, intermediate_size=1408, num_attention_heads=9, num_key_value_heads=3),
+    "long": dict(hidden_size=4224, intermediate_size=640, num_attention_heads=4, num_key_value_heads=1, num_hidden_layers=2),
+}
+# tokens in the cache in front of the step: none, one; the ends of eights, pages, the waves' 32 and 256 keys, a share, two and more
+CONTEXTS = [300, 1, 255, 256, 512, 513, 0, 31, 7, 16, 1100, 8, 64, 511, 767, 33]
+
+
+def _runner(model, **engine):
+    from rapid_llm_amd import EngineConfig, ModelRunner
+
+    engine = EngineConfig(**{**dict(dtype="bfloat16", max_seq_len=2048, page_size=16, num_pages=420, max_num_seqs=16), **engine})
+    return ModelRunner(model, engine, **({} if isinstance(model, str) else dict(load_format="random", weight_norm_std=0.1)))
+
+
+def _fill(runner, contexts, vocab):
+    """Requests with so many tokens in the cache, and the step that decodes one token of each."""
+    from rapid_llm_amd import StepEntry
+
+    tokens = {f"r{i}": random_tokens(n + 1, vocab, 31 + i) for i, n in enumerate(contexts)}
+    for rid, ids in tokens.items():
+        if len(ids) > 1:
+            runner.step([StepEntry(rid, ids[:-1])])
+    return tokens, [StepEntry(rid, ids[-1:], [0]) for rid, ids in tokens.items()]
+
+
+def _again(runner, tokens, entries):
+    logits = runner.step(entries).clone()
+    for rid, ids in tokens.items():
+        if len(ids) > 1:
+            runner.computed[rid] = len(ids) - 1
+        else:
+            runner.finish(rid)
+    return logits
+
+
+def _chains(runner):
+    return [e[3].static.get("decode_chain") for kinds in runner._graphs.values() for e in kinds.values()]
+
+
+@pytest.mark.parametrize("page", [8, 24])
+@pytest.mark.parametrize("which", list(SHAPES))
+def test_step_is_the_plain_implementations(tmp_path, which, page):
+    from rapid_llm_amd import write_random_model
+
+    cfg = {**BASE, **SHAPES[which]}
+    folder = str(write_random_model(cfg, 5, tmp_path / which, dtype="bfloat16"))
+    config, weights = plain_load(folder)
+    got, want = [], []
+    for rows in (1, 2, 3, 5, 8, 16):
+        runner = _runner(folder, page_size=page, num_pages=800)
+        tokens, entries = _fill(runner, CONTEXTS[:rows], cfg["vocab_size"])
+        got.append(_again(runner, tokens, entries).cpu())
+        assert all(c is not None for c in _chains(runner)) and len(_chains(runner)) == 1
+        # again, on the same and on other pages' contents: the same bits
+        assert torch.equal(_again(runner, tokens, entries).cpu(), got[-1])
+        want.append(torch.stack([plain_forward(config, weights, ids)[-1] for ids in tokens.values()]))
+    parity.assert_bf16_close(torch.cat(got), torch.cat(want), f"decode chain/{which}/{page}")
+
+
+@pytest.mark.parametrize("rows", [1, 2, 4, 16])
+def test_any_number_of_workgroups_gives_the_same(rows, monkeypatch):
+    from rapid_llm_amd.kernels import decode_chain, ops
+
+    cfg = {**BASE, "hidden_size": 1024, "num_attention_heads": 8, "intermediate_size": 1536}
+    results = []
+    for units in (None, 1, 3, 50, 255):
+        runner = _runner(cfg)
+        tokens, entries = _fill(runner, CONTEXTS[:rows], cfg["vocab_size"])
+        with monkeypatch.context() as m:
+            if units is not None:
+                # as many shares of the keys as ever, dealt to fewer workgroups: some have several of one request
+                real = decode_chain.DecodeChain.run
+
+                def run(self, *args, units=units, real=real):
+                    with pytest.MonkeyPatch.context() as inner:
+                        inner.setattr(decode_chain, "chip", lambda: ops.Chip(units))
+                        return real(self, *args)
+
+                m.setattr(decode_chain.DecodeChain, "run", run)
+            results.append(_again(runner, tokens, entries))
+        assert _chains(runner)[0] is not None
+        torch.cuda.synchronize()
+    for r in results[1:]:
+        assert torch.equal(r, results[0])
+
+
+def test_replays_between_other_steps():
+    from rapid_llm_amd import StepEntry
+
+    cfg = {**BASE, "hidden_size": 1024, "num_attention_heads": 8, "num_hidden_layers": 6, "intermediate_size": 1536}
+    runner = _runner(cfg)
+    steps = []
+    for k, rows in enumerate((1, 2, 7, 16)):  # recorded steps that share one space
+        tokens, entries = _fill(runner, CONTEXTS[:rows], cfg["vocab_size"])
+        want = runner.step(entries, use_graph=False).clone()
+        for rid in tokens:
+            runner.computed[rid] = len(tokens[rid]) - 1
+        first = _again(runner, tokens, entries)
+        parity.assert_bf16_close(first.cpu(), want.cpu(), f"decode chain against kernels/{rows}")
+        for _ in range(60):
+            again = _again(runner, tokens, entries)
+        assert torch.equal(again, first)
+        for rid in list(tokens):
+            runner.finish(rid)
+        steps.append((tokens, first))
+        runner.step([StepEntry("other", random_tokens(70, cfg["vocab_size"], k), [0])])
+        runner.finish("other")
+    for rows, (tokens, first) in zip((1, 2, 7, 16), steps):
+        t2, entries = _fill(runner, CONTEXTS[:rows], cfg["vocab_size"])
+        for _ in range(3):
+            assert torch.equal(_again(runner, t2, entries), first)
+        for rid in list(t2):
+            runner.finish(rid)
+
+
+def test_two_at_once():
+    """Two runners on streams and threads of their own: the chip cannot hold both launches' workgroups at a time."""
+    cfg = {**BASE, "hidden_size": 1024, "num_attention_heads": 8, "num_hidden_layers": 8, "intermediate_size": 3072}
+    pairs = []
+    for rows in (1, 6):
+        runner = _runner(cfg)
+        tokens, entries = _fill(runner, CONTEXTS[:rows], cfg["vocab_size"])
+        pairs.append((runner, tokens, entries, _again(runner, tokens, entries)))
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(runner, tokens, entries, want):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(80):
+                if not torch.equal(_again(runner, tokens, entries), want):
+                    wrong.append(len(tokens))
+
+    threads = [threading.Thread(target=work, args=p) for p in pairs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not wrong
+
+
+def test_layers_that_do_something_else_keep_their_kernels(monkeypatch):
+    cfg = {**BASE, "hidden_size": 512}
+    for change in (dict(head_dim=64), dict(num_attention_heads=10), dict(intermediate_size=392)):
+        runner = _runner({**cfg, **change})
+        tokens, entries = _fill(runner, [20, 3], cfg["vocab_size"])
+        _again(runner, tokens, entries)
+        assert _chains(runner) == [None], change
+    runner = _runner(cfg)
+    real, calls = runner.model.blocks[1].mixer.forward, []
+    runner.model.blocks[1].mixer.forward = lambda *a: calls.append(1) or real(*a)
+    tokens, entries = _fill(runner, [20, 3], cfg["vocab_size"])
+    before = len(calls)
+    _again(runner, tokens, entries)
+    assert _chains(runner) == [None] and len(calls) > before
