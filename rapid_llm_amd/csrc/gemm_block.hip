@@ -1,6 +1,7 @@
 // bfloat16 product for many rows (prompt steps): out[M,N] = X[M,K] * W[N,K]^T, float32 accumulation on
-// the matrix cores; with silu(gate) * up of the packed [gate | up] matrix in the epilogue, stored as bfloat16, or as
-// float32 runs of K.
+// the matrix cores; stored as bfloat16, with silu(gate) * up of the packed [gate | up] matrix in the epilogue, or as
+// float32 runs of K.  (As bfloat16, microseconds over weights from memory, the library's first: 2,048 rows of 6,144 x 4,096 84.7 /
+// 78.9, of 4,096 x 4,096 64.0 / 58.1; 8,926 of 4,096 x 1,024 82.8 / 81.0, of 1,024 x 3,072 62.0 / 55.4; ops.block_plain_plan has the rest.)
 //
 // What bounds it: the matrix cores, and with real operands the clock they run at (zeros: 2.05 PFLOP/s at
 // 8,192 x 8,192 x 8,192, random numbers: 1.55, 1.9 GHz; the library's kernel 2.26 and 1.62), so everything else is kept
@@ -200,7 +201,7 @@ __device__ __forceinline__ f32x4 rounded(f32x4 v, u16x2& most) {
     return __builtin_bit_cast(f32x4, (u32x4){a << 16, a & 0xffff0000u, b << 16, b & 0xffff0000u});
 }
 
-enum BlockOut { OUT_RUNS = 1, OUT_GLU = 2 };
+enum BlockOut { OUT_RUNS = 1, OUT_GLU = 2, OUT_PLAIN = 3 };
 
 // NW x NX pieces of 64 rows: a workgroup's tile is 64 NW weight rows x 64 NX rows of X.
 template <int NW, int NX, BlockOut OUT>
@@ -359,8 +360,8 @@ __global__ __launch_bounds__(BT) void gemm_block_kernel(BlockArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be on its way into LDS when it is given back
     if (wave < 4) __builtin_amdgcn_s_barrier();
     // ---- results: acc[u][t][x][i], row m0 + 64 x + 16 xi + r16 of X ----------------------------
-    const u32 elem = GLU ? 2 : 4;
-    char* base = (char*)a.out + ((GLU ? 0 : (size_t)split * a.M * a.ldo) + (size_t)m0 * a.ldo + n0) * elem;
+    const u32 elem = OUT == OUT_RUNS ? 4 : 2;
+    char* base = (char*)a.out + ((OUT != OUT_RUNS ? 0 : (size_t)split * a.M * a.ldo) + (size_t)m0 * a.ldo + n0) * elem;
     const int rows = min(64 * NX, a.M - m0), cols = a.N - n0;
     auto rs = __builtin_amdgcn_make_buffer_rsrc(base, 0, (u32)rows * (u32)a.ldo * elem, 0x00020000);
     // rows and columns that do not exist fall off the records
@@ -386,6 +387,12 @@ __global__ __launch_bounds__(BT) void gemm_block_kernel(BlockArgs a) {
             } else {
                 const int col = 32 * NW * wi + 32 * u + 8 * g;
                 const bool in = row < rows && col < cols;
+                if constexpr (OUT == OUT_PLAIN) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) o[i] = (__bf16)acc[u][i >> 2][x][i & 3];
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), rs, in ? (row * a.ldo + col) * 2 : -1, 0, 0);
+                    continue;
+                }
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[u][t][x]), rs,
@@ -418,18 +425,20 @@ static int launch_block(const BlockArgs& a, int kind, hipStream_t stream) {
     dim3 grid(a.tiles_w * a.tiles_x * a.splits), block(BT);
     if (kind == OUT_GLU)
         hipLaunchKernelGGL((gemm_block_kernel<NW, NX, OUT_GLU>), grid, block, 0, stream, a);
+    else if (kind == OUT_PLAIN)
+        hipLaunchKernelGGL((gemm_block_kernel<NW, NX, OUT_PLAIN>), grid, block, 0, stream, a);
     else
         hipLaunchKernelGGL((gemm_block_kernel<NW, NX, OUT_RUNS>), grid, block, 0, stream, a);
     return rl_launch_status();
 }
 
 // kind 1: out float32 [splits, M, N], run r of K's chunks in part r.  Kind 2: W = [gate | up] stacked, [2N, K], out
-// bfloat16 [M, N] = silu(gate) * up of the products rounded to bfloat16.
+// bfloat16 [M, N] = silu(gate) * up of the products rounded to bfloat16.  Kind 3: out bfloat16 [M, N].
 // nw, nx: pieces of 64 rows of a tile (2 to 4, 2 or 4; 2, 1).  K a multiple of 64, N of 8.
 extern "C" int rl_gemm_block(const void* X, const void* W, void* out, int M, int N, int K, int ldx, int ldw, int ldo,
                              int kind, int nw, int nx, int splits, hipStream_t stream) {
     if (M <= 0 || N <= 0) return RL_OK;
-    if ((kind != OUT_RUNS && kind != OUT_GLU) || !X || !W || !out || K < 64 || K % 64 || N % 8 || ldx % 8 || ldw % 8 || ldo % 8 || ldx < K ||
+    if ((kind != OUT_RUNS && kind != OUT_GLU && kind != OUT_PLAIN) || !X || !W || !out || K < 64 || K % 64 || N % 8 || ldx % 8 || ldw % 8 || ldo % 8 || ldx < K ||
         ldw < K || ldo < N || splits < 1 || (splits > 1 && kind != OUT_RUNS) ||
         ((uintptr_t)X | (uintptr_t)W | (uintptr_t)out) % 16)
         return RL_ERR_ARG;

@@ -28,6 +28,7 @@ STEP = 128  # every contraction is a multiple of it
 # up to 4,000 1,868 / 1,845; 1.7B (50.3 M) 1 / 2 / 4 / 8 / 16 requests 1,350 / 1,257, 1,375 / 1,361, 1,407 / 1,405, 1,518 / 1,485, 1,797 / 1,662;
 # 4B (101 M) 1 / 8 2,242 / 2,336, 2,572 / 2,763; 8B (193 M) 1 / 8 3,404 / 3,528, 3,762 / 3,982.
 MAX_LAYER_WEIGHTS = 64 << 20
+FEW_LAYER_WEIGHTS = 32 << 20  # of 2 to 7 rows: 1.7B with two of 42 to 546 keys 1,356 / 1,394
 
 _lib: ctypes.CDLL | None = None
 
@@ -49,7 +50,7 @@ def fits(rows: int, hidden: int, nq: int, nkv: int, d: int, inter: int, page_siz
     return (
         1 <= rows <= MAX_ROWS and d == HEAD_DIM and nkv >= 1 and nq % nkv == 0 and nq // nkv <= MAX_GROUP
         and hidden % STEP == 0 and inter % STEP == 0 and page_size % 8 == 0
-        and hidden * ((2 * nq + 2 * nkv) * d + 3 * inter) <= MAX_LAYER_WEIGHTS
+        and hidden * ((2 * nq + 2 * nkv) * d + 3 * inter) <= (FEW_LAYER_WEIGHTS if 2 <= rows < 8 else MAX_LAYER_WEIGHTS)
     )
 
 

@@ -7,8 +7,10 @@ GPU or without the compiled library these raise.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import functools
+import threading
 import os
 from typing import Optional
 
@@ -1440,7 +1442,8 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
 
     Up to 16 rows (decode) run the hand-written bandwidth-bound kernel, which can write
     float32 directly; so does the kernel for 17 to 64 rows over wide matrices.  Small matrices
-    run the one-launch tile product beyond, up to 512 rows.  Everything else goes to the library
+    run the one-launch tile product beyond, up to 512 rows, many rows the many-row product where its tiles fill the chip
+    (:func:`block_plain_plan`).  Everything else goes to the library
     product, as the reference's dense products do (``F.linear``).  A float32 result is written by the
     product itself, save the one-launch tile product's, which is bfloat16 and widened by the caller.
     ``x`` may be columns of a wider row."""
@@ -1491,16 +1494,21 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
             "rl_gemm_rows",
         )
         return out
+    if m * n >= _PLAIN_RESULTS and out_dtype == torch.bfloat16 and _aligned(x, w):  # (a question less for the host)
+        block = block_plain_plan(m, n, k, chip().units)
+        if block is not None:
+            return _block(x, w, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), "plain", block)
     return library_product(x, w, out_dtype)
 
 
 def library_takes(m: int, n: int, k: int) -> bool:
-    """Whether :func:`gemm_bf16` gives ``m`` rows over an ``[n, k]`` matrix to the library."""
+    """Whether :func:`gemm_bf16` gives ``m`` rows over an ``[n, k]`` matrix to the library (operands that begin inside a unit
+    of 16 bytes aside)."""
     if m <= SKINNY_MAX_ROWS and k % 8 == 0:
         return False
     if m <= ROWS_MAX_ROWS and rows_plan(m, n, k, swiglu=False) is not None:
         return False
-    return not _tile_applies(m, n, k, n)
+    return not _tile_applies(m, n, k, n) and block_plain_plan(m, n, k, chip().units) is None
 
 
 def gemm_bf16_wide(x: torch.Tensor, w: torch.Tensor, scaled=None) -> torch.Tensor:
@@ -1635,13 +1643,15 @@ def _tile_applies(m: int, weight_rows: int, k: int, cols: int) -> bool:
     first (over weights from memory at 17 / 37 / 64 rows, the tile product first: 4,096 x 1,024 7.1 / 4.9, 8.0 / 5.9, 8.9 / 6.5;
     2,048 x 1,024 5.7 / 4.1, 6.6 / 4.7, 7.5 / 5.6; at 17 and 64 rows 2,048 x 3,072 16.1 / 7.7, 20.2 / 12.0; 4,096 x 512 4.2 / 3.7,
     5.3 / 4.5; 8,192 x 128 3.1 / 3.4, 3.7 / 4.1; gate and up of 6,144 x 1,024 9.2 / 8.1, 10.9 / 9.2, 12.6 / 10.4, of 12,288
-    x 512 7.3 / 7.7, 10.1 / 9.8), hence from 512 k on, gate and up from 1,024."""
+    x 512 7.3 / 7.7, 10.1 / 9.8), hence from 512 k on, gate and up from 1,024.  A matrix of 8 M
+    elements comes here up to 320 rows inside :func:`own_products`: on the device the two are level."""
     return (
         SKINNY_MAX_ROWS < m <= TILE_MAX_ROWS
         and k % 128 == 0
         and cols % 4 == 0
         and cols * (weight_rows // cols) >= _TILE_MIN_COLS
-        and weight_rows * k <= _TILE_MAX_WEIGHTS
+        and (weight_rows * k <= _TILE_MAX_WEIGHTS
+             or (cols == weight_rows and _own(weight_rows, k) and m <= MID_SMALL_MAX_ROWS))
     )
 
 
@@ -1678,9 +1688,10 @@ _BLOCK_TILES = ((4, 4), (3, 4), (2, 4), (4, 2), (3, 2), (2, 2))
 _BLOCK_COSTS = {
     "gated": ((0.86, 0.49, 7.4), (0.74, 0.36, 5.9), (0.59, 0.24, 3.9), (0.745, 0.153, 2.5), (0.663, 0.068, 2.3), (0.518, 0.044, 1.9)),
     "runs": ((0.85, 0.47, 9.8), (0.73, 0.34, 6.2), (0.56, 0.25, 3.5), (0.64, 0.25, 4.0), (0.525, 0.19, 3.0), (0.42, 0.14, 2.3)),
+    "plain": ((0.942, 0.359, 7.2), (0.805, 0.265, 6.2), (0.637, 0.217, 3.8), (0.741, 0.136, 3.6), (0.62, 0.086, 3.0), (0.491, 0.052, 3.1)),
 }
 _BLOCK_RUN_ELEMENT = 1.1e-6
-BLOCK_RUNS_MIN_K = 6144  # shorter sums than this are never cut into its runs
+BLOCK_RUNS_MIN_K = 6144  # shorter sums than this are cut into its runs at some row counts only
 
 
 def block_plan(m: int, n: int, k: int, kind: str, units: int | None = None) -> tuple[int, int, int] | None:
@@ -1704,13 +1715,18 @@ def block_plan(m: int, n: int, k: int, kind: str, units: int | None = None) -> t
     48.7 / 24.0, 51.8 / 42.0, 82.4 / 64.3, 115 / 101; 1.7B (6,144) 18.6 / 18.3, 28.7 / 28.1, 43.5 / 41.4, and slower from
     there (1,500 rows 50.4 / 54.4).  Against the blocks of 64 rows of the mid-size product, at 65 / 128 / 192 rows:
     8B 42.4 / 30.2, 41.0 / 34.1, 54.6 / 38.9; 4B 23.7 / 21.8, 25.3 / 25.7, 32.3 / 26.2; 1.7B, which stays there up to
-    128 rows, 15.3 / 16.1, 16.6 / 17.9, 20.6 / 19.3.  Sums of 4,096 and less are level or the library's (8B output projection 33.6 / 32.9,
-    48.2 / 48.4, 74.9 / 73.7; 0.6B down 16.7 / 16.9, 19.8 / 21.4, 27.4 / 28.9)."""
-    return _block_plan(m, n, k, kind, chip().units if units is None else units)
+    128 rows, 15.3 / 16.1, 16.6 / 17.9, 20.6 / 19.3.  Sums of 4,096 k and more over matrices narrower
+    than that at 193 to 512 rows (4B output projection, the library's first, at 200 / 320 / 512 rows 25.3 / 18.8, 26.5 / 21.7, 29.0 / 26.7); other shorter ones
+    are level or the library's (8B output projection at 1,024 and 2,048 rows 51.2 / 51.1 and 78.0 / 83.5), and taken
+    inside :func:`own_products` alone (0.6B down at 450 / 700 / 1,024 rows 16.5 / 16.7, 18.5 / 18.3, 19.8 / 21.2, output 13.7 / 16.0,
+    15.2 / 16.4, 15.6 / 18.8).
+
+    ``"plain"``: stored as bfloat16 (:func:`block_plain_plan`)."""
+    return _block_plan(m, n, k, kind, chip().units if units is None else units, kind == "runs" and _own(n, k))
 
 
 @functools.lru_cache(maxsize=4096)
-def _block_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int, int] | None:
+def _block_plan(m: int, n: int, k: int, kind: str, units: int, own: bool = False) -> tuple[int, int, int] | None:
     if m <= ROWS_MAX_ROWS or n % 8 or k % 64 or k < 64:
         return None
     # offsets inside an operand are 32-bit in the kernel, those of rows beyond it too
@@ -1720,7 +1736,13 @@ def _block_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int
     runs = (1,)
     if kind == "runs":
         squares = -(-m // 256) * -(-n // 256)
-        if k < BLOCK_RUNS_MIN_K or (k < 8192 and (m <= 128 or squares > 32)) or squares > 128:
+        if own:
+            if m <= MID_SMALL_MAX_ROWS:
+                return None
+        elif k < BLOCK_RUNS_MIN_K:
+            if k < 4096 or 4 * n > 3 * k or not MID_MAX_ROWS < m <= 512:
+                return None
+        elif (k < 8192 and (m <= 128 or squares > 32)) or squares > 128:
             return None
         runs = (1, 2, 3, 4, 6, 8)
     best = None
@@ -1747,7 +1769,7 @@ def product_bytes(m: int, w: torch.Tensor) -> int:
     if w.dtype == torch.float32:
         return 4 * m * (n + k) + f32_product_bytes(m, n, k)
     plan = block_plan(m, n, k, "runs")
-    runs = plan[2] if plan is not None else mid_runs(n, k) if SKINNY_MAX_ROWS < m <= MID_MAX_ROWS else 0
+    runs = plan[2] if plan is not None else mid_runs(n, k) if SKINNY_MAX_ROWS < m <= mid_max_rows(n, k) else 0
     return 2 * m * (n + k) + 4 * m * n * runs
 
 
@@ -1770,7 +1792,77 @@ def block_few_plan(m: int, n: int, k: int, units: int | None = None) -> tuple[in
     return (2, 1, 1) if (2 * n + 256) * k * 2 <= 0x7FFFFFFF else None
 
 
-_BLOCK_KINDS = {"runs": 1, "gated": 2}  # as the kernel's entry point counts them
+_BLOCK_KINDS = {"runs": 1, "gated": 2, "plain": 3}  # as the kernel's entry point counts them
+
+
+class _Step(threading.local):
+    own_products = False  # the step that this thread is launching keeps to this package's products
+
+
+_step = _Step()
+MID_SMALL_MAX_ROWS = 320  # rows up to which the mid-size product takes small matrices of such a step
+_SMALL_WEIGHTS = 8 << 20  # elements of a matrix
+
+
+@contextlib.contextmanager
+def own_products():
+    """Inside the block, on this thread: small matrices go to this package's products wherever it has one, also where the
+    library's takes the device up to 4 us less."""
+    before, _step.own_products = _step.own_products, True
+    try:
+        yield
+    finally:
+        _step.own_products = before
+
+
+def runs_from_k() -> int:
+    """Shorter sums than this are never left as the many-row product's runs."""
+    return 1024 if _step.own_products else 4096
+
+
+def _own(n: int, k: int) -> bool:
+    """Whether the step's product over an ``[n, k]`` matrix is to be this package's."""
+    return _step.own_products and n * k <= _SMALL_WEIGHTS and min(n, k) >= 1024
+
+
+def mid_max_rows(n: int, k: int) -> int:
+    """Rows up to which the mid-size product takes an ``[n, k]`` matrix (beyond 192 inside :func:`own_products`: with
+    the norm, the library's first, at 200 / 256 / 320 rows 1,024 x 2,048 12.0 / 10.4, 12.1 / 10.9, 13.0 / 13.0; 1,024 x 3,072
+    12.4 / 13.8, 12.3 / 14.8, 15.8 / 15.5; 2,048 x 2,048 13.1 / 14.4, 13.7 / 15.5, 14.8 / 18.4)."""
+    return MID_SMALL_MAX_ROWS if _own(n, k) else MID_MAX_ROWS
+
+
+_PLAIN_RESULTS = 1 << 19  # results of which fewer are too few tiles on any chip
+
+
+def block_plain_plan(m: int, n: int, k: int, units: int) -> tuple[int, int, int] | None:
+    """The plan of the many-row product stored as bfloat16, ``None`` where the library's is the faster one.
+
+    A tile walks K alone and a unit has one, so the tiles decide: seven eighths of the units in one round, seven tenths of
+    several rounds.  Microseconds at 1,024 / 2,048 / 3,000 / 4,096 / 8,926 rows over weights from memory, the library's
+    first: 6,144 x 4,096 56.4 / 51.3, 84.7 / 78.9, 141 / 138, 167 / 156, 418 / 342; 4,096 x 4,096 42.5 / 41.3, 64.0 / 58.1,
+    ., 95.2 / 95.9, 334 / 248; 6,144 x 2,560 38.5 / 36.1, 57.9 / 54.8, 103 / 94.4, 112 / 105, 219 / 226; 4,096 x 2,048
+    24.9 / 22.8, 35.0 / 33.0, 44.9 / 46.4, 53.8 / 55.2, 129 / 137; 2,048 x 2,048 at 2,048 rows 20.8 / 20.3, at 8,926 83.4 /
+    75.6; 1,024 x 2,048 and 3,072 at 8,926 rows 44.2 / 38.8 and 62.0 / 55.4.  With three quarters of the units it is 0.9 to 1.07 of the
+    library's time (1.15 at 6,144 x 2,560 and 512 rows): so far for small matrices only, and with half of them inside
+    :func:`own_products` (4,096 x 1,024 at 600 rows 11.8 / 12.3).  Tiles of 256 x 256 over 1,024 k and less begin and end too much
+    (4,096 x 1,024 at 3,000 rows 25.5 / 27.6)."""
+    return _block_plain_plan(m, n, k, units, _own(n, k))
+
+
+@functools.lru_cache(maxsize=4096)
+def _block_plain_plan(m: int, n: int, k: int, units: int, own: bool) -> tuple[int, int, int] | None:
+    plan = _block_plan(m, n, k, "plain", units)
+    if plan is None:
+        return None
+    tiles = _block_tiles(m, n, "plain", plan)
+    rounds = -(-tiles // units)
+    if rounds > 1:
+        return plan if 10 * tiles >= 7 * rounds * units else None
+    if k <= 1024 and plan[:2] == (4, 4):
+        return None
+    share = 7 if n * k > _SMALL_WEIGHTS else 4 if own else 6
+    return plan if 8 * tiles >= share * units else None
 
 
 def _aligned(a: torch.Tensor, b: torch.Tensor) -> bool:
@@ -1784,7 +1876,6 @@ def block_reads(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.is_contiguous() and w.is_contiguous())
 
 
-@functools.lru_cache(maxsize=4096)
 def block_pays(m: int, n: int, k: int, units: int) -> bool:
     """Whether the ``"runs"`` form is faster, with the norm, than what else there is: the mid-size product up to 192 rows,
     where its workgroups (tiles times runs) have to cover five eighths of the units, the library's beyond, where three
@@ -1794,9 +1885,16 @@ def block_pays(m: int, n: int, k: int, units: int) -> bool:
     library's first: 512 columns of 12,288 k (64 and 96) 20.6 / 21.7, 26.0 / 22.1.  Beyond 1,280 rows sums of less than 9,216 k
     are 12% slower to 23% faster than the library's, as its kernels happen to fit (8,192 k at 1,500 rows: 2,048 columns 0.89
     of its speed, 1,536 1.23), and stay there.  Of 352 sizes, 512 to 8,192 columns at 65 to 2,048 rows, 3 are left slower, by 4%."""
-    plan = _block_plan(m, n, k, "runs", units)
-    if plan is None or (k < 9216 and m > 1280):
+    return _block_pays(m, n, k, units, _own(n, k))
+
+
+@functools.lru_cache(maxsize=4096)
+def _block_pays(m: int, n: int, k: int, units: int, own: bool) -> bool:
+    plan = _block_plan(m, n, k, "runs", units, own)
+    if plan is None or (BLOCK_RUNS_MIN_K <= k < 9216 and m > 1280):
         return False
+    if own:
+        return True
     share = 5 if m <= MID_MAX_ROWS and _mid_runs(n, k, units) > 0 else 3
     return 8 * plan[2] * _block_tiles(m, n, "runs", plan) >= share * units
 
@@ -1856,7 +1954,7 @@ def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor, copies: bool = True) -> to
             x, w = (t.clone() if t.data_ptr() & 15 else t for t in (x, w))
         return _block(x, w, torch.empty((plan[2], m, n), dtype=torch.float32, device=x.device), "runs", plan)
     ks = mid_runs(n, k)
-    if k != w.shape[1] or m > MID_MAX_ROWS or ks < 1:
+    if k != w.shape[1] or m > mid_max_rows(n, k) or ks < 1:
         raise KernelError(f"gemm_bf16_parts does not take x {tuple(x.shape)}, w {tuple(w.shape)}")
     return _mid_parts(x, w, ks)
 

@@ -38,6 +38,13 @@ REPEAT_MAX_TOKENS = 2048
 # behind its last use: bytes of them, as estimated, up to which that is done.  A quarter of what the engine leaves for a step's
 # activations, so that no step comes to need more than there is; steps that are this large are not bound by the host.
 REPEAT_MAX_BYTES = 1 << 28
+# Tokens times a layer's matrix elements up to which a step keeps to this package's products, where it can do without the
+# library's at all: a call of that costs the host 18 us, and a layer with one cannot be launched from native code, so
+# up to there the device waits for the host.  Microseconds a prompt step, with library products / without: 0.6B (15.7 M) at 200 /
+# 300 / 512 / 800 / 1,024 tokens 3,612 / 1,983, 3,609 / 2,239, 3,619 / 2,579, 3,998 / 2,948, 4,058 / 3,293 (at 1,500 level); 1.7B (50.3 M) at
+# 100 / 200 / 300 / 450 tokens 3,564 / 2,526, 3,414 / 2,776, 3,601 / 3,244, 3,484 / 3,632.  Recorded steps gain by fewer starts: 0.6B with 256
+# requests 5,272 / 5,127, 1.7B with 192 4,358 / 4,155.
+OWN_PRODUCTS_MAX = 20_000_000_000
 
 
 class CausalLM:
@@ -277,9 +284,25 @@ class CausalLM:
             return None
         return DeferredProduct(self.blocks[self.order[-1]].feed_forward.last_product, after) if lazy else after
 
+    def _own_products(self, ctx) -> bool:
+        """Whether the step keeps to this package's products (``OWN_PRODUCTS_MAX``)."""
+        block = self.blocks[self.order[0]]
+        if ctx.num_tokens <= ops.SKINNY_MAX_ROWS or block.launch_signature() is None:
+            return False
+        if ctx.num_tokens * sum(t.numel() for t in block.own_tensors() if t.dim() == 2) > OWN_PRODUCTS_MAX:
+            return False
+        with ops.own_products():
+            return not block.calls_library(ctx.num_tokens)
+
     def forward(self, ctx, caches) -> torch.Tensor:
         """Run the tokens of ``ctx`` through every layer (which writes their keys and values)
         and return float32 logits ``[len(ctx.logit_rows), vocab]``."""
+        if self._own_products(ctx):
+            with ops.own_products():
+                return self._forward(ctx, caches)
+        return self._forward(ctx, caches)
+
+    def _forward(self, ctx, caches) -> torch.Tensor:
         residual = self.embed.forward(ctx.token_ids, ctx)
         # the embedding's output, which later places take in again (the stream itself is updated
         # in place)

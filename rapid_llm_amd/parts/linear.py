@@ -13,7 +13,7 @@ Which product runs is decided by the weight's storage type:
 * bfloat16 weight: few rows (decode) go to the hand-written bandwidth-bound matrix-core
   kernel, more to kernels of this package for small and for wide matrices; a matrix whose result a norm adds
   to the residual may hand that norm float32 runs of K instead (``partial_sums``: 17 to 192 rows of a
-  narrow one, more where K is long).  What none of them takes goes to the library product, as in the reference, whose dense
+  narrow one, 320 of a small one, more where K is long).  What none of them takes goes to the library product, as in the reference, whose dense
   products are ``F.linear`` (rapid_llm/kernels/ops/gemm/linear.py:17-40).  The packed gate and up matrices have kernels of
   their own (``ops.gemm_bf16_swiglu``).
 """
@@ -71,8 +71,7 @@ class Linear:
         n, k = self.out_features, self.in_features
         if self.weight.dtype != torch.bfloat16:
             return False
-        if folded and ((rows <= ops.MID_MAX_ROWS and ops.mid_runs(n, k) > 0)
-                       or (k >= ops.BLOCK_RUNS_MIN_K and ops.block_pays(rows, n, k, ops.chip().units))):
+        if folded and ((rows <= ops.mid_max_rows(n, k) and ops.mid_runs(n, k) > 0) or ops.block_pays(rows, n, k, ops.chip().units)):
             return False
         return ops.library_takes(rows, n, k)
 
@@ -88,9 +87,10 @@ class Linear:
         rows = x.shape[0]
         if self.weight.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or rows <= ops.SKINNY_MAX_ROWS:
             return False
-        if rows <= ops.MID_MAX_ROWS and ops.mid_runs(self.out_features, self.in_features) > 0:
+        n, k = self.out_features, self.in_features
+        if rows <= ops.MID_SMALL_MAX_ROWS and rows <= ops.mid_max_rows(n, k) and ops.mid_runs(n, k) > 0:
             return True
-        return self.in_features >= ops.BLOCK_RUNS_MIN_K and ops.block_reads(x, self.weight)
+        return k >= ops.runs_from_k() and ops.block_reads(x, self.weight)
 
     def partial_sums(self, x: torch.Tensor) -> torch.Tensor:
         """``[runs, M, out]`` float32 whose sum over the runs is ``x W^T`` (without the bias)."""

@@ -10,6 +10,7 @@ def test_sizes():
     for name, (h, nq, nkv, inter) in family.items():
         for rows in (1, 16):
             assert chain.fits(rows, h, nq, nkv, 128, inter, 16) == (name in ("0.6b", "1.7b"))
+        assert chain.fits(2, h, nq, nkv, 128, inter, 16) == (name == "0.6b")
     assert not chain.fits(0, 1024, 16, 8, 128, 3072, 16) and not chain.fits(17, 1024, 16, 8, 128, 3072, 16)
     for sizes in ((1024, 16, 8, 64, 3072, 16), (1024, 16, 8, 128, 3008, 16), (1000, 16, 8, 128, 3072, 16), (1024, 16, 8, 128, 3072, 4),
                   (1024, 15, 8, 128, 3072, 16), (1024, 40, 8, 128, 3072, 16)):
