@@ -19,7 +19,14 @@
 // no visible key of a row leaves that row's state as it is, exactly (factor 1, terms 0), and so does
 // a span or a wave without visible keys in the fold.  A launch of few tiles (decoding) may therefore
 // give every span to a workgroup of its own, which leaves its waves' states to a second kernel that
-// folds them in the same order: the same bits.  Masked keys contribute exactly zero
+// folds them in the same order: the same bits.
+//
+// What bounds it: whole contexts of 2,048 keys, 32 query and 8 kv heads of 128 channels, take 404 us (85 TFLOP/s;
+// 5,000 keys 91).  The float32 matrix instructions hold the vector units for 53% of that, their rate, and the
+// other vector instructions for 36%, the weights of a tile above all; they do not overlap.  Two tiles of rows a
+// workgroup, which halve the keys that are read, leave one wave a SIMD and took 428 us.  Before, a tile's entry of the
+// block table was asked for and waited for with its keys and with its values, both behind every load in flight, at a
+// position that took a division, and the maximum and the sum of a row went through LDS: 514 us.  Masked keys contribute exactly zero
 // (rapid_llm/kernels/ops/attention/flashdecoding.py:223-237); scores are (q . k) / sqrt(d)
 // (rapid_llm/modules/attention.py:62), softmax over keys in float32
 // (rapid_llm/kernels/ops/attention/flashattention2_nopad.py:138-168).
@@ -48,14 +55,35 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ inline f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
 // the four lanes (r, g = 0..3) that share a row: the same bits in each of them
+// (exchanged between registers: through LDS, as a shuffle goes, each step waits for a round trip)
 __device__ inline float row_max(float v) {
-    v = fmaxf(v, __shfl_xor(v, 16, RL_WAVE));
-    return fmaxf(v, __shfl_xor(v, 32, RL_WAVE));
+    const unsigned u = __float_as_uint(v);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned w = __float_as_uint(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+    const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 __device__ inline float row_sum(float v) {
-    v += __shfl_xor(v, 16, RL_WAVE);
-    return v + __shfl_xor(v, 32, RL_WAVE);
+    const unsigned u = __float_as_uint(v);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned w = __float_as_uint(__uint_as_float(a[0]) + __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
+
+// A position of the cache that walks on by the keys between two tiles of a wave, without a division.
+struct Walk {
+    int key, page, off;
+    __device__ inline void step(int keys, int pages, int offs, int page_size) {
+        key += keys;
+        page += pages;
+        off += offs;
+        if (off >= page_size) {
+            off -= page_size;
+            ++page;
+        }
+    }
+};
 
 // (m, l, acc) folded with the state of later keys, (m2, l2, acc2); written out so that every kernel
 // rounds alike.  `none`: neither has seen a key.
@@ -84,12 +112,14 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
     const int* __restrict__ tile_info, const int* __restrict__ positions,
     const int* __restrict__ token_slot, const int* __restrict__ block_table, int table_stride,
     int page_size, int nq, int nkv, int window, float scale, int spans, int per, int held) {
-    const int tile = blockIdx.x;
-    const int hk = blockIdx.y;
+    // Whole contexts: neighbouring workgroups have different kv heads, so that with eight of them each of the
+    // chip's dies keeps one in its L2, and the last tiles, which have the most keys, begin first.
+    const int tile = SPLIT ? blockIdx.x : gridDim.x / nkv - 1 - blockIdx.x / nkv;
+    const int hk = SPLIT ? blockIdx.y : blockIdx.x % nkv;
     const int G = nq / nkv;
     const int at = tile_info[3 * tile], n = tile_info[3 * tile + 1], row0 = tile_info[3 * tile + 2];
     __shared__ float fold_ml[AW - 1][2][RL_WAVE];
-    __shared__ float fold_acc[AW - 1][DB * 4][RL_WAVE];
+    __shared__ f32x4 fold_acc[AW - 1][DB][RL_WAVE];
     const int lane = threadIdx.x & (RL_WAVE - 1);
     const int wave = threadIdx.x / RL_WAVE;
     const int r16 = lane & 15;
@@ -133,18 +163,26 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
 
     // operands of one tile of 16 keys: lane (key r16, g) reads channels 16c + 4g .. + 3 of its
     // key; lane (channel r16, g) reads keys kb + 4g .. + 3 of its channel in every block
-    auto load_keys = [&](int kb, f32x4 (&f)[DB]) {
-        const int key = min(kb + r16, hi - 1);  // beyond the cache: any real key, masked below
-        const float* krow =
-            k_cache + (((size_t)table[key / page_size] * nkv + hk) * page_size + key % page_size) * D + 4 * g;
+    // The entry of the block table is asked for a tile before (`ask`): the loads of a wave return in their
+    // order, so that asking and waiting for it here would wait for every load before it too.
+    const unsigned page_keys = (unsigned)page_size * D;
+    const int last_page = (hi - 1) / page_size, last_off = hi - 1 - last_page * page_size;
+    struct Place {
+        int entry, off;
+    };
+    auto ask_keys = [&](const Walk& w) -> Place {  // beyond the cache: any real key, masked below
+        return {table[w.key < hi ? w.page : last_page], w.key < hi ? w.off : last_off};
+    };
+    auto ask_values = [&](const Walk& w) -> Place {
+        return {table[w.key < hi ? w.page : last_page], w.key < hi ? w.off : last_off & ~3};
+    };
+    auto load_keys = [&](const Place& at_, f32x4 (&f)[DB]) {
+        const float* krow = k_cache + (size_t)((unsigned)at_.entry * nkv + hk) * page_keys + at_.off * D + 4 * g;
 #pragma unroll
         for (int c = 0; c < DB; ++c) f[c] = ld4(krow + 16 * c);
     };
-    auto load_values = [&](int kb, f32x4 (&f)[DB]) {
-        const int key4 = min(kb + 4 * g, (hi - 1) & ~3);
-        const float* vrow = v_cache +
-                            (((size_t)table[key4 / page_size] * nkv + hk) * D + r16) * page_size +
-                            key4 % page_size;
+    auto load_values = [&](const Place& at_, f32x4 (&f)[DB]) {
+        const float* vrow = v_cache + (size_t)((unsigned)at_.entry * nkv + hk) * page_keys + r16 * page_size + at_.off;
 #pragma unroll
         for (int b = 0; b < DB; ++b) f[b] = ld4(vrow + (size_t)16 * b * page_size);
     };
@@ -164,45 +202,54 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
         return (part[0] + part[1]) + (part[2] + part[3]);
     };
 
-    // softmax and second product of the tile at kb, given its scores and its values
-    auto finish_tile = [&](int kb, f32x4 s, const f32x4 (&vcur)[DB]) {
-        // ---- this lane's keys kb + 4g + i of its own row ------------------------------------
-        float tmax = -INFINITY;
+    // Softmax and second product of the tile at kb, given its scores and its values.  Tiles that every row sees whole,
+    // which are most, take no masks.
+    const int whole_from = window > 0 ? last_pos - window + 1 : 0;
+    auto whole = [&](int kb) { return kb >= whole_from && kb + 15 <= first_pos; };
+    auto finish_tile = [&](int kb, f32x4 s, f32x4 (&vals)[DB]) {
+#pragma clang fp contract(off)  // a score is rounded before the maximum is subtracted, in every kernel alike
+        const bool all = whole(kb);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int key = kb + 4 * g + i;
-            const bool seen = row_ok && key >= kstart && key < kend;
-            s[i] = seen ? s[i] * scale : -INFINITY;
-            tmax = fmaxf(tmax, s[i]);
-        }
-        tmax = row_max(tmax);
-        const float m_new = fmaxf(m, tmax);
-        float alpha = 1.f;  // no visible key so far and none here: nothing changes
-        f32x4 p = (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (m_new != -INFINITY) {
-            alpha = expf(m - m_new);  // m = -inf before the row's first key: 0
+        for (int i = 0; i < 4; ++i) s[i] *= scale;
+        if (!all) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) p[i] = expf(s[i] - m_new);  // masked: exactly 0
+            for (int i = 0; i < 4; ++i) {
+                const int key = kb + 4 * g + i;  // this lane's keys of its own row
+                if (!row_ok || key < kstart || key >= kend) s[i] = -INFINITY;
+            }
         }
+        const float m_new = fmaxf(m, row_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+        const bool none = m_new == -INFINITY;  // no visible key so far and none here: nothing changes
+        const float alpha = none ? 1.f : expf(m - m_new);  // m = -inf before the row's first key: 0
+        f32x4 p;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = none ? 0.f : expf(s[i] - m_new);  // masked: exactly 0
         l = fmaf(l, alpha, row_sum((p[0] + p[1]) + (p[2] + p[3])));
         m = m_new;
-        // ---- O^T = O^T alpha + V^T P^T --------------------------------------------------------
 #pragma unroll
-        for (int b = 0; b < DB; ++b) {
-            f32x4 vf = vcur[b];
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[b][i] *= alpha;
+        if (!all) {
             // keys no row of the tile sees (beyond the cache, or before the window, whose
             // pages may have been given back) may hold anything: 0 * it must be 0
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int key = kb + 4 * g + i;
-                if (key >= hi || key < first_key) vf[i] = 0.f;
-            }
+                if (key >= hi || key < first_key) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[b][i] *= alpha;
+                    for (int b = 0; b < DB; ++b) vals[b][i] = 0.f;
+                }
+            }
+        }
+        // ---- O^T += V^T P^T (two chains of dependent instructions in turn) ---------------------
+#pragma unroll
+        for (int b = 0; b < DB; b += 2)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[j], p[j], acc[b], 0, 0, 0);
-        }
+#pragma unroll
+                for (int u = b; u < b + 2 && u < DB; ++u)
+                    acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vals[u][j], p[j], acc[u], 0, 0, 0);
     };
 
     // a span is over: its state joins the wave's (a launch that walks whole contexts), or goes to memory
@@ -242,46 +289,51 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
         for (int b = 0; b < DB; ++b) acc[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
     };
 
-    // Software pipeline over the wave's tiles: while a tile goes through softmax and the second
-    // product, the scores of the next have been multiplied, and that tile's values and the keys of
-    // the one after are in flight (values travel a tile later than their keys: 32 registers fewer at 128
-    // channels, which keeps two waves a SIMD).  The last two tiles stand outside the loop, so that inside
-    // it the loads are issued without a condition and stay where they are written (behind a condition the
-    // compiler counts a load as absent and makes every older operand wait for it; left to
-    // itself the scheduler moves loads down to their use).
+    // Software pipeline over the wave's tiles: the scores of the next tile have been multiplied when a tile
+    // is finished, and the keys of the one after travel meanwhile; a tile's values travel while the scores
+    // of the next are multiplied.  Inside the loop the loads are issued without a condition and stay where they
+    // are written (behind a condition the compiler counts a load as absent and makes every older operand wait
+    // for it; left to itself the scheduler moves loads down to their use): the last tiles ask for the last
+    // keys again.
     constexpr int STEP = 16 * AW;
     const int mine = from + 16 * ((wave - from / 16) & (AW - 1));  // first tile >= from with index % AW == wave
     if (SPLIT && mine < upto && mine / SPAN > span) finish_span();  // no tile of this wave in the first span
     if (mine < upto) {
         int left = (upto - mine + STEP - 1) / STEP;  // tiles of this wave, the current one included
         int kb = mine;
-        f32x4 keys[DB], vcur[DB], vnext[DB];
-        load_keys(kb, keys);
-        load_values(kb, vcur);
+        const int step_pages = STEP / page_size, step_offs = STEP - step_pages * page_size;
+        Walk kw, vw;
+        kw.key = kb + r16, kw.page = kw.key / page_size, kw.off = kw.key - kw.page * page_size;
+        vw.key = kb + 4 * g, vw.page = vw.key / page_size, vw.off = vw.key - vw.page * page_size;
+        f32x4 keys[DB], vals[DB], s_next;
+        Place k_next = ask_keys(kw), v_next = ask_values(vw);
+        load_keys(k_next, keys);
+        load_values(v_next, vals);
+        kw.step(STEP, step_pages, step_offs, page_size);
+        vw.step(STEP, step_pages, step_offs, page_size);
+        k_next = ask_keys(kw);
+        v_next = ask_values(vw);
         f32x4 sc = scores(keys);
-        if (left > 1) load_keys(kb + STEP, keys);
-        while (left > 2) {
-            const f32x4 s_next = scores(keys);
-            load_values(kb + STEP, vnext);
-            load_keys(kb + 2 * STEP, keys);
+        if (left > 1) load_keys(k_next, keys);
+        kw.step(STEP, step_pages, step_offs, page_size);
+        k_next = ask_keys(kw);
+        while (--left > 0) {
+            s_next = scores(keys);
+            kw.step(STEP, step_pages, step_offs, page_size);
+            vw.step(STEP, step_pages, step_offs, page_size);
+            const Place k_ask = ask_keys(kw), v_ask = ask_values(vw);
+            load_keys(k_next, keys);
             __builtin_amdgcn_sched_barrier(0);
-            finish_tile(kb, sc, vcur);
+            finish_tile(kb, sc, vals);
+            load_values(v_next, vals);
+            __builtin_amdgcn_sched_barrier(0);
+            k_next = k_ask;
+            v_next = v_ask;
             sc = s_next;
-#pragma unroll
-            for (int b = 0; b < DB; ++b) vcur[b] = vnext[b];
             kb += STEP;
-            --left;
             if (kb % SPAN < STEP) finish_span();
         }
-        if (left == 2) {
-            const f32x4 s_next = scores(keys);
-            load_values(kb + STEP, vnext);
-            finish_tile(kb, sc, vcur);
-            if ((kb + STEP) % SPAN < STEP) finish_span();
-            finish_tile(kb + STEP, s_next, vnext);
-        } else {
-            finish_tile(kb, sc, vcur);
-        }
+        finish_tile(kb, sc, vals);
     }
     if (SPLIT) {
         // the last span, and one that holds no tile of this wave
@@ -295,9 +347,7 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
         fold_ml[wave - 1][0][lane] = m_all;
         fold_ml[wave - 1][1][lane] = l_all;
 #pragma unroll
-        for (int b = 0; b < DB; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) fold_acc[wave - 1][4 * b + i][lane] = acc_all[b][i];
+        for (int b = 0; b < DB; ++b) fold_acc[wave - 1][b][lane] = acc_all[b];
     }
     __syncthreads();
     if (wave > 0) return;
@@ -307,9 +357,11 @@ __global__ __launch_bounds__(AW* RL_WAVE) void attn_f32_kernel(
         l_all = fold_sum(l_all, fold_ml[w][1][lane], f);
         m_all = f.m;
 #pragma unroll
-        for (int b = 0; b < DB; ++b)
+        for (int b = 0; b < DB; ++b) {
+            const f32x4 other = fold_acc[w][b][lane];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc_all[b][i] = fold_sum(acc_all[b][i], fold_acc[w][4 * b + i][lane], f);
+            for (int i = 0; i < 4; ++i) acc_all[b][i] = fold_sum(acc_all[b][i], other[i], f);
+        }
     }
     if (!row_ok) return;
     // acc_all[b][i] is channel 16b + 4g + i of the lane's row
@@ -396,7 +448,8 @@ extern "C" int rl_attn_f32(const float* q, const float* k_cache, const float* v_
     if (spans < 0 || spans > 65535 || per < 1 || held < 1 || held > 16 || (spans && !states)) return RL_ERR_ARG;
     const dim3 block(AW * RL_WAVE);
     if (!spans) {
-        hipLaunchKernelGGL(attn_f32_kernel<false>, dim3(num_tiles, nkv), block, 0, stream, q, k_cache, v_cache, out,
+        if ((long long)num_tiles * nkv > 0xffffffffll / (AW * RL_WAVE)) return RL_ERR_ARG;
+        hipLaunchKernelGGL(attn_f32_kernel<false>, dim3(num_tiles * nkv), block, 0, stream, q, k_cache, v_cache, out,
                            states, tile_info, positions, token_slot, block_table, table_stride, page_size, nq, nkv,
                            window, scale, 0, 1, held);
         return rl_launch_status();

@@ -213,6 +213,26 @@ def test_attention_f32_split_states_of_decoding_requests(d, nq, nkv, monkeypatch
     torch.testing.assert_close(outs[0].cpu(), want, rtol=2e-5, atol=3e-6)
 
 
+@pytest.mark.parametrize("window", [0, 40, 200], ids=lambda w: f"w{w}")
+@pytest.mark.parametrize("d", [48, 128])
+def test_attention_f32_walks_pages_of_any_size(d, window, monkeypatch):
+    """A wave of the float32 attention steps through the block table by the 64 keys between its tiles: pages of
+    fewer keys than a tile, of a part of a step, of a step and of more, whole contexts and spans of their own,
+    at contexts of one tile of a wave, of two, and that end within a page: the same bits whatever the pages."""
+    ops = _ops()
+    seqs = [(0, 1), (0, 65), (63, 3), (64, 1), (127, 2), (190, 70), (255, 1), (600, 9)]
+    outs = []
+    for page in (16, 4, 12, 48, 64, 68, 148):
+        q, kc, vc, table, ctx, want = _paged_problem(seqs, 6, 2, d, page, torch.float32, d + window, window)
+        for spans in (0, 3):
+            monkeypatch.setattr(ops, "f32_spans", lambda *args: spans)
+            out = torch.full_like(q, float("nan"))
+            ops.attention_f32(q, kc, vc, out, ctx, table, page, 6, 2, d, window, 1.0 / math.sqrt(d))
+            outs.append(out)
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
+    torch.testing.assert_close(outs[0].cpu(), want, rtol=2e-5, atol=3e-6)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 def test_decode_attention_of_many_requests_of_mixed_lengths(dtype):
     """More workgroups than the chip holds at a time: the decode kernel then takes the requests
