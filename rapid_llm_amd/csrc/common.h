@@ -25,22 +25,19 @@ __device__ __host__ inline float bf16_to_float(bf16_t v) {
     return c.f;
 }
 
-// round to nearest, ties to even; NaN stays NaN
+// round to nearest, ties to even; NaN stays NaN (quiet, with its upper payload).  On the device one instruction,
+// which gives these bits for all 2^32 floats; written out it takes ten and a branch, in straight-line code that a short
+// kernel runs through once and waits for: the 64 stores of a lane of the prefill attention took 2.2 us.
 __device__ __host__ inline bf16_t float_to_bf16(float f) {
-    union {
-        uint32_t u;
-        float f;
-    } c;
-    c.f = f;
-    uint32_t u = c.u;
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_bit_cast(bf16_t, (__bf16)f);
+#else
+    const uint32_t u = __builtin_bit_cast(uint32_t, f);
     bf16_t r;
-    if ((u & 0x7fffffffu) > 0x7f800000u) {
-        r.bits = (uint16_t)((u >> 16) | 0x0040u);
-        return r;
-    }
-    u += 0x7fffu + ((u >> 16) & 1u);
-    r.bits = (uint16_t)(u >> 16);
+    r.bits = (u & 0x7fffffffu) > 0x7f800000u ? (uint16_t)((u >> 16) | 0x0040u)
+                                             : (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
     return r;
+#endif
 }
 
 __device__ inline float to_float(float v) { return v; }

@@ -2132,14 +2132,15 @@ class AttentionPlan:
             shape = self.shapes[(nkv, window)] = _prefill_shape(self, nkv, window, tile_rows_of(lib))
         return shape
 
-    def work_order(self, nkv: int, device, resident: int = 1) -> torch.Tensor:
+    def work_order(self, nkv: int, device, resident: int = 1) -> torch.Tensor | None:
         """Order in which the (tile, kv head) pairs of the prefill kernel are handed out:
         longest first, so that the short ones fill the gaps at the end.  Where a compute unit
         holds two workgroups at a time (``resident == 2``), the first round, one workgroup on
         every unit, takes the longest, and the second round, which joins them on the same
-        units, the shortest in ascending order, so that a unit's two workgroups add up alike."""
-        order = self.orders.get((nkv, resident))
-        if order is None:
+        units, the shortest in ascending order, so that a unit's two workgroups add up alike.  ``None``: in
+        the order of their numbers, as where every tile reads as many keys (one short prompt), for which
+        the kernel then need not wait."""
+        if (nkv, resident) not in self.orders:
             items = sorted(range(self.num_tiles * nkv), key=lambda i: (-self.tile_keys[i // nkv], i))
             if resident == 2:
                 round_one = chip().first_round
@@ -2148,9 +2149,9 @@ class AttentionPlan:
                 second = rest[::-1][:round_one]
                 middle = rest[: max(0, len(rest) - round_one)]
                 items = first + second + middle
-            order = upload_ints(items, device)
-            self.orders[(nkv, resident)] = order
-        return order
+            listed = items != list(range(len(items)))
+            self.orders[(nkv, resident)] = upload_ints(items, device) if listed else None
+        return self.orders[(nkv, resident)]
 
 
 # A decode launch splits the keys until it has a workgroup for every compute unit; the fewest

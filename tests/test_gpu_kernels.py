@@ -213,6 +213,26 @@ def test_attention_f32_split_states_of_decoding_requests(d, nq, nkv, monkeypatch
     torch.testing.assert_close(outs[0].cpu(), want, rtol=2e-5, atol=3e-6)
 
 
+@pytest.mark.parametrize("d,page", [(48, 12), (64, 16), (128, 16), (128, 12), (256, 16)])
+def test_attention_rounds_its_results_to_the_nearest_even(d, page):
+    """Two keys that weigh alike (the queries are 0): the result is half the sum of two bfloat16 values, a
+    tie between its neighbours in one of four, rounded once; prompts (one of which sees its first key alone), single
+    tokens, with workgroups in the order of their numbers and in one that the host lists."""
+    ops = _ops()
+    nq, nkv = 6, 2
+    for seqs in ([(0, 2)], [(0, 2), (1, 1), (1, 1), (0, 1)], [(0, 1), (0, 2), (1, 1)]):
+        q, kc, vc, table, ctx, _ = _paged_problem(seqs, nq, nkv, d, page, torch.bfloat16, d + page)
+        q.zero_()
+        out = torch.full_like(q, float("nan"))
+        ops.paged_attention(q, kc, vc, out, ctx, table, page, nq, nkv, d, 0, 1.0 / math.sqrt(d))
+        for t, (slot, pos) in enumerate(zip(ctx.token_slot.tolist(), ctx.positions.tolist())):
+            values = vc[int(table[slot, 0]), :, :, : pos + 1].float().sum(2) / (pos + 1)
+            want = values.bfloat16().repeat_interleave(nq // nkv, 0).reshape(-1)
+            assert torch.equal(out[t], want), (seqs, t)
+        if len(seqs) == 1:
+            assert ops.attention_plan(ctx, nq // nkv, d).work_order(nkv, q.device) is None
+
+
 @pytest.mark.parametrize("window", [0, 40, 200], ids=lambda w: f"w{w}")
 @pytest.mark.parametrize("d", [48, 128])
 def test_attention_f32_walks_pages_of_any_size(d, window, monkeypatch):
