@@ -28,7 +28,7 @@
 //     them asks for them until the number is right: one trip through memory, 1.3 to 1.5 us a phase where storing,
 //     waiting for the stores, a flag, seeing it and loading are 2.1 to 2.3 (256 workgroups, nothing else going on).  No
 //     place is written twice in a launch.
-//   * otherwise a workgroup stores, waits until that has reached memory and then says up to which phase it is done, in a
+//   * otherwise a workgroup stores, waits until that has reached memory and then says up to which phase of which launch it is done, in a
 //     line of its own (flags side by side in lines: 3.2 to 4.0 us a phase; stores to one line follow each other).  Rows of
 //     the products' inputs are then read through the L2: a line of them has one writer, who has written all of it, and
 //     nobody has asked for it before.
@@ -55,7 +55,7 @@ typedef __attribute__((address_space(3))) void* rl_lds_ptr;
 #define CH_KEYS (32 * SW)    // keys that the waves walk in one step
 #define CH_ALONE (2 * CH_KEYS)  // keys up to which a request's context is one share
 #define CH_MAX_WORKGROUPS 512
-#define FLAG_STRIDE 16       // words between two workgroups' flags
+#define FLAG_STRIDE 8        // words of 64 bits between two workgroups' flags
 #define PHASES 5
 #define AUX_SC1 16           // a load that passes by this die's L2
 
@@ -81,8 +81,11 @@ struct Control {
     u32 launch;
     u32 abort;     // of a launch that was given up: every later one ends at once
     u32 pad2[29];
-    u32 flags[CH_MAX_WORKGROUPS * FLAG_STRIDE];  // phases (over all launches) that a workgroup is done with
+    u64 flags[CH_MAX_WORKGROUPS * FLAG_STRIDE];  // phases that a workgroup is done with, and the tag of the launch that they are of
 };
+// Whether a workgroup's flag says that it is done with so many phases of the launch.  A flag names its launch: launches
+// that write none pass between two that do, any number of them, and a flag that was never written names none.
+__device__ __host__ inline bool done_with(u64 flag, u32 tag, u32 phases) { return (u32)(flag >> 32) == tag && (u32)flag >= phases; }
 
 // n / d for n below 2^32 / d: a multiplication
 struct Divisor {
@@ -796,8 +799,8 @@ __device__ __forceinline__ void wait_and_prepare(Args args, unsigned char* lds, 
     using S = Shape<XG>;
     const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
     const int G = args->nq / args->nkv;
-    const u32 rank = lds_get(&ctl->rank), workgroups = lds_get(&ctl->workgroups), launch = lds_get(&ctl->launch);
-    const u32 tag = launch + 1;
+    const u32 rank = lds_get(&ctl->rank), workgroups = lds_get(&ctl->workgroups);
+    const u32 tag = lds_get(&ctl->launch) + 1;
     u32 complete = 0;          // phases of the launch known to be complete
     u32 scaled = 0xffffffffu;  // the phase whose norm's factors were computed last
     for (int seq = 0;; ++seq) {
@@ -834,21 +837,20 @@ __device__ __forceinline__ void wait_and_prepare(Args args, unsigned char* lds, 
         }
         if (!TAGGED && complete < ph) {
             // every workgroup is done with the phase before
-            const u32 want = launch * (u32)(a->num_layers * PHASES) + ph;
-            const u32* flags = a->control->flags;
+            const u64* flags = a->control->flags;
             u32 turns = 0;
             for (u32 i0 = 0; i0 < workgroups; i0 += 64 * 4) {
                 bool left[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) left[j] = i0 + 64 * j + lane < workgroups;
                 for (;;) {
-                    u32 f[4];
+                    u64 f[4];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) f[j] = left[j] ? agent_load(flags + (i0 + 64 * j + lane) * FLAG_STRIDE) : want;
+                    for (int j = 0; j < 4; ++j) f[j] = left[j] ? agent_load(flags + (i0 + 64 * j + lane) * FLAG_STRIDE) : 0;
                     bool any = false;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        left[j] = left[j] && (int)(f[j] - want) < 0;
+                        left[j] = left[j] && !done_with(f[j], tag, ph);
                         any = any || left[j];
                     }
                     if (!__any(any)) break;
@@ -1114,16 +1116,15 @@ __device__ __forceinline__ void add_and_store(Args args, unsigned char* lds, Ctl
     using S = Shape<XG>;
     const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
     const f32x4* red = reinterpret_cast<const f32x4*>(lds + S::AT_SCRATCH);
-    const u32 rank = lds_get(&ctl->rank), workgroups = lds_get(&ctl->workgroups), launch = lds_get(&ctl->launch);
-    const u32 tag = launch + 1;
-    const u32 base = launch * (u32)(args->num_layers * PHASES);  // phases of the launches before
+    const u32 rank = lds_get(&ctl->rank), workgroups = lds_get(&ctl->workgroups);
+    const u32 tag = lds_get(&ctl->launch) + 1;
     if (!TAGGED) {  // the phases in front of its first item
         u32 done = (u32)(args->num_layers * PHASES);
         if (rank < args->total) {
             const Item it = item_of(args, rank);
             done = (u32)(it.layer * PHASES + it.phase);
         }
-        if (done > 0 && lane == 0) agent_store(args->control->flags + rank * FLAG_STRIDE, base + done);
+        if (done > 0 && lane == 0) agent_store(args->control->flags + rank * FLAG_STRIDE, pair64(done, tag));
     }
     for (int seq = 0;; ++seq) {
         const u32 t = rank + (u32)seq * workgroups;
@@ -1263,7 +1264,7 @@ __device__ __forceinline__ void add_and_store(Args args, unsigned char* lds, Ctl
         }
         if (tells) {
             stores_done();
-            if (lane == 0) agent_store(a->control->flags + rank * FLAG_STRIDE, base + done);
+            if (lane == 0) agent_store(a->control->flags + rank * FLAG_STRIDE, pair64(done, tag));
         }
     }
 }
@@ -1364,6 +1365,9 @@ extern "C" int rl_decode_chain_layer_bytes() { return (int)sizeof(ChainLayer); }
 extern "C" int rl_decode_chain_max_group() { return CH_MAX_GROUP; }
 extern "C" int rl_decode_chain_min_keys() { return CH_KEYS; }
 extern "C" int rl_decode_chain_control() { return (int)sizeof(Control); }
+extern "C" int rl_decode_chain_launch_word() { return (int)offsetof(Control, launch); }
+// (the waits' comparison, of launch number `launch`)
+extern "C" int rl_decode_chain_done(unsigned long long flag, unsigned launch, unsigned phases) { return done_with(flag, launch + 1, phases); }
 
 // Bytes for steps of these sizes: of rows, and of the attention's shares.
 extern "C" long long rl_decode_chain_space(int num_layers, int rows, int hidden, int nq, int nkv, int inter) {

@@ -1,5 +1,7 @@
 """The rules of the launch that runs all layers of a step of few tokens."""
 
+import ctypes
+
 import pytest
 
 from rapid_llm_amd.kernels import decode_chain as chain
@@ -25,3 +27,24 @@ def test_shares(units):
                 n = chain.shares(rows, nkv, span, units)
                 assert 1 <= n <= chain.MAX_SHARES and (n - 1) * chain.MIN_KEYS < span
                 assert n == 1 or n * rows * nkv <= units
+
+
+@pytest.mark.parametrize("layers", [2, 28, 64])
+def test_a_flag_speaks_of_its_own_launch_only(layers):
+    """Launches of one or two rows write no flags, any number of them: what the flags of the last launch that did say must
+    not be taken for this one's, also where a count of phases over all launches would have wrapped."""
+    phases = 5 * layers
+
+    def done(flag, launch, ph):
+        return chain._library().rl_decode_chain_done(ctypes.c_ulonglong(flag), ctypes.c_uint(launch), ctypes.c_uint(ph))
+
+    wraps = [2**31 // phases, 2**32 // phases, 2**31, 2**32 - 1]
+    launches = sorted({max(0, w + d) for w in wraps for d in (-2, -1, 0, 1) if w + d < 2**32 - 1} | {0, 1, 2})
+    for launch in launches:
+        for ph in (1, phases - 1):
+            assert not done(0, launch, ph)  # never written
+            for earlier in launches:
+                if earlier < launch:
+                    assert not done((earlier + 1) << 32 | phases, launch, ph), (earlier, launch)
+            for at in range(phases + 1):
+                assert done((launch + 1) << 32 | at, launch, ph) == (at >= ph)

@@ -108,6 +108,30 @@ def test_any_number_of_workgroups_gives_the_same(rows, monkeypatch):
         assert torch.equal(r, results[0])
 
 
+def _count_from(runner, launch):
+    """The number of the next launch, as if so many had gone before."""
+    from rapid_llm_amd.kernels import decode_chain
+
+    word = decode_chain._library().rl_decode_chain_launch_word() // 4
+    torch.cuda.synchronize()
+    runner.model._chain_space.control.view(torch.int32)[word] = launch - (1 << 32 if launch >= 1 << 31 else 0)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows", [1, 2, 4, 16])
+def test_results_do_not_depend_on_how_many_launches_went_before(rows):
+    layers = 4
+    cfg = {**BASE, "hidden_size": 1024, "num_attention_heads": 8, "intermediate_size": 1536, "num_hidden_layers": layers}
+    runner = _runner(cfg)
+    tokens, entries = _fill(runner, CONTEXTS[:rows], cfg["vocab_size"])
+    want = _again(runner, tokens, entries)
+    # (a count of the phases of all launches would be beyond 2^31, beyond 2^32; the launch's number beyond 2^31)
+    for launch in (2**31 // (5 * layers) + 1, 2**32 // (5 * layers) + 1, 2**31 + 5):
+        _count_from(runner, launch)
+        for _ in range(3):
+            assert torch.equal(_again(runner, tokens, entries), want), launch
+
+
 def test_replays_between_other_steps():
     from rapid_llm_amd import StepEntry
 
