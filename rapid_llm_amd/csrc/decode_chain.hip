@@ -72,6 +72,9 @@ struct ChainLayer {
 
 // what the workgroups of a launch know of each other; zeros before the first launch
 #define LIST_CLOSED 0x80000000u
+// The number of the last launch before they begin again at 0: tags, a launch's number + 1, are never 0, which lies where nobody
+// has stored yet.  When it ends, everything that holds tags is cleared, so that none is met a second time.
+#define LAST_LAUNCH 0xfffffffeu
 struct Control {
     u32 list;      // workgroups that have entered their names
     u32 pad0[31];
@@ -103,6 +106,8 @@ struct ChainArgs {
     unsigned char* space;   // a layer's rows and sums, layer_bytes each
     u64* shares;            // the attention's shares: numbers with the launch's
     Control* control;
+    u64* tagged;            // the space of steps of few rows, and how many words of it and of the shares hold tags
+    u64 tagged_words, share_words;
     int num_layers, M, H, nq, nkv, I, table_stride, page_size, nsplit;
     float scale_log2, qk_eps, norm_eps, ff_eps;
     // in a layer's space (the packed rows are at 0); at_res: the stream behind the output product (tagged)
@@ -1325,15 +1330,30 @@ __global__ __launch_bounds__(CH_THREADS) void decode_chain_kernel(ChainArgs) {
         for (size_t i = threadIdx.x; i < (size_t)a->M * a->H; i += CH_THREADS) a->out[i].bits = 0x7fc0;
         if (threadIdx.x == 0) agent_store(&control->abort, 1u);
     }
+    const u32 launch = lds_get(&ctl->launch);
+    if (launch == LAST_LAUNCH) {  // what any wave has stored is there before somebody clears it
+        stores_done();
+        __syncthreads();
+    }
+    u32 last = 0;
     if (threadIdx.x == 0) {
         stores_done();
         const u32 before = __hip_atomic_fetch_add(&control->left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (before + 1 == gridDim.x) {  // the last one: as the next launch wants to find it
+        last = before + 1 == gridDim.x;
+        if (last) {  // as the next launch wants to find it
             agent_store(&control->list, 0u);
             agent_store(&control->left, 0u);
-            agent_store(&control->launch, agent_load(&control->launch) + 1);
+            agent_store(&control->launch, launch == LAST_LAUNCH ? 0u : launch + 1);
         }
     }
+    if (launch != LAST_LAUNCH) return;
+    if (threadIdx.x == 0) ctl->rank = last;
+    __syncthreads();
+    if (!lds_get(&ctl->rank)) return;
+    for (u64 i = threadIdx.x; i < a->tagged_words; i += CH_THREADS) agent_store(a->tagged + i, (u64)0);
+    for (u64 i = threadIdx.x; i < a->share_words; i += CH_THREADS) agent_store(a->shares + i, (u64)0);
+    for (u32 i = threadIdx.x; i < CH_MAX_WORKGROUPS * FLAG_STRIDE; i += CH_THREADS) agent_store(control->flags + i, (u64)0);
+    if (threadIdx.x == 0) agent_store(&control->dealt, (u64)0);
 }
 
 // a layer's space; tagged results have a part of the space of their own, so that what lies in a number's place is always
@@ -1366,6 +1386,7 @@ extern "C" int rl_decode_chain_max_group() { return CH_MAX_GROUP; }
 extern "C" int rl_decode_chain_min_keys() { return CH_KEYS; }
 extern "C" int rl_decode_chain_control() { return (int)sizeof(Control); }
 extern "C" int rl_decode_chain_launch_word() { return (int)offsetof(Control, launch); }
+extern "C" unsigned rl_decode_chain_last_launch() { return LAST_LAUNCH; }
 // (the waits' comparison, of launch number `launch`)
 extern "C" int rl_decode_chain_done(unsigned long long flag, unsigned launch, unsigned phases) { return done_with(flag, launch + 1, phases); }
 
@@ -1379,14 +1400,17 @@ extern "C" long long rl_decode_chain_shares(int num_layers, int rows, int nq, in
 }
 
 // `tagged_space`, `space`, `shares`: as large as the two functions above say for up to CH_TAGGED_ROWS rows, for more, and for all.
-// `control` and the two that hold tags are zeros before the first launch; launches that share them follow each other.
+// `control` and the two that hold tags, of `tagged_bytes` and `shares_bytes`, are zeros before the first launch; launches that share
+// them follow each other.
 extern "C" int rl_decode_chain(const void* layers, const void* x, float* residual, void* out, const int* positions,
                                const int* token_slot, const int* block_table, const float* cos_tab, const float* sin_tab,
-                               void* tagged_space, void* space, void* shares, void* control, int num_layers, int rows, int hidden,
+                               void* tagged_space, long long tagged_bytes, void* space, void* shares, long long shares_bytes,
+                               void* control, int num_layers, int rows, int hidden,
                                int nq, int nkv, int inter, int table_stride, int page_size, int nsplit, float scale, float qk_eps,
                                float norm_eps, float ff_eps, int units, hipStream_t stream) {
     if (num_layers < 1 || rows < 1 || rows > CH_MAX_ROWS || nkv < 1 || nq % nkv || nq / nkv > CH_MAX_GROUP) return RL_ERR_ARG;
     if (hidden % KSTEP || inter % KSTEP || hidden < KSTEP || inter < KSTEP || page_size < 8 || page_size % 8) return RL_ERR_ARG;
+    if (tagged_bytes < 0 || shares_bytes < 0) return RL_ERR_ARG;
     if (nsplit < 1 || units < 1 || units > CH_MAX_WORKGROUPS || (cos_tab != nullptr) != (sin_tab != nullptr)) return RL_ERR_ARG;
     ChainArgs a;
     const long long layer_bytes = lay_out(a, rows, hidden, nq, nkv, inter);
@@ -1399,6 +1423,7 @@ extern "C" int rl_decode_chain(const void* layers, const void* x, float* residua
     a.space = (unsigned char*)(rows <= CH_TAGGED_ROWS ? tagged_space : space);
     a.shares = (u64*)shares;
     a.control = (Control*)control;
+    a.tagged = (u64*)tagged_space, a.tagged_words = tagged_bytes / 8, a.share_words = shares_bytes / 8;
     a.num_layers = num_layers, a.M = rows, a.H = hidden, a.nq = nq, a.nkv = nkv, a.I = inter;
     a.table_stride = table_stride, a.page_size = page_size, a.nsplit = nsplit;
     a.scale_log2 = scale * 1.4426950408889634f, a.qk_eps = qk_eps, a.norm_eps = norm_eps, a.ff_eps = ff_eps;

@@ -41,6 +41,7 @@ def _library() -> ctypes.CDLL:
         if limits != (MAX_GROUP, MIN_KEYS):
             raise KernelError(f"the decode chain's limits {limits} are not the launch rules'")
         lib.rl_decode_chain_space.restype = lib.rl_decode_chain_shares.restype = ctypes.c_longlong
+        lib.rl_decode_chain_last_launch.restype = ctypes.c_uint
         _lib = lib
     return _lib
 
@@ -151,7 +152,8 @@ class DecodeChain:
         _ok(
             _library().rl_decode_chain(
                 _p(self.table), _p(x), _p(residual), _p(out), _p(positions), _p(token_slot), _p(block_table), _p(cos), _p(sin),
-                _p(self.space.tagged), _p(self.space.rows), _p(self.space.shares), _p(self.space.control), self.num_layers, rows, hidden, self.nq, self.nkv, self.inter,
+                _p(self.space.tagged), ctypes.c_longlong(self.space.tagged.numel()), _p(self.space.rows),
+                _p(self.space.shares), ctypes.c_longlong(self.space.shares.numel()), _p(self.space.control), self.num_layers, rows, hidden, self.nq, self.nkv, self.inter,
                 block_table.stride(0), self.page_size, self.nsplit, ctypes.c_float(self.scale),
                 *(ctypes.c_float(e) for e in self.eps), chip().units, _stream(),
             ),

@@ -132,6 +132,39 @@ def test_results_do_not_depend_on_how_many_launches_went_before(rows):
             assert torch.equal(_again(runner, tokens, entries), want), launch
 
 
+@pytest.mark.parametrize("rows", [(1, 2), (2, 4), (16, 1)])
+def test_launch_numbers_begin_again(rows):
+    """Behind the last number everything that carries one is cleared: no place that was written under a number, or never,
+    is taken for written under the same number met again."""
+    from rapid_llm_amd.kernels import decode_chain
+
+    cfg = {**BASE, "hidden_size": 1024, "num_attention_heads": 8, "intermediate_size": 1536}
+    steps = []
+    runner = _runner(cfg)
+    for n in rows:
+        tokens, entries = _fill(runner, CONTEXTS[:n], cfg["vocab_size"])
+        steps.append((_again(runner, tokens, entries), n))
+        for rid in list(tokens):
+            runner.finish(rid)
+    space, last = runner.model._chain_space, decode_chain._library().rl_decode_chain_last_launch()
+    word = decode_chain._library().rl_decode_chain_launch_word() // 4
+    for before in (2, 0):  # launches in front of the last one
+        _count_from(runner, last - before)
+        for i in range(before + 3):
+            want, n = steps[i % 2]
+            tokens, entries = _fill(runner, CONTEXTS[:n], cfg["vocab_size"])
+            assert torch.equal(_again(runner, tokens, entries), want), (before, i)
+            for rid in list(tokens):
+                runner.finish(rid)
+            torch.cuda.synchronize()
+            number = int(space.control.view(torch.int32)[word]) & 0xFFFFFFFF
+            assert number == (last - before + i + 1 if i < before else i - before), (before, i)
+            if number == 0:
+                assert not space.tagged.any() and not space.shares.any()
+                control = space.control.view(torch.int32).clone()
+                assert not control.any()
+
+
 def test_replays_between_other_steps():
     from rapid_llm_amd import StepEntry
 
