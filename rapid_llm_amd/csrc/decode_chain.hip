@@ -11,8 +11,8 @@
 // Items are numbered in the order of their dependencies and dealt to the workgroups in turn.  That needs every workgroup that
 // has items to be running, whatever else the chip does: a workgroup enters its name when it starts; when all have, or
 // after some time, the list is closed, the items are dealt to those on it, and a workgroup that starts later leaves at once.
-// (Waits are bounded all the same: a workgroup that runs into the bound ends the launch, and the step's result
-// is NaN.)
+// (Waits are bounded all the same: a workgroup that runs into the bound ends the launch, the step's result is NaN, every
+// later launch ends at once, and a word in host memory says so.)
 //
 // A workgroup is eight waves that stream and multiply, and two that do what would stand in their way, because a
 // wave's loads return in order: one waits for other workgroups' results and prepares the attention's queries and the norms'
@@ -108,6 +108,7 @@ struct ChainArgs {
     Control* control;
     u64* tagged;            // the space of steps of few rows, and how many words of it and of the shares hold tags
     u64 tagged_words, share_words;
+    u32* notice;            // in host memory: set by a launch that is given up
     int num_layers, M, H, nq, nkv, I, table_stride, page_size, nsplit;
     float scale_log2, qk_eps, norm_eps, ff_eps;
     // in a layer's space (the packed rows are at 0); at_res: the stream behind the output product (tagged)
@@ -1328,7 +1329,10 @@ __global__ __launch_bounds__(CH_THREADS) void decode_chain_kernel(ChainArgs) {
     __syncthreads();
     if (lds_get(&ctl->ready[1])) {  // a wait ran into its bound
         for (size_t i = threadIdx.x; i < (size_t)a->M * a->H; i += CH_THREADS) a->out[i].bits = 0x7fc0;
-        if (threadIdx.x == 0) agent_store(&control->abort, 1u);
+        if (threadIdx.x == 0) {
+            agent_store(&control->abort, 1u);
+            __hip_atomic_store(a->notice, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
     const u32 launch = lds_get(&ctl->launch);
     if (launch == LAST_LAUNCH) {  // what any wave has stored is there before somebody clears it
@@ -1386,6 +1390,11 @@ extern "C" int rl_decode_chain_max_group() { return CH_MAX_GROUP; }
 extern "C" int rl_decode_chain_min_keys() { return CH_KEYS; }
 extern "C" int rl_decode_chain_control() { return (int)sizeof(Control); }
 extern "C" int rl_decode_chain_launch_word() { return (int)offsetof(Control, launch); }
+extern "C" int rl_decode_chain_abort_word() { return (int)offsetof(Control, abort); }
+// Where the device finds a word of pinned host memory.
+extern "C" int rl_decode_chain_notice(void* host, void** device) {
+    return hipHostGetDevicePointer(device, host, 0) == hipSuccess ? RL_OK : RL_ERR_ARG;
+}
 extern "C" unsigned rl_decode_chain_last_launch() { return LAST_LAUNCH; }
 // (the waits' comparison, of launch number `launch`)
 extern "C" int rl_decode_chain_done(unsigned long long flag, unsigned launch, unsigned phases) { return done_with(flag, launch + 1, phases); }
@@ -1401,16 +1410,16 @@ extern "C" long long rl_decode_chain_shares(int num_layers, int rows, int nq, in
 
 // `tagged_space`, `space`, `shares`: as large as the two functions above say for up to CH_TAGGED_ROWS rows, for more, and for all.
 // `control` and the two that hold tags, of `tagged_bytes` and `shares_bytes`, are zeros before the first launch; launches that share
-// them follow each other.
+// them follow each other.  `notice`: rl_decode_chain_notice's.
 extern "C" int rl_decode_chain(const void* layers, const void* x, float* residual, void* out, const int* positions,
                                const int* token_slot, const int* block_table, const float* cos_tab, const float* sin_tab,
                                void* tagged_space, long long tagged_bytes, void* space, void* shares, long long shares_bytes,
-                               void* control, int num_layers, int rows, int hidden,
+                               void* control, void* notice, int num_layers, int rows, int hidden,
                                int nq, int nkv, int inter, int table_stride, int page_size, int nsplit, float scale, float qk_eps,
                                float norm_eps, float ff_eps, int units, hipStream_t stream) {
     if (num_layers < 1 || rows < 1 || rows > CH_MAX_ROWS || nkv < 1 || nq % nkv || nq / nkv > CH_MAX_GROUP) return RL_ERR_ARG;
     if (hidden % KSTEP || inter % KSTEP || hidden < KSTEP || inter < KSTEP || page_size < 8 || page_size % 8) return RL_ERR_ARG;
-    if (tagged_bytes < 0 || shares_bytes < 0) return RL_ERR_ARG;
+    if (tagged_bytes < 0 || shares_bytes < 0 || !notice) return RL_ERR_ARG;
     if (nsplit < 1 || units < 1 || units > CH_MAX_WORKGROUPS || (cos_tab != nullptr) != (sin_tab != nullptr)) return RL_ERR_ARG;
     ChainArgs a;
     const long long layer_bytes = lay_out(a, rows, hidden, nq, nkv, inter);
@@ -1424,6 +1433,7 @@ extern "C" int rl_decode_chain(const void* layers, const void* x, float* residua
     a.shares = (u64*)shares;
     a.control = (Control*)control;
     a.tagged = (u64*)tagged_space, a.tagged_words = tagged_bytes / 8, a.share_words = shares_bytes / 8;
+    a.notice = (u32*)notice;
     a.num_layers = num_layers, a.M = rows, a.H = hidden, a.nq = nq, a.nkv = nkv, a.I = inter;
     a.table_stride = table_stride, a.page_size = page_size, a.nsplit = nsplit;
     a.scale_log2 = scale * 1.4426950408889634f, a.qk_eps = qk_eps, a.norm_eps = norm_eps, a.ff_eps = ff_eps;

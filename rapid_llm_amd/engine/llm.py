@@ -30,7 +30,8 @@ class PendingStep:
     """A step that has been queued on the device.  ``result()`` waits for it and returns its
     :class:`StepOutput`; until then the host is free to plan and queue the next step."""
 
-    def __init__(self, sampling: SamplingPlan, host: dict[str, torch.Tensor], asked: list[int]) -> None:
+    def __init__(self, runner, sampling: SamplingPlan, host: dict[str, torch.Tensor], asked: list[int]) -> None:
+        self._runner, self._lost = runner, runner.lost
         self._sampling = sampling
         self._host = host  # pinned copies of what the step chose and scored
         self._asked = asked
@@ -43,6 +44,7 @@ class PendingStep:
             return self._output
         # the step's one host synchronisation (rapid_llm/engine/scheduler.py:1000-1005)
         self._event.synchronize()
+        self._runner.check(self._lost)
         sampling, host = self._sampling, self._host
         out = StepOutput(host["ids"].tolist())
         if self._asked:
@@ -111,7 +113,7 @@ class GpuExecutor:
                 logits, sampling.prompt_targets, max(sampling.prompt_ks), row_index=sampling.prompt_rows
             )
             host.update(p_lp=self._to_host(lp), p_top_ids=self._to_host(top_ids), p_top_lp=self._to_host(top_lp))
-        return PendingStep(sampling, host, asked)
+        return PendingStep(runner, sampling, host, asked)
 
     def execute(self, entries, sampling: SamplingPlan) -> StepOutput:
         return self.launch(entries, sampling).result()

@@ -107,6 +107,11 @@ class StepOutput:
     prompt_logprobs: list[PositionLogprobs] | None = None  # parallel to prompt_rows
 
 
+class LostStep(RuntimeError):
+    """Raised by an executor's ``launch`` or by ``result()``: what the steps in flight chose cannot be had, and the cache
+    lacks what they would have written."""
+
+
 class _ReadFirst(Exception):
     """Planning met a shortage of pages while a step is in flight."""
 
@@ -430,7 +435,26 @@ class Scheduler:
     def step(self) -> list[Request]:
         """Plan one batch, run it, harvest chosen tokens.  Returns the requests that advanced
         or finished (rapid_llm/engine/scheduler.py:1405-1460).  Pipelined, the tokens harvested
-        are those of the step queued by the previous call (:818-933)."""
+        are those of the step queued by the previous call (:818-933).  Where that is lost (:class:`LostStep`) the
+        requests wait to be computed again from the tokens that are known, and the caller may go on."""
+        try:
+            return self._step()
+        except LostStep:
+            self._recompute()
+            raise
+
+    def _recompute(self) -> None:
+        """Nothing is in flight, and every running request is evicted."""
+        self._inflight = None
+        for request in self._held:
+            request.pending = request.discard = 0
+            self.executor.finish(request.request_id)
+        self._held = []
+        for request in sorted(self.running, key=lambda r: r.admission_number, reverse=True):
+            request.pending = 0
+            self._preempt(request, StepPlan())
+
+    def _step(self) -> list[Request]:
         if self.pipeline:
             try:
                 launched, advanced = self._launch()

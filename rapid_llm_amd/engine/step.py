@@ -33,6 +33,7 @@ from ..parts.runtime import Runtime
 from ..weights.loader import load_model_dir
 from ..weights.random_init import random_params
 from .feed import fed_token  # noqa: F401  (part of the step function's input convention)
+from .scheduler import LostStep
 
 _TORCH_DTYPE = {"bfloat16": torch.bfloat16, "float32": torch.float32}
 # batch sizes decode graphs are captured for; other sizes are padded up with filler rows
@@ -163,6 +164,7 @@ class ModelRunner:
         self.graph_library_products: dict[tuple[int, int], int] = {}
         # a part that does not promise to be replayable keeps every step eager
         self.graphs_allowed = self.model.replayable()
+        self.lost = 0  # times that steps were found lost (``check``)
         # workgroups a request gets in the launches that are laid out otherwise for contexts of unlike length
         self.ragged_workgroups = sorted({getattr(p, "deals_ragged_contexts", 0) for p in self.model.all_parts()} - {0})
         # where the sampling kernels leave their choices, one row per sampled request of a
@@ -278,6 +280,26 @@ class ModelRunner:
         if self.cache.has(request_id):
             self.cache.release(request_id)
         self.computed.pop(request_id, None)
+
+    def check(self, lost: int | None = None) -> None:
+        """Raise :class:`~rapid_llm_amd.engine.scheduler.LostStep` if a recorded step that has run to its end did not compute
+        its result: a launch that waits for its own workgroups gave up, the logits are NaN and the cache lacks the
+        step's keys and values.  For whoever reads a step's results, behind the wait for them, with ``runner.lost`` as
+        it was when the step was queued; the next step asks too.  Such launches are not made again: later steps are recorded anew, with
+        every layer's own kernels."""
+        if self.model.lost_launch():
+            torch.cuda.synchronize(self.device)  # (those queued behind it end at once)
+            for kinds in self._graphs.values():
+                for ragged in [r for r, entry in kinds.items() if entry[3].static.get("decode_chain") is not None]:
+                    del kinds[ragged]
+            self.model.give_up_chain()
+            self.lost += 1
+            lost = self.lost - 1
+        if lost is not None and lost != self.lost:
+            raise LostStep(
+                "a recorded step's launch of all layers gave up waiting for its own workgroups: the tokens of the steps "
+                "that were under way are not known, and their requests' keys and values are missing from the cache"
+            )
 
     # ------------------------------------------------------------------ the step
     def _prepare(self, entries: Sequence[StepEntry]) -> dict:
@@ -489,10 +511,11 @@ class ModelRunner:
         """Run one batch; returns float32 logits ``[wanted, vocab]`` in the order of the
         entries and of each entry's ``want``.  Raises :class:`OutOfPages`, with nothing
         changed, when slots or pages do not suffice.  The returned tensor may be reused by
-        the next step: read it (sample from it, copy it) before stepping again.
+        the next step: read it (sample from it, copy it) before stepping again, and :meth:`check` behind the wait for it.
         ``use_graph`` overrides the engine's setting for this one step."""
         if not entries:
             return torch.empty((0, self.vocab_size), dtype=torch.float32, device=self.device)
+        self.check()
         meta = self._prepare(entries)
         if (
             (self.engine.use_graph if use_graph is None else use_graph)

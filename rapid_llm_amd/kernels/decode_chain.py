@@ -70,6 +70,15 @@ class Space:
         sizes = space_bytes(layers, hidden, nq, nkv, inter, span)
         # (what lies in the place of a launch's number must be an earlier launch's)
         self.tagged, self.rows, self.shares, self.control = (torch.zeros(n, dtype=torch.uint8, device=device) for n in sizes)
+        # a launch that is given up leaves a word in host memory, which costs nothing to look at
+        self._notice = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._seen = self._notice.numpy()
+        self.notice = ctypes.c_void_p()
+        _ok(_library().rl_decode_chain_notice(_p(self._notice), ctypes.byref(self.notice)), "rl_decode_chain_notice")
+
+    def given_up(self) -> bool:
+        """Whether a launch that has ended was given up: its result, and that of every later one, is NaN."""
+        return bool(self._seen[0])
 
 
 def space_bytes(layers: int, hidden: int, nq: int, nkv: int, inter: int, span: int) -> tuple[int, int, int, int]:
@@ -153,7 +162,7 @@ class DecodeChain:
             _library().rl_decode_chain(
                 _p(self.table), _p(x), _p(residual), _p(out), _p(positions), _p(token_slot), _p(block_table), _p(cos), _p(sin),
                 _p(self.space.tagged), ctypes.c_longlong(self.space.tagged.numel()), _p(self.space.rows),
-                _p(self.space.shares), ctypes.c_longlong(self.space.shares.numel()), _p(self.space.control), self.num_layers, rows, hidden, self.nq, self.nkv, self.inter,
+                _p(self.space.shares), ctypes.c_longlong(self.space.shares.numel()), _p(self.space.control), self.space.notice, self.num_layers, rows, hidden, self.nq, self.nkv, self.inter,
                 block_table.stride(0), self.page_size, self.nsplit, ctypes.c_float(self.scale),
                 *(ctypes.c_float(e) for e in self.eps), chip().units, _stream(),
             ),

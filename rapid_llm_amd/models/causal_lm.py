@@ -80,6 +80,7 @@ class CausalLM:
                 if not 0 <= place < len(self.order):
                     raise ValueError(f"the embedding returns at place {place} of a run order of {len(self.order)}")
         self._chain_space: decode_chain.Space | None = None  # of the recorded steps that run all layers in one launch
+        self._chain_given_up = False  # (they keep their own kernels from there on)
         self._positions: dict[str, object] = {}
         self.blocks = []
         for i, layer in enumerate(spec.layers):
@@ -188,9 +189,17 @@ class CausalLM:
             ctx.static["decode_chain"] = self._new_chain(ctx, caches)
         return ctx.static["decode_chain"]
 
+    def lost_launch(self) -> bool:
+        """Whether a step's launch of all layers was given up, among those that have ended.  Asked behind the wait for a step."""
+        return self._chain_space is not None and self._chain_space.given_up()
+
+    def give_up_chain(self) -> None:
+        """No launch of all layers any more.  Asked for when none is under way and no recorded step holds one."""
+        self._chain_space, self._chain_given_up = None, True
+
     def chainable(self) -> bool:
         """Whether the layers are such that one launch may run them all (``decode_chain``), whatever a step's rows are."""
-        if self.offsets is not None or self.mixes is not None or self.returns or len(self.order) < 2:
+        if self._chain_given_up or self.offsets is not None or self.mixes is not None or self.returns or len(self.order) < 2:
             return False
         blocks = [self.blocks[li] for li in self.order]
         first = blocks[0].launch_signature()

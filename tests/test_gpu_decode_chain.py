@@ -165,6 +165,84 @@ def test_launch_numbers_begin_again(rows):
                 assert not control.any()
 
 
+def _give_up(model):
+    """What a launch leaves that ran into the bound of a wait: every later one ends at once."""
+    from rapid_llm_amd.kernels import decode_chain
+
+    torch.cuda.synchronize()
+    model._chain_space.control.view(torch.int32)[decode_chain._library().rl_decode_chain_abort_word() // 4] = 1
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows", [1, 4, 16])
+def test_a_launch_that_is_given_up_is_reported_and_not_made_again(rows):
+    from rapid_llm_amd.engine.scheduler import LostStep
+
+    cfg = {**BASE, "hidden_size": 512}
+    runner = _runner(cfg)
+    tokens, entries = _fill(runner, CONTEXTS[:rows], cfg["vocab_size"])
+    want = _again(runner, tokens, entries)
+    runner.check(runner.lost)
+    _give_up(runner.model)
+    before = runner.lost
+    assert _again(runner, tokens, entries).isnan().all()
+    torch.cuda.synchronize()
+    with pytest.raises(LostStep):  # whoever reads that step asks, ...
+        runner.check(before)
+    with pytest.raises(LostStep):  # ... also behind somebody else
+        runner.check(before)
+    runner.check(runner.lost)
+    got = _again(runner, tokens, entries)
+    assert _chains(runner) == [None]
+    parity.assert_bf16_close(got.cpu(), want.cpu(), f"kernels behind a lost launch/{rows}")
+    for _ in range(3):
+        assert torch.equal(_again(runner, tokens, entries), got)
+
+
+def test_the_next_step_reports_a_launch_that_was_given_up():
+    from rapid_llm_amd.engine.scheduler import LostStep
+
+    cfg = {**BASE, "hidden_size": 512}
+    runner = _runner(cfg)
+    tokens, entries = _fill(runner, CONTEXTS[:2], cfg["vocab_size"])
+    want = _again(runner, tokens, entries)
+    _give_up(runner.model)
+    _again(runner, tokens, entries)
+    torch.cuda.synchronize()
+    pages = runner.cache.num_free_pages()
+    with pytest.raises(LostStep):
+        runner.step(entries)
+    assert runner.cache.num_free_pages() == pages and runner.computed[entries[0].request_id] == len(tokens["r0"]) - 1
+    parity.assert_bf16_close(_again(runner, tokens, entries).cpu(), want.cpu(), "kernels behind a lost launch/next step")
+
+
+@pytest.mark.parametrize("pipeline", [False, True])
+def test_generation_goes_on_behind_a_launch_that_was_given_up(pipeline):
+    from rapid_llm_amd import LLM, SamplingParams
+    from rapid_llm_amd.engine.scheduler import LostStep
+
+    cfg = {**BASE, "hidden_size": 512}
+    llm = LLM(cfg, dtype="bfloat16", max_seq_len=256, max_num_seqs=8, num_pages=200, load_format="random", pipeline=pipeline)
+    prompts = [random_tokens(n, cfg["vocab_size"], 3 + n) for n in (5, 17, 40)]
+    params = SamplingParams(temperature=0.0, max_gen_len=24, ignore_eos=True)
+    want = [o.outputs[0].token_ids for o in llm.generate(prompts, params)]
+    requests = llm._submit(prompts, params)
+    scheduler = llm.scheduler
+    for _ in range(9):
+        scheduler.step()
+    known = [list(r.output_token_ids) for r in requests]
+    _give_up(scheduler.runner.model)
+    with pytest.raises(LostStep):
+        while scheduler.has_unfinished_requests():
+            scheduler.step()
+    # what had been read by then is right, and everything else is computed again
+    for r, k, w in zip(requests, known, want):
+        assert r.output_token_ids[: len(k)] == k == w[: len(k)] and r.output_token_ids == w[: len(r.output_token_ids)]
+    scheduler.run_to_completion()
+    assert all(len(r.output_token_ids) == 24 and r.finish_reason == "length" for r in requests)
+    assert all(c is None for c in _chains(scheduler.runner)) and scheduler.runner.lost == 1
+
+
 def test_replays_between_other_steps():
     from rapid_llm_amd import StepEntry
 

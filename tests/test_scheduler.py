@@ -11,7 +11,7 @@ from rapid_llm_amd.cache import CacheManager, GroupSpec
 from rapid_llm_amd.config import EngineConfig
 from rapid_llm_amd.engine.feed import fed_row, fed_token
 from rapid_llm_amd.engine.request import RequestStatus
-from rapid_llm_amd.engine.scheduler import Scheduler, StepOutput, detect_repetition
+from rapid_llm_amd.engine.scheduler import LostStep, Scheduler, StepOutput, detect_repetition
 from rapid_llm_amd.sampling import PositionLogprobs, SamplingParams
 
 EOS = 99
@@ -496,6 +496,64 @@ def test_pipeline_changes_no_token(seed, pool):
             for r in requests
         ])
         assert all(r.pending == 0 and r.discard == 0 for r in requests)
+    assert outcomes[0] == outcomes[1]
+
+
+class LosingExecutor(PipelinedExecutor):
+    """Some steps are lost: seen when they are read (those queued behind them are lost with them), or when the next is queued."""
+
+    def __init__(self, *args, read=(), queued=(), **kw):
+        super().__init__(*args, **kw)
+        self.read, self.queued, self.launches, self.lost = set(read), set(queued), 0, 0
+
+    def launch(self, entries, sampling):
+        self.launches += 1
+        if self.launches in self.queued:
+            self.lost += 1
+            raise LostStep("seen when the next step was queued")
+        number, lost, handle, executor = self.launches, self.lost, super().launch(entries, sampling), self
+
+        class Handle:
+            def result(self_inner):
+                out = handle.result()
+                if number in executor.read and lost == executor.lost:
+                    executor.lost += 1
+                if lost != executor.lost:
+                    raise LostStep("seen when it was read")
+                return out
+
+        return Handle()
+
+
+@pytest.mark.parametrize("pipeline", [False, True])
+@pytest.mark.parametrize("seed", range(3))
+def test_lost_steps_are_reported_and_computed_again(seed, pipeline):
+    outcomes = []
+    for read, queued in (((), ()), ((1, 7, 8, 30), (15, 16, 22))):
+        ex = LosingExecutor(60, 4, 3, 64, token=_token_with_stops, read=read, queued=queued)
+        config = EngineConfig(max_seq_len=64, page_size=4, num_pages=60, max_num_seqs=3, pipeline=pipeline,
+                              max_num_batched_tokens=24, max_chunk_size=8)
+        s = Scheduler(ex, config, stop_token_ids=[EOS])
+        requests = _workload(s, seed)
+        raised = steps = 0
+        while s.has_unfinished_requests():
+            try:
+                s.step()
+            except LostStep:
+                raised += 1
+                # nothing is held for anybody, and everybody who was not done waits
+                assert not s.running and not s._held and s._inflight is None and not ex.cache.live_requests()
+            steps += 1
+            assert steps < 2000
+        assert raised == ex.lost and bool(raised) == bool(read)
+        assert not ex.cache.live_requests() and all(r.pending == 0 and r.discard == 0 for r in requests)
+        ex.cache.check_invariants()
+        outcomes.append([
+            (r.output_token_ids, r.finish_reason,
+             None if r.output_logprobs is None else [x.token_id for x in r.output_logprobs],
+             None if r.prompt_logprobs is None else [x and x.token_id for x in r.prompt_logprobs])
+            for r in requests
+        ])
     assert outcomes[0] == outcomes[1]
 
 
