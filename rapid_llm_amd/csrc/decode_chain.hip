@@ -1385,6 +1385,12 @@ static long long lay_out(ChainArgs& a, int rows, int hidden, int nq, int nkv, in
     return at;
 }
 
+static long long items_of_layer(ChainArgs& a, int rows, int hidden, int nq, int nkv, int inter, int nsplit) {
+    const long long shares = (long long)rows * nkv * nsplit;
+    a.n[PH_QKV] = (nq + 2 * nkv) * (D / 16), a.n[PH_ATT] = (int)shares, a.n[PH_O] = a.n[PH_DOWN] = hidden / 16, a.n[PH_GU] = inter / 16;
+    return (nq + 2ll * nkv) * (D / 16) + shares + 2 * (hidden / 16) + inter / 16;
+}
+
 extern "C" int rl_decode_chain_layer_bytes() { return (int)sizeof(ChainLayer); }
 extern "C" int rl_decode_chain_max_group() { return CH_MAX_GROUP; }
 extern "C" int rl_decode_chain_min_keys() { return CH_KEYS; }
@@ -1408,6 +1414,19 @@ extern "C" long long rl_decode_chain_shares(int num_layers, int rows, int nq, in
     return nsplit < 2 ? 0 : 8ll * num_layers * rows * nsplit * nq * (D + 2);
 }
 
+// Whether the launch takes layers, steps and a cache of these sizes.  (The last line: every index is divided by a
+// multiplication, which is exact below 2^32 / divisor.)
+extern "C" int rl_decode_chain_takes(int num_layers, int rows, int hidden, int nq, int nkv, int inter, int table_stride,
+                                     int page_size, int nsplit, int units) {
+    if (num_layers < 1 || rows < 1 || rows > CH_MAX_ROWS || nkv < 1 || nq % nkv || nq / nkv > CH_MAX_GROUP) return 0;
+    if (hidden % KSTEP || inter % KSTEP || hidden < KSTEP || inter < KSTEP || page_size < 8 || page_size % 8) return 0;
+    if (nsplit < 1 || units < 1 || units > CH_MAX_WORKGROUPS || table_stride < 1) return 0;
+    ChainArgs a;
+    const long long per_layer = items_of_layer(a, rows, hidden, nq, nkv, inter, nsplit);
+    if (lay_out(a, rows, hidden, nq, nkv, inter) > 0x7fffffffll || per_layer * num_layers + units > 0x7fffffffll) return 0;
+    return (u64)(per_layer * num_layers + units) * per_layer < 0x100000000ull && (u64)table_stride * page_size * page_size < 0x100000000ull;
+}
+
 // `tagged_space`, `space`, `shares`: as large as the two functions above say for up to CH_TAGGED_ROWS rows, for more, and for all.
 // `control` and the two that hold tags, of `tagged_bytes` and `shares_bytes`, are zeros before the first launch; launches that share
 // them follow each other.  `notice`: rl_decode_chain_notice's.
@@ -1417,14 +1436,11 @@ extern "C" int rl_decode_chain(const void* layers, const void* x, float* residua
                                void* control, void* notice, int num_layers, int rows, int hidden,
                                int nq, int nkv, int inter, int table_stride, int page_size, int nsplit, float scale, float qk_eps,
                                float norm_eps, float ff_eps, int units, hipStream_t stream) {
-    if (num_layers < 1 || rows < 1 || rows > CH_MAX_ROWS || nkv < 1 || nq % nkv || nq / nkv > CH_MAX_GROUP) return RL_ERR_ARG;
-    if (hidden % KSTEP || inter % KSTEP || hidden < KSTEP || inter < KSTEP || page_size < 8 || page_size % 8) return RL_ERR_ARG;
-    if (tagged_bytes < 0 || shares_bytes < 0 || !notice) return RL_ERR_ARG;
-    if (nsplit < 1 || units < 1 || units > CH_MAX_WORKGROUPS || (cos_tab != nullptr) != (sin_tab != nullptr)) return RL_ERR_ARG;
+    if (!rl_decode_chain_takes(num_layers, rows, hidden, nq, nkv, inter, table_stride, page_size, nsplit, units)) return RL_ERR_ARG;
+    if (tagged_bytes < 0 || shares_bytes < 0 || !notice || (cos_tab != nullptr) != (sin_tab != nullptr)) return RL_ERR_ARG;
     ChainArgs a;
-    const long long layer_bytes = lay_out(a, rows, hidden, nq, nkv, inter);
-    const long long per_layer = (nq + 2ll * nkv) * (D / 16) + (long long)rows * nkv * nsplit + 2 * (hidden / 16) + inter / 16;
-    if (layer_bytes > 0x7fffffffll || per_layer * num_layers + units > 0x7fffffffll) return RL_ERR_ARG;
+    lay_out(a, rows, hidden, nq, nkv, inter);
+    const long long per_layer = items_of_layer(a, rows, hidden, nq, nkv, inter, nsplit);
     a.layers = (const RL_CONSTANT ChainLayer*)layers;
     a.x = (const bf16_t*)x, a.residual = residual, a.out = (bf16_t*)out;
     a.positions = positions, a.token_slot = token_slot, a.block_table = block_table;
@@ -1437,10 +1453,8 @@ extern "C" int rl_decode_chain(const void* layers, const void* x, float* residua
     a.num_layers = num_layers, a.M = rows, a.H = hidden, a.nq = nq, a.nkv = nkv, a.I = inter;
     a.table_stride = table_stride, a.page_size = page_size, a.nsplit = nsplit;
     a.scale_log2 = scale * 1.4426950408889634f, a.qk_eps = qk_eps, a.norm_eps = norm_eps, a.ff_eps = ff_eps;
-    a.n[PH_QKV] = (nq + 2 * nkv) * (D / 16), a.n[PH_ATT] = rows * nkv * nsplit, a.n[PH_O] = a.n[PH_DOWN] = hidden / 16, a.n[PH_GU] = inter / 16;
     a.per_layer.set((u32)per_layer), a.by_heads.set(nkv), a.by_rows.set(rows), a.by_page.set(page_size);
     a.total = (u32)(per_layer * num_layers);
-    if ((a.total + (u64)units) * per_layer >= 0x100000000ull || (u64)table_stride * page_size * page_size >= 0x100000000ull) return RL_ERR_ARG;
 #define RL_CHAIN(XG, TAGGED) hipLaunchKernelGGL((decode_chain_kernel<XG, TAGGED>), dim3(units), dim3(CH_THREADS), 0, stream, a)
     if (rows == 1)
         RL_CHAIN(0, true);

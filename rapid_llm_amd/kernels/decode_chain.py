@@ -62,6 +62,11 @@ def shares(rows: int, nkv: int, span: int, units: int | None = None) -> int:
     return max(1, min(-(-span // MIN_KEYS), units // (rows * nkv), MAX_SHARES))
 
 
+def takes(layers: int, rows: int, hidden: int, nq: int, nkv: int, inter: int, columns: int, page_size: int, span: int) -> bool:
+    """Whether the launch's index arithmetic reaches so many layers and so large a cache (``columns`` of the block table)."""
+    return bool(_library().rl_decode_chain_takes(layers, rows, hidden, nq, nkv, inter, columns, page_size, shares(rows, nkv, span), chip().units))
+
+
 class Space:
     """What the launches of a model's recorded steps share: rows between the products, shares of the attention, and
     what the workgroups of a launch know of each other.  One launch uses it at a time (a runner's steps follow each other)."""

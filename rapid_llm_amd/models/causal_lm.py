@@ -238,6 +238,9 @@ class CausalLM:
         sizes = (mixer.hidden_size, mixer.nq, mixer.nkv)
         if not decode_chain.fits(ctx.num_tokens, *sizes, mixer.d, ff.intermediate_size, caches[0].page_size):
             return None
+        columns = ctx.block_tables[caches[0].group_id].stride(0)
+        if not decode_chain.takes(len(blocks), ctx.num_tokens, *sizes, ff.intermediate_size, columns, caches[0].page_size, ctx.static["context_bound"]):
+            return None
         layers = [
             (b.mixer.qkv.weight, b.mixer.o.weight, b.feed_forward.gate_up.weight, b.feed_forward.down.weight, b.mixer.q_norm_w,
              b.mixer.k_norm_w, b.feed_forward_norm.weight, behind.mixer_norm.weight if behind is not None else None, c.k, c.v)

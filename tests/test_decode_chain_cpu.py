@@ -48,3 +48,12 @@ def test_a_flag_speaks_of_its_own_launch_only(layers):
                     assert not done((earlier + 1) << 32 | phases, launch, ph), (earlier, launch)
             for at in range(phases + 1):
                 assert done((launch + 1) << 32 | at, launch, ph) == (at >= ph)
+
+
+def test_indices_that_the_launch_does_not_reach():
+    """Divisions by a multiplication are exact below 2^32 / divisor: steps beyond keep their own kernels."""
+    sizes = (1024, 16, 8, 3072)
+    assert chain.takes(28, 1, *sizes, 256, 16, 4096)
+    assert chain.takes(28, 1, *sizes, 8, 16384, 4096) and not chain.takes(28, 1, *sizes, 3, 65536, 4096)  # keys times tokens a page
+    wide = (128, 1, 1, 131072)  # 8 k items a layer
+    assert chain.takes(8, 1, *wide, 256, 16, 4096) and not chain.takes(80, 1, *wide, 256, 16, 4096)

@@ -298,6 +298,15 @@ def test_two_at_once():
     assert not wrong
 
 
+def test_pages_beyond_the_launchs_indices_keep_their_kernels():
+    cfg = {**BASE, "max_position_embeddings": 131072}
+    runner = _runner(cfg, max_seq_len=131072, page_size=65536, num_pages=6, max_num_seqs=2)
+    tokens, entries = _fill(runner, [300, 20], cfg["vocab_size"])
+    got = _again(runner, tokens, entries)
+    assert _chains(runner) == [None]
+    parity.assert_bf16_close(got.cpu(), runner.step(entries, use_graph=False).cpu(), "pages of 65,536 tokens")
+
+
 def test_layers_that_do_something_else_keep_their_kernels(monkeypatch):
     cfg = {**BASE, "hidden_size": 512}
     for change in (dict(head_dim=64), dict(num_attention_heads=10), dict(intermediate_size=392)):
