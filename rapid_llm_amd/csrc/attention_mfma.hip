@@ -218,7 +218,7 @@ struct AskedQuery {
     bf16x8 raw[DC];
     float cs[DC / 2 + 1][8], sn[DC / 2 + 1][8];  // chunk c pairs with chunk c + DC / 2, same lane and slot
 };
-__device__ inline void ask_norm(float (&w)[DC][8], int g, const DecodeExtra& ex) {
+__device__ __forceinline__ void ask_norm(float (&w)[DC][8], int g, const DecodeExtra& ex) {
     if (ex.q_norm_w) {
 #pragma unroll
         for (int c = 0; c < DC; ++c)
@@ -227,7 +227,7 @@ __device__ inline void ask_norm(float (&w)[DC][8], int g, const DecodeExtra& ex)
     }
 }
 // (`qrow` can be read also where the row is not wanted)
-__device__ inline void ask_query(AskedQuery& a, const bf16_t* qrow, int pos, int g, const DecodeExtra& ex) {
+__device__ __forceinline__ void ask_query(AskedQuery& a, const bf16_t* qrow, int pos, int g, const DecodeExtra& ex) {
 #pragma unroll
     for (int c = 0; c < DC; ++c) a.raw[c] = load16(qrow + 32 * c + 8 * g);
     if (ex.cos_tab) {
@@ -241,7 +241,7 @@ __device__ inline void ask_query(AskedQuery& a, const bf16_t* qrow, int pos, int
             }
     }
 }
-__device__ inline void prepared_query(bf16x8 (&qf)[DC], const AskedQuery& a, const float (&w)[DC][8], bool row_ok,
+__device__ __forceinline__ void prepared_query(bf16x8 (&qf)[DC], const AskedQuery& a, const float (&w)[DC][8], bool row_ok,
                                       const DecodeExtra& ex) {
     float x[DC][8];
     float ss = 0.f;
@@ -277,6 +277,23 @@ __device__ inline void prepared_query(bf16x8 (&qf)[DC], const AskedQuery& a, con
     for (int c = 0; c < DC; ++c)
 #pragma unroll
         for (int j = 0; j < 8; ++j) qf[c][j] = (__bf16)x[c][j];
+}
+
+// The same in functions of their own, for kernels that have no registers left beside their accumulators: what is
+// written through a pointer stays in scratch memory, from where every step reads it again.
+__device__ __noinline__ void late_query(bf16x8 (&qf)[DC], const bf16_t* qrow, bool row_ok, int pos, int g, const DecodeExtra& ex) {
+    AskedQuery asked;
+    float w[DC][8];
+    ask_query(asked, qrow, pos, g, ex);
+    ask_norm(w, g, ex);
+    prepared_query(qf, asked, w, row_ok, ex);
+}
+__device__ __noinline__ void late_plain(bf16x8 (&qf)[DC], const bf16_t* qrow, bool row_ok, int g) {
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+        const bool chan_ok = !(D_TAIL && c == DC - 1 && g >= 2);
+        qf[c] = (row_ok && chan_ok) ? load16(qrow + 32 * c + 8 * g) : zero8();
+    }
 }
 
 // k_cache and v_cache carry no promise of being the only way to their memory: in the fused
@@ -779,10 +796,16 @@ attn_prefill_kernel(
     // prep_q: `q` holds the raw packed [q | k | v] rows, and the workgroup norms and rotates its
     // rows' heads itself, as the decode kernel does (the host asks for it only where
     // D % 64 == 0); else `q` holds finished queries.  Their loads go out before anything else and are
-    // waited for once the first tile has been asked for.
+    // waited for once the first tile has been asked for, up to heads of 192 channels.  Heads of 256 are read as they are
+    // finished: all asked for at once, they lay in scratch (1,488 bytes a lane; prompts of 37 / 200 / 2,048 tokens, 16 query
+    // heads, 49.5 / 101 / 417 us, now 15.7 / 58.0 / 350).  Two groups of waves have half the registers each, and at 224 and
+    // 256 channels are faster with the queries in scratch than with other things there (2,048 tokens 274 / 230 us and 379 / 350;
+    // at 208 and 240 with them in registers, 265 / 191 and 360 / 320; one group 15.9 / 9.7 and 21.7 / 15.7 at 37 tokens).
+    // Heads that are never finished here do without the code from 176 channels on (176: 133 / 113; 160: 87 / 91).
+    constexpr bool PREPARES = D % 64 == 0 || D <= 160, EARLY = D <= 192, CALLED = GROUPS == 2 && (D == 224 || D == 256);
     AskedQuery asked[PF_NQ];
     float norm_w[DC][8];
-    if (prep_q) {
+    if (PREPARES && EARLY && prep_q) {
 #pragma unroll
         for (int n = 0; n < PF_NQ; ++n)
             ask_query(asked[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_pos[n], g, ex);
@@ -792,8 +815,17 @@ attn_prefill_kernel(
     auto load_queries = [&]() {
 #pragma unroll
         for (int n = 0; n < PF_NQ; ++n) {
-            if (prep_q) {
-                prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex);
+            if (PREPARES && prep_q) {
+                if (EARLY)
+                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex);
+                else if (!CALLED) {
+                    ask_query(asked[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_pos[n], g, ex);
+                    ask_norm(norm_w, g, ex);
+                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex);
+                } else
+                    late_query(qf[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_ok[n], r_pos[n], g, ex);
+            } else if (CALLED && D == 224) {
+                late_plain(qf[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_ok[n], g);
             } else {
                 const bf16_t* qrow = q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D;
 #pragma unroll

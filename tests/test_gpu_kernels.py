@@ -105,6 +105,9 @@ ATTN_CASES = [
     # kv head): a single token over 9,000 keys, a portion of 512 behind 7,000, a two-token portion
     (64, 8, 128, 16, 0, [(9000, 1), (7000, 512), (5, 2)]),
     (40, 8, 128, 16, 0, [(9001, 1), (6990, 512), (0, 2)]),
+    # finished queries read by a function of its own (two groups of waves), and by the kernel itself
+    (6, 2, 224, 16, 0, [(0, 200), (300, 37), (9, 1)]),
+    (6, 2, 224, 16, 0, [(0, 37)]),
 ]
 
 
@@ -1530,6 +1533,10 @@ PREPARED_CASES = [
     (6, 3, 64, 8, 0, [(100, 40), (5, 1), (0, 2)]),
     (4, 4, 192, 32, 57, [(400, 3), (20, 90)]),             # window
     (32, 8, 128, 16, 0, [(1000, 600)]),                    # few, long tiles: the keys cut into runs
+    # heads whose queries are finished where they are read, with two groups of waves and with one
+    (4, 4, 256, 16, 0, [(0, 200), (300, 1), (40, 37)]),
+    (4, 4, 256, 16, 30, [(0, 37)]),
+    (12, 4, 256, 8, 0, [(0, 9)]),
 ]
 
 
