@@ -21,14 +21,26 @@ TAGGED_ROWS = 2  # rows up to which results travel with the launch's number
 MIN_KEYS = 256  # keys that a share of a request's context has at least
 MAX_SHARES = 16  # of a request's keys: whoever folds them asks for all
 STEP = 128  # every contraction is a multiple of it
-# Elements of a layer's matrices up to which the launch is the faster one.  What it saves are the starts and tails of six kernels
-# a layer; what it costs is that a phase's last workgroups leave the memory idle where weights keep it busy.  Microseconds a
-# step of the layers' own kernels / in one launch: Qwen3-0.6B (15.7 M) one request of 20 / 300 / 1,500 / 4,000 keys 975 / 710, 988 /
-# 808, 1,041 / 824, 1,124 / 903, 2 / 4 / 8 / 16 of 64 to 900 1,032 / 858, 1,053 / 958, 1,126 / 984, 1,316 / 1,147, 16 of
-# up to 4,000 1,868 / 1,845; 1.7B (50.3 M) 1 / 2 / 4 / 8 / 16 requests 1,350 / 1,257, 1,375 / 1,361, 1,407 / 1,405, 1,518 / 1,485, 1,797 / 1,662;
-# 4B (101 M) 1 / 8 2,242 / 2,336, 2,572 / 2,763; 8B (193 M) 1 / 8 3,404 / 3,528, 3,762 / 3,982.
-MAX_LAYER_WEIGHTS = 64 << 20
-FEW_LAYER_WEIGHTS = 32 << 20  # of 2 to 7 rows: 1.7B with two of 42 to 546 keys 1,356 / 1,394
+# Rows of a recorded step up to which: keys of its longest context up to which, and a layer's matrix elements (in units of 2^20) up to
+# which, the launch is the faster one.  What it saves are the starts and tails of six kernels a layer; what it costs is that a phase's
+# last workgroups leave the memory idle where weights, or the keys of many requests, keep it busy.  Time of the launch over that of
+# the layers' own kernels, 28 layers of 15.7 / 19.7 / 23.2 / 28.3 / 38.5 / 50.3 / 56.8 / 63.7 M elements (the first and the sixth
+# are Qwen3-0.6B's and 1.7B's; the dividing lines lie between a size below 1 and one above, 1.7B's own two rows and 2 to 8 of
+# 28 M among them):
+#   1 row, 300 keys 0.82 / 0.89 / 0.91 / 0.92 / 0.99 / 0.95 / 1.04 / 1.05, 8,000 0.90 / 0.93 / . / . / . / 0.98, 16,000 0.99 / 1.01,
+#   32,000 1.05; 2 rows, 42 to 546 keys 0.83 / 0.99 / 0.93 / 1.04 / 1.05 / 1.03 / . / 1.04, 2,000 to 4,000 0.92 / 1.00 / . / 1.06, 8,000 0.94 / 1.00,
+#   500 to 16,000 0.95 / 1.03; 4 rows, 64 to 900 0.91 / 1.00 / 1.05 / 1.05 / 1.04 / 1.00 / . / 1.08, 200 to 4,000 0.97 / 1.00 / . / 1.04, 8,000 0.97 / 1.02,
+#   500 to 16,000 0.99 / 1.05; 8 rows, 64 to 900 0.87 / 0.99 / 1.04 / 1.02 / 1.04 / 1.00 / . / 1.04, 1,000 to 2,000 0.93 / 0.96, 200 to 4,000 1.02 / 1.02;
+#   12 rows, 64 to 900 . / 0.99 / 0.99 / 0.99 / 1.03 / 1.01 / 1.07 / 1.05, 1,000 to 2,000 0.98 / 1.04, 200 to 4,000 1.10 / 1.16; 16 rows, 64 to 900
+#   0.87 / 0.95 / 0.93 / 0.93 / 0.97 / 0.96 / 0.97 / 0.98 (76.0 M: 1.02), 200 to 2,000 0.96 / 0.99 / . / 0.99 / 1.01 / 0.99, 200 to 4,000 1.01 / 1.04 / . / 1.03 / 1.04 / 1.01.
+_FASTER = {
+    1: ((8192, 50), (16384, 16)),
+    2: ((1024, 24), (4096, 20), (16384, 16)),
+    4: ((4096, 20), (16384, 16)),
+    8: ((2048, 20),),
+    15: ((1024, 32), (2048, 16)),
+    16: ((2048, 64),),
+}
 
 _lib: ctypes.CDLL | None = None
 
@@ -46,12 +58,18 @@ def _library() -> ctypes.CDLL:
     return _lib
 
 
-def fits(rows: int, hidden: int, nq: int, nkv: int, d: int, inter: int, page_size: int) -> bool:
-    """Whether the launch takes layers of these sizes, and is the faster one."""
+def faster(rows: int, weights: int, span: int) -> bool:
+    """Whether the launch is the faster one for ``rows`` rows over layers of ``weights`` matrix elements and contexts of up to ``span`` keys."""
+    limits = next(limits for most, limits in _FASTER.items() if rows <= most)
+    return weights <= next((limit << 20 for keys, limit in limits if span <= keys), 0)
+
+
+def fits(rows: int, hidden: int, nq: int, nkv: int, d: int, inter: int, page_size: int, span: int = 1) -> bool:
+    """Whether the launch takes layers of these sizes, and is the faster one over contexts of up to ``span`` keys."""
     return (
         1 <= rows <= MAX_ROWS and d == HEAD_DIM and nkv >= 1 and nq % nkv == 0 and nq // nkv <= MAX_GROUP
         and hidden % STEP == 0 and inter % STEP == 0 and page_size % 8 == 0
-        and hidden * ((2 * nq + 2 * nkv) * d + 3 * inter) <= (FEW_LAYER_WEIGHTS if 2 <= rows < 8 else MAX_LAYER_WEIGHTS)
+        and faster(rows, hidden * ((2 * nq + 2 * nkv) * d + 3 * inter), span)
     )
 
 
@@ -113,7 +131,7 @@ class DecodeChain:
         self.num_layers = len(layers)
         self.page_size = layers[0][8].shape[2]
         d = HEAD_DIM
-        if not fits(rows, hidden, nq, nkv, d, inter, self.page_size):
+        if not fits(rows, hidden, nq, nkv, d, inter, self.page_size, span):
             raise KernelError(f"the decode chain does not take {rows} rows of layers of {hidden} / {nq} / {nkv} / {inter}")
         shapes = (((nq + 2 * nkv) * d, hidden), (hidden, nq * d), (2 * inter, hidden), (hidden, inter))
         pages = layers[0][8].shape[0]

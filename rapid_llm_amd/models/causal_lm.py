@@ -219,7 +219,8 @@ class CausalLM:
             and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
             and ops.attention_prepares_queries(torch.bfloat16, mixer.d, 0 if cos is None else cos.shape[1],
                                                getattr(mixer.position, "pairing", "half_split") if cos is not None else "half_split")
-            and decode_chain.fits(1, mixer.hidden_size, mixer.nq, mixer.nkv, mixer.d, ff.intermediate_size, 8)
+            and any(decode_chain.fits(rows, mixer.hidden_size, mixer.nq, mixer.nkv, mixer.d, ff.intermediate_size, 8)
+                    for rows in range(1, decode_chain.MAX_ROWS + 1))
         )
 
     def chain_bytes(self, span: int) -> int:
@@ -236,7 +237,7 @@ class CausalLM:
         blocks = [self.blocks[li] for li in self.order]
         mixer, ff = blocks[0].mixer, blocks[0].feed_forward
         sizes = (mixer.hidden_size, mixer.nq, mixer.nkv)
-        if not decode_chain.fits(ctx.num_tokens, *sizes, mixer.d, ff.intermediate_size, caches[0].page_size):
+        if not decode_chain.fits(ctx.num_tokens, *sizes, mixer.d, ff.intermediate_size, caches[0].page_size, ctx.static["context_bound"]):
             return None
         columns = ctx.block_tables[caches[0].group_id].stride(0)
         if not decode_chain.takes(len(blocks), ctx.num_tokens, *sizes, ff.intermediate_size, columns, caches[0].page_size, ctx.static["context_bound"]):

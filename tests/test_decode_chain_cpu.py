@@ -57,3 +57,20 @@ def test_indices_that_the_launch_does_not_reach():
     assert chain.takes(28, 1, *sizes, 8, 16384, 4096) and not chain.takes(28, 1, *sizes, 3, 65536, 4096)  # keys times tokens a page
     wide = (128, 1, 1, 131072)  # 8 k items a layer
     assert chain.takes(8, 1, *wide, 256, 16, 4096) and not chain.takes(80, 1, *wide, 256, 16, 4096)
+
+
+def test_where_the_launch_is_the_faster_one():
+    """Microseconds of both ways, measured: (rows, millions of elements a layer, keys), and whether the launch was the faster."""
+    for rows, millions, keys, launch in (
+        (1, 15.7, 4096, True), (1, 50.3, 8192, True), (1, 56.8, 512, False), (1, 63.7, 2048, False), (1, 15.7, 16384, True), (1, 15.7, 32768, False),
+        (2, 23.2, 1024, True), (2, 28.3, 1024, False), (2, 28.3, 4096, False), (2, 50.3, 1024, False), (4, 19.7, 4096, True), (4, 23.2, 1024, False),
+        (4, 63.7, 1024, False), (8, 19.7, 2048, True), (8, 28.3, 1024, False), (8, 15.7, 4096, False), (12, 28.3, 1024, True), (12, 38.5, 1024, False),
+        (12, 15.7, 2048, True), (12, 19.7, 2048, False), (12, 15.7, 4096, False), (16, 63.7, 1024, True), (16, 76.0, 1024, False), (16, 28.3, 4096, False),
+    ):
+        assert chain.faster(rows, int(millions * 1e6), keys) == launch, (rows, millions, keys)
+    # more keys or larger layers never bring the launch back
+    for rows in range(1, 17):
+        for millions in (1, 15, 20, 30, 50, 66):
+            answers = [chain.faster(rows, millions * 1000000, 512 << i) for i in range(9)]
+            assert answers == sorted(answers, reverse=True) and not answers[-1]
+            assert answers[0] or not chain.faster(rows, millions * 1000000 + (8 << 20), 512)
