@@ -1,7 +1,8 @@
 // bfloat16 product for many rows (prompt steps): out[M,N] = X[M,K] * W[N,K]^T, float32 accumulation on
 // the matrix cores; stored as bfloat16, with silu(gate) * up of the packed [gate | up] matrix in the epilogue, or as
-// float32 runs of K.  (As bfloat16, microseconds over weights from memory, the library's first: 2,048 rows of 6,144 x 4,096 84.7 /
-// 78.9, of 4,096 x 4,096 64.0 / 58.1; 8,926 of 4,096 x 1,024 82.8 / 81.0, of 1,024 x 3,072 62.0 / 55.4; ops.block_plain_plan has the rest.)
+// float32 runs of K.  (As bfloat16, microseconds alone, operands from memory, the library's first: 2,048 rows of 6,144 x 4,096 84.7 /
+// 78.9, of 4,096 x 4,096 64.0 / 58.1; 8,926 of 4,096 x 1,024 82.8 / 81.0, of 1,024 x 3,072 62.0 / 55.4.  Inside a prompt step, where X has
+// just been written, the first is 2.0 us faster than the library's and the second level; ops.block_plain_plan has the rest.)
 //
 // What bounds it: the matrix cores, and with real operands the clock they run at (zeros: 2.05 PFLOP/s at
 // 8,192 x 8,192 x 8,192, random numbers: 1.55, 1.9 GHz; the library's kernel 2.26 and 1.62), so everything else is kept

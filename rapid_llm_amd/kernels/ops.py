@@ -1839,7 +1839,15 @@ def block_plain_plan(m: int, n: int, k: int, units: int) -> tuple[int, int, int]
     """The plan of the many-row product stored as bfloat16, ``None`` where the library's is the faster one.
 
     A tile walks K alone and a unit has one, so the tiles decide: seven eighths of the units in one round, seven tenths of
-    several rounds.  Microseconds at 1,024 / 2,048 / 3,000 / 4,096 / 8,926 rows over weights from memory, the library's
+    several rounds, more than three quarters of two rounds of 256 x 256.  What counts is the layer's time inside a prompt step, the two in
+    turn; microseconds by which this kernel's is the shorter at the rows given (2,048 / 3,000 / 4,096 / 5,000 / 7,000 / 8,926): 4,096 x 2,048
+    1.6 / 0.2 / -0.4 / 7.1 / 0.7 / -8.6 to -16.6 (at 8,720 and 8,800 14.9 and 17.1); 6,144 x 2,560 5.4 / 7.9 / 13.8 / 0.9 / 0.3 and, in another
+    run, -31.8 / -15.4 (at 8,500 37.0); 6,144 x 4,096 2.0 / 5.4 / 4.4 / 3.1 / -8.4 (8,500 68.2); 4,096 x 1,024 1.5 / . / . / 10.0 / 0.0 / 5.5; 2,560 x
+    4,096 1.3 / 1.8 / 2.0 / . / 0.8 / 2.1; 4,096 x 4,096 0.4 / . / -4.8 / -7.1 / -9.5 (-0.2 to -0.7% of the step, so far left here); 2,560
+    x 9,728 0.7 / -1.6 / -1.9 / . / 159 / 2.6; 4,096 x 12,288 0.1 / . / 1.7 / -18.9 / 69.1 (8,500 291).  The library's time changes by a
+    tenth between neighbouring numbers of rows, this kernel's does not.  Two rounds of 256 x 256 of which three quarters have a tile
+    (5,900 to 6,144 rows): 4,096 x 2,048 -4.9 to -2.4, 4,096 x 4,096 -14.8 to -7.2, 4,096 x 12,288 -30.0 to -12.0, not taken.
+    Alone, over weights from memory and rows that are as cold, microseconds at 1,024 / 2,048 / 3,000 / 4,096 / 8,926 rows, the library's
     first: 6,144 x 4,096 56.4 / 51.3, 84.7 / 78.9, 141 / 138, 167 / 156, 418 / 342; 4,096 x 4,096 42.5 / 41.3, 64.0 / 58.1,
     ., 95.2 / 95.9, 334 / 248; 6,144 x 2,560 38.5 / 36.1, 57.9 / 54.8, 103 / 94.4, 112 / 105, 219 / 226; 4,096 x 2,048
     24.9 / 22.8, 35.0 / 33.0, 44.9 / 46.4, 53.8 / 55.2, 129 / 137; 2,048 x 2,048 at 2,048 rows 20.8 / 20.3, at 8,926 83.4 /
@@ -1858,6 +1866,8 @@ def _block_plain_plan(m: int, n: int, k: int, units: int, own: bool) -> tuple[in
     tiles = _block_tiles(m, n, "plain", plan)
     rounds = -(-tiles // units)
     if rounds > 1:
+        if rounds == 2 and plan[:2] == (4, 4) and n * k >= _SMALL_WEIGHTS and 4 * tiles <= 6 * units:
+            return None
         return plan if 10 * tiles >= 7 * rounds * units else None
     if k <= 1024 and plan[:2] == (4, 4):
         return None

@@ -23,6 +23,16 @@ def test_plans_are_what_the_kernel_takes(units):
     assert ops.block_plain_plan(2048, 6140, 4096, units) is None and ops.block_plain_plan(2048, 6144, 4100, units) is None
 
 
+def test_two_rounds_of_large_tiles_that_three_quarters_of_the_units_have():
+    """Measured inside prompt steps: the library's products are the faster ones there, level or slower on both sides."""
+    for n, k in ((4096, 2048), (4096, 4096), (4096, 12288)):
+        for m in (5889, 6000, 6144):
+            assert ops._block_plan(m, n, k, "plain", 256)[:2] == (4, 4) and ops.block_plain_plan(m, n, k, 256) is None
+            assert ops.library_takes(m, n, k)
+        assert ops.block_plain_plan(6145, n, k, 256) is not None and ops.block_plain_plan(5500, n, k, 256) is not None
+    assert ops.block_plain_plan(6000, 2048, 2048, 256) is not None  # (one round)
+
+
 def test_small_models_library_products():
     layers = {"0.6b": ((4096, 1024), (1024, 2048), (1024, 3072)), "1.7b": ((4096, 2048), (2048, 2048), (2048, 6144))}
 
