@@ -129,6 +129,8 @@ class CausalLM:
                 )
             )
 
+        self._kinds = [self.blocks[li] for li in self.order]
+
     # ---- tensors ---------------------------------------------------------------
     def all_parts(self):
         yield self.embed
@@ -154,6 +156,13 @@ class CausalLM:
     def bind(self, params: dict[str, torch.Tensor], runtime) -> None:
         for part in self.all_parts():
             part.bind(params, runtime)
+        # a block of every kind that runs, for what depends on the sizes of a layer's matrices alone
+        kinds = {}
+        for li in self.order:
+            block = self.blocks[li]
+            plain = block.launch_signature() is not None
+            kinds.setdefault(tuple(t.shape for t in block.own_tensors() if t.dim() == 2) if plain else None, block)
+        self._kinds = list(kinds.values())
 
     def replayable(self) -> bool:
         """Whether a step of this model may be recorded into a graph: every part and every
@@ -298,14 +307,16 @@ class CausalLM:
         return DeferredProduct(self.blocks[self.order[-1]].feed_forward.last_product, after) if lazy else after
 
     def _own_products(self, ctx) -> bool:
-        """Whether the step keeps to this package's products (``OWN_PRODUCTS_MAX``)."""
-        block = self.blocks[self.order[0]]
-        if ctx.num_tokens <= ops.SKINNY_MAX_ROWS or block.launch_signature() is None:
+        """Whether the step keeps to this package's products (``OWN_PRODUCTS_MAX``): no layer needs the library's."""
+        if ctx.num_tokens <= ops.SKINNY_MAX_ROWS:
             return False
-        if ctx.num_tokens * sum(t.numel() for t in block.own_tensors() if t.dim() == 2) > OWN_PRODUCTS_MAX:
-            return False
+        for block in self._kinds:
+            if block.launch_signature() is None:
+                return False
+            if ctx.num_tokens * sum(t.numel() for t in block.own_tensors() if t.dim() == 2) > OWN_PRODUCTS_MAX:
+                return False
         with ops.own_products():
-            return not block.calls_library(ctx.num_tokens)
+            return not any(block.calls_library(ctx.num_tokens) for block in self._kinds)
 
     def forward(self, ctx, caches) -> torch.Tensor:
         """Run the tokens of ``ctx`` through every layer (which writes their keys and values)

@@ -3,9 +3,15 @@
 import random
 import threading
 
-import pytest
+from types import SimpleNamespace
 
+import pytest
+import torch
+
+from rapid_llm_amd.config.qwen3 import Qwen3Config
 from rapid_llm_amd.kernels import ops
+from rapid_llm_amd.models.causal_lm import CausalLM
+from rapid_llm_amd.models.qwen3 import build_qwen3_spec
 
 
 @pytest.mark.parametrize("units", [64, 256, 304])
@@ -55,3 +61,41 @@ def test_small_models_library_products():
         thread.start()
         thread.join()
     assert seen == [True]
+
+
+def test_a_step_keeps_to_own_products_only_if_every_layer_can():
+    """A later layer of another kind may need the library's product, or make more than its matrices' launches: the step
+    then waits for the host anyway, and every product is the one that is faster on the device."""
+    body = dict(
+        architectures=["Qwen3ForCausalLM"], model_type="qwen3", num_hidden_layers=4, hidden_size=1024, num_attention_heads=16,
+        num_key_value_heads=8, head_dim=128, intermediate_size=3072, vocab_size=97, rope_theta=10000.0, rms_norm_eps=1e-6,
+        tie_word_embeddings=True, max_position_embeddings=128, hidden_act="silu", attention_bias=False,
+    )
+    runtime = SimpleNamespace(device=torch.device("meta"), dtype=torch.bfloat16, max_seq_len=128, page_size=16)
+
+    def model(change=None):
+        m = CausalLM(build_qwen3_spec(Qwen3Config.from_dict(body)))
+        if change is not None:
+            change(m.blocks[2])
+        params = {s.name: torch.empty(s.shape, dtype=torch.float32 if s.role == "vector" else torch.bfloat16, device="meta") for s in m.param_specs()}
+        m._positions.clear()  # (their tables are made on the device)
+        m.bind(params, runtime)
+        return m
+
+    def own(m, tokens):
+        return m._own_products(SimpleNamespace(num_tokens=tokens))
+
+    plain = model()
+    assert len(plain._kinds) == 1 and own(plain, 300) and not own(plain, 16) and not own(plain, 4000)
+
+    def wide(block):  # an intermediate size that the library's product is needed for
+        ff = type(block.feed_forward)(1024, 20000, "model.layers.2.mlp.", name="layers.2.ff")
+        block.feed_forward = ff
+
+    def hooked(block):
+        block.mixer.forward = block.mixer.forward
+
+    mixed = model(wide)
+    assert len(mixed._kinds) == 2
+    assert any(b.calls_library(300) for b in mixed._kinds) and not own(mixed, 300)
+    assert not own(model(hooked), 300)
