@@ -108,6 +108,76 @@ def test_any_number_of_workgroups_gives_the_same(rows, monkeypatch):
         assert torch.equal(r, results[0])
 
 
+def _launched_with(units):
+    """A step's recorded launch has so many workgroups, and as many shares of the keys as ever."""
+    from rapid_llm_amd.kernels import decode_chain, ops
+
+    real, m = decode_chain.DecodeChain.run, pytest.MonkeyPatch()
+
+    def run(self, *args):
+        with pytest.MonkeyPatch.context() as inner:
+            inner.setattr(decode_chain, "chip", lambda: ops.Chip(units))
+            return real(self, *args)
+
+    m.setattr(decode_chain.DecodeChain, "run", run)
+    return m
+
+
+@pytest.mark.parametrize("rows", [1, 2, 4, 8, 16])
+def test_workgroups_that_start_too_late_leave(rows):
+    """A workgroup's LDS leaves no room for another one on its unit: of twice as many as there are units, the list is closed
+    without those that start when others have ended."""
+    from rapid_llm_amd.kernels import ops
+
+    cfg = {**BASE, "hidden_size": 1024, "num_attention_heads": 8, "intermediate_size": 1536}
+    units, dealt = ops.chip().units, 32  # (the word that holds how many workgroups the items were dealt to)
+    results = []
+    for launched in (units, min(2 * units, 512)):
+        runner = _runner(cfg)
+        tokens, entries = _fill(runner, CONTEXTS[:rows], cfg["vocab_size"])
+        m = _launched_with(launched)
+        try:
+            results.append(_again(runner, tokens, entries))
+        finally:
+            m.undo()
+        for _ in range(5):
+            assert torch.equal(_again(runner, tokens, entries), results[0])
+            assert 1 <= int(runner.model._chain_space.control.view(torch.int32)[dealt]) <= units
+        runner.check(runner.lost)
+    assert torch.equal(results[1], results[0])
+
+
+@pytest.mark.parametrize("kv_heads", [1, 2])
+def test_contexts_of_nine_to_sixteen_shares(tmp_path, kv_heads):
+    """Whoever folds a request's shares asks for eight at a time: contexts of 16, 9, 15 and 10 shares, each head folded by a workgroup
+    of its own, and (fewer workgroups than items) all by the last share's."""
+    from rapid_llm_amd import write_random_model
+
+    cfg = {**BASE, "num_key_value_heads": kv_heads, "num_hidden_layers": 2, "max_position_embeddings": 4096}
+    folder = str(write_random_model(cfg, 7, tmp_path / "long", dtype="bfloat16"))
+    config, weights = plain_load(folder)
+    contexts = [4089, 2303, 3839, 2304]
+    plain = None
+    for rows in (1, 2, 4):
+        got = []
+        for launched in (None, 5):
+            runner = _runner(folder, max_seq_len=4096, num_pages=900)
+            tokens, entries = _fill(runner, contexts[:rows], cfg["vocab_size"])
+            m = _launched_with(launched) if launched else pytest.MonkeyPatch()
+            try:
+                got.append(_again(runner, tokens, entries).cpu())
+            finally:
+                m.undo()
+            (chain,) = _chains(runner)
+            assert chain is not None and chain.nsplit == 16
+            assert torch.equal(_again(runner, tokens, entries).cpu(), got[-1])
+        assert torch.equal(got[0], got[1])
+        if plain is None:
+            every = [random_tokens(n + 1, cfg["vocab_size"], 31 + i) for i, n in enumerate(contexts)]
+            plain = torch.stack([plain_forward(config, weights, ids)[-1] for ids in every])
+        parity.assert_bf16_close(got[0], plain[:rows], f"decode chain/long/{kv_heads}/{rows}")
+
+
 def _count_from(runner, launch):
     """The number of the next launch, as if so many had gone before."""
     from rapid_llm_amd.kernels import decode_chain
