@@ -22,11 +22,11 @@
 // folds them in the same order: the same bits.
 //
 // What bounds it: whole contexts of 2,048 keys, 32 query and 8 kv heads of 128 channels, take 404 us (85 TFLOP/s;
-// 5,000 keys 91).  The float32 matrix instructions hold the vector units for 53% of that, their rate, and the
+// 5,000 keys 91) called alone, and 471 a layer in the prompt step under the profiler, where nothing of them is near.  The float32 matrix instructions hold the vector units for 53% of that, their rate, and the
 // other vector instructions for 36%, the weights of a tile above all; they do not overlap.  Two tiles of rows a
 // workgroup, which halve the keys that are read, leave one wave a SIMD and took 428 us.  Before, a tile's entry of the
 // block table was asked for and waited for with its keys and with its values, both behind every load in flight, at a
-// position that took a division, and the maximum and the sum of a row went through LDS: 514 us.  Masked keys contribute exactly zero
+// position that took a division, and the maximum and the sum of a row went through LDS: 514 us, 591 in the step.  Masked keys contribute exactly zero
 // (rapid_llm/kernels/ops/attention/flashdecoding.py:223-237); scores are (q . k) / sqrt(d)
 // (rapid_llm/modules/attention.py:62), softmax over keys in float32
 // (rapid_llm/kernels/ops/attention/flashattention2_nopad.py:138-168).

@@ -678,7 +678,7 @@ extern "C" int rl_gemm_skinny_residual(const void* X, const void* W, int M, int 
 }
 
 // =========================================================================== //
-// 17 .. 192 rows: the runs of K of a product whose result feeds the residual
+// 17 rows and more: the runs of K of a product whose result feeds the residual
 // =========================================================================== //
 // The library's product reads X once for every 16 or 32 weight rows at these sizes and
 // stays near 3 TB/s.  Here a workgroup is four waves with 16 weight rows each; the chunk of X
@@ -691,7 +691,7 @@ extern "C" int rl_gemm_skinny_residual(const void* X, const void* W, int M, int 
 // and 23.0 / 28.6.  The wide products (6,144 and 24,576 rows) gain nothing (18.3 / 18.1 and
 // 55 / 46) and stay with the library.  More than 64 rows run as blocks of 64 rows (grid.z), each
 // reading the weights again: up to about 192 rows that is still faster than the library's kernels
-// for such shapes (the host's rule holds the measurements).
+// for such shapes, and up to 320 level with them for small matrices (the host's rule, mid_max_rows, holds the measurements).
 #define MW 4  // waves per workgroup
 
 template <int MB>

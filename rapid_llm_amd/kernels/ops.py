@@ -1887,7 +1887,7 @@ def block_reads(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def block_pays(m: int, n: int, k: int, units: int) -> bool:
-    """Whether the ``"runs"`` form is faster, with the norm, than what else there is: the mid-size product up to 192 rows,
+    """Whether the ``"runs"`` form is faster, with the norm, than what else there is: the mid-size product up to ``MID_MAX_ROWS``,
     where its workgroups (tiles times runs) have to cover five eighths of the units, the library's beyond, where three
     eighths do.  Microseconds over weights from memory at 65 / 128 / 192 rows, the mid-size product first: 512 columns of
     12,288 k (32, 32 and 64 workgroups) 14.9 / 19.7, 15.3 / 20.7, 16.3 / 20.7; 1,536 of 9,728 (96, 96 and 192) 21.4 / 21.2,
@@ -1924,7 +1924,8 @@ def _block(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str, plan:
 # library's time jumps between neighbouring row counts (the 8B down projection: 51.8 at 144 rows,
 # 78.8 at 160, 55.4 at 176), this kernel's grows with the blocks of 64; from about 200 rows on
 # the library's best kernels are the faster ones.  Small matrices (the 0.6B and 1.7B shapes) are
-# within a microsecond either way from 144 rows on.
+# within a microsecond either way from 144 rows on; steps that keep to this package's products take them here up to
+# MID_SMALL_MAX_ROWS (mid_max_rows).
 MID_MAX_ROWS = 192
 _MID_BLOCK_ROWS = 64  # weight rows per workgroup of the mid-size product
 _MID_MAX_BLOCKS = 128  # wider matrices than this many workgroups stay with the library
@@ -1949,7 +1950,7 @@ def _mid_runs(n: int, k: int, units: int) -> int:
 
 
 def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor, copies: bool = True) -> torch.Tensor:
-    """``x[M,K] @ w[N,K]^T`` for 17 to 192 rows, or as many as :func:`block_plan` says, as float32 runs of K,
+    """``x[M,K] @ w[N,K]^T`` for 17 rows to :func:`mid_max_rows`, or as many as :func:`block_plan` says, as float32 runs of K,
     ``[runs, M, N]``: their sum is the product.  For products whose result goes into the residual: the norm that
     follows adds the runs (``add_rmsnorm_parts``).  The many-row product runs wherever it can, over copies of operands that
     begin inside a unit of 16 bytes; without ``copies`` only where :func:`block_reads` says so."""
@@ -1970,7 +1971,7 @@ def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor, copies: bool = True) -> to
 
 
 def _mid_parts(x: torch.Tensor, w: torch.Tensor, ks: int) -> torch.Tensor:
-    """The mid-size product of up to 192 rows in ``ks`` runs of K (:func:`mid_runs`)."""
+    """The mid-size product of up to :func:`mid_max_rows` rows in ``ks`` runs of K (:func:`mid_runs`)."""
     _need(x, "x", torch.bfloat16)
     m, k = x.shape
     _need(w, "w", torch.bfloat16, (None, k))

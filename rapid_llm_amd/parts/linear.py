@@ -13,7 +13,7 @@ Which product runs is decided by the weight's storage type:
 * bfloat16 weight: few rows (decode) go to the hand-written bandwidth-bound matrix-core
   kernel, more to kernels of this package for small and for wide matrices; a matrix whose result a norm adds
   to the residual may hand that norm float32 runs of K instead (``partial_sums``: 17 to 192 rows of a
-  narrow one, 320 of a small one, more where K is long).  What none of them takes goes to the library product, as in the reference, whose dense
+  narrow one, 320 of a small one inside ``ops.own_products``, more where K is long).  What none of them takes goes to the library product, as in the reference, whose dense
   products are ``F.linear`` (rapid_llm/kernels/ops/gemm/linear.py:17-40).  The packed gate and up matrices have kernels of
   their own (``ops.gemm_bf16_swiglu``).
 """
@@ -82,7 +82,7 @@ class Linear:
 
     def midsize(self, x) -> bool:
         """Whether ``x`` (more rows than the few-row kernel takes) may run as float32 runs of K that a norm adds: up to
-        192 rows over a narrow matrix (wide ones have nothing to gain), any number of them over long sums where the many-row
+        ``ops.mid_max_rows`` over a narrow matrix (wide ones have nothing to gain), any number of them over long sums where the many-row
         product is the faster one (``ops.block_reads``)."""
         rows = x.shape[0]
         if self.weight.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or rows <= ops.SKINNY_MAX_ROWS:
