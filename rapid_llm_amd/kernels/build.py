@@ -84,6 +84,11 @@ _HIPCC_FLAGS = (
     "-target-feature",
     "-Xclang",
     "-packed-fp32-ops",
+    # A kernel's first arguments come in scalar registers with the launch, without a trip to memory before anything else:
+    # steps of short kernels take 0.8 to 1.3% less (8B, 8 and 64 requests decoding 3,726 -> 3,695 and 6,794 -> 6,719 us;
+    # 0.6B, 256 requests 5,039 -> 4,999; 8B float32, 8 requests 7,442 -> 7,367).
+    "-mllvm",
+    "-amdgpu-kernarg-preload-count=16",
 )
 
 
