@@ -241,8 +241,9 @@ __device__ __forceinline__ void ask_query(AskedQuery& a, const bf16_t* qrow, int
             }
     }
 }
+// (`scale`: a factor of the scores that is taken into the query, before its only rounding)
 __device__ __forceinline__ void prepared_query(bf16x8 (&qf)[DC], const AskedQuery& a, const float (&w)[DC][8], bool row_ok,
-                                      const DecodeExtra& ex) {
+                                               const DecodeExtra& ex, float scale) {
     float x[DC][8];
     float ss = 0.f;
 #pragma unroll
@@ -255,11 +256,16 @@ __device__ __forceinline__ void prepared_query(bf16x8 (&qf)[DC], const AskedQuer
         }
     }
     if (ex.q_norm_w) {
-        const float rrms = rsqrtf(row_sum4(ss) / (float)D + ex.eps);
+        const float rrms = rsqrtf(row_sum4(ss) / (float)D + ex.eps) * scale;
 #pragma unroll
         for (int c = 0; c < DC; ++c)
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[c][j] *= rrms * w[c][j];
+    } else {
+#pragma unroll
+        for (int c = 0; c < DC; ++c)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[c][j] *= scale;
     }
     if (ex.cos_tab) {
         constexpr int HC = DC / 2;
@@ -281,12 +287,13 @@ __device__ __forceinline__ void prepared_query(bf16x8 (&qf)[DC], const AskedQuer
 
 // The same in functions of their own, for kernels that have no registers left beside their accumulators: what is
 // written through a pointer stays in scratch memory, from where every step reads it again.
-__device__ __noinline__ void late_query(bf16x8 (&qf)[DC], const bf16_t* qrow, bool row_ok, int pos, int g, const DecodeExtra& ex) {
+__device__ __noinline__ void late_query(bf16x8 (&qf)[DC], const bf16_t* qrow, bool row_ok, int pos, int g, const DecodeExtra& ex,
+                                        float scale) {
     AskedQuery asked;
     float w[DC][8];
     ask_query(asked, qrow, pos, g, ex);
     ask_norm(w, g, ex);
-    prepared_query(qf, asked, w, row_ok, ex);
+    prepared_query(qf, asked, w, row_ok, ex, scale);
 }
 __device__ __noinline__ void late_plain(bf16x8 (&qf)[DC], const bf16_t* qrow, bool row_ok, int g) {
 #pragma unroll
@@ -388,7 +395,7 @@ __global__ __launch_bounds__(WAVES* RL_WAVE) void attn_decode_kernel(
         // Q^T as B operand: lane (row col, group g) holds channels 32c + 8g .. + 7
         bf16x8 qf[DC];
         if (FUSED) {
-            prepared_query(qf, asked, norm_w, head_ok, ex);
+            prepared_query(qf, asked, norm_w, head_ok, ex, 1.f);
             // the token's own key and value: written by the split that holds its position
             // (with more than 16 heads on a kv head every chunk of heads writes the same bytes:
             // each reads them back after its own barrier only)
@@ -696,6 +703,7 @@ extern "C" int rl_attn_decode_fusable() { return D % 64 == 0 ? 1 : 0; }
 #define PF_WAVES 4                       // waves that share the rows of a tile
 #define PF_NQ RL_PF_NQ                   // 16-row blocks per wave
 #define PF_ROWS (PF_WAVES * PF_NQ * 16)  // rows per workgroup
+#define LAZY 8.f                         // powers of two a row's maximum may move by before its sums are rescaled
 #define PF_KEYS 64                       // keys per LDS tile and per softmax step
 #define PF_THREADS (PF_WAVES * RL_WAVE)  // threads of one wave group
 #define K_LD (D + 8)                     // padded row of the K tile (bfloat16 elements)
@@ -705,12 +713,18 @@ extern "C" int rl_attn_decode_fusable() { return D % 64 == 0 ? 1 : 0; }
 // Softmax is the arithmetic that competes with the matrix cores here, so a step covers 64
 // keys (one maximum, one rescale and one sum for 16 scores per lane), scores are masked only
 // in tiles that the diagonal, a window's edge or the end of the sequence crosses, and the
-// accumulators are rescaled only when some row's maximum moved.
+// accumulators are rescaled only when some row's maximum moved by more than LAZY: the weights are relative to what the
+// row's maximum was then, at most 2^LAZY, of which float32 sums and bfloat16 roundings have no less precision.  Queries
+// that are finished here (PREP) take the scores' factor in before their only rounding, and the scores' sums begin with
+// the negative maximum, so that a weight is one exponential of what the matrix cores leave (8,192 tokens of 32 query heads, all
+// of it and what follows here 0.89 -> 0.98 PFLOP/s).
 //
-// tile_info[4 * tile + {0,1,2,3}] = {first token of the request's portion in the flat batch,
-//   tokens of the request already in the cache, tokens in this portion, first row of the tile};
-// work_order (optional): workgroup b takes (tile, kv head) = (work_order[b] / nkv, % nkv), so
-// that the host decides which workgroups start together.
+// tile_info[8 * tile + {0..4}] = {first token of the request's portion in the flat batch, tokens of the
+//   request already in the cache, tokens in this portion, first row of the tile, the request's row of the
+//   block table (-1: token_slot has it)}, [6, 7]: the first row divided by the query heads of a kv head, and what is left;
+// work_order (optional): workgroup b takes the tile of work_order[8 * b ..], the same numbers, and the
+// kv head [5], so that the host decides which workgroups start together.  All of it lies side by side: every
+// further place to look something up is a trip to memory before a workgroup's first key is asked for.
 // Two waves per SIMD at most: the accumulators then live in ordinary vector registers, which
 // the rescale and the epilogue read directly (at the default budget of 128 the compiler parks
 // them in accumulation registers and moves them back and forth around every rescale).
@@ -740,35 +754,40 @@ constexpr int PF_DIRECT_TILE = PF_KEYS * D * 2;      // bytes of a key tile and 
 constexpr int PF_DIRECT_SET = 2 * PF_DIRECT_TILE;    // one step's tiles
 constexpr int PF_DIRECT_GROUP = 2 * PF_DIRECT_SET;   // a wave group's two sets
 
-template <int GROUPS, bool DIRECT>
+template <int GROUPS, bool DIRECT, bool PREP>
 __global__ __launch_bounds__(GROUPS* PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 2))) void
 attn_prefill_kernel(
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
-    const bf16_t* __restrict__ v_cache, bf16_t* __restrict__ out,
-    const int* __restrict__ tile_info, const int* __restrict__ work_order,
-    const int* __restrict__ token_slot, const int* __restrict__ block_table, int table_stride,
-    int page_size, unsigned page_magic, int nq, int nkv, int window, float scale_log2, int nsplit,
-    float* __restrict__ part_o, float* __restrict__ part_ml, int prep_q, DecodeExtra ex) {
+    const bf16_t* __restrict__ q, const int* __restrict__ tile_info, const int* __restrict__ work_order,
+    const int* __restrict__ block_table, int table_stride, unsigned page_magic, int page_size, int nkv,
+    const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, bf16_t* __restrict__ out,
+    const int* __restrict__ token_slot, int G, unsigned group_magic, int window, float scale_log2, int nsplit,
+    float* __restrict__ part_o, float* __restrict__ part_ml, DecodeExtra ex) {
     constexpr int GROUP_ELEMS = DIRECT ? PF_DIRECT_GROUP / 2 : PF_TILE_ELEMS;  // bfloat16 elements
     __shared__ __attribute__((aligned(1024))) bf16_t tiles[GROUPS * GROUP_ELEMS];
     __shared__ float fold_ml[GROUPS > 1 ? PF_WAVES * PF_NQ * 2 * RL_WAVE : 1];
 
-    const int G = nq / nkv;
+    // the arguments that do not come in registers, asked for together
+    asm volatile("" ::"s"(G), "s"(group_magic), "s"(nsplit), "s"(ex.qkv_stride), "s"(ex.q_norm_w), "s"(ex.cos_tab), "s"(k_cache));
+    const int nq = G * nkv;
     // nsplit > 1: the keys of every tile are cut into nsplit runs of whole 64-key steps, one
     // workgroup each; the runs' results go to part_o / part_ml (indexed by the token's place in
     // the step) and are folded by the merge kernel, as the decode kernel's splits are
-    const int split = blockIdx.x % nsplit;
-    const int wg = blockIdx.x / nsplit;
-    const int item = work_order ? work_order[wg] : wg;
-    const int tile = item / nkv;
-    const int hk = item % nkv;
-    const int tok0 = tile_info[4 * tile + 0];
-    const int start = tile_info[4 * tile + 1];
-    const int qlen = tile_info[4 * tile + 2];
-    const int row0 = tile_info[4 * tile + 3];
+    const int wg = nsplit > 1 ? blockIdx.x / nsplit : blockIdx.x;
+    const int split = blockIdx.x - wg * nsplit;
+    const int tile = (unsigned)wg / (unsigned)nkv;
+    const int* const work = work_order ? work_order + 8 * (size_t)wg : tile_info + 8 * (size_t)tile;
+    const int tok0 = work[0];
+    const int start = work[1];
+    const int qlen = work[2];
+    const int row0 = work[3];
+    const int slot = work[4];
+    const int hk = work_order ? work[5] : wg - tile * nkv;
+    const int row_tok = work[6], row_head = work[7];  // row0 / G, row0 % G
     const int rows = qlen * G;
     const int seq_end = start + qlen;  // keys at or beyond this were never written
-    const int* table = block_table + (size_t)token_slot[tok0] * table_stride;
+    const int* table = block_table + (size_t)(slot >= 0 ? slot : token_slot[tok0]) * table_stride;
+    // the portion's token that row row0 + i belongs to (group_magic = ceil(2^31 / G) divides by G: exact below 2^31 / G)
+    auto token_of = [&](int i) { return row_tok + (int)__umulhi(2u * (unsigned)(row_head + i), group_magic); };
 
     const int grp = GROUPS > 1 ? threadIdx.x / PF_THREADS : 0;  // wave group: which steps
     const int tid = threadIdx.x - grp * PF_THREADS;             // thread within the group
@@ -786,14 +805,15 @@ attn_prefill_kernel(
     bf16x8 qf[PF_NQ][DC];
 #pragma unroll
     for (int n = 0; n < PF_NQ; ++n) {
-        const int row = row0 + (wave * PF_NQ + n) * 16 + col;
-        r_ok[n] = row < rows;
-        const int rr = r_ok[n] ? row : rows - 1;
-        r_tok[n] = tok0 + rr / G;
-        r_head[n] = hk * G + rr % G;
-        r_pos[n] = start + rr / G;
+        const int row = (wave * PF_NQ + n) * 16 + col;  // of the tile
+        r_ok[n] = row0 + row < rows;
+        const int rr = r_ok[n] ? row : rows - 1 - row0;
+        const int tok = token_of(rr);
+        r_tok[n] = tok0 + tok;
+        r_head[n] = hk * G + row0 + rr - tok * G;
+        r_pos[n] = start + tok;
     }
-    // prep_q: `q` holds the raw packed [q | k | v] rows, and the workgroup norms and rotates its
+    // PREP: `q` holds the raw packed [q | k | v] rows, and the workgroup norms and rotates its
     // rows' heads itself, as the decode kernel does (the host asks for it only where
     // D % 64 == 0); else `q` holds finished queries.  Their loads go out before anything else and are
     // waited for once the first tile has been asked for, up to heads of 192 channels.  Heads of 256 are read as they are
@@ -801,11 +821,18 @@ attn_prefill_kernel(
     // heads, 49.5 / 101 / 417 us, now 15.7 / 58.0 / 350).  Two groups of waves have half the registers each, and at 224 and
     // 256 channels are faster with the queries in scratch than with other things there (2,048 tokens 274 / 230 us and 379 / 350;
     // at 208 and 240 with them in registers, 265 / 191 and 360 / 320; one group 15.9 / 9.7 and 21.7 / 15.7 at 37 tokens).
-    // Heads that are never finished here do without the code from 176 channels on (176: 133 / 113; 160: 87 / 91).
-    constexpr bool PREPARES = D % 64 == 0 || D <= 160, EARLY = D <= 192, CALLED = GROUPS == 2 && (D == 224 || D == 256);
-    AskedQuery asked[PF_NQ];
+    // Two groups hold the same rows: each finishes one block of them (SHARED) and hands it to the other through the second
+    // set of tiles, which nothing has been asked into yet.
+    constexpr bool EARLY = D <= 192, CALLED = GROUPS == 2 && (D == 224 || D == 256);
+    constexpr bool SHARED = GROUPS == 2 && PF_NQ == 2 && PREP && EARLY;
+    AskedQuery asked[SHARED ? 1 : PF_NQ];
     float norm_w[DC][8];
-    if (PREPARES && EARLY && prep_q) {
+    if constexpr (SHARED) {
+        const int tok = grp ? r_tok[1] : r_tok[0], head = grp ? r_head[1] : r_head[0], pos = grp ? r_pos[1] : r_pos[0];
+        ask_query(asked[0], q + (size_t)tok * ex.qkv_stride + (size_t)head * D, pos, g, ex);
+        ask_norm(norm_w, g, ex);
+        __builtin_amdgcn_sched_barrier(0);
+    } else if constexpr (EARLY && PREP) {
 #pragma unroll
         for (int n = 0; n < PF_NQ; ++n)
             ask_query(asked[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_pos[n], g, ex);
@@ -813,17 +840,33 @@ attn_prefill_kernel(
         __builtin_amdgcn_sched_barrier(0);
     }
     auto load_queries = [&]() {
+        if constexpr (SHARED) {
+            bf16x8 mine[DC];
+            prepared_query(mine, asked[0], norm_w, grp ? r_ok[1] : r_ok[0], ex, scale_log2);
+            constexpr int AT = DIRECT ? PF_DIRECT_SET / 2 : 0;  // (the padded tiles are stored behind the loop's first barrier)
+            static_assert(!DIRECT || PF_WAVES * PF_NQ * DC * RL_WAVE * 16 <= PF_DIRECT_SET, "the queries fit one set of tiles");
+            static_assert(DIRECT || PF_WAVES * PF_NQ * DC * RL_WAVE * 16 <= (int)sizeof(tiles), "the queries fit the tiles");
+            bf16x8* const handed = reinterpret_cast<bf16x8*>(tiles + AT) + wave * (PF_NQ * DC * RL_WAVE) + lane;
+#pragma unroll
+            for (int c = 0; c < DC; ++c) handed[(grp * DC + c) * RL_WAVE] = mine[c];
+            __syncthreads();
+#pragma unroll
+            for (int n = 0; n < PF_NQ; ++n)
+#pragma unroll
+                for (int c = 0; c < DC; ++c) qf[n][c] = handed[(n * DC + c) * RL_WAVE];
+            return;
+        }
 #pragma unroll
         for (int n = 0; n < PF_NQ; ++n) {
-            if (PREPARES && prep_q) {
+            if constexpr (PREP) {
                 if (EARLY)
-                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex);
+                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex, scale_log2);
                 else if (!CALLED) {
                     ask_query(asked[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_pos[n], g, ex);
                     ask_norm(norm_w, g, ex);
-                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex);
+                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex, scale_log2);
                 } else
-                    late_query(qf[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_ok[n], r_pos[n], g, ex);
+                    late_query(qf[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_ok[n], r_pos[n], g, ex, scale_log2);
             } else if (CALLED && D == 224) {
                 late_plain(qf[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_ok[n], g);
             } else {
@@ -838,21 +881,23 @@ attn_prefill_kernel(
     };
     // keys the tile needs: up to the position of its last row; from the window of its first
     const int last_row = min(row0 + PF_ROWS, rows) - 1;
-    const int tile_kend = start + last_row / G + 1;
-    const int first_pos = start + row0 / G;
+    const int tile_kend = start + token_of(last_row - row0) + 1;
+    const int first_pos = start + row_tok;
     const int tile_kstart = (window > 0 && first_pos - window + 1 > 0) ? first_pos - window + 1 : 0;
     // positions of this wave's rows (rows ascend with the position)
     const int w_first = min(row0 + wave * PF_NQ * 16, rows - 1);
     const int w_last = min(row0 + (wave + 1) * PF_NQ * 16, rows) - 1;
-    const int wave_min_pos = start + w_first / G;
-    const int wave_max_pos = start + (w_last > w_first ? w_last : w_first) / G;
+    const int wave_min_pos = start + token_of(w_first - row0);
+    const int wave_max_pos = start + token_of((w_last > w_first ? w_last : w_first) - row0);
 
     float m[PF_NQ], l[PF_NQ];
+    f32x4 below[PF_NQ];  // PREP: what the scores' sums begin with, -m
     f32x4 acc[PF_NQ][DB];
 #pragma unroll
     for (int n = 0; n < PF_NQ; ++n) {
         m[n] = -INFINITY;
         l[n] = 0.f;
+        below[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int b = 0; b < DB; ++b) acc[n][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
@@ -1091,7 +1136,7 @@ attn_prefill_kernel(
             }
 #pragma unroll
             for (int n = 0; n < PF_NQ; ++n) {
-                s[n][hb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                s[n][hb] = PREP ? below[n] : (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int c = 0; c < DC; ++c) s[n][hb] = mfma(kf[c], qf[n][c], s[n][hb]);
             }
@@ -1113,12 +1158,13 @@ attn_prefill_kernel(
             float mx = s[n][0][0];
 #pragma unroll
             for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[n][e >> 2][e & 3]);
-            mx = row_max4(mx) * scale_log2;  // the scale is positive: max commutes with it
-            const float m_new = fmaxf(m[n], mx);
-            // a row that has seen no visible key yet keeps m = -inf; exp2 of (-inf) - 0 is 0
-            const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
-            if (__any(m_new > m[n])) {
-                const float alpha = __builtin_amdgcn_exp2f(m[n] - m_safe);
+            mx = row_max4(mx);
+            const bool unset = m[n] == -INFINITY;  // the row has seen no visible key yet
+            if (!PREP) mx = mx * scale_log2 - (unset ? 0.f : m[n]);  // (the scale is positive)
+            if (__any(mx > LAZY || (unset && mx > -INFINITY))) {
+                const float up = (unset ? mx > -INFINITY : mx > 0.f) ? mx : 0.f;
+                const float alpha = unset ? 1.f : __builtin_amdgcn_exp2f(-up);  // (an unset row's sums are 0)
+                if (!unset || mx > -INFINITY) m[n] = (unset ? 0.f : m[n]) + up;
                 l[n] *= alpha;
 #pragma unroll
                 for (int b = 0; b < DB; ++b) {
@@ -1127,20 +1173,28 @@ attn_prefill_kernel(
                     acc[n][b][2] *= alpha;
                     acc[n][b][3] *= alpha;
                 }
-                m[n] = m_new;
+                if (PREP) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) s[n][e >> 2][e & 3] -= up;
+                    const float now = m[n] == -INFINITY ? 0.f : -m[n];
+                    below[n] = (f32x4){now, now, now, now};
+                }
             }
-            m_safe_n[n] = m_safe;
+            m_safe_n[n] = PREP || m[n] == -INFINITY ? 0.f : m[n];
         }
         // ---- the weights of the first 32 keys, then of the last 32; the products follow half by
         // half, so that the first half's matrix instructions run beside the second half's
         // exponentials (8,192 tokens: 701 -> 681 us) ---------------------------------------------
         float psum[PF_NQ];
+        auto weight = [&](int n, float score) {
+            return __builtin_amdgcn_exp2f(PREP ? score : fmaf(score, scale_log2, -m_safe_n[n]));
+        };
 #pragma unroll
         for (int n = 0; n < PF_NQ; ++n) {
             psum[n] = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float pe = __builtin_amdgcn_exp2f(fmaf(s[n][e >> 2][e & 3], scale_log2, -m_safe_n[n]));
+                const float pe = weight(n, s[n][e >> 2][e & 3]);
                 psum[n] += pe;
                 p[n][0][e] = (__bf16)pe;
             }
@@ -1149,7 +1203,7 @@ attn_prefill_kernel(
         for (int n = 0; n < PF_NQ; ++n) {
 #pragma unroll
             for (int e = 8; e < 16; ++e) {
-                const float pe = __builtin_amdgcn_exp2f(fmaf(s[n][e >> 2][e & 3], scale_log2, -m_safe_n[n]));
+                const float pe = weight(n, s[n][e >> 2][e & 3]);
                 psum[n] += pe;
                 p[n][1][e & 7] = (__bf16)pe;
             }
@@ -1170,48 +1224,53 @@ attn_prefill_kernel(
             }
         }
     }
-    if (GROUPS > 1) {
-        // group 1's state travels through the LDS that held the tiles: element j of a lane at
-        // [wave][j][lane]; group 0 folds it into its own
+    if constexpr (GROUPS > 1) {
+        // Each group folds and stores one block of rows: it hands its state of the other's through the LDS that held
+        // the tiles, element j of a lane at [group][wave][j][lane].  (One group folding both took 2.7 us, so 1.6.)
+        static_assert(PF_NQ == 2, "a block of rows for each group");
         float* fold_acc = reinterpret_cast<float*>(tiles);
-        constexpr int PER_LANE = PF_NQ * DB * 4;
-        static_assert(GROUPS == 1 || sizeof(float) * PF_WAVES * PER_LANE * RL_WAVE <= sizeof(tiles),
-                      "the accumulators of one group fit where the tiles were");
-        __syncthreads();  // every wave has read its last tile
-        if (grp == 1) {
+        constexpr int PER_LANE = DB * 4;
+        static_assert(sizeof(float) * 2 * PF_WAVES * PER_LANE * RL_WAVE <= sizeof(tiles),
+                      "the accumulators of one block of rows of each group fit where the tiles were");
+        if (grp == 1) {  // its own block first
 #pragma unroll
-            for (int n = 0; n < PF_NQ; ++n) {
-                fold_ml[((wave * PF_NQ + n) * 2 + 0) * RL_WAVE + lane] = m[n];
-                fold_ml[((wave * PF_NQ + n) * 2 + 1) * RL_WAVE + lane] = l[n];
-#pragma unroll
-                for (int b = 0; b < DB; ++b)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        fold_acc[(wave * PER_LANE + (n * DB + b) * 4 + i) * RL_WAVE + lane] = acc[n][b][i];
+            for (int b = 0; b < DB; ++b) {
+                const f32x4 t = acc[0][b];
+                acc[0][b] = acc[1][b];
+                acc[1][b] = t;
             }
+            const float tm = m[0], tl = l[0];
+            m[0] = m[1], l[0] = l[1], m[1] = tm, l[1] = tl;
+            r_tok[0] = r_tok[1], r_head[0] = r_head[1], r_ok[0] = r_ok[1];
         }
-        __syncthreads();
-        if (grp == 1) return;
-#pragma unroll
-        for (int n = 0; n < PF_NQ; ++n) {
-            const float m1 = fold_ml[((wave * PF_NQ + n) * 2 + 0) * RL_WAVE + lane];
-            const float l1 = fold_ml[((wave * PF_NQ + n) * 2 + 1) * RL_WAVE + lane];
-            const float m_new = fmaxf(m[n], m1);
-            const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
-            const float a0 = __builtin_amdgcn_exp2f(m[n] - m_safe);
-            const float a1 = __builtin_amdgcn_exp2f(m1 - m_safe);
-            m[n] = m_new;
-            l[n] = l[n] * a0 + l1 * a1;
+        __syncthreads();  // every wave has read its last tile
+        {
+            const int to = grp * PF_WAVES + wave;
+            fold_ml[(to * 2 + 0) * RL_WAVE + lane] = m[1];
+            fold_ml[(to * 2 + 1) * RL_WAVE + lane] = l[1];
 #pragma unroll
             for (int b = 0; b < DB; ++b)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    acc[n][b][i] = acc[n][b][i] * a0 +
-                                   fold_acc[(wave * PER_LANE + (n * DB + b) * 4 + i) * RL_WAVE + lane] * a1;
+                for (int i = 0; i < 4; ++i) fold_acc[(to * PER_LANE + b * 4 + i) * RL_WAVE + lane] = acc[1][b][i];
         }
+        __syncthreads();
+        const int from = (grp ^ 1) * PF_WAVES + wave;
+        const float m1 = fold_ml[(from * 2 + 0) * RL_WAVE + lane];
+        const float l1 = fold_ml[(from * 2 + 1) * RL_WAVE + lane];
+        const float m_new = fmaxf(m[0], m1);
+        const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
+        const float a0 = __builtin_amdgcn_exp2f(m[0] - m_safe);
+        const float a1 = __builtin_amdgcn_exp2f(m1 - m_safe);
+        m[0] = m_new;
+        l[0] = l[0] * a0 + l1 * a1;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[0][b][i] = acc[0][b][i] * a0 + fold_acc[(from * PER_LANE + b * 4 + i) * RL_WAVE + lane] * a1;
     }
 #pragma unroll
-    for (int n = 0; n < PF_NQ; ++n) {
+    for (int n = 0; n < (GROUPS > 1 ? 1 : PF_NQ); ++n) {
         const float lt = row_sum4(l[n]);
         const float inv = lt > 0.f ? 1.f / lt : 0.f;
         if (!r_ok[n]) continue;
@@ -1280,16 +1339,22 @@ extern "C" int rl_attn_prefill(const void* q, const void* k_cache, const void* v
     if ((long)num_tiles * nkv * nsplit > 0x7fffffffL) return RL_ERR_ARG;
     // the kernel's addresses are page id x elements of a page (32 bits) + an offset in the page
     if ((long)nkv * page_size * D > 0x7fffffffL) return RL_ERR_ARG;
+    // a row of a tile, and what is left of its first, divided by the group's heads: exact where (G + PF_ROWS) G < 2^31
+    const int G = nq / nkv;
+    if (G > 32768) return RL_ERR_ARG;
+    const unsigned group_magic = (unsigned)(((1ull << 31) + G - 1) / G);
     dim3 grid(num_tiles * nkv * nsplit), block(groups * PF_THREADS);
-    auto kernel = groups == 2 ? attn_prefill_kernel<2, false> : attn_prefill_kernel<1, false>;
+    constexpr bool PREPARES = D % 64 == 0;  // (else refused above)
+    auto kernel = prep_q ? (groups == 2 ? attn_prefill_kernel<2, false, PREPARES> : attn_prefill_kernel<1, false, PREPARES>)
+                         : (groups == 2 ? attn_prefill_kernel<2, false, false> : attn_prefill_kernel<1, false, false>);
     if constexpr (PF_DIRECT_OK) {
         if (page_size % 8 == 0)
-            kernel = groups == 2 ? attn_prefill_kernel<2, true> : attn_prefill_kernel<1, true>;
+            kernel = prep_q ? (groups == 2 ? attn_prefill_kernel<2, true, PREPARES> : attn_prefill_kernel<1, true, PREPARES>)
+                            : (groups == 2 ? attn_prefill_kernel<2, true, false> : attn_prefill_kernel<1, true, false>);
     }
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const bf16_t*)q, (const bf16_t*)k_cache,
-                       (const bf16_t*)v_cache, (bf16_t*)out, tile_info, work_order, token_slot,
-                       block_table, table_stride, page_size, page_magic, nq, nkv, window, scale_log2,
-                       nsplit, part_o, part_ml, prep_q ? 1 : 0, ex);
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const bf16_t*)q, tile_info, work_order, block_table,
+                       table_stride, page_magic, page_size, nkv, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
+                       (bf16_t*)out, token_slot, G, group_magic, window, scale_log2, nsplit, part_o, part_ml, ex);
     if (hipGetLastError() != hipSuccess) return RL_ERR_LAUNCH;
     if (nsplit > 1)
         hipLaunchKernelGGL(attn_merge_kernel, dim3(num_prefill_tokens, nq), dim3(D < 64 ? 64 : D), 0,

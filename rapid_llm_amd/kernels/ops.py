@@ -14,6 +14,7 @@ import threading
 import os
 from typing import Optional
 
+import numpy as np
 import torch
 
 from . import build
@@ -2062,7 +2063,7 @@ class AttentionPlan:
     (query heads per kv head): which requests are single tokens (decode kernel) and how the
     portions of the others are cut into row tiles (prefill kernel)."""
 
-    __slots__ = ("num_decode", "_contexts", "_ragged", "seq_token", "max_decode_ctx", "num_tiles", "tile_info", "tile_keys", "orders", "shapes",
+    __slots__ = ("num_decode", "_tiles", "_contexts", "_ragged", "seq_token", "max_decode_ctx", "num_tiles", "tile_info", "tile_keys", "orders", "shapes",
                  "_prefill_tokens", "_prefill_list", "_decode_order")
 
     def __init__(self, ctx, group: int, tile_rows: int) -> None:
@@ -2083,32 +2084,36 @@ class AttentionPlan:
             return
         dec_tokens: list[int] = []
         self._prefill_list, self._prefill_tokens = [], None
-        tile_list: list[tuple[int, int, int, int]] = []
+        tile_list: list[tuple[int, ...]] = []
         self.max_decode_ctx = 0
         contexts: list[int] = []
         at = 0
-        for start, n in zip(ctx.h_seq_starts, ctx.h_seq_lens):
+        slots = getattr(ctx, "h_seq_slots", None) or ()
+        if len(slots) != len(ctx.h_seq_lens):
+            slots = [-1] * len(ctx.h_seq_lens)  # the kernel looks it up
+        for start, n, slot in zip(ctx.h_seq_starts, ctx.h_seq_lens, slots):
             if n == 1:
                 dec_tokens.append(at)
                 self.max_decode_ctx = max(self.max_decode_ctx, start + 1)
                 contexts.append(start + 1)
             else:
                 for row0 in range(0, n * group, tile_rows):
-                    tile_list.append((at, start, n, row0))
+                    tile_list.append((at, start, n, row0, slot, 0, row0 // group, row0 % group))
                 self._prefill_list.extend(range(at, at + n))
             at += n
-        tiles = [v for t in tile_list for v in t]
+        self._tiles = np.asarray(tile_list, dtype=np.int32).reshape(-1, 8)
         # keys each tile reads: what its workgroups cost
         self.tile_keys = [t[1] + min(t[2], (t[3] + tile_rows) // group) for t in tile_list]
         self.orders = {}
         self.shapes = {}
         self.num_decode = len(dec_tokens)
         self._contexts, self._ragged = contexts, None
-        self.num_tiles = len(tiles) // 4
+        self.num_tiles = len(tile_list)
         device = ctx.token_ids.device
-        packed = upload_ints(dec_tokens + tiles, device)
+        pad = -len(dec_tokens) % 8  # a tile's numbers are read as one unit
+        packed = upload_ints(np.concatenate((np.asarray(dec_tokens + [0] * pad, dtype=np.int32), self._tiles.reshape(-1))), device)
         self.seq_token = packed[: self.num_decode]
-        self.tile_info = packed[self.num_decode :]
+        self.tile_info = packed[self.num_decode + pad :]
 
     def prefill_tokens(self, device) -> torch.Tensor:
         """Indices in the step of the tokens that belong to portions (not single tokens)."""
@@ -2140,28 +2145,33 @@ class AttentionPlan:
         """:func:`_prefill_shape` of the step, worked out once for all its layers of a kind."""
         shape = self.shapes.get((nkv, window))
         if shape is None:
-            shape = self.shapes[(nkv, window)] = _prefill_shape(self, nkv, window, tile_rows_of(lib))
+            shape = self.shapes[(nkv, window)] = _prefill_shape(self, nkv, window, tile_rows_of(lib), d=lib.rl_attn_head_dim())
         return shape
 
     def work_order(self, nkv: int, device, resident: int = 1) -> torch.Tensor | None:
-        """Order in which the (tile, kv head) pairs of the prefill kernel are handed out:
-        longest first, so that the short ones fill the gaps at the end.  Where a compute unit
+        """The (tile, kv head) pairs of the prefill kernel in the order in which they are handed out, eight numbers each
+        (the tile's, the kv head in the sixth place): longest first, so that the short ones fill the gaps at the end.  Where a compute unit
         holds two workgroups at a time (``resident == 2``), the first round, one workgroup on
         every unit, takes the longest, and the second round, which joins them on the same
         units, the shortest in ascending order, so that a unit's two workgroups add up alike.  ``None``: in
         the order of their numbers, as where every tile reads as many keys (one short prompt), for which
         the kernel then need not wait."""
         if (nkv, resident) not in self.orders:
-            items = sorted(range(self.num_tiles * nkv), key=lambda i: (-self.tile_keys[i // nkv], i))
+            keys = np.asarray(self.tile_keys, dtype=np.int64)
+            items = (np.argsort(-keys, kind="stable")[:, None] * nkv + np.arange(nkv)).reshape(-1)
             if resident == 2:
                 round_one = chip().first_round
                 first = items[:round_one]
                 rest = items[round_one:]
                 second = rest[::-1][:round_one]
                 middle = rest[: max(0, len(rest) - round_one)]
-                items = first + second + middle
-            listed = items != list(range(len(items)))
-            self.orders[(nkv, resident)] = upload_ints(items, device) if listed else None
+                items = np.concatenate((first, second, middle))
+            work = None
+            if (items != np.arange(items.size)).any():
+                work = self._tiles[items // nkv]
+                work[:, 5] = items % nkv
+                work = upload_ints(work, device)
+            self.orders[(nkv, resident)] = work
         return self.orders[(nkv, resident)]
 
 
@@ -2172,10 +2182,9 @@ class AttentionPlan:
 # time (``Chip.decode_resident``) hands them out longest request first.
 _MIN_SPLIT_KEYS = 128
 _MAX_SPLIT_PAGES = 1024  # page ids of one split are staged in LDS
-# The prefill kernel cuts its tiles' keys into runs when a launch has fewer workgroups than the
-# chip has slots for (``Chip.prefill_slots``) and tiles of at least twice this many keys (a
-# portion of one long prompt).
-_PREFILL_SPLIT_KEYS = 512
+# The prefill kernel may cut its tiles' keys into runs of at least this many when a launch has fewer workgroups than the
+# chip has slots for (``Chip.prefill_slots``): a portion behind a longer context.
+_PREFILL_SPLIT_KEYS = 128
 _PREFILL_MAX_SPLITS = 8
 
 
@@ -2184,46 +2193,63 @@ def tile_rows_of(lib) -> int:
 
 
 _PREFILL_STEP_KEYS = 64  # keys per step of the prefill kernel
-# what a step costs more when the two wave groups of a compute unit walk one tile in lockstep
-# than when they belong to two tiles and drift apart (measured: 3.17 against 2.83 us)
-_PREFILL_PAIRED_COST = 1.12
-# a tile that outlasts the others ends alone on its compute unit and steps faster there than
-# beside a second workgroup (2,048 tokens behind 2,048: 139 us with one wave group a tile,
-# 157 us with two, where whole steps at the shared rate would say 181 against 152)
-_PREFILL_ALONE = 0.8
-# what cutting the tiles' keys into runs costs, in steps: the runs' partial results are
-# written, and read and folded by a second kernel (1,024 tokens from their start: 33 us whole,
-# 47 us in two runs)
-_PREFILL_MERGE_STEPS = 5
+# Microseconds of the prefill kernel at heads of 128 channels, fitted to 86 launches (prompts of 37 to 4,096 tokens, 1 to 16
+# of them, portions of 64 to 1,000 behind 500 to 7,680; groups of two and four query heads); other heads scale all of it.  A
+# workgroup of one wave group: its start, the queries and the results, and a step of 64 keys; what a second one on the same unit
+# adds to that, and to a step if it has as many.  A launch with work for every unit: its start, a workgroup's own share that
+# the other does not hide, a step.  A workgroup of two wave groups (alone on its unit): the same, and what every
+# further one on the same unit costs beside its steps.
+_PREFILL_ONE, _PREFILL_ONE_STEP, _PREFILL_BESIDE, _PREFILL_BESIDE_STEP = 7.6, 1.63, 4.4, 0.3
+_PREFILL_FULL, _PREFILL_FULL_ITEM, _PREFILL_FULL_STEP = 4.0, 5.2, 0.99
+_PREFILL_TWO, _PREFILL_TWO_STEP, _PREFILL_TWO_ITEM = 8.4, 1.27, 7.2
+# what cutting the keys into runs costs: the runs' partial results are written, and read and folded by a second kernel
+_PREFILL_MERGE, _PREFILL_MERGE_BYTE = 2.0, 0.5e-6
 
 
 def _prefill_shape(plan: "AttentionPlan", nkv: int, window: int, tile_rows: int,
-                   units: int | None = None) -> tuple[int, int]:
+                   units: int | None = None, d: int = 128) -> tuple[int, int]:
     """(wave groups per workgroup, runs the keys of every tile are cut into) for a launch of
-    the prefill kernel, from an estimate of the launch's length in steps: the longest tile's
-    steps (halved where two wave groups share it, divided where its keys are cut into runs) or
-    the steps there are for every slot of the chip, whichever is more.  Few, long tiles (a
-    portion of one long prompt) come out with their keys cut into runs, folded by the merge
+    the prefill kernel, from an estimate of the launch's time: its longest workgroup (half the steps where two wave groups
+    share a tile, fewer where its keys are cut into runs) or the work there is for every unit, whichever is more.  Few, long
+    tiles (a portion of one long prompt) come out with their keys cut into runs, folded by the merge
     kernel; a prompt from its start, whose last rows alone see many keys, with two wave groups
-    a tile; a launch with work for every slot with neither."""
-    slots = (chip() if units is None else Chip(units)).prefill_slots
+    a tile while no unit gets many of them; a launch with work for every slot with neither.
+
+    Microseconds in one wave group / two / runs, the one taken last: one prompt of 2,048 tokens of 32 query heads 66.6 / 58.7,
+    four of 512 26.8 / 30.8, eight of 300 29.7 / 36.9; with 16 query heads one of 1,536 tokens 46.4 / 37.6 / 47.0, 64 tokens behind
+    2,000 58.9 / 46.5 / 20.2, four times 300 behind 2,000 73.5 / 56.9 / 53.2."""
+    chip_ = chip() if units is None else Chip(units)
+    units, slots = chip_.units, chip_.prefill_slots
     keys = plan.tile_keys
     if window > 0:
         keys = [min(k, window + tile_rows) for k in keys]
     items = plan.num_tiles * nkv
     steps = [-(-k // _PREFILL_STEP_KEYS) for k in keys]
     longest = max(steps)
-    share = nkv * sum(steps) / slots  # steps per slot if the work were spread evenly
-    best = (max(longest * _PREFILL_ALONE, share), 1, 1)
-    paired = max(-(-longest // 2), share) * _PREFILL_PAIRED_COST
-    if paired < best[0]:
-        best = (paired, 2, 1)
+    share = nkv * sum(steps) / units  # steps a unit if the work were spread evenly
+    even = (sum(steps) / (len(steps) * longest)) ** 2
+
+    def one(runs: int) -> float:
+        start, step = _PREFILL_ONE, _PREFILL_ONE_STEP
+        if items * runs > units:
+            start, step = start + _PREFILL_BESIDE, step + _PREFILL_BESIDE_STEP * even
+        return max(start + step * -(-longest // runs),
+                   _PREFILL_FULL + _PREFILL_FULL_ITEM * items * runs / units + _PREFILL_FULL_STEP * share)
+
+    best = (one(1), 1, 1)
+    two = _PREFILL_TWO + min(0.4 * (d / 128 - 1), 0.0) + _PREFILL_TWO_STEP * longest
+    if items > units:
+        rounds = -(-items // units)  # (workgroups of one length end together, and a round that is not full takes as long)
+        two = max(two, 2.0 + _PREFILL_TWO_ITEM * rounds + _PREFILL_TWO_STEP * share * (1.0 + even * (rounds * units / items - 1.0)))
+    if two < best[0]:
+        best = (two, 2, 1)
+    merged = _PREFILL_MERGE_BYTE * items * tile_rows * d * 4 / (0.55 + 0.45 * d / 128)  # (a step of 16 channels takes 0.6 of one of 128)
     if items < slots:
         most = min(_PREFILL_MAX_SPLITS, -(-slots // items), max(keys) // _PREFILL_SPLIT_KEYS)
-        for nsplit in range(2, most + 1):
-            cost = max(-(-longest // nsplit), share) + _PREFILL_MERGE_STEPS
+        for runs in range(2, most + 1):
+            cost = one(runs) + _PREFILL_MERGE + merged * runs
             if cost < best[0]:
-                best = (cost, 1, nsplit)
+                best = (cost, 1, runs)
     return best[1], best[2]
 
 
