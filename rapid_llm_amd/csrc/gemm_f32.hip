@@ -118,6 +118,22 @@ __device__ inline float finite_or_wide(float v, const float* a, const float* w, 
     return __builtin_isfinite(v) ? v * DOWN : wide_sum(a, w, K);
 }
 
+// GLU: W is a gate and an up matrix, N rows each, one behind the other, and a result is silu(gate) * up of the two
+// products.  Sixteen rows of a tile are the gate and up rows of eight columns, two and two in turn, so that a lane's four
+// results are two columns' pairs, whatever the tile.  The bits are those of the product and the activation's kernel one after
+// the other, which the results, twice as many, went through memory for: microseconds of a step before / with this, 0.6B
+// three prompts of 225 tokens 3,602 / 3,457, 8B a prompt of 2,048 140,050 / 138,250, eight requests decode 7,367 / 7,174.
+template <bool GLU>
+__device__ inline size_t row_of(int slot, int N) {
+    if (!GLU) return min(slot, N - 1);
+    const int col = (slot >> 4) * 8 + ((slot >> 1) & 6) + (slot & 1);
+    return (size_t)min(col, N - 1) + (slot & 2 ? N : 0);
+}
+__device__ inline float silu_mul(float g, float u) {
+    const Glu plain = {0.f, 0.f, 0, nullptr};
+    return glu_act(g, u, plain);
+}
+
 // 16 bytes from any address of a float: rows may begin anywhere (the hardware asks for 4-byte alignment)
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 __device__ inline f32x4 load4(const float* p) { return *reinterpret_cast<const f32x4u*>(p); }
@@ -154,7 +170,7 @@ __device__ inline f32x4 load_k4(const float* p, int at, int before, int K) {
 // (f32_plan says when NT is 2 or 3), with two for 17 to 32 rows over short ones and for any number of rows over at
 // most 256 k, where a wave has one chunk and the shared tiles below walk a chain of chunks or leave the runs to a second
 // kernel: 17 rows over 6,144 x 1,024 14.6 -> 11.5 us, over 1,024 x 128 6.0 -> 3.3, 225 rows 8.4 -> 4.4.
-template <int NT, int MT>
+template <int NT, int MT, bool GLU>
 __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_stream_kernel(
     const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
     int K, int lda, int ldw, int ldc) {
@@ -169,7 +185,7 @@ __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_stream_kernel(
     // rows beyond the matrices read the last row; their results are dropped at the end
     const float* wrow[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) wrow[nt] = W + (size_t)min(n0 + nt * 16 + r16, N - 1) * ldw + 8 * g;
+    for (int nt = 0; nt < NT; ++nt) wrow[nt] = W + row_of<GLU>(n0 + nt * 16 + r16, N) * ldw + 8 * g;
     const float* arow[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) arow[mt] = A + (size_t)min(m0 + mt * 16 + r16, M - 1) * lda + 8 * g;
@@ -288,6 +304,24 @@ __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_stream_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) red[wave][((nt * MT + mt) * 4 + i) * 64 + lane] = acc[nt][mt][i];
     __syncthreads();
+    if constexpr (GLU) {
+        for (int i = threadIdx.x; i < NT * MT * 128; i += FRUNS * RL_WAVE) {
+            const int ln = i & 63, tile = i >> 7, j = (i >> 6) & 1, e = tile * 256 + j * 64 + ln;
+            const int n = (n0 + tile / MT * 16) / 2 + 2 * (ln >> 4) + j;
+            const int m = m0 + tile % MT * 16 + (ln & 15);
+            if (n >= N || m >= M) continue;
+            float v[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                v[h] = red[0][e + 128 * h];
+#pragma unroll
+                for (int w = 1; w < FRUNS; ++w) v[h] = w & 1 ? v[h] - red[w][e + 128 * h] : v[h] + red[w][e + 128 * h];
+                v[h] = finite_or_wide(v[h], A + (size_t)m * lda, W + ((size_t)n + (h ? N : 0)) * ldw, K);
+            }
+            C[(size_t)m * ldc + n] = silu_mul(v[0], v[1]);
+        }
+        return;
+    }
     for (int e = threadIdx.x; e < NT * MT * 256; e += FRUNS * RL_WAVE) {
         const int ln = e & 63, tile = e >> 8;
         const int n = n0 + tile / MT * 16 + 4 * (ln >> 4) + ((e >> 6) & 3);
@@ -300,6 +334,54 @@ __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_stream_kernel(
     }
 }
 
+// The pairs of a wave's TN x TM blocks; row(y) and col(x): the lane's row, its first of two columns.  The few that are not
+// finite stand behind, once.
+template <int TN, int TM, typename ROW, typename COL>
+__device__ __forceinline__ void gated_results(const f32x4 (&total)[TN][TM], float* C, const float* A, const float* W, int M, int N, int K,
+                                              int lda, int ldw, int ldc, ROW row, COL col) {
+    uint32_t wide = 0;
+    static_assert(TN * TM * 2 <= 32, "a bit a pair");
+    const bool pairs = (ldc & 1) == 0 && (reinterpret_cast<uintptr_t>(C) & 7) == 0;
+#pragma unroll
+    for (int x = 0; x < TN; ++x)
+#pragma unroll
+        for (int y = 0; y < TM; ++y) {
+            const int m = row(y), n = col(x);
+            if (m >= M) continue;
+            f32x2 v;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float gate = total[x][y][j], up = total[x][y][2 + j];
+                if (!__builtin_isfinite(gate) || !__builtin_isfinite(up)) wide |= 1u << ((x * TM + y) * 2 + j);
+                v[j] = silu_mul(gate * DOWN, up * DOWN);
+            }
+            float* out = C + (size_t)m * ldc + n;
+            if (pairs && n + 1 < N) {
+                *reinterpret_cast<f32x2*>(out) = v;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    if (n + j < N) out[j] = v[j];
+            }
+        }
+    while (wide) {
+        const int e = __ffs(wide) - 1;
+        wide &= wide - 1;
+        float gate = 0.f, up = 0.f;
+        int m = 0, n = 0;
+#pragma unroll
+        for (int x = 0; x < TN; ++x)
+#pragma unroll
+            for (int y = 0; y < TM; ++y)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    if (e == (x * TM + y) * 2 + j) gate = total[x][y][j], up = total[x][y][2 + j], m = row(y), n = col(x) + j;
+        if (n >= N) continue;
+        const float* a = A + (size_t)m * lda;
+        C[(size_t)m * ldc + n] = silu_mul(finite_or_wide(gate, a, W + (size_t)n * ldw, K), finite_or_wide(up, a, W + ((size_t)n + N) * ldw, K));
+    }
+}
+
 // ---- more rows: tiles whose operands are split once and shared through LDS ---------------------
 // A workgroup of four waves owns 32 TM x 32 TN results, a wave 16 TM x 16 TN of them.  A chunk's rows of
 // A and W travel through registers, where they are split, into LDS in the order in which the matrix
@@ -308,7 +390,7 @@ __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_stream_kernel(
 // cover each other's barriers and the next chunk's rows are asked for before this one is multiplied.
 // Small ones, whose chunks are short: LDS holds two chunks (one barrier a chunk), and three chunks' rows
 // are on their way.
-template <int TM, int TN, Length L, bool RUNS>
+template <int TM, int TN, Length L, bool RUNS, bool GLU>
 __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(
     const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
     int K, int lda, int ldw, int ldc, int tiles_m, int tiles_n, int runs) {
@@ -349,7 +431,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(
 #pragma unroll
     for (int i = 0; i < PW; ++i) {
         const int row = (threadIdx.x >> 2) + 64 * i;
-        from_w[i] = W + (size_t)min(n0 + row, N - 1) * ldw + 8 * piece;
+        from_w[i] = W + row_of<GLU>(n0 + row, N) * ldw + 8 * piece;
         to_w[i] = place(row);
     }
     const int wm = (wave & 1) * TM, wn = (wave >> 1) * TN;  // the wave's first 16-row blocks
@@ -491,6 +573,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(
     }
     while (run < run_hi) finish_run();  // runs without a chunk: zeros
     if (RUNS) return;
+    if constexpr (GLU) {
+        gated_results<TN, TM>(total, C, A, W, M, N, K, lda, ldw, ldc, [&](int y) { return m0 + (wm + y) * 16 + r16; },
+                              [&](int x) { return (n0 + (wn + x) * 16) / 2 + 2 * g; });
+        return;
+    }
     // which of the lane's results are not finite: they are few or none, so their sums stand behind, once
     uint64_t wide = 0;
     const bool pieces = (ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
@@ -604,7 +691,7 @@ __device__ __forceinline__ void read_a2(bf16x8 (&a)[2][3], uint32_t at) {
 // Microseconds at 2,048 rows, the tiles of 128 x 128 / this with A's pieces made: 6,144 x 4,096 521 / 453, 4,096 x 4,096
 // 326 / 279, 24,576 x 4,096 1,957 / 1,624, 4,096 x 12,288 1,006 / 817.  TN = 3 is for matrices whose tiles of
 // 128 columns leave a short last round (ops.f32_wide has the rule).
-template <int TN>
+template <int TN, bool GLU>
 __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restrict__ A, const __bf16* __restrict__ P,
                                                             const float* __restrict__ W, float* __restrict__ C, int M,
                                                             int N, int K, int lda, int ldw, int ldc, int tiles_m,
@@ -651,7 +738,7 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
     // W: 8 k of a row a thread, through registers (where the rows are fewer, the last threads carry what others do:
     // every wave has the same loads on their way)
     const int piece = tid & 3, row = (tid >> 2) < BN ? tid >> 2 : (tid >> 2) - 32;
-    const float* from_w = W + (size_t)min(n0 + row, N - 1) * ldw + 8 * piece;
+    const float* from_w = W + row_of<GLU>(n0 + row, N) * ldw + 8 * piece;
     unsigned char* to_w = lds + 2 * WIDE_A + (row >> 4) * 1024 + (piece * 16 + ((row & 15) ^ (2 * piece))) * 16;
     f32x4 raw[2];
     auto load_w = [&](int c) {
@@ -740,6 +827,11 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
     wait_loads<0>();  // nothing may still be on its way into LDS when it is given back
     if (wave < 4) __builtin_amdgcn_s_barrier();
 
+    if constexpr (GLU) {
+        gated_results<TN, 4>(total, C, A, W, M, N, K, lda, ldw, ldc, [&](int y) { return m0 + wm * 64 + y * 16 + r16; },
+                             [&](int x) { return (n0 + (wn * TN + x) * 16) / 2 + 2 * g; });
+        return;
+    }
     uint64_t wide = 0;
     const bool whole = (ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
 #pragma unroll
@@ -773,19 +865,29 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
 }
 
 // the runs of the tile kernel added in their order
+template <bool GLU>
 __global__ __launch_bounds__(256) void gemm_f32_add_runs_kernel(
     const float* __restrict__ parts, const float* __restrict__ A, const float* __restrict__ W,
     float* __restrict__ C, int M, int N, int K, int lda, int ldw, int ldc) {
     const int m = blockIdx.y;
     const int n = blockIdx.x * 256 + threadIdx.x;
-    if (n >= N) return;
-    float v = parts[(size_t)m * N + n];
+    if (n >= (GLU ? N / 2 : N)) return;  // (a gated product's parts hold the gate's and up's columns)
+    float run[GLU ? 2 : 1][FRUNS], v[GLU ? 2 : 1];
 #pragma unroll
-    for (int r = 1; r < FRUNS; ++r) {
-        const float x = parts[((size_t)r * M + m) * N + n];
-        v = r & 1 ? v - x : v + x;
+    for (int h = 0; h < (GLU ? 2 : 1); ++h)
+#pragma unroll
+        for (int r = 0; r < FRUNS; ++r) run[h][r] = parts[((size_t)r * M + m) * N + n + h * (N / 2)];
+#pragma unroll
+    for (int h = 0; h < (GLU ? 2 : 1); ++h) {
+        v[h] = run[h][0];
+#pragma unroll
+        for (int r = 1; r < FRUNS; ++r) v[h] = r & 1 ? v[h] - run[h][r] : v[h] + run[h][r];
+        v[h] = finite_or_wide(v[h], A + (size_t)m * lda, W + ((size_t)n + h * (N / 2)) * ldw, K);
     }
-    C[(size_t)m * ldc + n] = finite_or_wide(v, A + (size_t)m * lda, W + (size_t)n * ldw, K);
+    if constexpr (GLU)
+        C[(size_t)m * ldc + n] = silu_mul(v[0], v[1]);
+    else
+        C[(size_t)m * ldc + n] = v[0];
 }
 
 // The same sums where a norm follows: added to the residual in place (with the product's bias, where it has one), whose rows
@@ -865,46 +967,92 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
     }
 }
 
-template <int NT>
+// 16-row blocks of W of a product of N result columns
+template <bool GLU>
+static int w_blocks(int N) {
+    return GLU ? (N + 7) / 8 : (N + 15) / 16;
+}
+
+template <int NT, bool GLU>
 static int launch_stream(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw,
                          int ldc, hipStream_t stream) {
     const int mt = M <= 16 ? 1 : 2;
-    const dim3 grid((N + 16 * NT - 1) / (16 * NT), (M + 16 * mt - 1) / (16 * mt)), block(FRUNS * RL_WAVE);
+    const dim3 grid((w_blocks<GLU>(N) + NT - 1) / NT, (M + 16 * mt - 1) / (16 * mt)), block(FRUNS * RL_WAVE);
     if (grid.y > 65535) return RL_ERR_ARG;
     if (mt == 1)
-        hipLaunchKernelGGL((gemm_f32_stream_kernel<NT, 1>), grid, block, 0, stream, A, W, C, M, N, K, lda, ldw, ldc);
+        hipLaunchKernelGGL((gemm_f32_stream_kernel<NT, 1, GLU>), grid, block, 0, stream, A, W, C, M, N, K, lda, ldw, ldc);
     else
-        hipLaunchKernelGGL((gemm_f32_stream_kernel<NT, 2>), grid, block, 0, stream, A, W, C, M, N, K, lda, ldw, ldc);
+        hipLaunchKernelGGL((gemm_f32_stream_kernel<NT, 2, GLU>), grid, block, 0, stream, A, W, C, M, N, K, lda, ldw, ldc);
     return rl_launch_status();
 }
 
-template <int TM, int TN, Length L>
+template <int TM, int TN, Length L, bool GLU>
 static int launch_tile_of(const float* A, const float* W, float* C, float* parts, int M, int N, int K, int lda,
                        int ldw, int ldc, int groups, hipStream_t stream) {
-    const int tm = (M + 32 * TM - 1) / (32 * TM), tn = (N + 32 * TN - 1) / (32 * TN);
-    if ((long long)tm * tn > 0x7fffffffLL / 16) return RL_ERR_ARG;
+    const int tm = (M + 32 * TM - 1) / (32 * TM);
     const dim3 block(256);
     if (groups == 1) {
-        hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TN, L, false>), dim3(tm * tn), block, 0, stream, A, W, C, M, N,
+        const int tn = (w_blocks<GLU>(N) + 2 * TN - 1) / (2 * TN);
+        if ((long long)tm * tn > 0x7fffffffLL / 16) return RL_ERR_ARG;
+        hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TN, L, false, GLU>), dim3(tm * tn), block, 0, stream, A, W, C, M, N,
                            K, lda, ldw, ldc, tm, tn, FRUNS);
         return rl_launch_status();
     }
+    const int rows = GLU ? 2 * N : N, tn = (rows + 32 * TN - 1) / (32 * TN);  // (the runs are those of the plain product)
+    if ((long long)tm * tn > 0x7fffffffLL / 16) return RL_ERR_ARG;
     if (!parts || M > 65535) return RL_ERR_ARG;
-    hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TN, L, true>), dim3(tm * tn, groups), block, 0, stream, A, W, parts,
-                       M, N, K, lda, ldw, ldc, tm, tn, FRUNS / groups);
+    hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TN, L, true, false>), dim3(tm * tn, groups), block, 0, stream, A, W, parts,
+                       M, rows, K, lda, ldw, ldc, tm, tn, FRUNS / groups);
     if (int code = rl_launch_status()) return code;
     if (!C) return RL_OK;  // (rl_gemm_f32_add_rmsnorm adds them)
-    hipLaunchKernelGGL(gemm_f32_add_runs_kernel, dim3((N + 255) / 256, M), block, 0, stream, parts, A, W, C, M, N,
+    hipLaunchKernelGGL(gemm_f32_add_runs_kernel<GLU>, dim3((N + 255) / 256, M), block, 0, stream, parts, A, W, C, M, rows,
                        K, lda, ldw, ldc);
     return rl_launch_status();
 }
 
-template <int TM, int TN>
+template <int TM, int TN, bool GLU = false>
 static int launch_tile(const float* A, const float* W, float* C, float* parts, int M, int N, int K, int lda,
                        int ldw, int ldc, int groups, hipStream_t stream) {
-    if (K % 4) return launch_tile_of<TM, TN, ELEMENTS>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
-    if (K % FCH) return launch_tile_of<TM, TN, PIECES>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
-    return launch_tile_of<TM, TN, WHOLE>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
+    if (K % 4) return launch_tile_of<TM, TN, ELEMENTS, GLU>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
+    if (K % FCH) return launch_tile_of<TM, TN, PIECES, GLU>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
+    return launch_tile_of<TM, TN, WHOLE, GLU>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
+}
+
+template <bool GLU>
+static int launch_product(const float* A, const float* W, float* C, float* parts, int M, int N, int K, int lda,
+                          int ldw, int ldc, int tile, int groups, hipStream_t stream) {
+    if (tile <= 3) {
+        if (groups != 1) return RL_ERR_ARG;
+        if (tile == 1) return launch_stream<1, GLU>(A, W, C, M, N, K, lda, ldw, ldc, stream);
+        if (tile == 2) return launch_stream<2, GLU>(A, W, C, M, N, K, lda, ldw, ldc, stream);
+        if (tile == 3) return launch_stream<3, GLU>(A, W, C, M, N, K, lda, ldw, ldc, stream);
+        return RL_ERR_ARG;
+    }
+    if (tile == 32) return launch_tile<1, 2, GLU>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
+    if (tile == 64) return launch_tile<2, 2, GLU>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
+    if (tile == 128) return launch_tile<4, 4, GLU>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
+    return RL_ERR_ARG;
+}
+
+template <bool GLU>
+static int launch_wide(const float* A, const float* W, float* C, void* pieces, int M, int N, int K, int lda,
+                       int ldw, int ldc, int cols, hipStream_t stream) {
+    const int chunks = K / FCH, blocks = (M + 15) / 16;
+    if (!pieces || (uintptr_t)pieces % 16 || K <= 0 || K % FCH || lda < K || ldw < K || ldc < N || (cols != 128 && cols != 96))
+        return RL_ERR_ARG;
+    const int tm = (M + 255) / 256, tn = (w_blocks<GLU>(N) + cols / 16 - 1) / (cols / 16);
+    // the pieces of a tile are addressed with 32 bits
+    if (K > 1 << 20 || blocks > 65535 || (long long)tm * tn > 0x7fffffffLL / 16) return RL_ERR_ARG;
+    hipLaunchKernelGGL(gemm_f32_pieces_kernel, dim3((chunks + 3) / 4, blocks), dim3(256), 0, stream, A, (__bf16*)pieces, M,
+                       chunks, lda, (chunks + FRUNS - 1) / FRUNS);
+    if (int code = rl_launch_status()) return code;
+    if (cols == 128)
+        hipLaunchKernelGGL((gemm_f32_wide_kernel<4, GLU>), dim3(tm * tn), dim3(512), 0, stream, A, (const __bf16*)pieces, W, C,
+                           M, N, K, lda, ldw, ldc, tm, tn);
+    else
+        hipLaunchKernelGGL((gemm_f32_wide_kernel<3, GLU>), dim3(tm * tn), dim3(512), 0, stream, A, (const __bf16*)pieces, W, C,
+                           M, N, K, lda, ldw, ldc, tm, tn);
+    return rl_launch_status();
 }
 
 // Rows of A and W may be strided; the inner dimension is contiguous.  `tile`: 1, 2 and 3 stream the
@@ -921,17 +1069,16 @@ extern "C" int rl_gemm_f32(const float* A, const float* W, float* C, float* part
                            C, M, N, K, lda, ldw, ldc);
         return rl_launch_status();
     }
-    if (tile <= 3) {
-        if (groups != 1) return RL_ERR_ARG;
-        if (tile == 1) return launch_stream<1>(A, W, C, M, N, K, lda, ldw, ldc, stream);
-        if (tile == 2) return launch_stream<2>(A, W, C, M, N, K, lda, ldw, ldc, stream);
-        if (tile == 3) return launch_stream<3>(A, W, C, M, N, K, lda, ldw, ldc, stream);
-        return RL_ERR_ARG;
-    }
-    if (tile == 32) return launch_tile<1, 2>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
-    if (tile == 64) return launch_tile<2, 2>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
-    if (tile == 128) return launch_tile<4, 4>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
-    return RL_ERR_ARG;
+    return launch_product<false>(A, W, C, parts, M, N, K, lda, ldw, ldc, tile, groups, stream);
+}
+
+// The same with silu(gate) * up of the packed [gate | up] matrix W[2 N, K]; `parts` [8, M, 2 N].
+extern "C" int rl_gemm_f32_gated(const float* A, const float* W, float* C, float* parts, int M, int N, int K, int lda,
+                                 int ldw, int ldc, int tile, int groups, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return RL_OK;
+    if (K <= FEW || lda < K || ldw < K || ldc < N || !C || N > 0x3fffffff) return RL_ERR_ARG;
+    if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return RL_ERR_ARG;
+    return launch_product<true>(A, W, C, parts, M, N, K, lda, ldw, ldc, tile, groups, stream);
 }
 
 // The same for many rows and K a multiple of 32: `pieces` holds 96 K bytes for every 16 rows of A; `cols` (128 or 96) are
@@ -939,22 +1086,14 @@ extern "C" int rl_gemm_f32(const float* A, const float* W, float* C, float* part
 extern "C" int rl_gemm_f32_wide(const float* A, const float* W, float* C, void* pieces, int M, int N, int K, int lda,
                                 int ldw, int ldc, int cols, hipStream_t stream) {
     if (M <= 0 || N <= 0) return RL_OK;
-    const int chunks = K / FCH, blocks = (M + 15) / 16;
-    if (!pieces || (uintptr_t)pieces % 16 || K <= 0 || K % FCH || lda < K || ldw < K || ldc < N || (cols != 128 && cols != 96))
-        return RL_ERR_ARG;
-    const int tm = (M + 255) / 256, tn = (N + cols - 1) / cols;
-    // the pieces of a tile are addressed with 32 bits
-    if (K > 1 << 20 || blocks > 65535 || (long long)tm * tn > 0x7fffffffLL / 16) return RL_ERR_ARG;
-    hipLaunchKernelGGL(gemm_f32_pieces_kernel, dim3((chunks + 3) / 4, blocks), dim3(256), 0, stream, A, (__bf16*)pieces, M,
-                       chunks, lda, (chunks + FRUNS - 1) / FRUNS);
-    if (int code = rl_launch_status()) return code;
-    if (cols == 128)
-        hipLaunchKernelGGL(gemm_f32_wide_kernel<4>, dim3(tm * tn), dim3(512), 0, stream, A, (const __bf16*)pieces, W, C, M, N,
-                           K, lda, ldw, ldc, tm, tn);
-    else
-        hipLaunchKernelGGL(gemm_f32_wide_kernel<3>, dim3(tm * tn), dim3(512), 0, stream, A, (const __bf16*)pieces, W, C, M, N,
-                           K, lda, ldw, ldc, tm, tn);
-    return rl_launch_status();
+    return launch_wide<false>(A, W, C, pieces, M, N, K, lda, ldw, ldc, cols, stream);
+}
+
+extern "C" int rl_gemm_f32_wide_gated(const float* A, const float* W, float* C, void* pieces, int M, int N, int K, int lda,
+                                      int ldw, int ldc, int cols, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return RL_OK;
+    if (N > 0x3fffffff) return RL_ERR_ARG;
+    return launch_wide<true>(A, W, C, pieces, M, N, K, lda, ldw, ldc, cols, stream);
 }
 
 // residual[M, N] += A W^T (+ bias) in place and out[M, N] = rmsnorm(residual) * weight, where f32_plan cuts the product into

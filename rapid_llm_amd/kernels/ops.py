@@ -1160,27 +1160,49 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
     n, k2 = w.shape
     if k != k2 or out.shape != (m, n):
         raise KernelError(f"gemm_f32 shapes do not agree: a {tuple(a.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)}")
-    cols = f32_wide(m, n, k, chip().units)
+    _f32_product(a, w, out, n, False)
+
+
+def gemm_f32_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor | None:
+    """``silu(x Wg^T) * (x Wu^T)`` for the packed ``[gate | up]`` matrix in float32, by the product's own kernels and with the bits
+    of :func:`gemm_f32` and :func:`swiglu`; ``None`` for sums of a few products, which have a kernel without it."""
+    for t, name in ((x, "x"), (w_gate_up, "w_gate_up")):
+        if not t.is_cuda or t.dtype != torch.float32 or t.dim() != 2 or t.stride(1) != 1:
+            raise KernelError(f"gemm_f32 operand {name} must be a float32 GPU matrix with unit inner stride")
+    m, k = x.shape
+    two_i = w_gate_up.shape[0]
+    if k != w_gate_up.shape[1] or two_i % 2:
+        raise KernelError(f"gemm_f32_swiglu shapes do not agree: x {tuple(x.shape)}, w {tuple(w_gate_up.shape)}")
+    if k < 4 or two_i < 2:
+        return None
+    out = torch.empty((m, two_i // 2), dtype=torch.float32, device=x.device)
+    _f32_product(x, w_gate_up, out, two_i, True)
+    return out
+
+
+def _f32_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows_of_w: int, gated: bool) -> None:
+    """The launches of :func:`gemm_f32` or of its gated form, laid out for so many rows of ``w``."""
+    m, k = a.shape
+    n = out.shape[1]
+    strides = (a.stride(0), w.stride(0), out.stride(0))
+    cols = f32_wide(m, rows_of_w, k, chip().units)
     if cols:
         rows = _f32_piece_rows(m, k)
         pieces = torch.empty(96 * k * -(-min(m, rows) // 16), dtype=torch.uint8, device=a.device)
         for lo in range(0, m, rows):
-            _ok(
-                core().rl_gemm_f32_wide(
-                    _p(a[lo:]), _p(w), _p(out[lo:]), _p(pieces), min(rows, m - lo), n, k, a.stride(0), w.stride(0), out.stride(0), cols,
-                    _stream()
-                ),
-                "rl_gemm_f32_wide",
-            )
+            args = (_p(a[lo:]), _p(w), _p(out[lo:]), _p(pieces), min(rows, m - lo), n, k, *strides, cols, _stream())
+            if gated:
+                _ok(core().rl_gemm_f32_wide_gated(*args), "rl_gemm_f32_wide_gated")
+            else:
+                _ok(core().rl_gemm_f32_wide(*args), "rl_gemm_f32_wide")
         return
-    tile, groups = f32_plan(m, n, k, chip().units)
-    parts = torch.empty((8, m, n), dtype=torch.float32, device=a.device) if groups > 1 else None
-    _ok(
-        core().rl_gemm_f32(
-            _p(a), _p(w), _p(out), _p(parts), m, n, k, a.stride(0), w.stride(0), out.stride(0), tile, groups, _stream()
-        ),
-        "rl_gemm_f32",
-    )
+    tile, groups = f32_plan(m, rows_of_w, k, chip().units)
+    parts = torch.empty((8, m, rows_of_w), dtype=torch.float32, device=a.device) if groups > 1 else None
+    args = (_p(a), _p(w), _p(out), _p(parts), m, n, k, *strides, tile, groups, _stream())
+    if gated:
+        _ok(core().rl_gemm_f32_gated(*args), "rl_gemm_f32_gated")
+    else:
+        _ok(core().rl_gemm_f32(*args), "rl_gemm_f32")
 
 
 def f32_runs(m: int, n: int, k: int) -> bool:

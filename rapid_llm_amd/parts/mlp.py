@@ -111,6 +111,10 @@ class SwiGLU(FeedForward):
                    else ops.gemm_bf16_swiglu(x, w, **glu))
             if act is not None:
                 return self.down.deferred(act, ctx)
+        if w.dtype == torch.float32 and x.dtype == torch.float32 and self.activation == "silu" and not self.limit and not self.has_bias:
+            act = ops.gemm_f32_swiglu(x, w)
+            if act is not None:
+                return self.down.deferred(act, ctx)
         gu = self.gate_up(x)
         act = torch.empty((x.shape[0], self.intermediate_size), dtype=gu.dtype, device=x.device)
         ops.swiglu(gu, act, self.limit, self.alpha, activation=self.activation, bias=self.gate_up_bias)

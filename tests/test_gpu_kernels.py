@@ -796,6 +796,33 @@ def test_gemm_f32_for_many_rows(shape, cols):
     torch.testing.assert_close(out[:, :n], want, rtol=0, atol=0, equal_nan=True)
 
 
+@pytest.mark.parametrize("tile,groups", [(1, 1), (2, 1), (3, 1), (32, 1), (32, 8), (64, 1), (64, 4), (128, 1), (128, 2), (128, 0), (96, 0)])
+@pytest.mark.parametrize("m,inter,k", [(1, 24, 64), (16, 40, 36), (33, 100, 4), (129, 203, 288), (257, 136, 1056), (40, 1, 333)])
+def test_gemm_f32_gated(m, inter, k, tile, groups):
+    """The float32 product with silu(gate) * up behind it, in every kernel that makes it (groups 0: the many-row kernel): the
+    bits of the product and the activation one after the other, also where a gate or an up value has no finite pieces,
+    for columns that end inside a pair, a block and a tile, and nothing behind the results."""
+    ops = _ops()
+    if groups == 0 and k % 32:
+        pytest.skip("the many-row kernel takes sums of a multiple of 32")
+    gen = torch.Generator().manual_seed(m + inter)
+    a, w = torch.randn(m, k, generator=gen).to(DEV), torch.randn(2 * inter, k, generator=gen).to(DEV)
+    a[m // 2, k // 2], w[inter // 2, k - 1], w[inter + inter // 3, 0] = float("inf"), 2.0**104, -(2.0**110)
+    gate_up, want = torch.empty((m, 2 * inter), device=DEV), torch.empty((m, inter), device=DEV)
+    ops.gemm_f32(a, w, gate_up)
+    ops.swiglu(gate_up, want)
+    out = torch.full((m, inter + 3), 7.0, device=DEV)
+    parts, pieces = torch.empty((8, m, 2 * inter), device=DEV), torch.empty(96 * k * -(-m // 16), dtype=torch.uint8, device=DEV)
+    lib, p = ops.core(), ops._p
+    if groups:
+        code = lib.rl_gemm_f32_gated(p(a), p(w), p(out), p(parts), m, inter, k, k, k, inter + 3, tile, groups, ops._stream())
+    else:
+        code = lib.rl_gemm_f32_wide_gated(p(a), p(w), p(out), p(pieces), m, inter, k, k, k, inter + 3, tile, ops._stream())
+    assert code == 0 and bool((out[:, inter:] == 7.0).all())
+    torch.testing.assert_close(out[:, :inter], want, rtol=0, atol=0, equal_nan=True)
+    torch.testing.assert_close(ops.gemm_f32_swiglu(a, w), want, rtol=0, atol=0, equal_nan=True)
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 1024, 1000), (64, 4096, 288), (225, 1024, 3072), (300, 2052, 2048), (130, 4100, 4096)])
 def test_gemm_f32_whose_runs_the_norm_adds(m, n, k):
     """Every tile and sharing: the bits of the product, its bias and the norm as kernels of their own, an infinite row too."""
