@@ -49,6 +49,7 @@ CORE_SOURCES = (
     "gemm_bf16.hip",
     "gemm_rows.hip",
     "gemm_block.hip",
+    "gemm_pair.hip",
     "repeat.hip",
     "latent.hip",
     "router.hip",

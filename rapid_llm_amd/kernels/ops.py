@@ -1499,6 +1499,9 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, scaled=N
     x = whole_rows(x)
     if scaled is not None:
         raise KernelError(f"scaled rows need the few-row product: {m} rows over {k}")
+    halves = pair(m, n, k, "plain") if out_dtype == torch.bfloat16 else None
+    if halves is not None and _aligned(x, w):
+        return _pair(x, w, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), "plain", halves)
     plan = rows_plan(m, n, k, swiglu=False) if m <= ROWS_MAX_ROWS else None
     if _tile_applies(m, n, k, n) and not (plan is not None and k >= 512 and out_dtype == torch.bfloat16 and _aligned(x, w)):
         out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
@@ -1531,7 +1534,8 @@ def library_takes(m: int, n: int, k: int) -> bool:
         return False
     if m <= ROWS_MAX_ROWS and rows_plan(m, n, k, swiglu=False) is not None:
         return False
-    return not _tile_applies(m, n, k, n) and block_plain_plan(m, n, k, chip().units) is None
+    return (not _tile_applies(m, n, k, n) and pair(m, n, k, "plain") is None
+            and block_plain_plan(m, n, k, chip().units) is None)
 
 
 def gemm_bf16_wide(x: torch.Tensor, w: torch.Tensor, scaled=None) -> torch.Tensor:
@@ -1791,7 +1795,7 @@ def product_bytes(m: int, w: torch.Tensor) -> int:
     n, k = w.shape
     if w.dtype == torch.float32:
         return 4 * m * (n + k) + f32_product_bytes(m, n, k)
-    plan = block_plan(m, n, k, "runs")
+    plan = pair_plan(m, n, k, "runs", chip().units) or block_plan(m, n, k, "runs")
     runs = plan[2] if plan is not None else mid_runs(n, k) if SKINNY_MAX_ROWS < m <= mid_max_rows(n, k) else 0
     return 2 * m * (n + k) + 4 * m * n * runs
 
@@ -1820,6 +1824,7 @@ _BLOCK_KINDS = {"runs": 1, "gated": 2, "plain": 3}  # as the kernel's entry poin
 
 class _Step(threading.local):
     own_products = False  # the step that this thread is launching keeps to this package's products
+    shared_tiles = False  # this thread is launching a model's step
 
 
 _step = _Step()
@@ -1836,6 +1841,24 @@ def own_products():
         yield
     finally:
         _step.own_products = before
+
+
+@contextlib.contextmanager
+def shared_tiles():
+    """Inside the block, on this thread: products go to the one whose waves share a tile over halves of K wherever
+    :func:`pair_plan` has a plan.  A model's step is such a block; a product by itself keeps to what the plans beside it say."""
+    before, _step.shared_tiles = _step.shared_tiles, True
+    try:
+        yield
+    finally:
+        _step.shared_tiles = before
+
+
+def pair(m: int, n: int, k: int, kind: str) -> tuple[int, int, int] | None:
+    """:func:`pair_plan` inside :func:`shared_tiles`; stored as bfloat16 only where the tile product is not level with it."""
+    if not _step.shared_tiles or m <= ROWS_MAX_ROWS or (kind == "plain" and m < TILE_GATED_MAX_ROWS and _tile_applies(m, n, k, n)):
+        return None
+    return pair_plan(m, n, k, kind, chip().units)
 
 
 def runs_from_k() -> int:
@@ -1896,6 +1919,87 @@ def _block_plain_plan(m: int, n: int, k: int, units: int, own: bool) -> tuple[in
         return None
     share = 7 if n * k > _SMALL_WEIGHTS else 4 if own else 6
     return plan if 8 * tiles >= share * units else None
+
+
+# The product whose two groups of waves hold one tile over halves of K: tiles (32 weight rows x 32 rows of X, so many of each)
+# and microseconds of a launch of one round: a chunk of 64 k with next to no unit busy, what all of them add (first
+# whatever rows of X there are, then for those there are: rows beyond the last cost nothing), the launch, and
+# ("runs", the norm that adds them included) a million elements of runs.  Fitted to 2,600 launches over 19 matrices at 66
+# to 1,024 rows: within 8% as a rule, 24% at worst.
+_PAIR_COSTS = {
+    "plain": {(4, 4): (0.597, -0.725, 0.773, 1.807), (3, 4): (0.501, -0.517, 0.574, 2.195), (2, 4): (0.413, -0.243, 0.271, 2.326),
+              (4, 2): (0.462, -0.326, 0.352, 1.437), (3, 2): (0.356, -0.18, 0.243, 2.19), (2, 2): (0.286, -0.13, 0.161, 2.23)},
+    "runs": {(4, 4): (0.436, 0.088, 0.113, 7.349, 1.834), (3, 4): (0.362, 0.04, 0.131, 6.656, 2.095), (2, 4): (0.305, 0.019, 0.08, 6.171, 2.379),
+             (4, 2): (0.322, 0.212, -0.091, 5.777, 2.315), (3, 2): (0.252, 0.123, -0.013, 5.818, 2.473), (2, 2): (0.193, 0.04, 0.044, 5.719, 2.226)},
+    "gated": {(2, 4): (0.498, -0.161, 0.194, 2.579), (4, 2): (0.561, -0.243, 0.249, 1.998), (2, 2): (0.29, 0.218, 0.1, 0.018)},
+}
+
+
+@functools.lru_cache(maxsize=4096)
+def pair_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int, int] | None:
+    """(tiles of 32 weight rows, of 32 rows of X, runs of K) of the product whose waves share a tile over halves of K, for ``m``
+    rows and ``n`` result columns (``kind`` as for :func:`block_plan`); ``None`` where another product is the faster one.
+
+    It reads its operands from LDS half as often as the many-row product does at tiles of 64 to 128 rows, and is for what one
+    round of such tiles covers.  Microseconds over weights from memory, what was there before first (runs with their norm):
+    ``"plain"`` at 66 / 150 / 192 / 256 / 450 rows: 6,144 x 4,096 23.1 / 18.2, 39.3 / 24.4, 33.5 / 26.1, 40.0 / 27.5, 32.6 / 31.2;
+    6,144 x 2,560 16.5 / 13.3, 26.2 / 18.0, 24.1 / 19.5, 30.9 / 22.0; 4,096 x 2,048 12.4 / 10.6, 13.3 / 11.1, 21.5 / 12.4, 13.4 / 12.6,
+    16.7 / 15.2; 4,096 x 1,024 from 128 rows on, below it the tile product is level (6.4 / 6.7), 7.4 / 6.8, 7.2 / 6.8, 7.4 /
+    7.0, 11.1 / 8.9.  With tiles for fewer than half of the units, narrow matrices five eighths, the library's kernels cut K
+    (1,024 x 2,048 at 320 / 768 rows 8.9 / 9.5, 10.3 / 9.8; 2,048 x 2,048 at 225 / 320 9.2 / 9.5, 10.3 / 9.7).  Beyond 256 rows over large matrices the library's tiles fit as well: only with tiles for 13 of 16 units
+    (192 tiles at 384 rows: 4,096 x 4,096 24.9 / 28.3) and rows of a multiple of 2 KB (6,144 x 2,560 at 300 / 512 rows 22.3 / 23.3, 26.9 / 28.7).
+    ``"runs"`` at the same rows: 4,096 x 4,096 17.4 / 14.7, 22.1 / 19.7, 23.4 / 20.7, 26.5 / 23.6, 33.4 / 30.9; 2,560 x 4,096 15.1 / 12.9, 18.6 / 15.4,
+    19.6 / 17.0, 19.6 / 18.4; 1,024 x 3,072 from 129 rows on 11.1 / 10.3, 11.8 / 10.6, 11.7 / 11.0, 15.0 / 12.8; below them matrices of up
+    to 4 M elements stay with the mid-size product (8.9 / 9.7), of up to 2 M up to 192 rows.  The many-row product keeps long sums:
+    beyond 6,144 k all but 128 rows of up to 32 M elements (2,560 x 9,728 at 66 / 192 rows 23.1 / 19.2, 26.1 / 28.0; 4,096 x
+    12,288 at 66 rows 29.8 / 29.8), below 300 rows on (2,048 x 6,144 at 256 / 512 rows 21.7 / 20.5, 28.5 / 29.0).
+    ``"gated"``: 3,072 x 1,024 9.3 / 7.9, 12.6 / 10.1, 12.8 / 10.3, 13.6 / 10.9; 6,144 x 2,048 up to 128 rows 22.6 / 17.2, 24.3 / 19.2; tiles of
+    128 x 128 are slower than the many-row product's (9,728 x 2,560 at 66 rows 32.2 / 34.1)."""
+    if not ROWS_MAX_ROWS < m <= 1024 or n % 8 or k % 64 or k < 256:
+        return None
+    if max((m + 128) * k, ((2 if kind == "gated" else 1) * n + 256) * k) * 2 > 0x7FFFFFFF:
+        return None
+    size, runs = n * k, (1,)
+    if kind == "runs":
+        runs = (1, 2, 3, 4, 5, 6, 8)
+        if m > 512 or size <= (1 << 21 if m > 128 else 1 << 22) and m <= MID_MAX_ROWS and _mid_runs(n, k, units) > 0:
+            return None
+        if _block_plan(m, n, k, "runs", units) is not None and not (m <= 300 if k <= 6144 else m <= 128 and size <= 1 << 25):
+            return None
+    best = None
+    for (tw, tx), cost in _PAIR_COSTS[kind].items():
+        across, down = -(-n // ((16 if kind == "gated" else 32) * tw)), -(-m // (32 * tx))
+        for ks in runs:
+            per = -(-(k // 64) // ks)
+            if across * down * ks > units or (ks > 1 and (per < 3 or per * (ks - 1) >= k // 64)):
+                continue
+            busy = across * down * ks / units
+            time = per * (cost[0] + busy * (cost[1] + cost[2] * m / (32 * tx * down))) + cost[3]
+            if kind == "runs":
+                time += cost[4] * 1e-6 * m * n * ks
+            if best is None or time < best[0]:
+                best = (time, (tw, tx, ks), across * down * ks)
+    if best is None:
+        return None
+    if kind == "plain" and 8 * best[2] < (4 if n >= 4096 else 5) * units:
+        return None
+    if kind != "gated" and m > 256 and size >= _SMALL_WEIGHTS and (16 * best[2] < 13 * units or k % 1024):
+        return None
+    return best[1]
+
+
+def _pair(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str, plan: tuple[int, int, int]) -> torch.Tensor:
+    m, k = x.shape
+    n = out.shape[-1]
+    _ok(core().rl_gemm_pair(_p(x), _p(w), _p(out), m, n, k, k, k, n, _BLOCK_KINDS[kind], *plan, _stream()), "rl_gemm_pair")
+    return out
+
+
+def pair_reads(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether a layer's product goes to the ``"runs"`` form of :func:`pair_plan`'s product: it is the faster one, and takes
+    the operands as they are, rows side by side in whole units of 16 bytes."""
+    return (pair(x.shape[0], w.shape[0], w.shape[1], "runs") is not None and _aligned(x, w)
+            and x.is_contiguous() and w.is_contiguous())
 
 
 def _aligned(a: torch.Tensor, b: torch.Tensor) -> bool:
@@ -1979,6 +2083,11 @@ def gemm_bf16_parts(x: torch.Tensor, w: torch.Tensor, copies: bool = True) -> to
     begin inside a unit of 16 bytes; without ``copies`` only where :func:`block_reads` says so."""
     m, k = x.shape
     n = w.shape[0]
+    if k == w.shape[1] and pair_reads(x, w):
+        _need(x, "x", torch.bfloat16)
+        _need(w, "w", torch.bfloat16)
+        halves = pair(m, n, k, "runs")
+        return _pair(x, w, torch.empty((halves[2], m, n), dtype=torch.float32, device=x.device), "runs", halves)
     plan = block_plan(m, n, k, "runs") if k == w.shape[1] and (copies or block_reads(x, w)) else None
     if plan is not None:
         _need(x, "x", torch.bfloat16)
@@ -2048,6 +2157,9 @@ def gemm_bf16_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, scaled=None, limi
         plan = rows_plan(m, inter, k, swiglu=True) if m <= ROWS_MAX_ROWS else None
         tile = _tile_applies(m, two_i, k, inter) and not (plan is not None and k >= 1024 and _aligned(x, w_gate_up))
         if activation == "silu" and limit <= 0 and bias is None:
+            halves = pair(m, inter, k, "gated")
+            if halves is not None and _aligned(x, w_gate_up):
+                return _pair(x, w_gate_up, torch.empty((m, inter), dtype=torch.bfloat16, device=x.device), "gated", halves)
             block = _gated_block(m, inter, k, tile, chip().units)
             if block is not None and _aligned(x, w_gate_up):
                 return _block(x, w_gate_up, torch.empty((m, inter), dtype=torch.bfloat16, device=x.device), "gated", block)

@@ -321,10 +321,11 @@ class CausalLM:
     def forward(self, ctx, caches) -> torch.Tensor:
         """Run the tokens of ``ctx`` through every layer (which writes their keys and values)
         and return float32 logits ``[len(ctx.logit_rows), vocab]``."""
-        if self._own_products(ctx):
-            with ops.own_products():
-                return self._forward(ctx, caches)
-        return self._forward(ctx, caches)
+        with ops.shared_tiles():
+            if self._own_products(ctx):
+                with ops.own_products():
+                    return self._forward(ctx, caches)
+            return self._forward(ctx, caches)
 
     def _forward(self, ctx, caches) -> torch.Tensor:
         residual = self.embed.forward(ctx.token_ids, ctx)

@@ -71,7 +71,8 @@ class Linear:
         n, k = self.out_features, self.in_features
         if self.weight.dtype != torch.bfloat16:
             return False
-        if folded and ((rows <= ops.mid_max_rows(n, k) and ops.mid_runs(n, k) > 0) or ops.block_pays(rows, n, k, ops.chip().units)):
+        if folded and ((rows <= ops.mid_max_rows(n, k) and ops.mid_runs(n, k) > 0) or ops.block_pays(rows, n, k, ops.chip().units)
+                       or ops.pair(rows, n, k, "runs") is not None):
             return False
         return ops.library_takes(rows, n, k)
 
@@ -82,15 +83,16 @@ class Linear:
 
     def midsize(self, x) -> bool:
         """Whether ``x`` (more rows than the few-row kernel takes) may run as float32 runs of K that a norm adds: up to
-        ``ops.mid_max_rows`` over a narrow matrix (wide ones have nothing to gain), any number of them over long sums where the many-row
-        product is the faster one (``ops.block_reads``)."""
+        ``ops.mid_max_rows`` over a narrow matrix (wide ones have nothing to gain), some hundred where the product that shares its
+        tiles over halves of K is the faster one (``ops.pair_reads``), any number of them over long sums where the many-row
+        product is (``ops.block_reads``)."""
         rows = x.shape[0]
         if self.weight.dtype != torch.bfloat16 or x.dtype != torch.bfloat16 or rows <= ops.SKINNY_MAX_ROWS:
             return False
         n, k = self.out_features, self.in_features
         if rows <= ops.MID_SMALL_MAX_ROWS and rows <= ops.mid_max_rows(n, k) and ops.mid_runs(n, k) > 0:
             return True
-        return k >= ops.runs_from_k() and ops.block_reads(x, self.weight)
+        return ops.pair_reads(x, self.weight) or (k >= ops.runs_from_k() and ops.block_reads(x, self.weight))
 
     def partial_sums(self, x: torch.Tensor) -> torch.Tensor:
         """``[runs, M, out]`` float32 whose sum over the runs is ``x W^T`` (without the bias)."""

@@ -1,0 +1,95 @@
+"""The product whose waves share a tile over halves of K: what its plans ask of the kernel, and the kernel against 64 bits."""
+
+import random
+
+import pytest
+import torch
+
+from rapid_llm_amd.kernels import ops
+
+
+@pytest.mark.parametrize("kind", ["plain", "runs", "gated"])
+def test_plans_are_what_the_kernel_takes(kind):
+    rng = random.Random(1)
+    found = 0
+    for _ in range(4000):
+        m, n, k = rng.randint(1, 1400), 8 * rng.randint(1, 1600), 64 * rng.randint(1, 200)
+        plan = ops.pair_plan(m, n, k, kind, 256)
+        if plan is None:
+            continue
+        found += 1
+        tw, tx, ks = plan
+        assert ops.ROWS_MAX_ROWS < m <= 1024 and tw in (2, 3, 4) and tx in (2, 4) and (kind != "gated" or tw % 2 == 0) and (kind == "runs" or ks == 1)
+        chunks = k // 64
+        assert -(-chunks // ks) * (ks - 1) < chunks  # every run holds a chunk
+        tiles = -(-n // ((16 if kind == "gated" else 32) * tw)) * -(-m // (32 * tx))
+        assert tiles * ks <= 256 and (m + 128) * k * 2 <= 0x7FFFFFFF
+    assert found > 100
+    assert ops.pair_plan(200, 4092, 2048, kind, 256) is None and ops.pair_plan(200, 4096, 2080, kind, 256) is None
+
+
+def test_only_steps_of_a_model_go_there():
+    assert ops.pair(200, 6144, 4096, "plain") is None and ops.library_takes(200, 6144, 4096)
+    with ops.shared_tiles():
+        assert ops.pair(200, 6144, 4096, "plain") == ops.pair_plan(200, 6144, 4096, "plain", ops.chip().units) is not None
+        assert not ops.library_takes(200, 6144, 4096) and ops.pair(64, 6144, 4096, "plain") is None
+        assert ops.pair(100, 4096, 1024, "plain") is None  # the tile product is level there
+    assert ops.pair(200, 6144, 4096, "plain") is None
+
+
+# One chunk and an odd number of them (the second group multiplies zeros), fewer chunks than buffers and more; rows and columns that end
+# inside a tile of 16, a wave's tiles and a workgroup's; several tiles on both sides.
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (70, 72, 128), (129, 200, 192), (257, 1000, 320), (65, 520, 704), (300, 264, 4096)])
+@pytest.mark.parametrize("tile", [(4, 4), (3, 4), (2, 4), (4, 2), (3, 2), (2, 2)])
+def test_kernel(m, n, k, tile):
+    gen = torch.Generator().manual_seed(m + k)
+    dev = "cuda"
+    x, w, w2 = ((torch.randn(r, k, generator=gen) * s).to(torch.bfloat16).to(dev) for r, s in ((m, 1.0), (n, 0.1), (2 * n, 0.1)))
+    lib, p = ops.core(), ops._p
+    want = x.double() @ w.double().t()
+
+    def launch(weight, out, kind, ks=1):
+        assert lib.rl_gemm_pair(p(x), p(weight), p(out), m, n, k, k, k, n, kind, *tile, ks, ops._stream()) == 0
+
+    # bfloat16 results: half a unit in the last place of each, 2^-9, and the float32 sums before it
+    out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=dev)
+    launch(w, out, 3)
+    assert bool((out[m] == 7.0).all())
+    assert float(((out[:m].double() - want).abs() - want.abs() / 256).max()) <= 1e-5 * float(want.abs().max())
+    # float32 runs: sums of k terms in float32, in an order of their own: sqrt(k) roundings of 2^-24 of the largest, eight times over
+    for ks in (1, 2, 3):
+        if -(-(k // 64) // ks) * (ks - 1) >= k // 64:
+            continue
+        runs = torch.full((ks * m + 1, n), 7.0, device=dev)
+        launch(w, runs, 1, ks)
+        assert bool((runs[ks * m] == 7.0).all())
+        got = runs[: ks * m].view(ks, m, n).double().sum(0)
+        assert float((got - want).abs().max()) <= 8 * k**0.5 * 2.0**-24 * float(want.abs().max())
+    if tile[0] % 2 == 0:
+        # gate and up are rounded to bfloat16 first: off by 2^-8 of themselves where a sum on the edge goes the other way, and by
+        # what the sums may be off, as above; silu's slope is 1.1 at most; then the result is rounded
+        both = (x.double() @ w2.double().t()).to(torch.bfloat16).double()
+        gate, up, off = both[:, :n], both[:, n:], 8 * k**0.5 * 2.0**-24 * float(both.abs().max())
+        act = torch.nn.functional.silu(gate) * up
+        out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=dev)
+        launch(w2, out, 2)
+        assert bool((out[m] == 7.0).all())
+        slack = 1.1 * up.abs() * (gate.abs() / 256 + off) + torch.nn.functional.silu(gate).abs() * (up.abs() / 256 + off) + act.abs() / 256
+        assert bool(((out[:m].double() - act).abs() <= slack).all())
+
+
+@pytest.mark.gpu
+def test_sizes_the_kernel_refuses():
+    lib, p = ops.core(), ops._p
+    x, w, out = (torch.zeros(256, 256, dtype=torch.bfloat16, device="cuda") for _ in range(3))
+    ok = dict(M=64, N=64, K=64, ldx=256, ldw=256, ldo=256, kind=3, tw=2, tx=2, splits=1)
+
+    def code(**change):
+        a = {**ok, **change}
+        return lib.rl_gemm_pair(p(x), p(w), p(out), a["M"], a["N"], a["K"], a["ldx"], a["ldw"], a["ldo"], a["kind"], a["tw"], a["tx"], a["splits"], ops._stream())
+
+    assert code() == 0 and code(M=0) == 0
+    for change in (dict(K=96), dict(N=60), dict(ldx=60), dict(ldo=63), dict(kind=0), dict(kind=2, tw=3), dict(tw=5), dict(tx=3), dict(splits=2),
+                   dict(kind=1, splits=2), dict(ldx=100)):
+        assert code(**change) != 0, change
