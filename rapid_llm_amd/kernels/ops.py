@@ -1856,7 +1856,7 @@ def shared_tiles():
 
 def pair(m: int, n: int, k: int, kind: str) -> tuple[int, int, int] | None:
     """:func:`pair_plan` inside :func:`shared_tiles`; stored as bfloat16 only where the tile product is not level with it."""
-    if not _step.shared_tiles or m <= ROWS_MAX_ROWS or (kind == "plain" and m < TILE_GATED_MAX_ROWS and _tile_applies(m, n, k, n)):
+    if not _step.shared_tiles or m <= SKINNY_MAX_ROWS or (kind == "plain" and m < TILE_GATED_MAX_ROWS and _tile_applies(m, n, k, n)):
         return None
     return pair_plan(m, n, k, kind, chip().units)
 
@@ -1954,11 +1954,26 @@ def pair_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int, 
     beyond 6,144 k all but 128 rows of up to 32 M elements (2,560 x 9,728 at 66 / 192 rows 23.1 / 19.2, 26.1 / 28.0; 4,096 x
     12,288 at 66 rows 29.8 / 29.8), below 300 rows on (2,048 x 6,144 at 256 / 512 rows 21.7 / 20.5, 28.5 / 29.0).
     ``"gated"``: 3,072 x 1,024 9.3 / 7.9, 12.6 / 10.1, 12.8 / 10.3, 13.6 / 10.9; 6,144 x 2,048 up to 128 rows 22.6 / 17.2, 24.3 / 19.2; tiles of
-    128 x 128 are slower than the many-row product's (9,728 x 2,560 at 66 rows 32.2 / 34.1)."""
-    if not ROWS_MAX_ROWS < m <= 1024 or n % 8 or k % 64 or k < 256:
+    128 x 128 are slower than the many-row product's (9,728 x 2,560 at 66 rows 32.2 / 34.1).
+    At 17 / 40 / 64 rows, tiles of 64 x 64 against the kernel that keeps X in registers: ``"gated"`` up to 2,048 k, where one round holds
+    them, 3,072 x 1,024 7.7 / 7.7, 8.9 / 8.0, 10.2 / 8.5, 6,144 x 2,048 15.3 / 13.6, 16.7 / 14.2, 19.7 / 15.3 (9,728 x 2,560, which takes larger
+    tiles, 23.8 / 26.6, 28.4 / 28.9); against the mid-size product, with the norm, ``"runs"`` beyond 6,144 k 2,560 x 9,728 17.1 / 15.7, 17.6 / 16.9,
+    18.5 / 17.9, 4,096 x 12,288 26.5 / 23.8, 27.2 / 25.2, 28.6 / 27.5 (2,048 x 6,144 11.8 / 11.6, 13.3 / 13.5); ``"plain"`` is the slower one
+    throughout (6,144 x 4,096 15.2 / 18.3)."""
+    if not SKINNY_MAX_ROWS < m <= 1024 or n % 8 or k % 64 or k < 256:
         return None
     if max((m + 128) * k, ((2 if kind == "gated" else 1) * n + 256) * k) * 2 > 0x7FFFFFFF:
         return None
+    if m <= ROWS_MAX_ROWS:
+        tiles = -(-n // (32 if kind == "gated" else 64))
+        if kind == "gated":
+            return (2, 2, 1) if k <= 2048 and 3 * units <= 8 * tiles <= 8 * units else None
+        if kind == "plain" or k <= 6144 or 4 * tiles > units or 8 * tiles < units:
+            return None
+        ks = min(8, units // tiles)
+        while -(-(k // 64) // ks) * (ks - 1) >= k // 64:  # every run holds a chunk
+            ks -= 1
+        return 2, 2, ks
     size, runs = n * k, (1,)
     if kind == "runs":
         runs = (1, 2, 3, 4, 5, 6, 8)

@@ -13,13 +13,13 @@ def test_plans_are_what_the_kernel_takes(kind):
     rng = random.Random(1)
     found = 0
     for _ in range(4000):
-        m, n, k = rng.randint(1, 1400), 8 * rng.randint(1, 1600), 64 * rng.randint(1, 200)
+        m, n, k = rng.choice((rng.randint(1, 1400), rng.randint(1, 80))), 8 * rng.randint(1, 1600), 64 * rng.randint(1, 200)
         plan = ops.pair_plan(m, n, k, kind, 256)
         if plan is None:
             continue
         found += 1
         tw, tx, ks = plan
-        assert ops.ROWS_MAX_ROWS < m <= 1024 and tw in (2, 3, 4) and tx in (2, 4) and (kind != "gated" or tw % 2 == 0) and (kind == "runs" or ks == 1)
+        assert ops.SKINNY_MAX_ROWS < m <= 1024 and tw in (2, 3, 4) and tx in (2, 4) and (kind != "gated" or tw % 2 == 0) and (kind == "runs" or ks == 1)
         chunks = k // 64
         assert -(-chunks // ks) * (ks - 1) < chunks  # every run holds a chunk
         tiles = -(-n // ((16 if kind == "gated" else 32) * tw)) * -(-m // (32 * tx))
@@ -33,6 +33,7 @@ def test_only_steps_of_a_model_go_there():
     with ops.shared_tiles():
         assert ops.pair(200, 6144, 4096, "plain") == ops.pair_plan(200, 6144, 4096, "plain", ops.chip().units) is not None
         assert not ops.library_takes(200, 6144, 4096) and ops.pair(64, 6144, 4096, "plain") is None
+        assert ops.pair(64, 4096, 12288, "runs") == (2, 2, 4) and ops.pair(17, 3072, 1024, "gated") == (2, 2, 1) and ops.pair(16, 3072, 1024, "gated") is None
         assert ops.pair(100, 4096, 1024, "plain") is None  # the tile product is level there
     assert ops.pair(200, 6144, 4096, "plain") is None
 
