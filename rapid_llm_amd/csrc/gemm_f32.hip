@@ -10,7 +10,7 @@
 // come to a sixth of 2.5 PFLOP/s, of which bfloat16 products of real operands reach 0.6.  Measured at 2,048
 // rows: 6,144 x 4,096 1,018 -> 453 us, 24,576 x 4,096 4,259 -> 1,624 us, 4,096 x 12,288 2,007 -> 817 us
 // (227 to 254 TFLOP/s); at 225 rows of a small model 6,144 x 1,024 53 -> 36 us and 1,024 x 3,072 68 -> 20
-// us.  Error against 64 bits over normal operands, relative to the result: K = 4,096 4.1e-7 -> 3.4e-7,
+// us (22 and 18 where a wave has a run).  Error against 64 bits over normal operands, relative to the result: K = 4,096 4.1e-7 -> 3.4e-7,
 // K = 12,288 7.0e-7 -> 6.0e-7.
 //
 // One order of summation for every output element, whatever M, the tile it falls in or what
@@ -610,6 +610,194 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(
     }
 }
 
+// ---- some rows: a wave a run, nothing shared ------------------------------------------
+// The tiles above walk K as a chain of chunks, each split, stored to LDS, waited for and read back, or leave their runs to
+// a second kernel.  Here the eight waves of a workgroup hold the same 16 NT x 16 MT results, each over its run of K, and no
+// wave waits for another.  A wave's rows go from memory straight into its own part of LDS, eight lanes a row (asked for into
+// registers as the instruction takes them, lane by lane from another row, a unit gets 16 bytes a cycle: 6,144 x 4,096 at 225 rows
+// 87 us, so 77), and from there to its registers, where they are split; a place is asked for again as soon as it has been
+// read, D chunks ahead.
+// What bounds it: splitting and multiplying, 208 (NT + MT) and 96 NT MT cycles a wave and chunk, which take about as long as
+// one after the other (at 225 rows of 6,144 x 4,096 the splits alone 38 us, the loads alone 43, all 77), so the tiles
+// are as large as the rows and the number of units allow.  The next split between the products 77 -> 74, the first four waves
+// ahead of the others on their SIMDs 60 -> 56 (4,096 x 4,096).
+// Microseconds, the other kernels / this: ops.f32_waves; steps: 0.6B three prompts of 225 tokens 3,453 -> 2,732, 8B eight
+// requests decode 7,159 -> 6,977.
+typedef __attribute__((address_space(3))) void* rl_lds_ptr;
+#define RUNS_LDS (160 * 1024)
+
+// Sixteen rows' chunks from LDS, the lane's eight k each; the wait stands in the block that asks, so that the compiler adds
+// none for loads that are on their way into LDS.
+__device__ __forceinline__ void read_rows(f32x4 (&r)[1][2], uint32_t at) {
+    asm volatile("ds_read_b128 %0, %2\n ds_read_b128 %1, %3\n s_waitcnt lgkmcnt(0)" : "=&v"(r[0][0]), "=&v"(r[0][1]) : "v"(at), "v"(at ^ 16) : "memory");
+}
+__device__ __forceinline__ void read_rows(f32x4 (&r)[2][2], uint32_t at) {
+    asm volatile(
+        "ds_read_b128 %0, %4\n ds_read_b128 %1, %5\n ds_read_b128 %2, %4 offset:2048\n ds_read_b128 %3, %5 offset:2048\n s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0][0]), "=&v"(r[0][1]), "=&v"(r[1][0]), "=&v"(r[1][1])
+        : "v"(at), "v"(at ^ 16)
+        : "memory");
+}
+
+template <int NT, int MT, bool GLU>
+__global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_runs_kernel(
+    const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K, int lda, int ldw,
+    int ldc, int tiles_m, int tiles_n) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the host pass does not know the LDS loads)
+    constexpr int T = NT + MT, SLOT = 2048, CHUNK = T * SLOT;  // a place: sixteen rows' chunk
+    constexpr int FIT = RUNS_LDS / (FRUNS * CHUNK), D = FIT < 3 ? FIT : 3;
+    constexpr int GA = MT % 2 ? 1 : 2, GW = NT % 2 ? 1 : 2;  // places read together
+    constexpr int BLOCKS = NT * MT, ROUNDS = (BLOCKS + FRUNS - 1) / FRUNS;
+    static_assert(D >= 1 && 2 * D * T <= 64, "a chunk fits, and the counter");
+    constexpr int SUMS = (ROUNDS > 1 ? 2 : 1) * FRUNS * FRUNS * RL_WAVE * 16, BYTES = FRUNS * D * CHUNK > SUMS ? FRUNS * D * CHUNK : SUMS;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[BYTES];
+
+    const int lane = threadIdx.x & (RL_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / RL_WAVE);
+    const int r16 = lane & 15, g = lane >> 4;
+    // the order of the tiles: as in gemm_f32_tile_kernel
+    const int tiles = tiles_m * tiles_n;
+    int t = blockIdx.x;
+    {
+        const int share = tiles / 8, rest = tiles % 8, die = t % 8;
+        t = die * share + min(die, rest) + t / 8;
+    }
+    const int band = t / (8 * tiles_n), first = band * 8, high = min(8, tiles_m - first);
+    const int m0 = (first + t % (8 * tiles_n) % high) * (16 * MT);
+    const int n0 = t % (8 * tiles_n) / high * (16 * NT);
+
+    const int chunks = K / FCH, per = (chunks + FRUNS - 1) / FRUNS;
+    const int c_lo = min(chunks, wave * per), c_hi = min(chunks, c_lo + per);
+
+    // A load lays a wave's 64 x 16 bytes side by side: eight rows, unit u of row r at u ^ (r / 2), so that reads meet every
+    // bank once.  Rows beyond the matrices find no records: zeros, whose results are dropped.
+    const int row0 = GLU ? n0 / 2 : n0;
+    const uint32_t w_bytes = ((uint32_t)((GLU ? 2 * N : N) - row0 - 1) * ldw + K) * 4, a_bytes = ((uint32_t)(M - m0 - 1) * lda + K) * 4;
+    const float *w_from = W + (size_t)row0 * ldw, *a_from = A + (size_t)m0 * lda;
+    uint32_t w_off[2], a_off[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = 8 * i + (lane >> 3);
+        const uint32_t unit = ((lane & 7) ^ (r >> 1)) * 16;
+        w_off[i] = (uint32_t)(GLU ? ((r >> 1) & 6) + (r & 1) + (r & 2 ? N : 0) : r) * (uint32_t)ldw * 4 + unit;
+        a_off[i] = (uint32_t)r * (uint32_t)lda * 4 + unit;
+    }
+    const uint32_t w_step = (uint32_t)(GLU ? 8 : 16) * (uint32_t)ldw * 4, a_step = 16 * (uint32_t)lda * 4;
+    unsigned char* const own = lds + wave * (D * CHUNK);
+    // the rows of places MT .. MT + NT - 1 are W's; behind the last chunk no records are found
+    auto ask = [&](int place, int c, uint32_t at) {
+        const bool is_a = place < MT;
+        const auto rs = is_a ? __builtin_amdgcn_make_buffer_rsrc((void*)a_from, 0, c < c_hi ? a_bytes : 0u, 0x00020000)
+                             : __builtin_amdgcn_make_buffer_rsrc((void*)w_from, 0, c < c_hi ? w_bytes : 0u, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t off = is_a ? a_off[i] + place * a_step : w_off[i] + (place - MT) * w_step;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (rl_lds_ptr)(own + at + place * SLOT + i * 1024), 16, off, c * (FCH * 4), 0, 0);
+        }
+    };
+
+    f32x4 acc[NT][MT];
+#pragma unroll
+    for (int x = 0; x < NT; ++x)
+#pragma unroll
+        for (int y = 0; y < MT; ++y) acc[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int p = 0; p < T; ++p) ask(p, c_lo + d, d * CHUNK);
+    const uint32_t l0 = (uint32_t)(uintptr_t)(rl_lds_ptr)own + r16 * 128 + ((2 * g) ^ (r16 >> 1)) * 16;
+    const float up = wave & 1 ? -UP : UP;
+    uint32_t at = 0;
+    if (wave < 4) __builtin_amdgcn_s_setprio(1);  // a SIMD's two waves split and multiply in turn rather than both at a time
+#pragma unroll 1
+    for (int c = c_lo; c < c_hi; ++c) {
+        // of the newest 2 D T loads all but those of the places read next may be missing
+        Split as[MT];
+#pragma unroll
+        for (int y = 0; y < MT; y += GA) {
+            f32x4 raw[GA][2];
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (D * T - GA)) : "memory");
+            read_rows(raw, l0 + at + y * SLOT);
+#pragma unroll
+            for (int j = 0; j < GA; ++j) ask(y + j, c + D, at);
+#pragma unroll
+            for (int j = 0; j < GA; ++j) as[y + j] = split8(raw[j][0], raw[j][1], up);
+        }
+        Split ws[2][GW];
+        auto take = [&](int x, Split (&to)[GW]) {
+            f32x4 raw[GW][2];
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (D * T - GW)) : "memory");
+            read_rows(raw, l0 + at + (MT + x) * SLOT);
+#pragma unroll
+            for (int j = 0; j < GW; ++j) ask(MT + x + j, c + D, at);
+#pragma unroll
+            for (int j = 0; j < GW; ++j) to[j] = split8(raw[j][0], raw[j][1]);
+        };
+        take(0, ws[0]);
+#pragma unroll
+        for (int x = 0; x < NT; x += GW) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (x + GW < NT) take(x + GW, ws[(x / GW + 1) & 1]);
+#pragma unroll
+            for (int s = 0; s < 6; ++s)
+#pragma unroll
+                for (int j = 0; j < GW; ++j)
+#pragma unroll
+                    for (int y = 0; y < MT; ++y)
+                        acc[x + j][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[x / GW & 1][j].p[PIECE_W[s]], as[y].p[PIECE_A[s]], acc[x + j][y], 0, 0, 0);
+            if (x + GW < NT) {  // three vector instructions of the next split behind every product
+#pragma unroll
+                for (int i = 0; i < 6 * GW * MT; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(2, 3, 0);
+                }
+            }
+        }
+        at = at == (D - 1) * CHUNK ? 0 : at + CHUNK;
+    }
+    __builtin_amdgcn_s_setprio(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be on its way to where the sums go
+    __syncthreads();
+
+    // The runs are added in their order, a block a wave, eight blocks a round.
+    f32x4* const sums = reinterpret_cast<f32x4*>(lds);  // [2][block][run][lane]
+#pragma unroll
+    for (int round = 0; round < ROUNDS; ++round) {
+        f32x4* const here = sums + (round & 1) * (FRUNS * FRUNS * RL_WAVE) + lane;
+#pragma unroll
+        for (int b = 0; b < FRUNS; ++b)
+            if (FRUNS * round + b < BLOCKS) here[(b * FRUNS + wave) * RL_WAVE] = acc[(FRUNS * round + b) / MT][(FRUNS * round + b) % MT];
+        __syncthreads();
+        const int block = FRUNS * round + wave;
+        if (block >= BLOCKS) break;
+        f32x4 total[1][1];
+        total[0][0] = here[wave * FRUNS * RL_WAVE];
+#pragma unroll
+        for (int r = 1; r < FRUNS; ++r) {
+            const f32x4 v = here[(wave * FRUNS + r) * RL_WAVE];
+            total[0][0] = r & 1 ? total[0][0] - v : total[0][0] + v;
+        }
+        const int m = m0 + block % MT * 16 + r16, n = n0 + block / MT * 16 + (GLU ? 0 : 4 * g);
+        if constexpr (GLU) {
+            gated_results<1, 1>(total, C, A, W, M, N, K, lda, ldw, ldc, [&](int) { return m; }, [&](int) { return n / 2 + 2 * g; });
+        } else if (m < M) {
+            f32x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = n + i < N ? finite_or_wide(total[0][0][i], A + (size_t)m * lda, W + (size_t)(n + i) * ldw, K) : 0.f;
+            float* out = C + (size_t)m * ldc + n;
+            if ((ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 && n + 3 < N) {
+                *reinterpret_cast<f32x4*>(out) = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < N) out[i] = v[i];
+            }
+        }
+    }
+#endif
+}
+
 // ---- many rows: the pieces of A laid out before, eight waves in two halves ----------------------
 // One kernel splits A once, instead of every workgroup that reads its rows, and lays the pieces down as the matrix
 // instruction reads them (bound by memory, 10 bytes an element: 10 us for 2,048 x 4,096): [16 rows][chunk][hi, mid, lo][64 lanes][8 k], 1 KB a piece.  Rows behind the last are zeros.
@@ -630,7 +818,6 @@ __global__ __launch_bounds__(256) void gemm_f32_pieces_kernel(const float* __res
     for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(out + p * 512) = s.p[p];
 }
 
-typedef __attribute__((address_space(3))) void* rl_lds_ptr;
 #define WIDE_A (256 * FCH * 6)  // bytes of a chunk's pieces of A
 
 template <int N>
@@ -1018,6 +1205,43 @@ static int launch_tile(const float* A, const float* W, float* C, float* parts, i
     return launch_tile_of<TM, TN, WHOLE, GLU>(A, W, C, parts, M, N, K, lda, ldw, ldc, groups, stream);
 }
 
+template <int NT, int MT, bool GLU>
+static int launch_runs_of(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc, hipStream_t stream) {
+    const int tm = (M + 16 * MT - 1) / (16 * MT), tn = (w_blocks<GLU>(N) + NT - 1) / NT;
+    if ((long long)tm * tn > 0x7fffffffLL / 16) return RL_ERR_ARG;
+    hipLaunchKernelGGL((gemm_f32_runs_kernel<NT, MT, GLU>), dim3(tm * tn), dim3(FRUNS * RL_WAVE), 0, stream, A, W, C, M, N, K,
+                       lda, ldw, ldc, tm, tn);
+    return rl_launch_status();
+}
+
+template <bool GLU>
+static int launch_runs(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc, int nt, int mt,
+                       hipStream_t stream) {
+    // offsets are 32-bit, those of a tile's rows beyond the matrices too
+    const long long limit = 0xffffffffll / 4;
+    if (K % FCH || ((GLU ? 2ll : 1ll) * N + 256) * ldw > limit || (M + 256ll) * lda > limit) return RL_ERR_ARG;
+#define RL_RUNS(NTV, MTV) \
+    if (nt == NTV && mt == MTV) return launch_runs_of<NTV, MTV, GLU>(A, W, C, M, N, K, lda, ldw, ldc, stream)
+    RL_RUNS(1, 1);
+    RL_RUNS(2, 1);
+    RL_RUNS(3, 1);
+    RL_RUNS(6, 1);
+    RL_RUNS(1, 2);
+    RL_RUNS(2, 2);
+    RL_RUNS(3, 2);
+    RL_RUNS(4, 2);
+    RL_RUNS(6, 2);
+    RL_RUNS(2, 3);
+    RL_RUNS(3, 3);
+    RL_RUNS(4, 3);
+    RL_RUNS(3, 4);
+    RL_RUNS(4, 4);
+    RL_RUNS(6, 4);
+    RL_RUNS(4, 5);
+#undef RL_RUNS
+    return RL_ERR_ARG;
+}
+
 template <bool GLU>
 static int launch_product(const float* A, const float* W, float* C, float* parts, int M, int N, int K, int lda,
                           int ldw, int ldc, int tile, int groups, hipStream_t stream) {
@@ -1079,6 +1303,21 @@ extern "C" int rl_gemm_f32_gated(const float* A, const float* W, float* C, float
     if (K <= FEW || lda < K || ldw < K || ldc < N || !C || N > 0x3fffffff) return RL_ERR_ARG;
     if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return RL_ERR_ARG;
     return launch_product<true>(A, W, C, parts, M, N, K, lda, ldw, ldc, tile, groups, stream);
+}
+
+// The same for K a multiple of 32, a wave a run: a tile is 16 nt weight rows x 16 mt rows of A.
+extern "C" int rl_gemm_f32_runs(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc, int nt,
+                                int mt, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return RL_OK;
+    if (K < FCH || lda < K || ldw < K || ldc < N || !A || !W || !C) return RL_ERR_ARG;
+    return launch_runs<false>(A, W, C, M, N, K, lda, ldw, ldc, nt, mt, stream);
+}
+
+extern "C" int rl_gemm_f32_runs_gated(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
+                                      int nt, int mt, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return RL_OK;
+    if (K < FCH || lda < K || ldw < K || ldc < N || !A || !W || !C || N > 0x3fffffff) return RL_ERR_ARG;
+    return launch_runs<true>(A, W, C, M, N, K, lda, ldw, ldc, nt, mt, stream);
 }
 
 // The same for many rows and K a multiple of 32: `pieces` holds 96 K bytes for every 16 rows of A; `cols` (128 or 96) are

@@ -1108,9 +1108,70 @@ _F32_PIECE_BYTES = 1e7  # bytes a microsecond at which A is read and its pieces 
 _F32_MOST_PIECES = 1 << 28  # bytes of pieces beyond which a product is cut into launches of fewer rows
 
 
+# The float32 product of a wave a run: tiles (16 weight rows x 16 rows of A, so many of each) and microseconds of a launch, of a round of
+# workgroups, of a chunk of 32 k of every round with next to no unit busy, and what all of them add.  Fitted to 3,000 launches over 20
+# matrices at 1 to 640 rows (3 to 8% off, root mean square); the weights' bytes bound it.
+_F32_WAVES = {
+    (1, 1): (1.44, 1.72, 0.46, 0.23), (1, 2): (1.78, 2.03, 0.75, 0.13), (2, 2): (1.72, 2.09, 1.10, 0.15),
+    (3, 2): (2.06, 2.23, 1.35, 0.29), (4, 2): (1.49, 2.19, 1.69, 0.26), (6, 2): (2.41, 2.17, 2.24, 0.49),
+    (2, 3): (1.96, 2.48, 1.33, 0.23), (3, 3): (2.27, 1.94, 1.61, 0.40), (4, 3): (1.73, 2.76, 2.00, 0.39),
+    (3, 4): (1.99, 2.54, 1.95, 0.46), (4, 4): (1.61, 3.26, 2.46, 0.49), (6, 4): (1.27, 4.71, 3.20, 0.83),
+    (4, 5): (0.98, 4.70, 2.84, 0.62),
+}
+# What the estimates of the other kernels are multiplied by, and what is added, to be times of the same machine: the tiles whose runs
+# are shared, those whose are not, the many-row product (218 of those launches, 4 to 8% off).
+_F32_OTHERS = {"shared": (1.09, 1.8), "tiles": (1.1, 3.7), "wide": (1.04, 4.3)}
+
+
+@functools.lru_cache(maxsize=4096)
+def f32_waves(m: int, n: int, k: int, units: int, normed: bool = False) -> tuple[int, int] | None:
+    """(tiles of 16 weight rows, of 16 rows of A) of the float32 product whose waves have a run of K each, ``None`` where the
+    kernels of :func:`f32_plan` and :func:`f32_wide` are the faster ones; ``normed``: where a norm could add those kernels' runs.  The
+    bits are the same either way.
+
+    Its operands reach the registers that multiply them without a barrier and no second kernel adds its runs; every
+    wave splits what it reads, so it loses where many rows make the large tiles' shared splitting pay, and where few tiles over
+    long sums leave most units without work.  Microseconds, the others / this: at 40 rows 4,096 x 1,024 13.7 / 9.2, 24,576 x 4,096 121.7 /
+    87.4; at 64 6,144 x 1,024 17.4 / 11.9, 6,144 x 4,096 34.8 / 32.2, 2,048 x 6,144 23.7 / 26.5, 4,096 x 12,288 59.8 / 69.9;
+    at 128 6,144 x 2,560 38.7 / 30.0; at 225 4,096 x 1,024 26.3 / 16.7, 6,144 x 1,024 34.3 / 21.9, 1,024 x 2,048 18.3 / 13.1, 1,024 x 3,072 20.7
+    / 18.1, 6,144 x 4,096 88.8 / 70.4, 24,576 x 4,096 240.8 / 287.9; at 450 4,096 x 2,048 62.8 / 53.7, 12,288 x 2,048 125.4 / 150.4.
+
+    Up to 16 rows against the kernel that streams the weights through registers: it is ahead from 1,536 k on (8 rows of 1,024 x 3,072
+    11.3 / 9.9, 6,144 x 4,096 24.4 / 21.2, 2,560 x 9,728 31.3 / 26.4, 151,936 x 4,096 424 / 410; 4,096 x 1,024 6.3 / 6.5), with up to four
+    rows, whose A the other reads for next to nothing, only over wide matrices of long sums (one row of 4,096 x 2,048 8.6 / 9.3,
+    6,144 x 4,096 24.1 / 22.2, 24,576 x 4,096 78.5 / 68.9)."""
+    if k % 32 or k < 512 or m > 1024 or (n + 256) * k > 1 << 30:
+        return None
+    tiles = -(-n // 16)
+    if m <= 16:
+        if k < 1536 or (m <= 4 and (n < 6144 or k < 2560)):
+            return None
+        # one round where that is possible; beyond, tiles of three keep the last round short
+        return next((nt for nt in (1, 2, 3, 6) if tiles <= nt * units), 3), 1
+    best, floor = None, 2.0 + 4.0 * n * k / 6e6
+    for (nt, mt), (launch, per_round, few, full) in _F32_WAVES.items():
+        if 16 * (mt - 1) >= m:
+            continue
+        count = -(-tiles // nt) * -(-m // (16 * mt))
+        rounds, busy = -(-count // units), count / units
+        time = launch + rounds * per_round + -(-k // 256) * (rounds * few + busy * full)
+        if best is None or (max(time, floor), time) < best[0]:
+            best = ((max(time, floor), time), (nt, mt))
+    others, cols = _f32_wide(m, n, k, units)
+    kind = "wide"
+    if not cols:
+        others, _, groups = _f32_tile_plan(m, n, k, units)
+        kind = "shared" if groups > 1 else "tiles"
+    scale, more = _F32_OTHERS[kind]
+    others = scale * others + more
+    if normed and kind == "shared":
+        others -= 1.3 + 1e-5 * m * n  # the norm's own kernel, and the product's way through memory
+    return best[1] if best[0][0] < 0.93 * others else None
+
+
 @functools.lru_cache(maxsize=4096)
 def f32_wide(m: int, n: int, k: int, units: int) -> int:
-    """Rows of W a tile of the float32 product for many rows takes, 0 where the tiles of ``f32_plan`` are the faster
+    """Rows of W a tile of the float32 product for many rows takes, 0 where ``f32_plan``'s tiles or ``f32_waves``' are the faster
     ones.  The bits are the same either way.
 
     Its tiles are two and one and a half times the largest there and a unit holds one, so they pay where they fill the
@@ -1120,8 +1181,13 @@ def f32_wide(m: int, n: int, k: int, units: int) -> int:
     4,096 x 1,024 67 / 61, 90 / 81, 175 / 159; 1,024 x 3,072 48 / 143, 85 / 149, 156 / 161.  Up to 512 k the making of A's
     pieces is not paid back (256 k: 3,120 weight rows at 1,982 rows, 11,272 at 259, 0.92 of the other tiles' speed), and the
     estimate has to be lower by 8%: of 289 sizes drawn, 34 go here, 1.04 to 1.41 times as fast."""
+    return 0 if f32_waves(m, n, k, units) is not None else _f32_wide(m, n, k, units)[1]
+
+
+def _f32_wide(m: int, n: int, k: int, units: int) -> tuple[float, int]:
+    """(estimated microseconds, rows of W a tile takes) of that product; 0 rows where the tiles of ``f32_plan`` are faster."""
     if m <= 64 or k % 32 or k <= 512 or k > 1 << 20:
-        return 0
+        return 0.0, 0
     best, cols = 0.92 * (_f32_tile_plan(m, n, k, units)[0] + _F32_WIDE_ROUND), 0
     for width, (few, full) in _F32_WIDE.items():
         rounds, rest = divmod(-(-m // 256) * -(-n // width), units)
@@ -1129,7 +1195,7 @@ def f32_wide(m: int, n: int, k: int, units: int) -> int:
         time = chunk * (k // 32) + _F32_WIDE_ROUND * (rounds + (rest > 0)) + 2.0 + 10.0 * m * k / _F32_PIECE_BYTES
         if time < best:
             best, cols = time, width
-    return cols
+    return best, cols
 
 
 def _f32_piece_rows(m: int, k: int) -> int:
@@ -1140,7 +1206,7 @@ def _f32_piece_rows(m: int, k: int) -> int:
 
 def f32_product_bytes(m: int, n: int, k: int) -> int:
     """What a float32 product of ``m`` rows over ``[n, k]`` weights takes beside its result."""
-    if f32_wide(m, n, k, chip().units):
+    if f32_wide(m, n, k, chip().units) or _f32_wide(m, n, k, chip().units)[1]:  # (operands that f32_waves' kernel does not take)
         return 96 * k * -(-min(m, _f32_piece_rows(m, k)) // 16)
     return f32_scratch_bytes(m, n, k)
 
@@ -1185,7 +1251,19 @@ def _f32_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows_of_w:
     m, k = a.shape
     n = out.shape[1]
     strides = (a.stride(0), w.stride(0), out.stride(0))
-    cols = f32_wide(m, rows_of_w, k, chip().units)
+    units = chip().units
+    cols = f32_wide(m, rows_of_w, k, units)
+    waves = f32_waves(m, rows_of_w, k, units) if not cols else None
+    if waves is not None:
+        # it reads whole units of 16 bytes, at offsets of 32 bits
+        if _aligned(a, w) and not (strides[0] | strides[1]) & 3 and max((m + 256) * strides[0], (rows_of_w + 256) * strides[1]) <= 1 << 30:
+            args = (_p(a), _p(w), _p(out), m, n, k, *strides, *waves, _stream())
+            if gated:
+                _ok(core().rl_gemm_f32_runs_gated(*args), "rl_gemm_f32_runs_gated")
+            else:
+                _ok(core().rl_gemm_f32_runs(*args), "rl_gemm_f32_runs")
+            return
+        cols = _f32_wide(m, rows_of_w, k, units)[1]
     if cols:
         rows = _f32_piece_rows(m, k)
         pieces = torch.empty(96 * k * -(-min(m, rows) // 16), dtype=torch.uint8, device=a.device)
@@ -1196,7 +1274,7 @@ def _f32_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows_of_w:
             else:
                 _ok(core().rl_gemm_f32_wide(*args), "rl_gemm_f32_wide")
         return
-    tile, groups = f32_plan(m, rows_of_w, k, chip().units)
+    tile, groups = f32_plan(m, rows_of_w, k, units)
     parts = torch.empty((8, m, rows_of_w), dtype=torch.float32, device=a.device) if groups > 1 else None
     args = (_p(a), _p(w), _p(out), _p(parts), m, n, k, *strides, tile, groups, _stream())
     if gated:
@@ -1207,7 +1285,10 @@ def _f32_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows_of_w:
 
 def f32_runs(m: int, n: int, k: int) -> bool:
     """Whether a float32 product leaves runs of K that a kernel behind it adds: the norm that follows can be that one."""
-    return not f32_wide(m, n, k, chip().units) and f32_plan(m, n, k, chip().units)[1] > 1
+    units = chip().units
+    if f32_waves(m, n, k, units) is not None:
+        return f32_waves(m, n, k, units, True) is None and f32_plan(m, n, k, units)[1] > 1
+    return not f32_wide(m, n, k, units) and f32_plan(m, n, k, units)[1] > 1
 
 
 def gemm_f32_add_rmsnorm(a: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
