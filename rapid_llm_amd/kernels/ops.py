@@ -1109,14 +1109,14 @@ _F32_MOST_PIECES = 1 << 28  # bytes of pieces beyond which a product is cut into
 
 
 # The float32 product of a wave a run: tiles (16 weight rows x 16 rows of A, so many of each) and microseconds of a launch, of a round of
-# workgroups, of a chunk of 32 k of every round with next to no unit busy, and what all of them add.  Fitted to 3,000 launches over 20
-# matrices at 1 to 640 rows (3 to 8% off, root mean square); the weights' bytes bound it.
+# workgroups, of a chunk of 32 k of every round with next to no unit busy, and what all of them add.  Fitted to 1,900 launches over 18
+# matrices at 8 to 640 rows (3 to 8% off, root mean square); the weights' bytes bound it.
 _F32_WAVES = {
-    (1, 1): (1.44, 1.72, 0.46, 0.23), (1, 2): (1.78, 2.03, 0.75, 0.13), (2, 2): (1.72, 2.09, 1.10, 0.15),
-    (3, 2): (2.06, 2.23, 1.35, 0.29), (4, 2): (1.49, 2.19, 1.69, 0.26), (6, 2): (2.41, 2.17, 2.24, 0.49),
-    (2, 3): (1.96, 2.48, 1.33, 0.23), (3, 3): (2.27, 1.94, 1.61, 0.40), (4, 3): (1.73, 2.76, 2.00, 0.39),
-    (3, 4): (1.99, 2.54, 1.95, 0.46), (4, 4): (1.61, 3.26, 2.46, 0.49), (6, 4): (1.27, 4.71, 3.20, 0.83),
-    (4, 5): (0.98, 4.70, 2.84, 0.62),
+    (1, 1): (2.98, 0.18, 0.48, 0.12), (1, 2): (1.76, 1.68, 0.73, 0.16), (2, 2): (3.44, 0.01, 1.02, 0.18),
+    (3, 2): (3.68, 0.00, 1.28, 0.31), (4, 2): (1.40, 2.30, 1.67, 0.33), (6, 2): (2.47, 2.16, 2.24, 0.57),
+    (2, 3): (3.91, 0.07, 1.30, 0.23), (3, 3): (1.82, 2.36, 1.61, 0.44), (4, 3): (1.41, 3.10, 1.98, 0.49),
+    (3, 4): (1.50, 3.00, 1.94, 0.52), (4, 4): (1.38, 3.48, 2.45, 0.60), (6, 4): (1.23, 4.80, 3.23, 0.91),
+    (4, 5): (0.51, 5.28, 2.88, 0.72),
 }
 # What the estimates of the other kernels are multiplied by, and what is added, to be times of the same machine: the tiles whose runs
 # are shared, those whose are not, the many-row product (218 of those launches, 4 to 8% off).
@@ -1136,15 +1136,15 @@ def f32_waves(m: int, n: int, k: int, units: int, normed: bool = False) -> tuple
     at 128 6,144 x 2,560 38.7 / 30.0; at 225 4,096 x 1,024 26.3 / 16.7, 6,144 x 1,024 34.3 / 21.9, 1,024 x 2,048 18.3 / 13.1, 1,024 x 3,072 20.7
     / 18.1, 6,144 x 4,096 88.8 / 70.4, 24,576 x 4,096 240.8 / 287.9; at 450 4,096 x 2,048 62.8 / 53.7, 12,288 x 2,048 125.4 / 150.4.
 
-    Up to 16 rows against the kernel that streams the weights through registers: it is ahead from 1,536 k on (8 rows of 1,024 x 3,072
-    11.3 / 9.9, 6,144 x 4,096 24.4 / 21.2, 2,560 x 9,728 31.3 / 26.4, 151,936 x 4,096 424 / 410; 4,096 x 1,024 6.3 / 6.5), with up to four
+    Up to 16 rows against the kernel that streams the weights through registers: it is ahead from 1,024 k on (8 rows of 1,024 x 3,072
+    11.3 / 9.4, 6,144 x 4,096 24.4 / 21.4, 2,560 x 9,728 31.3 / 26.4, 6,144 x 1,024 8.7 / 8.0; 151,936 x 4,096 424 / 410, x 1,024 115 / 122), with up to four
     rows, whose A the other reads for next to nothing, only over wide matrices of long sums (one row of 4,096 x 2,048 8.6 / 9.3,
     6,144 x 4,096 24.1 / 22.2, 24,576 x 4,096 78.5 / 68.9)."""
     if k % 32 or k < 512 or m > 1024 or (n + 256) * k > 1 << 30:
         return None
     tiles = -(-n // 16)
     if m <= 16:
-        if k < 1536 or (m <= 4 and (n < 6144 or k < 2560)):
+        if k < 1024 or (k < 1536 and n > 6144) or (m <= 4 and (n < 6144 or k < 2560)):
             return None
         # one round where that is possible; beyond, tiles of three keep the last round short
         return next((nt for nt in (1, 2, 3, 6) if tiles <= nt * units), 3), 1
