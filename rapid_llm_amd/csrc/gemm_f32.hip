@@ -687,15 +687,17 @@ __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_runs_kernel(
     }
     const uint32_t w_step = (uint32_t)(GLU ? 8 : 16) * (uint32_t)ldw * 4, a_step = 16 * (uint32_t)lda * 4;
     unsigned char* const own = lds + wave * (D * CHUNK);
-    // the rows of places MT .. MT + NT - 1 are W's; behind the last chunk no records are found
+    // the rows of places MT .. MT + NT - 1 are W's; behind the last chunk no records are found, and no chunk is asked for: the
+    // unit compares a load's own offset with the records less the scalar offset, which would wrap
     auto ask = [&](int place, int c, uint32_t at) {
-        const bool is_a = place < MT;
-        const auto rs = is_a ? __builtin_amdgcn_make_buffer_rsrc((void*)a_from, 0, c < c_hi ? a_bytes : 0u, 0x00020000)
-                             : __builtin_amdgcn_make_buffer_rsrc((void*)w_from, 0, c < c_hi ? w_bytes : 0u, 0x00020000);
+        const bool is_a = place < MT, there = c < c_hi;
+        const auto rs = is_a ? __builtin_amdgcn_make_buffer_rsrc((void*)a_from, 0, there ? a_bytes : 0u, 0x00020000)
+                             : __builtin_amdgcn_make_buffer_rsrc((void*)w_from, 0, there ? w_bytes : 0u, 0x00020000);
+        const int chunk = there ? c * (FCH * 4) : 0;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const uint32_t off = is_a ? a_off[i] + place * a_step : w_off[i] + (place - MT) * w_step;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (rl_lds_ptr)(own + at + place * SLOT + i * 1024), 16, off, c * (FCH * 4), 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (rl_lds_ptr)(own + at + place * SLOT + i * 1024), 16, off, chunk, 0, 0);
         }
     };
 

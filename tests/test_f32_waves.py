@@ -73,3 +73,27 @@ def test_operands_that_it_does_not_take(m, n, k):
         out = torch.empty_like(first)
         ops.gemm_f32(*moved, out)
         assert torch.equal(out, first)
+
+
+# What is asked for ahead of a wave's last chunk is not there: operands that end with their memory, where the last wave's run ends
+# with the rows (64 chunks), where it is shorter than the others' (61) and where waves have none (3).
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [2048, 1952, 96])
+@pytest.mark.parametrize("tile", [(1, 1), (1, 2), (6, 1), (4, 5)])
+def test_operands_that_end_with_their_memory(tile, k):
+    m, n = 37, 150
+    lib, p = ops.core(), ops._p
+    gen = torch.Generator().manual_seed(k)
+
+    def at_the_end(rows):
+        held = torch.empty(24 << 20, dtype=torch.uint8, device="cuda")  # (an allocation of its own, whole pages of 2 MB)
+        t = held[held.numel() - rows * k * 4 :].view(torch.float32).view(rows, k)
+        return t.copy_(torch.randn(rows, k, generator=gen))
+
+    for gated in (False, True):
+        a, w = at_the_end(m), at_the_end(2 * n if gated else n)
+        want, out = torch.empty((m, n), device="cuda"), torch.empty((m, n), device="cuda")
+        entry, runs = (lib.rl_gemm_f32_gated, lib.rl_gemm_f32_runs_gated) if gated else (lib.rl_gemm_f32, lib.rl_gemm_f32_runs)
+        assert entry(p(a), p(w), p(want), None, m, n, k, k, k, n, 64, 1, ops._stream()) == 0
+        assert runs(p(a), p(w), p(out), m, n, k, k, k, n, *tile, ops._stream()) == 0
+        assert torch.equal(out, want)
