@@ -1118,6 +1118,7 @@ _F32_WAVES = {
     (3, 4): (1.50, 3.00, 1.94, 0.52), (4, 4): (1.38, 3.48, 2.45, 0.60), (6, 4): (1.23, 4.80, 3.23, 0.91),
     (4, 5): (0.51, 5.28, 2.88, 0.72),
 }
+_F32_WAVES_REACH = 0xFFFFFFFF // 4  # elements that an offset of that kernel reaches, rows of a tile behind the last included
 # What the estimates of the other kernels are multiplied by, and what is added, to be times of the same machine: the tiles whose runs
 # are shared, those whose are not, the many-row product (218 of those launches, 4 to 8% off).
 _F32_OTHERS = {"shared": (1.09, 1.8), "tiles": (1.1, 3.7), "wide": (1.04, 4.3)}
@@ -1140,7 +1141,7 @@ def f32_waves(m: int, n: int, k: int, units: int, normed: bool = False) -> tuple
     11.3 / 9.4, 6,144 x 4,096 24.4 / 21.4, 2,560 x 9,728 31.3 / 26.4, 6,144 x 1,024 8.7 / 8.0; 151,936 x 4,096 424 / 410, x 1,024 115 / 122), with up to four
     rows, whose A the other reads for next to nothing, only over wide matrices of long sums (one row of 4,096 x 2,048 8.6 / 9.3,
     6,144 x 4,096 24.1 / 22.2, 24,576 x 4,096 78.5 / 68.9)."""
-    if k % 32 or k < 512 or m > 1024 or (n + 256) * k > 1 << 30:
+    if k % 32 or k < 512 or m > 1024 or (n + 256) * k > _F32_WAVES_REACH:
         return None
     tiles = -(-n // 16)
     if m <= 16:
@@ -1256,7 +1257,8 @@ def _f32_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows_of_w:
     waves = f32_waves(m, rows_of_w, k, units) if not cols else None
     if waves is not None:
         # it reads whole units of 16 bytes, at offsets of 32 bits
-        if _aligned(a, w) and not (strides[0] | strides[1]) & 3 and max((m + 256) * strides[0], (rows_of_w + 256) * strides[1]) <= 1 << 30:
+        reach = max((m + 256) * strides[0], (rows_of_w + 256) * strides[1])
+        if _aligned(a, w) and not (strides[0] | strides[1]) & 3 and reach <= _F32_WAVES_REACH:
             args = (_p(a), _p(w), _p(out), m, n, k, *strides, *waves, _stream())
             if gated:
                 _ok(core().rl_gemm_f32_runs_gated(*args), "rl_gemm_f32_runs_gated")

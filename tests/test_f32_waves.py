@@ -22,11 +22,35 @@ def test_plans_are_what_the_kernel_takes():
             continue
         found.add(plan)
         assert plan in TILES and m <= 1024 and k >= 512 and 16 * (plan[1] - 1) < m and ops.f32_wide(m, n, k, units) == 0
-        assert (n + 256) * k <= 1 << 30 and (m + 256) * k <= 1 << 30
+        assert (n + 256) * k < 1 << 30 and (m + 256) * k < 1 << 30  # (the entry point's limit: offsets of 32 bits)
         # the norm that would add the others' runs only makes those better
         assert ops.f32_waves(m, n, k, units, True) in (plan, None)
     assert len(found) > 10
     assert ops.f32_waves(225, 4096, 1000, 256) is None and ops.f32_waves(225, 4096, 480, 256) is None and ops.f32_waves(40, 1 << 20, 4096, 256) is None
+
+
+@pytest.mark.parametrize("m,n,k", [(8, 261888, 4096), (8, 130816, 8192), (300, 261888, 4096)])
+def test_matrices_whose_last_offset_is_one_too_many(m, n, k):
+    assert (n + 256) * k == 1 << 30 and ops.f32_waves(m, n, k, 256) is None
+    assert ops.f32_waves(m, n - 16, k, 256) is not None or m > 16
+
+
+@pytest.mark.parametrize("rows_a,rows_w,ld_a,ld_w", [(256, 1024, 1 << 21, 1024), (256, 768, 1024, 1 << 20), (256, 1024, (1 << 21) - 4, 1024)])
+def test_rows_whose_last_offset_is_one_too_many(rows_a, rows_w, ld_a, ld_w, monkeypatch):
+    """Strided rows that reach the limit go to the kernels behind, one stride less does not."""
+    called = []
+
+    class Library:
+        def __getattr__(self, name):
+            return lambda *args: called.append(name) or 0
+
+    monkeypatch.setattr(ops, "core", Library)
+    monkeypatch.setattr(ops, "_stream", lambda: None)
+    a, w = (torch.empty_strided((rows, 1024), (ld, 1), device="meta") for rows, ld in ((rows_a, ld_a), (rows_w, ld_w)))
+    assert ops.f32_waves(rows_a, rows_w, 1024, 256) is not None
+    ops._f32_product(a, w, torch.empty((rows_a, rows_w), device="meta"), rows_w, False)
+    over = max((rows_a + 256) * ld_a, (rows_w + 256) * ld_w) > 0xFFFFFFFF // 4
+    assert called == (["rl_gemm_f32"] if over else ["rl_gemm_f32_runs"]) and over == (ld_a != (1 << 21) - 4)
 
 
 # One chunk (seven waves without), runs of unlike length, fewer chunks than are asked for ahead and more; rows and columns that
