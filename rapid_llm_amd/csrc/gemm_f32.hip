@@ -1222,9 +1222,9 @@ static int launch_runs_of(const float* A, const float* W, float* C, int M, int N
 template <bool GLU>
 static int launch_runs(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc, int nt, int mt,
                        hipStream_t stream) {
-    // offsets are 32-bit, those of a tile's rows beyond the matrices too
+    // whole units of 16 bytes are loaded; offsets are 32-bit, those of a tile's rows beyond the matrices too
     const long long limit = 0xffffffffll / 4;
-    if (K % FCH || ((GLU ? 2ll : 1ll) * N + 256) * ldw > limit || (M + 256ll) * lda > limit) return RL_ERR_ARG;
+    if (((uintptr_t)A | (uintptr_t)W) % 16 || (lda | ldw) % 4 || K % FCH || ((GLU ? 2ll : 1ll) * N + 256) * ldw > limit || (M + 256ll) * lda > limit) return RL_ERR_ARG;
 #define RL_RUNS(NTV, MTV) \
     if (nt == NTV && mt == MTV) return launch_runs_of<NTV, MTV, GLU>(A, W, C, M, N, K, lda, ldw, ldc, stream)
     RL_RUNS(1, 1);
@@ -1310,7 +1310,8 @@ extern "C" int rl_gemm_f32_gated(const float* A, const float* W, float* C, float
     return launch_product<true>(A, W, C, parts, M, N, K, lda, ldw, ldc, tile, groups, stream);
 }
 
-// The same for K a multiple of 32, a wave a run: a tile is 16 nt weight rows x 16 mt rows of A.
+// The same for K a multiple of 32 and rows that begin with whole units of 16 bytes, a wave a run: a tile is 16 nt weight rows x
+// 16 mt rows of A.
 extern "C" int rl_gemm_f32_runs(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc, int nt,
                                 int mt, hipStream_t stream) {
     if (M <= 0 || N <= 0) return RL_OK;

@@ -1,6 +1,7 @@
 """The float32 product whose waves have a run of K each: what its plans ask of the kernel, and the kernel's bits against the
 shared tiles'."""
 
+import ctypes
 import random
 
 import pytest
@@ -51,6 +52,18 @@ def test_rows_whose_last_offset_is_one_too_many(rows_a, rows_w, ld_a, ld_w, monk
     ops._f32_product(a, w, torch.empty((rows_a, rows_w), device="meta"), rows_w, False)
     over = max((rows_a + 256) * ld_a, (rows_w + 256) * ld_w) > 0xFFFFFFFF // 4
     assert called == (["rl_gemm_f32"] if over else ["rl_gemm_f32_runs"]) and over == (ld_a != (1 << 21) - 4)
+
+
+def test_what_the_entry_points_refuse():
+    """Rows that begin inside a unit of 16 bytes, sums that are no whole chunks, offsets beyond 32 bits, tiles that there are not: an
+    error before anything is launched."""
+    lib, at = ops.core(), 1 << 20  # (addresses that nothing reads)
+    good = dict(A=at, W=at, C=at, M=8, N=64, K=512, lda=512, ldw=512, ldc=64, nt=1, mt=1)
+    changes = [dict(A=at + 4), dict(W=at + 8), dict(lda=513), dict(ldw=514), dict(K=500), dict(lda=508), dict(N=(1 << 21) - 256),
+               dict(ldw=1 << 22), dict(lda=1 << 23, M=24), dict(nt=5), dict(mt=0), dict(A=0), dict(ldc=63)]
+    for entry in (lib.rl_gemm_f32_runs, lib.rl_gemm_f32_runs_gated):
+        for change in changes:
+            assert entry(*(v if name in ("M", "N", "K", "lda", "ldw", "ldc", "nt", "mt") else ctypes.c_void_p(v) for name, v in {**good, **change}.items()), None) == 1, change
 
 
 # One chunk (seven waves without), runs of unlike length, fewer chunks than are asked for ahead and more; rows and columns that
