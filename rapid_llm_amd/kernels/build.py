@@ -62,7 +62,7 @@ RECURRENT_SOURCES = ("recurrent.hip",)
 LINEAR_ATTENTION_SOURCES = ("linear_attention.hip",)
 ATTENTION_TILE_SOURCES = ("attention_tile.hip",)
 DECODE_CHAIN_SOURCES = ("decode_chain.hip",)
-HEADERS = ("common.h", "static_entry.h")
+HEADERS = ("common.h", "silu.h", "static_entry.h")
 
 # head sizes built ahead of time by build_all(): every one the kernels take.  A fresh
 # checkout compiles only the head size of the model it is asked to run.

@@ -81,6 +81,28 @@ def test_kernel(m, n, k, tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile", [(2, 2), (2, 4), (4, 2)])
+def test_every_gate_has_the_activation_of_the_many_row_product(tile):
+    """All bfloat16 gates against sixty factors, infinities and NaN among both: bit for bit what the other product with an activation
+    stores, whose form is the more exact one (a wave's numbers below 87, some beyond and all of them)."""
+    lib, p = ops.core(), ops._p
+    gates = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    gen = torch.Generator().manual_seed(3)
+    ups = torch.cat((torch.randn(40, generator=gen), torch.randn(20, generator=gen) * 100, torch.tensor([0.0, -0.0, float("inf"), float("nan")]))).to(torch.bfloat16)
+    m, n, k = gates.numel(), ups.numel(), 64
+    x, w = torch.zeros(m, k, dtype=torch.bfloat16), torch.zeros(2 * n, k, dtype=torch.bfloat16)
+    # gate * 1 and 1 * up, beside products with 0: NaN for a number that is not finite
+    x[:, 0], x[:, 1], w[:n, 0], w[n:, 1] = gates, 1.0, 1.0, ups
+    x, w = x.cuda(), w.cuda()
+    want, out = (torch.full((m, n), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    assert lib.rl_gemm_block(p(x), p(w), p(want), m, n, k, k, k, n, 2, 2, 2, 1, ops._stream()) == 0
+    assert lib.rl_gemm_pair(p(x), p(w), p(out), m, n, k, k, k, n, 2, *tile, 1, ops._stream()) == 0
+    assert torch.equal(out.isnan(), want.isnan())
+    same = (out.view(torch.int16) == want.view(torch.int16)) | want.isnan()
+    assert bool(same.all()), int((~same).sum())
+
+
+@pytest.mark.gpu
 def test_sizes_the_kernel_refuses():
     lib, p = ops.core(), ops._p
     x, w, out = (torch.zeros(256, 256, dtype=torch.bfloat16, device="cuda") for _ in range(3))
