@@ -241,7 +241,7 @@ __device__ __forceinline__ void ask_query(AskedQuery& a, const bf16_t* qrow, int
             }
     }
 }
-// (`scale`: a factor of the scores that is taken into the query, before its only rounding)
+// (`scale`: a factor of the scores that a norm's takes in; without a norm a query's numbers may be stored as they are)
 __device__ __forceinline__ void prepared_query(bf16x8 (&qf)[DC], const AskedQuery& a, const float (&w)[DC][8], bool row_ok,
                                                const DecodeExtra& ex, float scale) {
     float x[DC][8];
@@ -261,11 +261,6 @@ __device__ __forceinline__ void prepared_query(bf16x8 (&qf)[DC], const AskedQuer
         for (int c = 0; c < DC; ++c)
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[c][j] *= rrms * w[c][j];
-    } else {
-#pragma unroll
-        for (int c = 0; c < DC; ++c)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) x[c][j] *= scale;
     }
     if (ex.cos_tab) {
         constexpr int HC = DC / 2;
@@ -715,9 +710,11 @@ extern "C" int rl_attn_decode_fusable() { return D % 64 == 0 ? 1 : 0; }
 // in tiles that the diagonal, a window's edge or the end of the sequence crosses, and the
 // accumulators are rescaled only when some row's maximum moved by more than LAZY: the weights are relative to what the
 // row's maximum was then, at most 2^LAZY, of which float32 sums and bfloat16 roundings have no less precision.  Queries
-// that are finished here (PREP) take the scores' factor in before their only rounding, and the scores' sums begin with
-// the negative maximum, so that a weight is one exponential of what the matrix cores leave (8,192 tokens of 32 query heads, all
-// of it and what follows here 0.89 -> 0.98 PFLOP/s).
+// that are normed here (PF_NORMED) take the scores' factor in with the norm's, before their only rounding, and the scores' sums
+// begin with the negative maximum, so that a weight is one exponential of what the matrix cores leave (8,192 tokens of 32 query
+// heads, all of it and what follows here 0.89 -> 0.98 PFLOP/s).  Without a norm a query, or the channels of it that turn
+// slowly, can be bfloat16 numbers as they lie: the factor would round them (1,024 normal keys of 128 channels, error of the
+// outputs against 64 bits 2.24e-3 -> 2.79e-3), so it stays with the scores.
 //
 // tile_info[8 * tile + {0..4}] = {first token of the request's portion in the flat batch, tokens of the
 //   request already in the cache, tokens in this portion, first row of the tile, the request's row of the
@@ -754,7 +751,10 @@ constexpr int PF_DIRECT_TILE = PF_KEYS * D * 2;      // bytes of a key tile and 
 constexpr int PF_DIRECT_SET = 2 * PF_DIRECT_TILE;    // one step's tiles
 constexpr int PF_DIRECT_GROUP = 2 * PF_DIRECT_SET;   // a wave group's two sets
 
-template <int GROUPS, bool DIRECT, bool PREP>
+// the queries are finished, the kernel rotates them (or not), the kernel norms them and rotates them (or not)
+enum PrefillQueries { PF_FINISHED, PF_TURNED, PF_NORMED };
+
+template <int GROUPS, bool DIRECT, PrefillQueries QUERIES>
 __global__ __launch_bounds__(GROUPS* PF_THREADS) __attribute__((amdgpu_waves_per_eu(1, 2))) void
 attn_prefill_kernel(
     const bf16_t* __restrict__ q, const int* __restrict__ tile_info, const int* __restrict__ work_order,
@@ -762,6 +762,7 @@ attn_prefill_kernel(
     const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, bf16_t* __restrict__ out,
     const int* __restrict__ token_slot, int G, unsigned group_magic, int window, float scale_log2, int nsplit,
     float* __restrict__ part_o, float* __restrict__ part_ml, DecodeExtra ex) {
+    constexpr bool PREP = QUERIES != PF_FINISHED, FOLDED = QUERIES == PF_NORMED;
     constexpr int GROUP_ELEMS = DIRECT ? PF_DIRECT_GROUP / 2 : PF_TILE_ELEMS;  // bfloat16 elements
     __shared__ __attribute__((aligned(1024))) bf16_t tiles[GROUPS * GROUP_ELEMS];
     __shared__ float fold_ml[GROUPS > 1 ? PF_WAVES * PF_NQ * 2 * RL_WAVE : 1];
@@ -839,10 +840,11 @@ attn_prefill_kernel(
         ask_norm(norm_w, g, ex);
         __builtin_amdgcn_sched_barrier(0);
     }
+    const float query_scale = FOLDED ? scale_log2 : 1.f;
     auto load_queries = [&]() {
         if constexpr (SHARED) {
             bf16x8 mine[DC];
-            prepared_query(mine, asked[0], norm_w, grp ? r_ok[1] : r_ok[0], ex, scale_log2);
+            prepared_query(mine, asked[0], norm_w, grp ? r_ok[1] : r_ok[0], ex, query_scale);
             constexpr int AT = DIRECT ? PF_DIRECT_SET / 2 : 0;  // (the padded tiles are stored behind the loop's first barrier)
             static_assert(!DIRECT || PF_WAVES * PF_NQ * DC * RL_WAVE * 16 <= PF_DIRECT_SET, "the queries fit one set of tiles");
             static_assert(DIRECT || PF_WAVES * PF_NQ * DC * RL_WAVE * 16 <= (int)sizeof(tiles), "the queries fit the tiles");
@@ -860,13 +862,13 @@ attn_prefill_kernel(
         for (int n = 0; n < PF_NQ; ++n) {
             if constexpr (PREP) {
                 if (EARLY)
-                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex, scale_log2);
+                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex, query_scale);
                 else if (!CALLED) {
                     ask_query(asked[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_pos[n], g, ex);
                     ask_norm(norm_w, g, ex);
-                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex, scale_log2);
+                    prepared_query(qf[n], asked[n], norm_w, r_ok[n], ex, query_scale);
                 } else
-                    late_query(qf[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_ok[n], r_pos[n], g, ex, scale_log2);
+                    late_query(qf[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_ok[n], r_pos[n], g, ex, query_scale);
             } else if (CALLED && D == 224) {
                 late_plain(qf[n], q + (size_t)r_tok[n] * ex.qkv_stride + (size_t)r_head[n] * D, r_ok[n], g);
             } else {
@@ -891,7 +893,7 @@ attn_prefill_kernel(
     const int wave_max_pos = start + token_of((w_last > w_first ? w_last : w_first) - row0);
 
     float m[PF_NQ], l[PF_NQ];
-    f32x4 below[PF_NQ];  // PREP: what the scores' sums begin with, -m
+    f32x4 below[PF_NQ];  // FOLDED: what the scores' sums begin with, -m
     f32x4 acc[PF_NQ][DB];
 #pragma unroll
     for (int n = 0; n < PF_NQ; ++n) {
@@ -1136,7 +1138,7 @@ attn_prefill_kernel(
             }
 #pragma unroll
             for (int n = 0; n < PF_NQ; ++n) {
-                s[n][hb] = PREP ? below[n] : (f32x4){0.f, 0.f, 0.f, 0.f};
+                s[n][hb] = FOLDED ? below[n] : (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int c = 0; c < DC; ++c) s[n][hb] = mfma(kf[c], qf[n][c], s[n][hb]);
             }
@@ -1160,7 +1162,7 @@ attn_prefill_kernel(
             for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[n][e >> 2][e & 3]);
             mx = row_max4(mx);
             const bool unset = m[n] == -INFINITY;  // the row has seen no visible key yet
-            if (!PREP) mx = mx * scale_log2 - (unset ? 0.f : m[n]);  // (the scale is positive)
+            if (!FOLDED) mx = mx * scale_log2 - (unset ? 0.f : m[n]);  // (the scale is positive)
             if (__any(mx > LAZY || (unset && mx > -INFINITY))) {
                 const float up = (unset ? mx > -INFINITY : mx > 0.f) ? mx : 0.f;
                 const float alpha = unset ? 1.f : __builtin_amdgcn_exp2f(-up);  // (an unset row's sums are 0)
@@ -1173,21 +1175,21 @@ attn_prefill_kernel(
                     acc[n][b][2] *= alpha;
                     acc[n][b][3] *= alpha;
                 }
-                if (PREP) {
+                if (FOLDED) {
 #pragma unroll
                     for (int e = 0; e < 16; ++e) s[n][e >> 2][e & 3] -= up;
                     const float now = m[n] == -INFINITY ? 0.f : -m[n];
                     below[n] = (f32x4){now, now, now, now};
                 }
             }
-            m_safe_n[n] = PREP || m[n] == -INFINITY ? 0.f : m[n];
+            m_safe_n[n] = FOLDED || m[n] == -INFINITY ? 0.f : m[n];
         }
         // ---- the weights of the first 32 keys, then of the last 32; the products follow half by
         // half, so that the first half's matrix instructions run beside the second half's
         // exponentials (8,192 tokens: 701 -> 681 us) ---------------------------------------------
         float psum[PF_NQ];
         auto weight = [&](int n, float score) {
-            return __builtin_amdgcn_exp2f(PREP ? score : fmaf(score, scale_log2, -m_safe_n[n]));
+            return __builtin_amdgcn_exp2f(FOLDED ? score : fmaf(score, scale_log2, -m_safe_n[n]));
         };
 #pragma unroll
         for (int n = 0; n < PF_NQ; ++n) {
@@ -1303,6 +1305,15 @@ attn_prefill_kernel(
     }
 }
 
+template <PrefillQueries QUERIES>
+static auto prefill_kernel(int groups, int page_size) {
+    auto kernel = groups == 2 ? attn_prefill_kernel<2, false, QUERIES> : attn_prefill_kernel<1, false, QUERIES>;
+    if constexpr (PF_DIRECT_OK) {
+        if (page_size % 8 == 0) kernel = groups == 2 ? attn_prefill_kernel<2, true, QUERIES> : attn_prefill_kernel<1, true, QUERIES>;
+    }
+    return kernel;
+}
+
 extern "C" int rl_attn_prefill_rows() { return PF_ROWS; }
 
 // groups: 1 or 2 wave groups per workgroup (a compute unit then holds 2 or 1 workgroups).
@@ -1344,13 +1355,9 @@ extern "C" int rl_attn_prefill(const void* q, const void* k_cache, const void* v
     if (G > 32768) return RL_ERR_ARG;
     const unsigned group_magic = (unsigned)(((1ull << 31) + G - 1) / G);
     dim3 grid(num_tiles * nkv * nsplit), block(groups * PF_THREADS);
-    constexpr bool PREPARES = D % 64 == 0;  // (else refused above)
-    auto kernel = prep_q ? (groups == 2 ? attn_prefill_kernel<2, false, PREPARES> : attn_prefill_kernel<1, false, PREPARES>)
-                         : (groups == 2 ? attn_prefill_kernel<2, false, false> : attn_prefill_kernel<1, false, false>);
-    if constexpr (PF_DIRECT_OK) {
-        if (page_size % 8 == 0)
-            kernel = prep_q ? (groups == 2 ? attn_prefill_kernel<2, true, PREPARES> : attn_prefill_kernel<1, true, PREPARES>)
-                            : (groups == 2 ? attn_prefill_kernel<2, true, false> : attn_prefill_kernel<1, true, false>);
+    auto kernel = prefill_kernel<PF_FINISHED>(groups, page_size);
+    if constexpr (D % 64 == 0) {  // (else refused above)
+        if (prep_q) kernel = q_norm_w ? prefill_kernel<PF_NORMED>(groups, page_size) : prefill_kernel<PF_TURNED>(groups, page_size);
     }
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const bf16_t*)q, tile_info, work_order, block_table,
                        table_stride, page_magic, page_size, nkv, (const bf16_t*)k_cache, (const bf16_t*)v_cache,

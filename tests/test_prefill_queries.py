@@ -1,0 +1,63 @@
+"""Queries that the prefill attention finishes itself, as it reads them from the packed rows."""
+
+import random
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from rapid_llm_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+SHAPES = [(1, 1), (2, 1), (1, 3), (2, 3)]  # wave groups, runs of keys
+EPS = 3e-6
+
+
+def _problem(seqs, nq, nkv, d, page, seed, change=None):
+    """Packed rows whose keys and values are in the caches already; ``change(i, keys)`` may change those of request i."""
+    gen, rng = torch.Generator().manual_seed(seed), random.Random(seed)
+    pages = [-(-(a + n) // page) for a, n in seqs]
+    ids, slots = list(range(1, sum(pages) + 1)), list(range(len(seqs) + 3))
+    rng.shuffle(ids)
+    rng.shuffle(slots)
+    table = torch.zeros(len(slots), max(pages) + 1, dtype=torch.int32)
+    kc, vc = torch.full((len(ids) + 1, nkv, page, d), float("nan")), torch.full((len(ids) + 1, nkv, d, page), float("nan"))
+    rows, requests, positions, token_slot = [], [], [], []
+    for i, (a, n) in enumerate(seqs):
+        k, v = (torch.randn(a + n, nkv, d, generator=gen) for _ in range(2))
+        if change is not None:
+            change(i, k)
+        k, v = k.bfloat16().float(), v.bfloat16().float()
+        for p in range(pages[i]):
+            pid = ids.pop()
+            table[slots[i], p] = pid
+            lo, hi = p * page, min(a + n, (p + 1) * page)
+            kc[pid, :, : hi - lo], vc[pid, :, :, : hi - lo] = k[lo:hi].transpose(0, 1), v[lo:hi].permute(1, 2, 0)
+        rows.append(torch.randn(n, (nq + 2 * nkv) * d, generator=gen).bfloat16())
+        requests.append((k, v, torch.arange(a, a + n)))
+        positions += range(a, a + n)
+        token_slot += [slots[i]] * n
+    ctx = SimpleNamespace(
+        positions=torch.tensor(positions, dtype=torch.int32, device=DEV), token_slot=torch.tensor(token_slot, dtype=torch.int32, device=DEV),
+        token_ids=torch.zeros(len(positions), dtype=torch.int32, device=DEV), h_seq_starts=[a for a, _ in seqs], h_seq_lens=[n for _, n in seqs],
+        max_position=max(positions), extra={},
+    )
+    return torch.cat(rows), requests, slots[: len(seqs)], kc.bfloat16().to(DEV), vc.bfloat16().to(DEV), table.to(DEV), ctx
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"g{s[0]}n{s[1]}")
+@pytest.mark.parametrize("nq,nkv,d,page", [(8, 2, 64, 16), (8, 2, 128, 16), (6, 3, 128, 12), (4, 2, 192, 8), (4, 4, 256, 16)])
+def test_queries_that_nothing_changes_are_not_rounded(nq, nkv, d, page, shape, monkeypatch):
+    """Without a norm, and without a rotation or with one by no angle, a query is the bfloat16 numbers of its row: bit for bit what
+    the kernel gives for queries that were written out."""
+    monkeypatch.setattr(ops, "_prefill_shape", lambda *a, **k: shape)
+    seqs = [(0, 70), (300, 37), (5, 1), (0, 2)]
+    rows, _, _, kc, vc, table, ctx = _problem(seqs, nq, nkv, d, page, d + page)
+    cos, sin = torch.ones(400, d // 2, device=DEV), torch.zeros(400, d // 2, device=DEV)
+    outs = []
+    for q, prepare in ((rows[:, : nq * d].contiguous(), None), (rows, (None, None, None, EPS)), (rows, (None, cos, sin, EPS))):
+        out = torch.full((len(rows), nq * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.paged_attention(q.to(DEV), kc, vc, out, ctx, table, page, nq, nkv, d, 0, d**-0.5, prepare=prepare)
+        outs.append(out)
+    assert bool(outs[0].isfinite().all()) and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
