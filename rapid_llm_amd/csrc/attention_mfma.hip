@@ -1356,9 +1356,10 @@ extern "C" int rl_attn_prefill(const void* q, const void* k_cache, const void* v
     const unsigned group_magic = (unsigned)(((1ull << 31) + G - 1) / G);
     dim3 grid(num_tiles * nkv * nsplit), block(groups * PF_THREADS);
     auto kernel = prefill_kernel<PF_FINISHED>(groups, page_size);
-    if constexpr (D % 64 == 0) {  // (else refused above)
-        if (prep_q) kernel = q_norm_w ? prefill_kernel<PF_NORMED>(groups, page_size) : prefill_kernel<PF_TURNED>(groups, page_size);
-    }
+    constexpr bool PREPARES = D % 64 == 0;  // (else refused above)
+    if (prep_q)
+        kernel = q_norm_w ? prefill_kernel<PREPARES ? PF_NORMED : PF_FINISHED>(groups, page_size)
+                          : prefill_kernel<PREPARES ? PF_TURNED : PF_FINISHED>(groups, page_size);
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const bf16_t*)q, tile_info, work_order, block_table,
                        table_stride, page_magic, page_size, nkv, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
                        (bf16_t*)out, token_slot, G, group_magic, window, scale_log2, nsplit, part_o, part_ml, ex);
