@@ -1243,7 +1243,6 @@ attn_prefill_kernel(
             }
             const float tm = m[0], tl = l[0];
             m[0] = m[1], l[0] = l[1], m[1] = tm, l[1] = tl;
-            r_tok[0] = r_tok[1], r_head[0] = r_head[1], r_ok[0] = r_ok[1];
         }
         __syncthreads();  // every wave has read its last tile
         {
@@ -1271,13 +1270,18 @@ attn_prefill_kernel(
             for (int i = 0; i < 4; ++i)
                 acc[0][b][i] = acc[0][b][i] * a0 + fold_acc[(from * PER_LANE + b * 4 + i) * RL_WAVE + lane] * a1;
     }
+    int late_col = col;
+    asm volatile("" : "+v"(late_col));
 #pragma unroll
     for (int n = 0; n < (GROUPS > 1 ? 1 : PF_NQ); ++n) {
         const float lt = row_sum4(l[n]);
         const float inv = lt > 0.f ? 1.f / lt : 0.f;
-        if (!r_ok[n]) continue;
+        // (the row's place once more: kept through the loop it would take registers that large heads do not have)
+        const int row = (wave * PF_NQ + (GROUPS > 1 ? grp : n)) * 16 + late_col;
+        if (row0 + row >= rows) continue;
+        const int tok = token_of(row), row_at = (tok0 + tok) * nq + hk * G + row0 + row - tok * G;
         if (nsplit > 1) {
-            const size_t slot = ((size_t)r_tok[n] * nq + r_head[n]) * nsplit + split;
+            const size_t slot = (size_t)row_at * nsplit + split;
             if (lt > 0.f) {
                 float* prow = part_o + slot * D;
 #pragma unroll
@@ -1292,7 +1296,7 @@ attn_prefill_kernel(
             }
             continue;
         }
-        bf16_t* orow = out + ((size_t)r_tok[n] * nq + r_head[n]) * D;
+        bf16_t* orow = out + (size_t)row_at * D;
 #pragma unroll
         for (int b = 0; b < DB; ++b) {
             struct {
