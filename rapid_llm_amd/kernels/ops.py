@@ -2434,8 +2434,16 @@ _PREFILL_STEP_KEYS = 64  # keys per step of the prefill kernel
 _PREFILL_ONE, _PREFILL_ONE_STEP, _PREFILL_BESIDE, _PREFILL_BESIDE_STEP = 7.6, 1.63, 4.4, 0.3
 _PREFILL_FULL, _PREFILL_FULL_ITEM, _PREFILL_FULL_STEP = 4.0, 5.2, 0.99
 _PREFILL_TWO, _PREFILL_TWO_STEP, _PREFILL_TWO_ITEM = 8.4, 1.27, 7.2
+# Two wave groups have half the registers each: beyond 160 channels their state lies in scratch.  A workgroup of one / of two, one
+# prompt of 2,048 tokens of 32 query heads / sixteen of 197 of 24: 160 channels 116 / 99, 34.1 / 43.0; 176 125 / 126, 35.7 / 50.5; 192
+# 136 / 167, 49.5 / 68.1; 224 159 / 293, 45.2 / 109; 256 190 / 458, 66.5 / 173.
+_PREFILL_TWO_LARGE = 0.016  # of it all, for each channel more
 # what cutting the keys into runs costs: the runs' partial results are written, and read and folded by a second kernel
 _PREFILL_MERGE, _PREFILL_MERGE_BYTE = 2.0, 0.5e-6
+# what a last round of runs that leaves slots without one costs, of what it would if nothing of it fitted beside the one before
+# (110 launches of 260 to 510 workgroups without runs, heads of 64 to 256: whole / two runs, 64 channels 43.9 / 51.4, 80 210 / 241, 128
+# 106 / 124, 192 169 / 202; but 112 channels 144 / 105, 128 312 / 191)
+_PREFILL_LAST_ROUND = 0.4
 
 
 def _prefill_shape(plan: "AttentionPlan", nkv: int, window: int, tile_rows: int,
@@ -2463,16 +2471,20 @@ def _prefill_shape(plan: "AttentionPlan", nkv: int, window: int, tile_rows: int,
 
     def one(runs: int) -> float:
         start, step = _PREFILL_ONE, _PREFILL_ONE_STEP
-        if items * runs > units:
-            start, step = start + _PREFILL_BESIDE, step + _PREFILL_BESIDE_STEP * even
-        return max(start + step * -(-longest // runs),
-                   _PREFILL_FULL + _PREFILL_FULL_ITEM * items * runs / units + _PREFILL_FULL_STEP * share)
+        if items * runs <= units:
+            return start + step * -(-longest // runs)
+        start, step = start + _PREFILL_BESIDE, step + _PREFILL_BESIDE_STEP * even
+        full = _PREFILL_FULL + _PREFILL_FULL_ITEM * items * runs / units + _PREFILL_FULL_STEP * share
+        if runs > 1 and items * runs > slots:  # runs are of one length: a last round that is not full
+            full *= 1.0 + _PREFILL_LAST_ROUND * (-(-items * runs // slots) * slots / (items * runs) - 1.0)
+        return max(start + step * -(-longest // runs), full)
 
     best = (one(1), 1, 1)
     two = _PREFILL_TWO + min(0.4 * (d / 128 - 1), 0.0) + _PREFILL_TWO_STEP * longest
     if items > units:
         rounds = -(-items // units)  # (workgroups of one length end together, and a round that is not full takes as long)
         two = max(two, 2.0 + _PREFILL_TWO_ITEM * rounds + _PREFILL_TWO_STEP * share * (1.0 + even * (rounds * units / items - 1.0)))
+    two *= 1.0 + _PREFILL_TWO_LARGE * max(d - 160, 0)
     if two < best[0]:
         best = (two, 2, 1)
     merged = _PREFILL_MERGE_BYTE * items * tile_rows * d * 4 / (0.55 + 0.45 * d / 128)  # (a step of 16 channels takes 0.6 of one of 128)

@@ -157,6 +157,35 @@ def test_prefill_launch_shapes_follow_an_estimate_of_the_launch():
     assert shape([(16000, 150)], window=256) == (2, 1)
 
 
+@pytest.mark.parametrize("d,groups", [(64, 2), (128, 2), (160, 2), (192, 1), (224, 1), (256, 1)])
+def test_prefill_launch_shapes_of_large_heads(d, groups):
+    """Two wave groups of large heads keep their state in scratch: one prompt goes to one wave group a tile."""
+    from types import SimpleNamespace
+
+    from rapid_llm_amd.kernels import ops
+
+    for n, nkv, group in ((2048, 8, 4), (1024, 8, 4), (300, 8, 4), (600, 16, 1)):
+        keys = [min(n, (row0 + 128) // group) for row0 in range(0, n * group, 128)]
+        assert ops._prefill_shape(SimpleNamespace(tile_keys=keys, num_tiles=len(keys)), nkv, 0, 128, 256, d=d) == (groups, 1)
+
+
+def test_prefill_launch_shapes_of_short_tiles_and_of_last_rounds():
+    """As many tiles of one step as there are units: one wave group each.  Tiles for one round and a part of the next are
+    not cut into runs that leave most of a last round without work."""
+    from types import SimpleNamespace
+
+    from rapid_llm_amd.kernels import ops
+
+    def shape(seqs, nkv, group, d):
+        keys = [start + min(n, (row0 + 128) // group) for start, n in seqs for row0 in range(0, n * group, 128)]
+        return ops._prefill_shape(SimpleNamespace(tile_keys=keys, num_tiles=len(keys)), nkv, 0, 128, 256, d=d)
+
+    assert shape([(0, 8)] * 16, 16, 4, 160) == (1, 1) and shape([(0, 13)] * 16, 16, 1, 128) == (1, 1)
+    lengths = (730, 604, 791, 988, 1082, 706, 766, 912)
+    assert shape([(6019, n) for n in lengths], 8, 1, 80) == (1, 1)
+    assert shape([(0, 10752)], 4, 1, 128) == (1, 2)  # (the longest tiles are many times the others)
+
+
 def test_which_products_run_in_one_launch_of_this_package():
     """The host's rule for the tile product (17 to 512 rows over a matrix of a few megabytes with
     enough result columns for every compute unit): the smallest model's QKV and gate/up products
