@@ -2375,9 +2375,10 @@ class AttentionPlan:
 
     def prefill_shape(self, nkv: int, window: int, lib) -> tuple[int, int]:
         """:func:`_prefill_shape` of the step, worked out once for all its layers of a kind."""
-        shape = self.shapes.get((nkv, window))
+        d = lib.rl_attn_head_dim()
+        shape = self.shapes.get((nkv, window, d))
         if shape is None:
-            shape = self.shapes[(nkv, window)] = _prefill_shape(self, nkv, window, tile_rows_of(lib), d=lib.rl_attn_head_dim())
+            shape = self.shapes[(nkv, window, d)] = _prefill_shape(self, nkv, window, tile_rows_of(lib), d=d)
         return shape
 
     def work_order(self, nkv: int, device, resident: int = 1) -> torch.Tensor | None:
