@@ -111,7 +111,8 @@ class SwiGLU(FeedForward):
                    else ops.gemm_bf16_swiglu(x, w, **glu))
             if act is not None:
                 return self.down.deferred(act, ctx)
-        if w.dtype == torch.float32 and x.dtype == torch.float32 and self.activation == "silu" and not self.limit and not self.has_bias:
+        if (w.dtype == torch.float32 and x.dtype == torch.float32 and self.activation == "silu" and not self.limit
+                and not self.has_bias and self.gate_up.bias is None and plain_products(self.gate_up, self.gate_up)):
             act = ops.gemm_f32_swiglu(x, w)
             if act is not None:
                 return self.down.deferred(act, ctx)

@@ -500,3 +500,42 @@ def test_tiles_a_workgroup_of_the_product_for_tens_of_rows():
     assert plan(33, 12288, 4096, True) == (3, 256) and ops.rows_plan(33, 12288, 4096, True, units=304) == (3, 304)
     assert plan(16, 12288, 4096, True) is None and plan(65, 12288, 4096, True) is None
     assert plan(33, 12296, 4096, True) is None and plan(33, 12288, 4160, True) is None
+
+
+@pytest.mark.parametrize("change", ["none", "derived", "replaced", "biased"])
+def test_a_float32_feed_forward_asks_its_gate_and_up_product(change, monkeypatch):
+    """Product and activation are one launch only where the product is nothing but its weight: a derived product, one with
+    a call of its own and one with a bias are asked."""
+    from rapid_llm_amd.kernels import ops
+    from rapid_llm_amd.parts.mlp import SwiGLU
+
+    ff = SwiGLU(4, 6, "mlp.")
+    ff.down.deferred = lambda act, ctx: act
+    gate_up, called = torch.randn(12, 4), []
+
+    class Doubled(Linear):
+        def product(self, x, out_dtype=None):
+            called.append("derived")
+            return 2 * (x @ self.weight.T)
+
+    if change == "derived":
+        ff.gate_up = Doubled(4, 12)
+    ff.gate_up.bind(gate_up, torch.ones(12) if change == "biased" else None)
+    if change == "replaced":
+        ff.gate_up.product = lambda x, out_dtype=None: called.append("replaced") or 2 * (x @ gate_up.T)
+
+    def swiglu(gu, act, *args, **kwargs):
+        act.copy_(torch.nn.functional.silu(gu[:, :6]) * gu[:, 6:])
+
+    monkeypatch.setattr(ops, "swiglu", swiglu)
+    monkeypatch.setattr(ops, "gemm_f32", lambda x, w, out: out.copy_(x @ w.T))
+    monkeypatch.setattr(ops, "add_bias", lambda y, bias: y.add_(bias))
+    monkeypatch.setattr(ops, "gemm_f32_swiglu", lambda x, w: called.append("one launch") or torch.zeros(x.shape[0], 6))
+    x = torch.randn(3, 4)
+    got = ff.forward(x, None)
+    if change == "none":
+        assert called == ["one launch"]
+        return
+    gu = x @ gate_up.T + 1.0 if change == "biased" else 2 * (x @ gate_up.T)
+    assert called == ([] if change == "biased" else [change])
+    torch.testing.assert_close(got, torch.nn.functional.silu(gu[:, :6]) * gu[:, 6:])
