@@ -787,8 +787,10 @@ attn_prefill_kernel(
     const int rows = qlen * G;
     const int seq_end = start + qlen;  // keys at or beyond this were never written
     const int* table = block_table + (size_t)(slot >= 0 ? slot : token_slot[tok0]) * table_stride;
-    // the portion's token that row row0 + i belongs to (group_magic = ceil(2^31 / G) divides by G: exact below 2^31 / G)
-    auto token_of = [&](int i) { return row_tok + (int)__umulhi(2u * (unsigned)(row_head + i), group_magic); };
+    // the portion's token that row row0 + i belongs to: (row_head + i) / G by a product with group_magic = ceil(2^(31 + s) / G),
+    // s = floor(log2 G), exact below 2^30
+    const int group_shift = 31 - __builtin_clz(G);
+    auto token_of = [&](int i) { return row_tok + (int)(__umulhi(2u * (unsigned)(row_head + i), group_magic) >> group_shift); };
 
     const int grp = GROUPS > 1 ? threadIdx.x / PF_THREADS : 0;  // wave group: which steps
     const int tid = threadIdx.x - grp * PF_THREADS;             // thread within the group
@@ -1354,10 +1356,8 @@ extern "C" int rl_attn_prefill(const void* q, const void* k_cache, const void* v
     if ((long)num_tiles * nkv * nsplit > 0x7fffffffL) return RL_ERR_ARG;
     // the kernel's addresses are page id x elements of a page (32 bits) + an offset in the page
     if ((long)nkv * page_size * D > 0x7fffffffL) return RL_ERR_ARG;
-    // a row of a tile, and what is left of its first, divided by the group's heads: exact where (G + PF_ROWS) G < 2^31
     const int G = nq / nkv;
-    if (G > 32768) return RL_ERR_ARG;
-    const unsigned group_magic = (unsigned)(((1ull << 31) + G - 1) / G);
+    const unsigned group_magic = (unsigned)(((1ull << (62 - __builtin_clz(G))) + G - 1) / G);
     dim3 grid(num_tiles * nkv * nsplit), block(groups * PF_THREADS);
     auto kernel = prefill_kernel<PF_FINISHED>(groups, page_size);
     constexpr bool PREPARES = D % 64 == 0;  // (else refused above)

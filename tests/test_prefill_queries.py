@@ -61,3 +61,22 @@ def test_queries_that_nothing_changes_are_not_rounded(nq, nkv, d, page, shape, m
         ops.paged_attention(q.to(DEV), kc, vc, out, ctx, table, page, nq, nkv, d, 0, d**-0.5, prepare=prepare)
         outs.append(out)
     assert bool(outs[0].isfinite().all()) and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("group", [32769, 46347])
+def test_as_many_query_heads_as_there_may_be_on_a_kv_head(group):
+    """Rows of a portion are divided by the group's heads: more heads than the square root of what a 32-bit product reaches."""
+    d, page, seqs = 16, 16, [(0, 2), (5, 3)]
+    _, requests, _, kc, vc, table, ctx = _problem(seqs, 1, 1, d, page, 3)
+    gen = torch.Generator().manual_seed(group)
+    q = torch.randn(5, group, d, generator=gen).bfloat16().to(DEV)
+    out = torch.full((5, group * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention(q.view(5, -1), kc, vc, out, ctx, table, page, group, 1, d, 0, d**-0.5)
+    at = 0
+    for k, v, positions in requests:
+        for pos in positions.tolist():
+            k1, v1 = k[: pos + 1, 0].to(DEV).double(), v[: pos + 1, 0].to(DEV).double()
+            want = torch.softmax(q[at].double() @ k1.T.contiguous() * d**-0.5, dim=1) @ v1
+            # weights and results are rounded to bfloat16, 2^-9 each, and the weights' sum is not of the rounded ones
+            assert bool(((out[at].view(group, d).double() - want).abs() <= 2.0**-7 * v1.abs().amax()).all())
+            at += 1
