@@ -1929,7 +1929,9 @@ def own_products():
 @contextlib.contextmanager
 def shared_tiles():
     """Inside the block, on this thread: products go to the one whose waves share a tile over halves of K wherever
-    :func:`pair_plan` has a plan.  A model's step is such a block; a product by itself keeps to what the plans beside it say."""
+    :func:`pair_plan` has a plan.  A model's step is such a block.  A product by itself keeps what its callers count on and
+    that one does not give: :func:`gemm_bf16_parts` leaves as many runs as :func:`mid_runs` or :func:`block_plan` say, operands
+    that begin inside a unit of 16 bytes have the bits of others, and :func:`library_takes` names the library's products."""
     before, _step.shared_tiles = _step.shared_tiles, True
     try:
         yield

@@ -80,6 +80,63 @@ def test_kernel(m, n, k, tile):
         assert bool(((out[:m].double() - act).abs() <= slack).all())
 
 
+# A kind's smallest and largest rows of a plan, and sizes in between.
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,m,n,k", [("plain", 65, 6144, 2560), ("plain", 200, 4096, 2048), ("plain", 1023, 1024, 1024), ("gated", 17, 3072, 1024),
+                                        ("gated", 129, 3072, 1024), ("runs", 18, 2560, 9728), ("runs", 100, 2560, 4096), ("runs", 500, 1024, 3072)])
+def test_a_layers_products_go_there_with_operands_of_any_place(kind, m, n, k, monkeypatch):
+    """Through the entry points that the layers call: rows side by side in whole units of 16 bytes go there, rows that are columns
+    of wider ones as a copy (runs: elsewhere), operands that begin inside a unit elsewhere.  All of them give the product."""
+    from rapid_llm_amd.parts.linear import Linear
+
+    went, launch = [], ops._pair
+    monkeypatch.setattr(ops, "_pair", lambda *args: went.append(args[3]) or launch(*args))
+    gen = torch.Generator().manual_seed(m + n)
+    rows = 2 * n if kind == "gated" else n
+    room_x, room_w = torch.randn(m * k + 8, generator=gen).to(torch.bfloat16).cuda(), (torch.randn(rows * k + 8, generator=gen) * k**-0.5).to(torch.bfloat16).cuda()
+
+    def operands(x_at, w_at, apart):
+        x, w = room_x[x_at : x_at + m * k].view(m, k), room_w[w_at : w_at + rows * k].view(rows, k)
+        if apart:
+            wider = torch.full((m, k + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+            wider[:, :k] = x
+            x = wider[:, :k]
+        return x, w
+
+    for x_at, w_at, apart in ((0, 0, False), (8, 8, False), (1, 0, False), (0, 3, False), (0, 0, True)):
+        if apart and (kind == "gated" or kind == "runs" and m <= ops.mid_max_rows(n, k)):
+            continue  # (refused, as they were: a layer's rows are side by side)
+        x, w = operands(x_at, w_at, apart)
+        linear = Linear(k, rows)
+        linear.bind(w)
+        went.clear()
+        with ops.shared_tiles():
+            there = x_at % 8 == 0 and w_at % 8 == 0 and not (apart and kind == "runs")
+            if kind == "gated":
+                got = ops.gemm_bf16_swiglu(x, w)
+                if got is None:
+                    got = ops.gemm_bf16(x, w, torch.bfloat16)
+                    gate, up = got[:, :n].double(), got[:, n:].double()
+                    got = torch.nn.functional.silu(gate) * up
+            elif kind == "runs":
+                assert ops.pair_reads(x, w) == there
+                got = linear.partial_sums(x).double().sum(0) if linear.midsize(x) else linear(x)
+            else:
+                got = linear(x)
+        assert went == ([kind] if there else [])
+        want = x.double() @ w.double().t().contiguous()
+        # float32 sums in an order of their own, as above; rounded to bfloat16 where they are stored as that
+        off = 8 * k**0.5 * 2.0**-24 * float(want.abs().max())
+        if kind == "gated":
+            both = want.to(torch.bfloat16).double()
+            gate, up = both[:, :n], both[:, n:]
+            want = torch.nn.functional.silu(gate) * up
+            bound = 1.1 * up.abs() * (gate.abs() / 256 + off) + torch.nn.functional.silu(gate).abs() * (up.abs() / 256 + off) + want.abs() / 256
+        else:
+            bound = want.abs() / 256 + off
+        assert bool(((got.double() - want).abs() <= bound).all()), (x_at, w_at, apart)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tile", [(2, 2), (2, 4), (4, 2)])
 def test_every_gate_has_the_activation_of_the_many_row_product(tile):
