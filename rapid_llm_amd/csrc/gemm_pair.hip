@@ -273,7 +273,7 @@ static int launch_pair(const PairArgs& a, int kind, hipStream_t stream) {
         hipLaunchKernelGGL((gemm_pair_kernel<TW, TX, PAIR_PLAIN>), grid, block, 0, stream, a);
     else if (kind == PAIR_RUNS)
         hipLaunchKernelGGL((gemm_pair_kernel<TW, TX, PAIR_RUNS>), grid, block, 0, stream, a);
-    else if constexpr (TW % 2 == 0)
+    else if constexpr (TW % 2 == 0 && TW * TX < 16)  // (gated tiles of 128 x 128 are slower than the many-row product's)
         hipLaunchKernelGGL((gemm_pair_kernel<TW, TX, PAIR_GLU>), grid, block, 0, stream, a);
     else
         return RL_ERR_ARG;
@@ -282,7 +282,7 @@ static int launch_pair(const PairArgs& a, int kind, hipStream_t stream) {
 
 // kind 1: out float32 [splits, M, N], run r of K's chunks in part r.  Kind 2: W = [gate | up] stacked, [2N, K], out
 // bfloat16 [M, N] = silu(gate) * up of the products rounded to bfloat16.  Kind 3: out bfloat16 [M, N].
-// tw, tx: a tile is 32 tw weight rows x 32 tx rows of X.  K a multiple of 64, N of 8.
+// tw, tx: a tile is 32 tw weight rows x 32 tx rows of X (kind 2: (2, 2), (2, 4) or (4, 2)).  K a multiple of 64, N of 8.
 extern "C" int rl_gemm_pair(const void* X, const void* W, void* out, int M, int N, int K, int ldx, int ldw, int ldo,
                             int kind, int tw, int tx, int splits, hipStream_t stream) {
     if (M <= 0 || N <= 0) return RL_OK;
