@@ -2040,6 +2040,14 @@ def pair_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int, 
     12,288 at 66 rows 29.8 / 29.8), below 300 rows on (2,048 x 6,144 at 256 / 512 rows 21.7 / 20.5, 28.5 / 29.0).
     ``"gated"``: 3,072 x 1,024 9.3 / 7.9, 12.6 / 10.1, 12.8 / 10.3, 13.6 / 10.9; 6,144 x 2,048 up to 128 rows 22.6 / 17.2, 24.3 / 19.2; tiles of
     128 x 128 are slower than the many-row product's (9,728 x 2,560 at 66 rows 32.2 / 34.1).
+    Of 520 sizes drawn, 16 to 1,024 rows of 350 to 16,000 columns and k, what the lines for other matrices than those leave out: ``"gated"``
+    beyond 2,048 k tiles for less than a quarter of the units, which the library's kernels or the many-row product share better (512 x
+    2,560 at 87 rows, 32 tiles, 10.4 / 11.3; 64 tiles 19.0 / 15.5), beyond 4,096 for less than five eighths (35 sizes 0.68 to 1.42 of the
+    other's time, the library's kernels fitting or not: 768 x 4,352 at 120 rows 16.8 / 22.7, 664 x 16,128 at 618 67.3 / 95.8; with
+    more 13 sizes 0.66 to 1.07); ``"runs"`` of short sums over wide matrices, whose float32 results are most of the bytes (10,328 x 320 at
+    359 rows 18.0 / 23.2, 14,648 x 576 at 180 17.6 / 20.9, 2,560 x 512 at 332 8.9 / 10.1, 3,800 x 768 at 459 15.3 / 16.0, 14,336 x 768 at 225
+    20.9 / 24.1, 15,360 x 1,408 at 160 26.0 / 27.9; but 3,840 x 768 at 306 14.0 / 13.4, 9,728 x 768 at 128 16.7 / 16.1, 13,056 x 1,536 at 129
+    28.4 / 26.5).  What is left is 0.4 to 1.07 of the other's time.
     At 17 / 40 / 64 rows, tiles of 64 x 64 against the kernel that keeps X in registers: ``"gated"`` up to 2,048 k, where one round holds
     them, 3,072 x 1,024 7.7 / 7.7, 8.9 / 8.0, 10.2 / 8.5, 6,144 x 2,048 15.3 / 13.6, 16.7 / 14.2, 19.7 / 15.3 (9,728 x 2,560, which takes larger
     tiles, 23.8 / 26.6, 28.4 / 28.9); against the mid-size product, with the norm, ``"runs"`` beyond 6,144 k 2,560 x 9,728 17.1 / 15.7, 17.6 / 16.9,
@@ -2082,6 +2090,10 @@ def pair_plan(m: int, n: int, k: int, kind: str, units: int) -> tuple[int, int, 
     if best is None:
         return None
     if kind == "plain" and 8 * best[2] < (4 if n >= 4096 else 5) * units:
+        return None
+    if kind == "gated" and k > 2048 and 8 * best[2] < (2 if k <= 4096 else 5) * units:
+        return None
+    if kind == "runs" and n >= 2048 and (k < 768 or (k <= 1024 and m > 256) or (n >= 10240 and m > 128)):
         return None
     if kind != "gated" and m > 256 and size >= _SMALL_WEIGHTS and (16 * best[2] < 13 * units or k % 1024):
         return None

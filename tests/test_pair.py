@@ -28,6 +28,15 @@ def test_plans_are_what_the_kernel_takes(kind):
     assert ops.pair_plan(200, 4092, 2048, kind, 256) is None and ops.pair_plan(200, 4096, 2080, kind, 256) is None
 
 
+@pytest.mark.parametrize("kind,m,n,k,there", [
+    ("gated", 87, 512, 2560, False), ("gated", 113, 1024, 2560, True), ("gated", 120, 768, 4352, False), ("gated", 708, 1224, 4608, True),
+    ("gated", 618, 664, 16128, False), ("gated", 74, 1024, 4608, False), ("runs", 359, 10328, 320, False), ("runs", 332, 2560, 512, False), ("runs", 265, 1624, 512, True),
+    ("runs", 459, 3800, 768, False), ("runs", 128, 9728, 768, True), ("runs", 225, 14336, 768, False), ("runs", 87, 11624, 1920, True)])
+def test_sizes_that_other_products_are_faster_at(kind, m, n, k, there):
+    """Widths of no one model: few tiles over long sums, and results of short sums that are most of the bytes."""
+    assert (ops.pair_plan(m, n, k, kind, 256) is not None) == there
+
+
 def test_only_steps_of_a_model_go_there():
     assert ops.pair(200, 6144, 4096, "plain") is None and ops.library_takes(200, 6144, 4096)
     with ops.shared_tiles():
