@@ -616,7 +616,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(
 // wave waits for another.  A wave's rows go from memory straight into its own part of LDS, eight lanes a row (asked for into
 // registers as the instruction takes them, lane by lane from another row, a unit gets 16 bytes a cycle: 6,144 x 4,096 at 225 rows
 // 87 us, so 77), and from there to its registers, where they are split; a place is asked for again as soon as it has been
-// read, one or two chunks ahead.
+// read, one chunk ahead or two.
 // What bounds it: splitting and multiplying, 208 (NT + MT) and 96 NT MT cycles a wave and chunk, which take about as long as
 // one after the other (at 225 rows of 6,144 x 4,096 the splits alone 38 us, the loads alone 43, all 77), so the tiles
 // are as large as the rows and the number of units allow.  The next split between the products 77 -> 74, the first four waves
@@ -645,14 +645,17 @@ __global__ __launch_bounds__(FRUNS* RL_WAVE) void gemm_f32_runs_kernel(
     int ldc, int tiles_m, int tiles_n) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass does not know the LDS loads)
     constexpr int T = NT + MT, SLOT = 2048, CHUNK = T * SLOT;  // a place: sixteen rows' chunk
-    // One chunk ahead, and 64 to 80 KB of LDS, so that a unit holds two workgroups of small tiles; two where a chunk is so small that it
-    // does not cover memory's answer.  (Three as far as they fit / this, us: 8 rows of 4,096 x 12,288 43.0 / 39.5, 6,144 x 4,096 22.9 / 21.4;
-    // 225 of 1,024 x 3,072 19.5 / 17.9, of 1,536 x 512 10.8 / 7.9; one everywhere: 8 rows of 4,096 x 4,096 14.8 / 16.3.)
-    constexpr int D = NT == 1 && MT <= 2 ? 2 : 1;
+    // One chunk ahead, so that a unit holds two workgroups of tiles of up to eight blocks and five places, 64 to 80 KB each ((4, 2)
+    // and (6, 1) take 96 and 112 KB, more blocks 128 and more for the sums alone); two for the smallest tile, whose chunk does not
+    // cover memory's answer.  (Three as far as they fit / this, us: 8 rows of 4,096 x 12,288 43.0 / 39.5, 6,144 x 4,096 22.9 / 21.4; 225 of
+    // 1,024 x 3,072 19.5 / 17.9, of 1,536 x 512 10.8 / 7.9; one for the smallest too: 8 rows of 4,096 x 4,096 14.8 / 16.3; two at (1, 2), 96 KB: 17 / 32 rows
+    // of 4,096 x 1,024 7.0 / 6.4, 8.3 / 7.7, of 4,096 x 4,096 20.1 / 19.5, 22.5 / 21.4.)
+    constexpr int D = NT == 1 && MT == 1 ? 2 : 1;
     constexpr int GA = MT % 2 ? 1 : 2, GW = NT % 2 ? 1 : 2;  // places read together
     constexpr int BLOCKS = NT * MT, ROUNDS = (BLOCKS + FRUNS - 1) / FRUNS;
     static_assert(FRUNS * D * CHUNK <= RUNS_LDS && 2 * D * T <= 64, "the chunks fit, and the counter");
     constexpr int SUMS = (ROUNDS > 1 ? 2 : 1) * FRUNS * FRUNS * RL_WAVE * 16, BYTES = FRUNS * D * CHUNK > SUMS ? FRUNS * D * CHUNK : SUMS;
+    static_assert(BLOCKS > FRUNS || T > 5 || 2 * BYTES <= RUNS_LDS, "two workgroups a unit");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[BYTES];
 
     const int lane = threadIdx.x & (RL_WAVE - 1);
