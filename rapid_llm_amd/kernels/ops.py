@@ -2387,9 +2387,8 @@ class AttentionPlan:
         # a step is recorded for the part that has most to gain; where this one has few workgroups it has nothing
         return self._ragged and 4 * self.num_decode * each >= chip().units
 
-    def prefill_shape(self, nkv: int, window: int, lib) -> tuple[int, int]:
-        """:func:`_prefill_shape` of the step, worked out once for all its layers of a kind."""
-        d = lib.rl_attn_head_dim()
+    def prefill_shape(self, nkv: int, window: int, lib, d: int) -> tuple[int, int]:
+        """:func:`_prefill_shape` of the step, worked out once for all its layers of a kind (``lib``: of heads of ``d``)."""
         shape = self.shapes.get((nkv, window, d))
         if shape is None:
             shape = self.shapes[(nkv, window, d)] = _prefill_shape(self, nkv, window, tile_rows_of(lib), d=d)
@@ -2861,7 +2860,7 @@ def paged_attention(
     group = nq // nkv
     plan = attention_plan(ctx, group, d)
     if plan.num_tiles:
-        groups, nsplit = plan.prefill_shape(nkv, window, lib)
+        groups, nsplit = plan.prefill_shape(nkv, window, lib, d)
         part_o = part_ml = tokens_list = None
         if nsplit > 1:
             part_o = torch.empty((tokens, nq, nsplit, d), dtype=torch.float32, device=q.device)

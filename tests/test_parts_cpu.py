@@ -192,14 +192,12 @@ def test_layers_of_unlike_heads_have_launch_shapes_of_their_own():
 
     from rapid_llm_amd.kernels import ops
 
-    def library(d):
-        return SimpleNamespace(rl_attn_head_dim=lambda: d, rl_attn_prefill_rows=lambda: 128)
-
+    lib = SimpleNamespace(rl_attn_prefill_rows=lambda: 128)
     for first, second in ((64, 256), (256, 64)):
         plan = ops.AttentionPlan.__new__(ops.AttentionPlan)
         plan.shapes, plan.tile_keys, plan.num_tiles = {}, [min(2048, row0 // 4 + 32) for row0 in range(0, 8192, 128)], 64
         for d in (first, second, first):
-            assert plan.prefill_shape(8, 0, library(d)) == ops._prefill_shape(plan, 8, 0, 128, d=d) == ((2, 1) if d == 64 else (1, 1))
+            assert plan.prefill_shape(8, 0, lib, d) == ops._prefill_shape(plan, 8, 0, 128, d=d) == ((2, 1) if d == 64 else (1, 1))
 
 
 def test_which_products_run_in_one_launch_of_this_package():
