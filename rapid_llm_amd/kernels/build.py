@@ -86,8 +86,9 @@ _HIPCC_FLAGS = (
     "-Xclang",
     "-packed-fp32-ops",
     # A kernel's first arguments come in scalar registers with the launch, without a trip to memory before anything else:
-    # steps of short kernels take 0.8 to 1.3% less (8B, 8 and 64 requests decoding 3,726 -> 3,695 and 6,794 -> 6,719 us;
-    # 0.6B, 256 requests 5,039 -> 4,999; 8B float32, 8 requests 7,442 -> 7,367).
+    # steps of short kernels take 0.6 to 2.4% less (without / with, microseconds, two runs of each side in turn: 8B, one, 8 and 64
+    # requests decoding 3,477 / 3,433, 3,729 / 3,699 and 6,687 / 6,641; 0.6B, 256 requests 4,933 / 4,899; float32, 8B, 8
+    # requests 6,976 / 6,895, 0.6B, prompts of 225 tokens 2,912 / 2,844).
     "-mllvm",
     "-amdgpu-kernarg-preload-count=16",
 )
